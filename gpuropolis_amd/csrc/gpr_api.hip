@@ -561,6 +561,14 @@ static hipError_t launch_buckets(gpr_ctx *c, const GprMHArgs &a) {
     return e;
 }
 
+// Reference semantics, lane schedule: every chain in one launch, four points per lane where
+// a dataset has more than one chunk of 64.
+static hipError_t launch_ref_lane(gpr_ctx *c, const GprMHArgs &a) {
+    int nmax = 0;
+    for (const GprDataset &g : c->hds) nmax = std::max(nmax, g.n);
+    return gpr_launch_mh_ref_lane(a, nmax <= 64 ? 1 : 4, c->stream);
+}
+
 // One MCMC block on the context stream.  on_device: step and block come from the
 // device clock, which a final kernel advances (the form captured into graphs); else
 // from the host counters, advanced here.
@@ -575,7 +583,7 @@ static int launch_block(gpr_ctx *c, int steps, int32_t block_seed, bool on_devic
     if (c->cfg.rng == GPR_RNG_LCG && sched != GPR_SCHED_LANE)
         return fail(GPR_E_ARG, "the LCG stream is sequential per chain: it needs the lane schedule");
     if (sched == GPR_SCHED_LANE) {
-        if (ref) HIP_TRY(gpr_launch_mh_ref_lane(a, c->stream));
+        if (ref) HIP_TRY(launch_ref_lane(c, a));
         else {
             if (c->cfg.proposal == GPR_PROP_MALA)
                 return fail(GPR_E_UNSUPPORTED, "MALA runs on the wave schedule only");
@@ -895,7 +903,7 @@ extern "C" int gpr_autotune(gpr_ctx *c, int steps, gpr_tune *out, int max_out, i
         TUNE_TRY(copy_all(false));
         TUNE_TRY(hipEventRecord(c->ev0, c->stream));
         if (c->cfg.semantics == GPR_SEM_REFERENCE) {
-            TUNE_TRY(gpr_launch_mh_ref_lane(a, c->stream));
+            TUNE_TRY(launch_ref_lane(c, a));
         } else {
             int capmax = 1;
             for (const GprDataset &g : c->hds) capmax = std::max(capmax, g.cap);

@@ -61,7 +61,7 @@ struct GprMHArgs {
     double *ll;             // [N]
     int nchains;            // N, the stride
     const float *dx, *dy, *dw;
-    const float *dsd;       // sd per point (reference lane kernel)
+    const float *dsd;       // sd per point (reference lane schedule)
     const double *lnc;      // 0.5*(logf(2 pi) + 2 logf(sd)) per point, host libm (main.cu:300)
     const GprDataset *ds;
     const GprMetric *metric;  // [ndatasets] or null (identity metric everywhere)
@@ -139,7 +139,7 @@ struct GprResampleArgs {
 hipError_t gpr_launch_mh_config_wave(const GprMHArgs &a, int kc, bool hi, bool mala, bool small, int grid,
                                      hipStream_t s);
 hipError_t gpr_launch_mh_config_lane(const GprMHArgs &a, int cap_max, hipStream_t s);
-hipError_t gpr_launch_mh_ref_lane(const GprMHArgs &a, hipStream_t s);
+hipError_t gpr_launch_mh_ref_lane(const GprMHArgs &a, int kc, hipStream_t s);
 hipError_t gpr_launch_mh_ref_wave(const GprMHArgs &a, int kc, int grid, hipStream_t s);
 hipError_t gpr_launch_eval_wave(const GprEvalArgs &a, hipStream_t s);
 // header (n, kc, lconst, wconst, ...) and per-point weights of one dataset from its sd

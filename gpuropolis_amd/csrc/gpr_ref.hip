@@ -8,11 +8,14 @@
 // random_int / random_float / random_normal / random_geometric (main.cu:218-254) and
 // the host variants (main.cu:262-284) with the shared spec math.
 //
-//   k_mh_ref_lane  one lane per chain, the literal bottom-up fold over 31 slots per
-//                  datum (as the reference evaluates); Philox or LCG.
-//   k_mh_ref_wave  one wave per chain: heap in VGPRs (lane = slot), lane-parallel
-//                  heap -> postfix decode of the reachable tree, the shared wave
-//                  evaluator, per-constant proposals in parallel lanes.
+// Two kernels, both one wave per chain: heap in VGPRs (lane = slot), lane-parallel
+// heap -> postfix decode of the reachable tree, the shared wave interpreter, per-constant
+// proposals in parallel lanes.
+//   k_mh_ref_literal  the lane schedule: the reference's likelihood arithmetic (FP64 terms
+//                     of every point, main.cu:454-468) and its order of draws; Philox or LCG.
+//   k_mh_ref_wave     the wave schedule: FP32 compensated terms with early rejection.
+#include <algorithm>
+
 #include "gpr_device.h"
 
 // gpr_logf of the node counts 0 .. 31 (-inf at 0), filled once per device by
@@ -49,17 +52,8 @@ __device__ __forceinline__ float r_pow10(int order) {  // powf(10, order), order
 }
 
 // ---------------------------------------------------------------- draw sources
-struct LcgSrc {
-    uint32_t rx;
-    __device__ __forceinline__ uint32_t rand31() { rx = (rx * 1103515245u + 12345u) & 0x7fffffffu; return rx; }
-};
 struct PhiloxSrc {
     gpr_rstream st;
-    __device__ __forceinline__ uint32_t rand31() { return st.next() >> 1; }
-};
-// the same words, drawn 64 at a time on the vector unit (wave-uniform draws)
-struct WavePhiloxSrc {
-    WaveStream st;
     __device__ __forceinline__ uint32_t rand31() { return st.next() >> 1; }
 };
 
@@ -69,18 +63,24 @@ template <class S> __device__ __forceinline__ int r_random_int(int n, S &s) {
     do { r = (int)(s.rand31() / div); } while (r >= n);
     return r;
 }
-template <class S> __device__ __forceinline__ float r_random_float(S &s) {
-    return (float)((double)(float)r_random_int(1000000, s) / 1000000.0);
-}
-template <class S> __device__ __forceinline__ float r_random_normal(S &s) {
+// random_float of random_int(1000000) = r: the reference divides in double and rounds to
+// float; the product with the double 1e-6 rounds to the same float for every one of the
+// million values of r (tests/test_gpu_ref_edges.py), in one instruction instead of a division
+#define R_FLOAT_N 1000000
+#define R_FLOAT_DIV (0x7fffffffu / (R_FLOAT_N + 1))
+__device__ __forceinline__ float r_float_of(int r) { return (float)((double)r * 1e-6); }
+template <class S> __device__ __forceinline__ float r_random_float(S &s) { return r_float_of(r_random_int(R_FLOAT_N, s)); }
+__device__ __forceinline__ float r_box_muller(float u, float v) {
 #pragma clang fp contract(off)
-    const float u = r_random_float(s);
-    const float v = r_random_float(s);
     return sqrtf(-2.0f * gpr_logf(u)) * gpr_sin2pi(v);
 }
-template <class S> __device__ __forceinline__ float r_random_geometric(S &s) {
-    return ceilf(gpr_logf(r_random_float(s)) / R_LOG01_F);
+template <class S> __device__ __forceinline__ float r_random_normal(S &s) {
+    const float u = r_random_float(s);
+    const float v = r_random_float(s);
+    return r_box_muller(u, v);
 }
+__device__ __forceinline__ float r_geometric_of(float u) { return ceilf(gpr_logf(u) / R_LOG01_F); }
+template <class S> __device__ __forceinline__ float r_random_geometric(S &s) { return r_geometric_of(r_random_float(s)); }
 template <class S> __device__ __forceinline__ int r_host_random_int(int limit, S &s) {
     const uint32_t div = (uint32_t)(0x7fffffff / limit);
     int r;
@@ -95,6 +95,87 @@ template <class S> __device__ __forceinline__ float r_host_random_normal(S &s) {
     const float u = r_host_random_float(s);
     const float v = r_host_random_float(s);
     return sqrtf(-2.0f * gpr_logf(u)) * gpr_sin2pi(v);
+}
+
+// Orders this wave's LDS accesses before the call against those after it (LDS operations
+// of one wave execute in order; this keeps the compiler from moving them).
+__device__ __forceinline__ void r_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// One serial stream of 31-bit words, 64 of them at a time: lane k holds word k of the
+// current batch and pos is the next word.  A draw that rejects values (random_int) makes
+// the number of words it takes depend on them; take() finds the accepted ones by ballot, so
+// that the words go where the serial loop over the stream would put them.
+template <class Words>
+struct WaveDraws {
+    Words src;
+    uint32_t raw;   // this lane's word of the batch
+    int pos;
+    __device__ __forceinline__ void refill() { raw = src.batch(); pos = 0; }
+    // the next random_int(N)
+    template <int N> __device__ __forceinline__ int next_int() {
+        constexpr uint32_t div = 0x7fffffffu / (N + 1);
+        int r;
+        do {
+            if (pos == 64) refill();
+            r = (int)((uint32_t)rl_i((int)raw, pos++) / div);
+        } while (r >= N);
+        return r;
+    }
+    // buf[0 .. m-1] = the next m values of random_int(n), div = 0x7fffffff / (n + 1); every
+    // iteration of the loop consumes the rest of a batch or ends it
+    __device__ __forceinline__ void take(int m, int n, uint32_t div, int *buf) {
+        const int l = lane_id();
+        int got = 0;
+        while (got < m) {
+            if (pos == 64) refill();
+            const int r = (int)(raw / div);
+            const uint64_t ok = ballot(l >= pos && r < n);
+            const int at = got + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(ok >> 32),
+                                                                __builtin_amdgcn_mbcnt_lo((uint32_t)ok, 0u));
+            const bool mine = ((ok >> l) & 1ull) != 0 && at < m;
+            if (mine) buf[at] = r;
+            const uint64_t last = ballot(mine && at == m - 1);
+            pos = last ? __builtin_ctzll(last) + 1 : 64;
+            got += __popcll(ok);
+        }
+    }
+};
+
+// words of a Philox substream, in order
+struct PhiloxWords {
+    uint64_t seed;
+    uint32_t chain, step, c2, base;
+    __device__ __forceinline__ uint32_t batch() {
+        const int k = lane_id();
+        const gpr_u4 b = gpr_philox(chain, step, c2, 16u * base + (uint32_t)(k >> 2), (uint32_t)seed, (uint32_t)(seed >> 32));
+        base++;
+        return gpr_u4_word(b, k & 3) >> 1;
+    }
+};
+__device__ __forceinline__ WaveDraws<PhiloxWords> philox_draws(uint64_t seed, uint32_t chain, uint32_t step, uint32_t purpose) {
+    return {{seed, chain, step, purpose << 24, 0u}, 0u, 64};
+}
+// the reference's LCG (main.cu:213-216): lane k jumps k + 1 steps ahead of the batch's
+// start, x -> mul x + add (mod 2^31)
+struct LcgWords {
+    uint32_t x, mul, add;
+    __device__ __forceinline__ uint32_t batch() {
+        const uint32_t w = (mul * x + add) & 0x7fffffffu;
+        x = (uint32_t)rl_i((int)w, 63);
+        return w;
+    }
+};
+__device__ __forceinline__ WaveDraws<LcgWords> lcg_draws(uint32_t seed) {
+    uint32_t m = 1, c = 0, pm = 1103515245u, pc = 12345u;
+    for (int e = lane_id() + 1; e; e >>= 1) {
+        if (e & 1) { m *= pm; c = c * pm + pc; }
+        pc = pc * pm + pc;
+        pm *= pm;
+    }
+    return {{seed, m, c}, 0u, 64};
 }
 
 // ---------------------------------------------------------------- densities (main.cu:299-309)
@@ -117,44 +198,50 @@ __device__ __forceinline__ double r_logplusexp(double a, double b) {  // main.cu
 }
 __device__ __forceinline__ bool r_valid(double x) { return __builtin_isfinite(x); }
 
-// One constant proposal of the constant step (main.cu:746-785).  Returns the forward and
-// backward terms this constant adds (forward/backward accumulate over constants).
-template <class S>
-__device__ __forceinline__ void r_const_prop(S &s, float &C, double &ft, double &bt) {
+// One constant proposal of the constant step (main.cu:746-785) from its four random_float
+// draws: the first decides for the mixture (always: P_PROPOSE_C_GEOMETRIC = 1), the second
+// for an integer (PROPOSE_INT), the others make the value.  A proposal does not depend on
+// the constant it replaces.  ft: its forward term.
+__device__ __forceinline__ float r_const_prop(float f1, float f2, float f3, double &ft) {
 #pragma clang fp contract(off)
-    const float oldC = C;
-    ft = 0.0;
-    bt = 0.0;
-    if (r_random_float(s) < 1.0f) {                 // P_PROPOSE_C_GEOMETRIC = 1: always
-        if (r_random_float(s) < 0.15f) {            // PROPOSE_INT
-            const float sgn = r_random_float(s) < 0.5f ? -1.0f : 1.0f;
-            C = sgn * r_random_geometric(s) - 1.0f;
-            ft = r_lgeom(C + 1.0f) + (C == 0.0f ? 0.0 : R_LOG2_D) + (double)R_LOG015_F;
-        } else {
-            C = 1.0f * r_random_normal(s);
-            ft = r_lnormal1(C / 1.0f) + R_LOG1M015_D;
-        }
-        if (r_is_int(oldC)) {
-            bt = r_logplusexp(r_lgeom(oldC + 1.0f) + (C == 0.0f ? 0.0 : R_LOG2_D) + (double)R_LOG015_F,
-                              r_lnormal1(oldC / 1.0f) + R_LOG1M015_D);
-        } else {
-            bt = r_lnormal1(oldC / 1.0f) + R_LOG1M015_D;
-        }
-    } else {                                        // unreachable, main.cu:779-784
-        const int order = r_random_int(8, s) - 4;
-        C = C + 1.0f * r_pow10(order) * r_random_normal(s);
+    if (f1 < 0.15f) {
+        const float c = (f2 < 0.5f ? -1.0f : 1.0f) * r_geometric_of(f3) - 1.0f;
+        ft = r_lgeom(c + 1.0f) + (c == 0.0f ? 0.0 : R_LOG2_D) + (double)R_LOG015_F;
+        return c;
+    }
+    const float c = 1.0f * r_box_muller(f2, f3);
+    ft = r_lnormal1(c / 1.0f) + R_LOG1M015_D;
+    return c;
+}
+// The backward terms of a constant: for a proposal other than 0, and for 0 (main.cu:768-778).
+__device__ __forceinline__ void r_const_back(float oldC, double &bt, double &bt0) {
+#pragma clang fp contract(off)
+    bt = bt0 = r_lnormal1(oldC / 1.0f) + R_LOG1M015_D;
+    if (r_is_int(oldC)) {
+        const double g = r_lgeom(oldC + 1.0f);
+        bt = r_logplusexp(g + R_LOG2_D + (double)R_LOG015_F, bt0);
+        bt0 = r_logplusexp(g + 0.0 + (double)R_LOG015_F, bt0);
+    }
+}
+// The four random_float draws of a constant's Philox substream (chain, step, CPROP, slot):
+// one block, unless a word is rejected (about 1 in 4400).
+__device__ __forceinline__ void r_const_floats(uint64_t seed, uint32_t chain, uint32_t step, uint32_t slot, float (&f)[4]) {
+    const gpr_u4 b = gpr_philox(chain, step, ((uint32_t)GPR_P_CPROP << 24) | slot, 0u, (uint32_t)seed, (uint32_t)(seed >> 32));
+    const int r0 = (int)((b.x >> 1) / R_FLOAT_DIV), r1 = (int)((b.y >> 1) / R_FLOAT_DIV), r2 = (int)((b.z >> 1) / R_FLOAT_DIV),
+              r3 = (int)((b.w >> 1) / R_FLOAT_DIV);
+    f[0] = r_float_of(r0); f[1] = r_float_of(r1); f[2] = r_float_of(r2); f[3] = r_float_of(r3);
+    if (max(max(r0, r1), max(r2, r3)) >= R_FLOAT_N) {
+        PhiloxSrc pc;
+        pc.st.init(seed, chain, step, GPR_P_CPROP, slot);
+        for (int k = 0; k < 4; k++) f[k] = r_random_float(pc);
     }
 }
 
-__device__ __forceinline__ bool r_is_descendant(int n, int k) {  // main.cu:660-677
-    if (k == n) return true;
-    n = n + 1;
-    k = k + 1;
-    while (k > n) {
-        k >>= 1;
-        if (k == n) return true;
-    }
-    return false;
+// Is slot k (0-based) the slot n or one of its descendants (main.cu:660-677)?  Slot numbers
+// from 1 shifted right by the difference of their bit lengths.
+__device__ __forceinline__ bool r_is_descendant(int n, int k) {
+    const int n1 = n + 1, k1 = k + 1, d = __builtin_clz(n1) - __builtin_clz(k1);
+    return d >= 0 && (k1 >> d) == n1;
 }
 
 // reference op code -> postfix op code (A, B: -1, pass-through)
@@ -195,58 +282,7 @@ __device__ __forceinline__ float r_tape_const(int o, float hc) {
     return gpr_ref_is_physical(o) ? gpr_ref_physical_value(o) : (o == GPR_REF_HALF ? 0.5f : hc);
 }
 
-// ---------------------------------------------------------------- lane schedule
-typedef float gpr_f32v __attribute__((ext_vector_type(32)));
-typedef int gpr_i32v __attribute__((ext_vector_type(32)));
-
-// dispatch_eval (main.cu:397-444), one lane
-__device__ __forceinline__ float r_dispatch_eval(int o, float a, float b, float C) {
-    switch (o) {
-    case GPR_REF_ONE: return 1.0f;
-    case GPR_REF_CONST: return C;
-    case GPR_REF_INV: return 1.0f / a;
-    case GPR_REF_A: return a;
-    case GPR_REF_B: return b;
-    case GPR_REF_PLUS: return a + b;
-    case GPR_REF_CPLUS: return a + C;
-    case GPR_REF_MINUS: return a - b;
-    case GPR_REF_RMINUS: return b - a;
-    case GPR_REF_TIMES: return a * b;
-    case GPR_REF_CTIMES: return C * a;
-    case GPR_REF_DIV: return a / b;
-    case GPR_REF_RDIV: return b / a;
-    case GPR_REF_SQRT: return sqrtf(a);
-    case GPR_REF_LOG: return logf(a);
-    case GPR_REF_SIN: return sinf(a);
-    case GPR_REF_ASIN: return asinf(a);
-    case GPR_REF_COS: return cosf(a);
-    case GPR_REF_ACOS: return acosf(a);
-    case GPR_REF_TAN: return tanf(a);
-    case GPR_REF_ATAN: return atanf(a);
-    case GPR_REF_EXP: return expf(a);
-    case GPR_REF_POW: return powf(a, b);
-    case GPR_REF_CPOW: return powf(a, C);
-    case GPR_REF_RPOW: return powf(b, a);
-    case GPR_REF_CRPOW: return powf(C, a);
-    case GPR_REF_ABS: return fabsf(a);
-    case GPR_REF_HALF: return (float)((double)a / 2.0);
-    default: return gpr_ref_is_physical(o) ? gpr_ref_physical_value(o) : __builtin_nanf("");
-    }
-}
-
-// program_fold (main.cu:371-393) of the eval, length and count dispatchers, one lane.
-// The slot index is uniform across the wave, so the register arrays are indexed with
-// s_set_gpr_idx.
-__device__ float r_fold_eval(const gpr_i32v &P, const gpr_f32v &C, float x) {
-    gpr_f32v buf;
-    for (int i = GPR_REF_SLOTS; i >= 1; i--) {
-        const int l = 2 * i;
-        const float lv = l > GPR_REF_SLOTS ? x : buf[l & 31];
-        const float rv = l > GPR_REF_SLOTS ? x : buf[(l + 1) & 31];
-        buf[i] = r_dispatch_eval(P[i - 1], lv, rv, C[i - 1]);
-    }
-    return buf[1];
-}
+// ---------------------------------------------------------------- heap decode
 __device__ __forceinline__ int r_len_kind(int o) {  // 0 leaf, 1 A, 2 B, 3 unary, 4 C-op, 5 binary
     if (gpr_ref_is_physical(o)) return 0;              // PHYSICAL_CONSTANT_LENGTH_PRIOR = 1
     switch (o) {
@@ -259,167 +295,6 @@ __device__ __forceinline__ int r_len_kind(int o) {  // 0 leaf, 1 A, 2 B, 3 unary
     default: return 3;
     }
 }
-// dispatch_length (main.cu:477-526) and dispatch_countnodes (main.cu:553-601) folds
-__device__ void r_fold_len_count(const gpr_i32v &P, float &length, int &count) {
-    gpr_f32v bl;
-    gpr_i32v bc;
-    for (int i = GPR_REF_SLOTS; i >= 1; i--) {
-        const int l = 2 * i;
-        const float la = l > GPR_REF_SLOTS ? 1.0f : bl[l & 31], lb = l > GPR_REF_SLOTS ? 1.0f : bl[(l + 1) & 31];
-        const int ca = l > GPR_REF_SLOTS ? 0 : bc[l & 31], cb = l > GPR_REF_SLOTS ? 0 : bc[(l + 1) & 31];
-        const int k = r_len_kind(P[i - 1]);
-        float lv;
-        int cv;
-        switch (k) {
-        case 0: lv = 1.0f; cv = 1; break;
-        case 1: lv = la; cv = ca; break;
-        case 2: lv = lb; cv = cb; break;
-        case 3: lv = 1.0f + la; cv = 1 + ca; break;
-        case 4: lv = 1.0f + la + 1.0f; cv = ca + 1; break;
-        default: lv = 1.0f + la + lb; cv = 1 + ca + cb; break;
-        }
-        bl[i] = lv;
-        bc[i] = cv;
-    }
-    length = bl[1];
-    count = bc[1];
-}
-
-// compute_prior (main.cu:529-544) and compute_likelihood (main.cu:454-468), one lane.
-// lnc[i] = 0.5*(logf(2 pi) + 2 logf(sd_i)) is precomputed on the host with the host libm.
-__device__ double r_prior(const gpr_i32v &P, const gpr_f32v &C, double lnops) {
-#pragma clang fp contract(off)
-    float length;
-    int count;
-    r_fold_len_count(P, length, count);
-    double prior = -(double)(1.0f * length) * lnops;
-    for (int c = 0; c < GPR_REF_SLOTS; c++) prior += gpr_lcauchy(C[c]);
-    return prior;
-}
-__device__ double r_likelihood(const gpr_i32v &P, const gpr_f32v &C, const float *x, const float *y, const float *sd,
-                               const double *lnc, int n) {
-#pragma clang fp contract(off)
-    double ll = 0.0;
-    for (int i = 0; i < n; i++) {
-        const float fx = r_fold_eval(P, C, x[i]);
-        if (!__builtin_isfinite(fx)) return -GPR_INF;
-        const float r = fx - y[i];
-        const double s = (double)sd[i];
-        const double l = -(double)(r * r) / (2.0 * s * s) - lnc[i];
-        if (!__builtin_isfinite(l)) return -GPR_INF;
-        ll += l;
-    }
-    return ll;
-}
-
-template <class S>
-__device__ __forceinline__ bool r_accept(S &s, double ppost, double cur, double acc) {
-    return (r_valid(ppost) && (acc > 0.0 || r_random_float(s) < gpr_expf((float)acc))) || !r_valid(cur);
-}
-
-template <int RNG>
-__global__ void __launch_bounds__(128) k_mh_ref_lane(GprMHArgs a) {
-    const uint32_t step0 = a.clock ? a.clock[0] : a.step0;
-    const int nops = gpr_opset_nops(a.opset);
-    const int chain = blockIdx.x * blockDim.x + threadIdx.x;
-    if (chain >= a.nchains) return;
-    int di = 0;
-    while (a.ds[di].chain0 + a.ds[di].nchains <= chain) di++;
-    const GprDataset d = a.ds[di];
-    const float *x = a.dx + d.off, *y = a.dy + d.off, *sdv = a.dsd + d.off;
-    const double *lc = a.lnc + d.off;
-    const int N = a.nchains;
-    gpr_i32v P;
-    gpr_f32v C;
-    for (int i = 0; i < GPR_REF_SLOTS; i++) {
-        P[i] = a.ops[(size_t)i * N + chain];
-        C[i] = a.cs[(size_t)i * N + chain];
-    }
-    double cur_prior = r_prior(P, C, a.ref_lnops);
-    double cur_ll = r_likelihood(P, C, x, y, sdv, lc, d.n);
-    double cur_post = cur_prior + cur_ll;
-    LcgSrc lcg{(uint32_t)a.block_seed + (uint32_t)chain};
-    gpr_i32v oldP;
-    gpr_f32v oldC;
-    double forward = 0.0, backward = 0.0;
-    unsigned long long n_sprop = 0, n_sacc = 0, n_cprop = 0, n_cacc = 0;
-    for (int mcmci = 0; mcmci < a.steps; mcmci++) {
-        const uint32_t step = step0 + (uint32_t)mcmci;
-        if (mcmci % 5 == 0) {
-            n_sprop++;
-            float length;
-            int count;
-            r_fold_len_count(P, length, count);
-            forward = -(double)gpr_logf((float)count);
-            PhiloxSrc ph;
-            ph.st.init(a.seed, (uint32_t)chain, step, GPR_P_STRUCT, 0);
-            int nn;
-            if (RNG == GPR_RNG_LCG) nn = !r_valid(cur_post) ? 0 : r_random_int(GPR_REF_SLOTS, lcg);
-            else nn = !r_valid(cur_post) ? 0 : r_random_int(GPR_REF_SLOTS, ph);
-            for (int i = 0; i < GPR_REF_SLOTS; i++) {
-                oldP[i] = P[i];
-                if (i >= nn && r_is_descendant(nn, i)) {
-                    P[i] = gpr_opset_code(a.opset, RNG == GPR_RNG_LCG ? r_random_int(nops, lcg) : r_random_int(nops, ph));
-                }
-            }
-            r_fold_len_count(P, length, count);
-            backward = -(double)gpr_logf((float)count);
-            const double pp = r_prior(P, C, a.ref_lnops);
-            const double pl = r_likelihood(P, C, x, y, sdv, lc, d.n);
-            const double ppost = pp + pl;
-            const double acc = ppost - cur_post + backward - forward;
-            bool ok;
-            if (RNG == GPR_RNG_LCG) ok = r_accept(lcg, ppost, cur_post, acc);
-            else { PhiloxSrc pa; pa.st.init(a.seed, (uint32_t)chain, step, GPR_P_ACCEPT, 0); ok = r_accept(pa, ppost, cur_post, acc); }
-            if (ok) { cur_post = ppost; cur_ll = pl; cur_prior = pp; n_sacc++; }
-            else P = oldP;
-        } else {
-            n_cprop++;
-            for (int c = 0; c < GPR_REF_SLOTS; c++) {
-                oldC[c] = C[c];
-                float cv = C[c];
-                double ft, bt;
-                if (RNG == GPR_RNG_LCG) r_const_prop(lcg, cv, ft, bt);
-                else { PhiloxSrc pc; pc.st.init(a.seed, (uint32_t)chain, step, GPR_P_CPROP, (uint32_t)c); r_const_prop(pc, cv, ft, bt); }
-                C[c] = cv;
-                forward += ft;
-                backward += bt;
-            }
-            const double pp = r_prior(P, C, a.ref_lnops);
-            const double pl = r_likelihood(P, C, x, y, sdv, lc, d.n);
-            const double ppost = pp + pl;
-            const double acc = ppost - cur_post + backward - forward;
-            bool ok;
-            if (RNG == GPR_RNG_LCG) ok = r_accept(lcg, ppost, cur_post, acc);
-            else { PhiloxSrc pa; pa.st.init(a.seed, (uint32_t)chain, step, GPR_P_ACCEPT, 0); ok = r_accept(pa, ppost, cur_post, acc); }
-            if (ok) { cur_post = ppost; cur_ll = pl; cur_prior = pp; n_cacc++; }
-            else C = oldC;
-        }
-    }
-    for (int i = 0; i < GPR_REF_SLOTS; i++) {
-        a.ops[(size_t)i * N + chain] = (uint8_t)P[i];
-        a.cs[(size_t)i * N + chain] = C[i];
-    }
-    a.prior[chain] = cur_prior;
-    a.ll[chain] = cur_ll;
-    if (a.counters) {
-        atomicAdd(&a.counters[GPR_CNT_SPROP], n_sprop);
-        atomicAdd(&a.counters[GPR_CNT_SACC], n_sacc);
-        atomicAdd(&a.counters[GPR_CNT_CPROP], n_cprop);
-        atomicAdd(&a.counters[GPR_CNT_CACC], n_cacc);
-        atomicAdd(&a.counters[GPR_CNT_STEPS], (unsigned long long)a.steps);
-        atomicAdd(&a.counters[GPR_CNT_EVALS], (unsigned long long)a.steps * (unsigned long long)(GPR_REF_SLOTS * d.n));
-    }
-}
-
-hipError_t gpr_launch_mh_ref_lane(const GprMHArgs &a, hipStream_t s) {
-    const int grid = (a.nchains + 127) / 128;
-    if (a.rng == GPR_RNG_LCG) hipLaunchKernelGGL((k_mh_ref_lane<GPR_RNG_LCG>), dim3(grid), dim3(128), 0, s, a);
-    else hipLaunchKernelGGL((k_mh_ref_lane<GPR_RNG_PHILOX>), dim3(grid), dim3(128), 0, s, a);
-    return hipGetLastError();
-}
-
-// ---------------------------------------------------------------- wave schedule
 // Lane-parallel decode of the heap held one slot per lane (lane i = slot i+1, i < 31)
 // into the postfix tape of the reachable tree, one token per lane.  Subtree token
 // counts are folded bottom-up and start positions pushed top-down, level by level;
@@ -428,6 +303,8 @@ hipError_t gpr_launch_mh_ref_lane(const GprMHArgs &a, hipStream_t s) {
 struct RefTape {
     WaveProg p;     // ops and constants of the tape, o0/c0 per lane
     int slot;       // heap slot of each token (255 for x)
+    int src;        // heap slot whose constant the token carries, or -1: its constant does
+                    // not change with the heap's (none, a physical constant, halving's 0.5)
     int count;      // reachable non-pass-through ops: count_nodes (main.cu:604-608)
     int dl;         // description length: tokens + C-op tokens (dispatch_length fold)
 };
@@ -494,7 +371,10 @@ __device__ RefTape r_decode_wave(int hop, float hc) {
     rt.p.o1 = 0;
     rt.p.c1 = 0.0f;
     const float cs = shfl_all(r_tape_const(hop, hc), rt.slot & 31);
-    rt.p.c0 = (valid && gpr_has_const(rt.p.o0)) ? cs : 0.0f;
+    const int ho = shfl_all(hop, rt.slot & 31);
+    const bool holds = valid && gpr_has_const(rt.p.o0);
+    rt.p.c0 = holds ? cs : 0.0f;
+    rt.src = holds && !gpr_ref_is_physical(ho) && ho != GPR_REF_HALF ? rt.slot : -1;
     rt.count = len - __popcll(ballot(valid && rt.p.o0 == GPR_OP_X));
     // description length: tokens plus the C-op tokens (dispatch_length kind 4; halving is
     // a c* token of length 1 + a)
@@ -503,29 +383,289 @@ __device__ RefTape r_decode_wave(int hop, float hc) {
     return rt;
 }
 
-// refresh the tape's constants from the heap constants
-__device__ __forceinline__ void r_tape_consts(RefTape &rt, int hop, float hc) {
-    const float cs = shfl_all(r_tape_const(hop, hc), rt.slot & 31);
-    rt.p.c0 = (lane_id() < rt.p.len && gpr_has_const(rt.p.o0)) ? cs : 0.0f;
+// the tape with other heap constants: slot c's at lane base + c of v
+__device__ __forceinline__ float r_tape_consts(const RefTape &rt, float v, int base) {
+    const float cv = shfl_all(v, base + max(rt.src, 0));
+    return rt.src >= 0 ? cv : rt.p.c0;
 }
 
-// prior: -length*log(NOPS+1) + sum over all 31 constants in slot order (main.cu:529-544)
-__device__ __forceinline__ double r_prior_wave(int dl, float hc, double lnops) {
+// ---------------------------------------------------------------- serial sums
+// The prior and the proposal densities add 31 terms each in slot order (FP64, the order is
+// part of the result).  A sum by lane reads costs two readlanes and an add per term; here
+// the terms go through LDS, S[row][slot] with 32 doubles a row, and one lane does one
+// serial sum, so that the sums of a step (or of the four constant steps between two structure
+// moves) share every instruction.  Only the lanes that sum may be active: with the other
+// lanes reading along (one address for all of them) the LDS took about 80 cycles an
+// instruction, and a block of the batch of NIST sizes 7.4 ms instead of 3.9.
+#define R_ROW 32
+__device__ __forceinline__ double r_add_row(const double *row, double acc) {
 #pragma clang fp contract(off)
-    const double lc = gpr_lcauchy(hc);
-    double prior = -(double)(1.0f * (float)dl) * lnops;
-    for (int c = 0; c < GPR_REF_SLOTS; c++) prior += rl_d(lc, c);
-    return prior;
+#pragma unroll
+    for (int c = 0; c < 24; c += 8) {
+        double v[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) v[k] = row[c + k];
+#pragma unroll
+        for (int k = 0; k < 8; k++) acc += v[k];
+    }
+    double v[7];
+#pragma unroll
+    for (int k = 0; k < 7; k++) v[k] = row[24 + k];
+#pragma unroll
+    for (int k = 0; k < 7; k++) acc += v[k];
+    return acc;
+}
+__device__ __forceinline__ double r_prior_start(int dl, double lnops) {
+#pragma clang fp contract(off)
+    return -(double)(1.0f * (float)dl) * lnops;
+}
+// prior: -length*log(NOPS+1) + sum over all 31 constants in slot order (main.cu:529-544);
+// lc: slot c's term at lane c.
+__device__ __forceinline__ double r_prior_wave(int dl, double lc, double lnops, double *S) {
+    r_lds_order();
+    if (lane_id() < R_ROW) S[lane_id()] = lc;
+    r_lds_order();
+    double acc = r_prior_start(dl, lnops);
+    if (lane_id() == 0) acc = r_add_row(S, acc);
+    return rl_d(acc, 0);
 }
 
+// LDS of one wave: the interpreter's stack for programs of depth at most 6 (heap-31 programs
+// are trees of at most five levels; levels -2 .. 3 of wave_eval_ls), then the sums' rows
+// and results (the random_int buffers of a structure move share the rows)
+#define R_LEVELS 6
+#define R_SUM_ROWS 12
+#define R_SUM_DOUBLES (R_SUM_ROWS * R_ROW + 12)
+__host__ __device__ constexpr size_t r_lds_floats(int kc) { return (size_t)R_LEVELS * 64 * kc + 2 * R_SUM_DOUBLES; }
+extern __shared__ float r_lds[];
+
+// The structure move's new ops (main.cu:717-730): a node drawn from the slots (the root when
+// the current state is invalid), then a new op for it and each of its descendants in slot order.
+template <class D>
+__device__ __forceinline__ int r_struct_draw(D &dr, bool valid, int hop, int opset, int nops, int *buf) {
+    const int l = lane_id();
+    const int nn = valid ? dr.template next_int<GPR_REF_SLOTS>() : 0;
+    const bool desc = l < GPR_REF_SLOTS && r_is_descendant(nn, l);
+    const uint64_t dm = ballot(desc);
+    r_lds_order();
+    dr.take(__popcll(dm), nops, (uint32_t)(0x7fffffff / (nops + 1)), buf);
+    r_lds_order();
+    const int k = (int)__builtin_amdgcn_mbcnt_lo((uint32_t)dm, 0u);   // slots lie in the low lanes
+    return desc ? gpr_opset_code(opset, buf[min(k, GPR_REF_SLOTS)]) : hop;
+}
+
+// ---------------------------------------------------------------- lane schedule
+// Likelihood as main.cu:454-468: per point an FP64 term -(f - y)^2 / (2 sd^2) - lnc with the
+// float square, -inf as soon as a value or a term is not finite.  Lanes compute their
+// points' terms; the sum runs over them in point order, as the reference adds them (a
+// program with an LL near -1e22 is accepted or not by the last bit of it), through the 64
+// doubles of S.
 template <int KC>
-__global__ void __launch_bounds__(GPR_WG) __attribute__((amdgpu_waves_per_eu(KC == 1 ? 4 : 1)))
-k_mh_ref_wave(GprMHArgs a) {
+__device__ __forceinline__ double r_loglik64(const WaveProg &p, const OpMasks &m, float *ls, double *S, const float *x,
+                                             const float *y, const float *sd, const double *lnc, int n) {
+#pragma clang fp contract(off)
+    const int l = lane_id();
+    double s = 0.0;
+    for (int base = 0; base < n; base += 64 * KC) {
+        float xs[KC], T[KC];
+#pragma unroll
+        for (int k = 0; k < KC; k++) {
+            const int i = base + 64 * k + l;
+            xs[k] = i < n ? x[i] : 0.0f;
+        }
+        wave_eval_ls<KC, false>(p, xs, T, ls, m);
+#pragma unroll
+        for (int k = 0; k < KC; k++) {
+            const int i = base + 64 * k + l, left = n - (base + 64 * k);
+            if (left <= 0) break;
+            double t = 0.0;              // adding +0 past the last point changes nothing
+            if (i < n) {
+                const float r = T[k] - y[i];
+                const double e = (double)sd[i];
+                t = __builtin_isfinite(T[k]) ? -(double)(r * r) / (2.0 * e * e) - lnc[i] : -GPR_INF;
+            }
+            r_lds_order();
+            S[l] = t;
+            r_lds_order();
+            if (l == 0) for (int c = 0; c < min(left, 64); c += 8) {
+                double v[8];
+#pragma unroll
+                for (int q = 0; q < 8; q++) v[q] = S[c + q];
+#pragma unroll
+                for (int q = 0; q < 8; q++) s += v[q];
+            }
+        }
+    }
+    s = rl_d(s, 0);
+    return __builtin_isfinite(s) ? s : -GPR_INF;
+}
+
+// One wave per chain, one wave per workgroup, chains blockIdx.x, blockIdx.x + gridDim.x, ...
+// The draws of a step depend on the step before it (a rejected value and the accept test
+// take a varying number of LCG words), so steps are serial and only the work inside a step
+// is spread over the lanes: 64 words of the stream at once, a constant per lane, a point per
+// lane, the three serial sums in three lanes.  Bound by the latency of that chain at the
+// command line's default of 1024 chains (four waves per CU).  One lane per chain, folding
+// all 31 slots at every point with every lane's own ops, took 4600 us a step on 37 points
+// at 1024 chains; this takes 11.
+template <int KC, int RNG>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_mh_ref_literal(GprMHArgs a) {
+    const uint32_t step0 = a.clock ? a.clock[0] : a.step0;
+    const int nops = gpr_opset_nops(a.opset);
+    const int l = lane_id();
+    const int N = a.nchains;
+    const bool live = l < GPR_REF_SLOTS;
+    float *ls = r_lds;
+    double *S = (double *)(r_lds + R_LEVELS * 64 * KC);
+    int *buf = (int *)S;
+    unsigned long long n_sprop = 0, n_sacc = 0, n_cprop = 0, n_cacc = 0, n_steps = 0, n_evals = 0;
+    for (int ch = (int)blockIdx.x; ch < N; ch += (int)gridDim.x) {
+        const uint32_t chain = (uint32_t)ch;
+        int di = 0;
+        while (a.ds[di].chain0 + a.ds[di].nchains <= ch) di++;
+        const int n = a.ds[di].n, off = a.ds[di].off;
+        const float *x = a.dx + off, *y = a.dy + off, *sdv = a.dsd + off;
+        const double *lc = a.lnc + off;
+        int hop = live ? a.ops[(size_t)l * N + chain] : 0;
+        float hc = live ? a.cs[(size_t)l * N + chain] : 0.0f;
+        RefTape cur = r_decode_wave(hop, hc);
+        OpMasks cm = op_masks<false>(cur.p);
+        double cur_prior = r_prior_wave(cur.dl, gpr_lcauchy(hc), a.ref_lnops, S);
+        double cur_ll = r_loglik64<KC>(cur.p, cm, ls, S, x, y, sdv, lc, n);
+        double cur_post = cur_prior + cur_ll;
+        double bt, bt0;
+        r_const_back(hc, bt, bt0);
+        WaveDraws<LcgWords> lcg = lcg_draws((uint32_t)a.block_seed + chain);
+        double forward = 0.0, backward = 0.0;
+        int phase = 0;
+        for (int mcmci = 0; mcmci < a.steps; mcmci++) {
+            const uint32_t step = step0 + (uint32_t)mcmci;
+            int php = hop;
+            float phc = hc;
+            RefTape prop = cur;
+            OpMasks pm = cm;
+            double pp;
+            const bool structural = phase == 0;
+            phase = phase == 4 ? 0 : phase + 1;
+            if (structural) {
+                n_sprop++;
+                forward = -(double)gpr_ref_logint[cur.count];
+                if (RNG == GPR_RNG_LCG) {
+                    php = r_struct_draw(lcg, r_valid(cur_post), hop, a.opset, nops, buf);
+                } else {
+                    WaveDraws<PhiloxWords> ph = philox_draws(a.seed, chain, step, GPR_P_STRUCT);
+                    php = r_struct_draw(ph, r_valid(cur_post), hop, a.opset, nops, buf);
+                }
+                prop = r_decode_wave(php, hc);
+                pm = op_masks<false>(prop.p);
+                backward = -(double)gpr_ref_logint[prop.count];
+                pp = r_prior_wave(prop.dl, gpr_lcauchy(hc), a.ref_lnops, S);
+            } else {
+                n_cprop++;
+                float f[4];
+                if (RNG == GPR_RNG_LCG) {
+                    r_lds_order();
+                    lcg.take(4 * GPR_REF_SLOTS, R_FLOAT_N, R_FLOAT_DIV, buf);
+                    r_lds_order();
+#pragma unroll
+                    for (int k = 0; k < 4; k++) f[k] = r_float_of(buf[min(4 * l, 4 * GPR_REF_SLOTS) + k]);
+                } else {
+                    r_const_floats(a.seed, chain, step, (uint32_t)(l & 31), f);
+                }
+                double ft;
+                phc = r_const_prop(f[1], f[2], f[3], ft);
+                if (!live) phc = 0.0f;
+                // rows: prior, forward, backward; lane q sums row q
+                r_lds_order();
+                if (l < R_ROW) {
+                    S[l] = gpr_lcauchy(phc);
+                    S[R_ROW + l] = ft;
+                    S[2 * R_ROW + l] = phc == 0.0f ? bt0 : bt;
+                }
+                r_lds_order();
+                double acc = l == 0 ? r_prior_start(cur.dl, a.ref_lnops) : (l == 1 ? forward : backward);
+                if (l < 3) acc = r_add_row(S + l * R_ROW, acc);
+                pp = rl_d(acc, 0);
+                forward = rl_d(acc, 1);
+                backward = rl_d(acc, 2);
+                prop.p.c0 = r_tape_consts(cur, phc, 0);
+            }
+            const double pl = r_loglik64<KC>(prop.p, pm, ls, S, x, y, sdv, lc, n);
+            const double ppost = pp + pl;
+            const double acc = ppost - cur_post + backward - forward;
+            bool ok = !r_valid(cur_post);
+            if (r_valid(ppost)) {
+                if (acc > 0.0) {
+                    ok = true;
+                } else {
+                    float u;
+                    if (RNG == GPR_RNG_LCG) {
+                        u = r_float_of(lcg.next_int<R_FLOAT_N>());
+                    } else {
+                        PhiloxSrc pa;
+                        pa.st.init(a.seed, chain, step, GPR_P_ACCEPT, 0);
+                        u = r_random_float(pa);
+                    }
+                    ok = ok || u < gpr_expf((float)acc);
+                }
+            }
+            if (uni(ok)) {
+                cur_post = ppost; cur_ll = pl; cur_prior = pp;
+                hop = php; hc = phc; cur = prop; cm = pm;
+                if (structural) n_sacc++;
+                else { n_cacc++; r_const_back(hc, bt, bt0); }
+            }
+        }
+        n_steps += (unsigned long long)a.steps;
+        n_evals += (unsigned long long)a.steps * (unsigned long long)(GPR_REF_SLOTS * n);
+        if (live) { a.ops[(size_t)l * N + chain] = (uint8_t)hop; a.cs[(size_t)l * N + chain] = hc; }
+        if (l == 0) { a.prior[chain] = cur_prior; a.ll[chain] = cur_ll; }
+    }
+    if (l == 0 && a.counters) {
+        atomicAdd(&a.counters[GPR_CNT_SPROP], n_sprop);
+        atomicAdd(&a.counters[GPR_CNT_SACC], n_sacc);
+        atomicAdd(&a.counters[GPR_CNT_CPROP], n_cprop);
+        atomicAdd(&a.counters[GPR_CNT_CACC], n_cacc);
+        atomicAdd(&a.counters[GPR_CNT_STEPS], n_steps);
+        atomicAdd(&a.counters[GPR_CNT_EVALS], n_evals);
+    }
+}
+
+// kc: points per lane per pass of the interpreter, 1 or 4 (the largest dataset's: a pass
+// over at most 64 points with four per lane would interpret three empty ones)
+hipError_t gpr_launch_mh_ref_lane(const GprMHArgs &a, int kc, hipStream_t s) {
+    // a bounded grid: 64 lanes per chain would pass the 2^32 threads of a launch
+    const dim3 grid(std::min(a.nchains, 1 << 20));
+    const bool lcg = a.rng == GPR_RNG_LCG;
+#define R_L(K, R) hipLaunchKernelGGL((k_mh_ref_literal<K, R>), grid, dim3(64), sizeof(float) * r_lds_floats(K), s, a)
+    if (kc == 1) { if (lcg) R_L(1, GPR_RNG_LCG); else R_L(1, GPR_RNG_PHILOX); }
+    else { if (lcg) R_L(4, GPR_RNG_LCG); else R_L(4, GPR_RNG_PHILOX); }
+#undef R_L
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------- wave schedule
+// One wave per chain, persistent over the tiles of a size class.  Bound by instruction
+// issue.  A constant proposal does not depend on the constants it replaces, so the moves of
+// the (up to four) constant steps between two structure steps are drawn together: a lane per
+// constant and step (two steps a pass), the accept draws of all five steps in one Philox
+// evaluation, and the steps' priors and running forward and backward sums by six lanes side
+// by side.  Only the backward terms depend on the current constants; they are computed when
+// those change (two per constant: for a proposal of 0 and for any other) and summed again
+// for the steps that are left.  16384 chains x 100 steps: 2.9 ms at n = 20 and 4.1 at 236,
+// where one step at a time, its sums by lane reads and the value stack in indexed registers
+// took 4.4 and 7.6 (VALU instructions per chain-step halved).  Four waves per SIMD: the
+// compiler takes 140 VGPRs (three waves) when left alone.
+template <int KC>
+__global__ void __launch_bounds__(GPR_WG) __attribute__((amdgpu_waves_per_eu(4))) k_mh_ref_wave(GprMHArgs a) {
     const uint32_t step0 = a.clock ? a.clock[0] : a.step0;
     const int nops = gpr_opset_nops(a.opset);
     const int wave = uni((int)(threadIdx.x >> 6));
     const int l = lane_id();
     const int N = a.nchains;
+    const int slot = l & 31, half = l >> 5;
+    float *ls = r_lds + (size_t)wave * r_lds_floats(KC);
+    double *S = (double *)(ls + R_LEVELS * 64 * KC), *R = S + R_SUM_ROWS * R_ROW;
     unsigned long long n_sprop = 0, n_sacc = 0, n_cprop = 0, n_cacc = 0, n_evals = 0, n_steps = 0, n_flops = 0;
     for (;;) {
         __shared__ int s_tile;
@@ -536,91 +676,155 @@ k_mh_ref_wave(GprMHArgs a) {
         if (tile_idx >= a.ntiles) break;
         const GprTile tile = a.tiles[tile_idx];
         if (wave >= tile.count) continue;
-        const GprDataset d = a.ds[tile.dataset];
+        const GprDataset d = uni_dataset(a.ds[uni(tile.dataset)]);
         const uint32_t chain = (uint32_t)uni(tile.chain0 + wave);
         const float *dx = a.dx + d.off, *dy = a.dy + d.off, *dw = a.dw + d.off;
         const int nchunks = (d.n + 64 * KC - 1) / (64 * KC);
         Chunk<KC> c0;
         c0.load(dx, dy, dw, d.n, 0);
-        const bool live = l < GPR_REF_SLOTS;
-        int hop = live ? a.ops[(size_t)l * N + chain] : 0;
-        float hc = live ? a.cs[(size_t)l * N + chain] : 0.0f;
+        // slot c's constant sits at lanes c and 32 + c
+        const bool live = slot < GPR_REF_SLOTS;
+        int hop = l < GPR_REF_SLOTS ? a.ops[(size_t)l * N + chain] : 0;
+        float hc = live ? a.cs[(size_t)slot * N + chain] : 0.0f;
         RefTape cur = r_decode_wave(hop, hc);
-        double cur_prior = r_prior_wave(cur.dl, hc, a.ref_lnops);
-        double cur_ll = wave_loglik<KC, false>(cur.p, d, dx, dy, dw, c0, nchunks);
+        OpMasks cm = op_masks<false>(cur.p);
+        int opq, nconst;
+        prog_counts<false>(cur.p, opq, nconst);
+        double cur_prior = r_prior_wave(cur.dl, gpr_lcauchy(hc), a.ref_lnops, S);
+        double cur_ll = wave_loglik<KC, false, true>(cur.p, d, dx, dy, dw, c0, nchunks, ls, &cm);
         double cur_post = cur_prior + cur_ll;
+        double bt, bt0;
+        r_const_back(hc, bt, bt0);
         double forward = 0.0, backward = 0.0;
+        float pc[2] = {0.0f, 0.0f};   // proposals of constant steps 0, 1 (halves) and 2, 3
+        double sums = 0.0;            // lane u, 4 + u, 8 + u: prior, forward, backward of constant step u
+        float au = 0.0f, alu = 0.0f;  // lane u: accept draw of step u of the five, and its log
+        int phase = 0;
         for (int mcmci = 0; mcmci < a.steps; mcmci++) {
             const uint32_t step = step0 + (uint32_t)mcmci;
             int php = hop;
-            float phc = hc;
             RefTape prop = cur;
-            bool structural = (mcmci % 5) == 0;
+            OpMasks pm = cm;
+            double pp;
+            int p_opq = opq, p_nconst = nconst;
+            const int ph5 = phase;
+            const bool structural = ph5 == 0;
+            phase = phase == 4 ? 0 : phase + 1;
             if (structural) {
                 n_sprop++;
                 forward = -(double)gpr_ref_logint[cur.count];
-                WavePhiloxSrc ph;
-                ph.st.init(a.seed, chain, step, GPR_P_STRUCT, 0);
-                const int nn = !r_valid(cur_post) ? 0 : r_random_int(GPR_REF_SLOTS, ph);
-                for (int i = nn; i < GPR_REF_SLOTS; i++) {
-                    if (r_is_descendant(nn, i)) php = wl_i(php, gpr_opset_code(a.opset, r_random_int(nops, ph)), i);
-                }
-                prop = r_decode_wave(php, phc);
+                WaveDraws<PhiloxWords> ph = philox_draws(a.seed, chain, step, GPR_P_STRUCT);
+                php = r_struct_draw(ph, r_valid(cur_post), hop, a.opset, nops, (int *)S);
+                prop = r_decode_wave(php, hc);
+                pm = op_masks<false>(prop.p);
+                prog_counts<false>(prop.p, p_opq, p_nconst);
                 backward = -(double)gpr_ref_logint[prop.count];
+                pp = r_prior_wave(prop.dl, gpr_lcauchy(hc), a.ref_lnops, S);
+                // the accept draw of step u is the first random_float of its ACCEPT substream
+                {
+                    const uint32_t st = step + (uint32_t)min(l, 4);
+                    int r = (int)((gpr_first(a.seed, chain, st, GPR_P_ACCEPT, 0) >> 1) / R_FLOAT_DIV);
+                    if (r >= R_FLOAT_N) {
+                        PhiloxSrc pa;
+                        pa.st.init(a.seed, chain, st, GPR_P_ACCEPT, 0);
+                        r = r_random_int(R_FLOAT_N, pa);
+                    }
+                    au = r_float_of(r);
+                    alu = gpr_logf(au);
+                }
             } else {
                 n_cprop++;
-                double ft = 0.0, bt = 0.0;
-                if (live) {
-                    PhiloxSrc pc;
-                    pc.st.init(a.seed, chain, step, GPR_P_CPROP, (uint32_t)l);
-                    r_const_prop(pc, phc, ft, bt);
+                const int u = ph5 - 1;
+                if (u == 0) {
+                    // every constant step up to the next structure step or the block's end
+                    const int nw = min(4, a.steps - mcmci);
+                    r_lds_order();
+#pragma unroll
+                    for (int p = 0; p < 2; p++) {
+                        if (2 * p >= nw) break;
+                        const int v = 2 * p + half;
+                        float f[4];
+                        r_const_floats(a.seed, chain, step + (uint32_t)v, (uint32_t)slot, f);
+                        double ft;
+                        pc[p] = r_const_prop(f[1], f[2], f[3], ft);
+                        S[v * R_ROW + slot] = gpr_lcauchy(pc[p]);
+                        S[(4 + v) * R_ROW + slot] = ft;
+                        S[(8 + v) * R_ROW + slot] = pc[p] == 0.0f ? bt0 : bt;
+                    }
+                    r_lds_order();
+                    // lanes 0-3: the steps' priors; lane 4: forward, lane 5: backward, running
+                    // over the steps
+                    double acc = l < 4 ? r_prior_start(cur.dl, a.ref_lnops) : (l == 4 ? forward : backward);
+                    if (l < 6) {
+                        for (int v = 0; v < nw; v++) {
+                            acc = r_add_row(S + (l < 4 ? l : (l == 4 ? 4 + v : 8 + v)) * R_ROW, acc);
+                            if (l >= 4) R[(l - 3) * 4 + v] = acc;
+                            else if (v == 0) R[l] = acc;
+                        }
+                    }
+                    r_lds_order();
+                    if (l < 12) sums = R[l];
                 }
-                for (int c = 0; c < GPR_REF_SLOTS; c++) {   // slot order, as the sequential loop
-                    forward += rl_d(ft, c);
-                    backward += rl_d(bt, c);
-                }
-                r_tape_consts(prop, php, phc);
+                pp = rl_d(sums, u);
+                forward = rl_d(sums, 4 + u);
+                backward = rl_d(sums, 8 + u);
+                prop.p.c0 = r_tape_consts(cur, (u & 2) ? pc[1] : pc[0], (u & 1) * 32);
             }
-            const double pp = r_prior_wave(prop.dl, phc, a.ref_lnops);
-            // The accept draw u is the first random_float of the step's ACCEPT substream,
-            // the same value whenever it is taken, so it is drawn before the evaluation.  A
-            // valid current state accepts only if acc > 0 or u < expf(acc), and either needs
-            // acc >= log u - 1 (u > 0) or acc >= -105 (u = 0: expf(acc) underflows to 0
-            // below -103.98).  That bounds the proposal's LL from below: the evaluation
-            // stops once its partial sum proves the LL under the bound (wave_loglik), and
-            // the proposal is rejected as it would be after the full sum.
-            float u = 0.0f;
+            // A valid current state accepts only if acc > 0 or u < expf(acc), and either needs
+            // acc >= log u - 1 (u > 0) or acc >= -105 (u = 0: expf(acc) underflows to 0 below
+            // -103.98).  That bounds the proposal's LL from below: the evaluation stops once
+            // its partial sum proves the LL under the bound (wave_loglik), and the proposal is
+            // rejected as it would be after the full sum.
+            const float u01 = rl_f(au, ph5);
             double reject_below = -GPR_INF;
             if (r_valid(cur_post)) {
-                WavePhiloxSrc pa;
-                pa.st.init(a.seed, chain, step, GPR_P_ACCEPT, 0);
-                u = r_random_float(pa);
-                const double amin = u > 0.0f ? (double)gpr_logf(u) - 1.0 : -105.0;
+                const double amin = u01 > 0.0f ? (double)rl_f(alu, ph5) - 1.0 : -105.0;
                 if (r_valid(pp) && r_valid(forward) && r_valid(backward))
                     reject_below = cur_post - backward + forward - pp + amin -
                                    1e-12 * (__builtin_fabs(cur_post) + __builtin_fabs(backward) +
                                             __builtin_fabs(forward) + __builtin_fabs(pp));
             }
             int pts = d.n;
-            const double pl = wave_loglik<KC, false>(prop.p, d, dx, dy, dw, c0, nchunks, nullptr, nullptr,
-                                                     reject_below, &pts);
+            const double pl = wave_loglik<KC, false, true>(prop.p, d, dx, dy, dw, c0, nchunks, ls, &pm, reject_below, &pts);
             pts = min(pts, d.n);
             n_evals += (unsigned long long)prop.p.len * (unsigned long long)pts;
-            {
-                const int nleaf = __popcll(ballot(l < prop.p.len && prop.p.o0 <= GPR_OP_ONE));
-                const int nconst = __popcll(ballot(l < prop.p.len && gpr_has_const(prop.p.o0)));
-                n_flops += (unsigned long long)(prop.p.len - nleaf + 4) * (unsigned long long)pts + (unsigned long long)nconst;
-            }
+            n_flops += (unsigned long long)p_opq * (unsigned long long)pts + (unsigned long long)p_nconst;
             const double ppost = pp + pl;
             const double acc = ppost - cur_post + backward - forward;
-            if ((r_valid(ppost) && (acc > 0.0 || u < gpr_expf((float)acc))) || !r_valid(cur_post)) {
+            if ((r_valid(ppost) && (acc > 0.0 || u01 < gpr_expf((float)acc))) || !r_valid(cur_post)) {
                 cur_post = ppost; cur_ll = pl; cur_prior = pp;
-                hop = php; hc = phc; cur = prop;
-                if (structural) n_sacc++; else n_cacc++;
+                cur = prop;
+                if (structural) {
+                    n_sacc++;
+                    hop = php;
+                    cm = pm;
+                    opq = p_opq;
+                    nconst = p_nconst;
+                } else {
+                    n_cacc++;
+                    const int u = ph5 - 1, nw = min(4, a.steps - (mcmci - u));
+                    hc = shfl_all((u & 2) ? pc[1] : pc[0], (u & 1) * 32 + slot);
+                    if (!live) hc = 0.0f;
+                    r_const_back(hc, bt, bt0);
+                    if (u + 1 < nw) {
+                        // backward terms and sums of the steps that are left
+                        r_lds_order();
+#pragma unroll
+                        for (int p = 0; p < 2; p++)
+                            if (2 * p + half > u) S[(8 + 2 * p + half) * R_ROW + slot] = pc[p] == 0.0f ? bt0 : bt;
+                        r_lds_order();
+                        if (l == 0) {
+                            double back = backward;
+                            for (int v = u + 1; v < nw; v++) R[8 + v] = back = r_add_row(S + (8 + v) * R_ROW, back);
+                        }
+                        r_lds_order();
+                        if (l < 12) sums = R[l];
+                    }
+                }
             }
         }
         n_steps += (unsigned long long)a.steps;
-        if (live) { a.ops[(size_t)l * N + chain] = (uint8_t)hop; a.cs[(size_t)l * N + chain] = hc; }
+        if (l < GPR_REF_SLOTS) { a.ops[(size_t)l * N + chain] = (uint8_t)hop; a.cs[(size_t)l * N + chain] = hc; }
         if (l == 0) { a.prior[chain] = cur_prior; a.ll[chain] = cur_ll; }
     }
     if (l == 0 && a.counters) {
@@ -636,9 +840,10 @@ k_mh_ref_wave(GprMHArgs a) {
 
 hipError_t gpr_launch_mh_ref_wave(const GprMHArgs &a, int kc, int grid, hipStream_t s) {
     const dim3 wg(64 * a.wpg);
-    if (kc == 1) hipLaunchKernelGGL((k_mh_ref_wave<1>), dim3(grid), wg, 0, s, a);
-    else if (kc == 2) hipLaunchKernelGGL((k_mh_ref_wave<2>), dim3(grid), wg, 0, s, a);
-    else hipLaunchKernelGGL((k_mh_ref_wave<4>), dim3(grid), wg, 0, s, a);
+    const size_t sh = sizeof(float) * r_lds_floats(kc) * (size_t)a.wpg;
+    if (kc == 1) hipLaunchKernelGGL((k_mh_ref_wave<1>), dim3(grid), wg, sh, s, a);
+    else if (kc == 2) hipLaunchKernelGGL((k_mh_ref_wave<2>), dim3(grid), wg, sh, s, a);
+    else hipLaunchKernelGGL((k_mh_ref_wave<4>), dim3(grid), wg, sh, s, a);
     return hipGetLastError();
 }
 
