@@ -173,118 +173,10 @@ struct WaveProg {
     int len;
 };
 
-// Per-lane value stack: KC vector values of GPR_MAX_DEPTH floats.  Element access
-// with the uniform stack pointer lowers to s_set_gpr_idx moves; nothing goes through
-// an alloca, so nothing is spilled to scratch.
-typedef float gpr_f16v __attribute__((ext_vector_type(GPR_MAX_DEPTH)));
-template <int KC>
-struct VStack {
-    gpr_f16v s0, s1, s2, s3;
-    __device__ __forceinline__ float get(int k, int i) const {
-        return k == 0 ? s0[i] : (k == 1 ? s1[i] : (k == 2 ? s2[i] : s3[i]));
-    }
-    __device__ __forceinline__ void put(int k, int i, float v) {
-        if (k == 0) s0[i] = v; else if (k == 1) s1[i] = v; else if (k == 2) s2[i] = v; else s3[i] = v;
-    }
-};
-
 #define GPR_KLOOP(expr)                              \
     do {                                             \
         _Pragma("unroll") for (int k = 0; k < KC; k++) T[k] = (expr); \
     } while (0)
-
-// Interpret the tape at KC points per lane.  op is wave-uniform: every branch below is
-// a scalar branch and only the selected operation executes.  Taken branches cost far
-// more than VALU work here, so the two common token classes take one branch each and
-// no nested switch: leaves (x, constant, one) select their value, and +, -, * compute
-// a + s*b (s = +-1, exact, so one rounding like a +- b) or a*b and select.  Every other
-// op goes through the full switch.
-template <int KC, bool HI>
-__device__ __forceinline__ void wave_eval(const WaveProg &p, const float (&xs)[KC], float (&T)[KC]) {
-    VStack<KC> S;
-    int sp = 0;
-#pragma unroll
-    for (int k = 0; k < KC; k++) T[k] = 0.0f;
-    for (int t = 0; t < p.len; t++) {
-        const int l = t & 63;
-        const bool h = HI && t >= 64;
-        const int op = h ? rl_i(p.o1, l) : rl_i(p.o0, l);
-        if (op <= GPR_OP_ONE) {
-            // the write index is bounded for malformed tapes; valid ones (depth <= 16) never hit it
-            const int wi = min(sp, GPR_MAX_DEPTH - 1);
-#pragma unroll
-            for (int k = 0; k < KC; k++) S.put(k, wi, T[k]);
-            sp = min(sp + 1, GPR_MAX_DEPTH);
-            const float cv = h ? rl_f(p.c1, l) : rl_f(p.c0, l);
-            const float sv = op == GPR_OP_CONST ? cv : 1.0f;
-            const bool isx = op == GPR_OP_X;
-            GPR_KLOOP(isx ? xs[k] : sv);
-        } else if (op <= GPR_OP_MUL) {
-            sp = max(sp - 1, 0);
-            const bool mul = op == GPR_OP_MUL;
-            const float sgn = op == GPR_OP_SUB ? -1.0f : 1.0f;
-#pragma unroll
-            for (int k = 0; k < KC; k++) {
-                const float a = S.get(k, sp);
-                const float pm = __builtin_fmaf(sgn, T[k], a);
-                const float pr = a * T[k];
-                T[k] = mul ? pr : pm;
-            }
-        } else if (op <= GPR_OP_RPOW) {
-            sp = max(sp - 1, 0);
-            switch (op) {
-            case GPR_OP_DIV: GPR_KLOOP(S.get(k, sp) / T[k]); break;
-            case GPR_OP_RSUB: GPR_KLOOP(T[k] - S.get(k, sp)); break;
-            case GPR_OP_RDIV: GPR_KLOOP(T[k] / S.get(k, sp)); break;
-            case GPR_OP_POW: GPR_KLOOP(powf(S.get(k, sp), T[k])); break;
-            default: GPR_KLOOP(powf(T[k], S.get(k, sp))); break;
-            }
-        } else {
-            const float c = op >= GPR_OP_CADD ? (h ? rl_f(p.c1, l) : rl_f(p.c0, l)) : 0.0f;
-            switch (op) {
-            case GPR_OP_NEG: GPR_KLOOP(-T[k]); break;
-            case GPR_OP_EXP: GPR_KLOOP(expf(T[k])); break;
-            case GPR_OP_LOG: GPR_KLOOP(logf(T[k])); break;
-            case GPR_OP_INV: GPR_KLOOP(1.0f / T[k]); break;
-            case GPR_OP_SQRT: GPR_KLOOP(sqrtf(T[k])); break;
-            case GPR_OP_SIN: GPR_KLOOP(sinf(T[k])); break;
-            case GPR_OP_ASIN: GPR_KLOOP(asinf(T[k])); break;
-            case GPR_OP_COS: GPR_KLOOP(cosf(T[k])); break;
-            case GPR_OP_ACOS: GPR_KLOOP(acosf(T[k])); break;
-            case GPR_OP_TAN: GPR_KLOOP(tanf(T[k])); break;
-            case GPR_OP_ATAN: GPR_KLOOP(atanf(T[k])); break;
-            case GPR_OP_ABS: GPR_KLOOP(fabsf(T[k])); break;
-            case GPR_OP_CADD: GPR_KLOOP(T[k] + c); break;
-            case GPR_OP_CMUL: GPR_KLOOP(c * T[k]); break;
-            case GPR_OP_CPOW: GPR_KLOOP(powf(T[k], c)); break;
-            case GPR_OP_CRPOW: GPR_KLOOP(powf(c, T[k])); break;
-            default: GPR_KLOOP(__builtin_nanf("")); break;
-            }
-        }
-    }
-}
-
-// The same interpreter with the value stack in LDS: the top two entries stay in VGPRs
-// (T, U) and the rest live in this wave's slab ls[level][lane][KC] (GPR_MAX_DEPTH + 2
-// levels; levels 0 and 1 take the stores and loads of an empty U, so the pushes and
-// pops need no test).  A push spills U to the slab, a binary op refills U from it; both
-// are one 16-byte LDS access per lane at KC = 4.  Saves the 16*KC VGPRs of the indexed
-// stack (occupancy) and the indexing-mode switches.  Same operations on the same
-// operands as wave_eval, so the values are bit-identical.  The tape must be well formed
-// with stack depth at most GPR_MAX_DEPTH: the sampler's programs are (init, proposals
-// and gpr_write_state check it), and the stack pointer is not clamped.
-template <int KC>
-__device__ __forceinline__ void ls_store(float *q, const float (&v)[KC]) {
-    if (KC == 4) *(float4 *)q = make_float4(v[0], v[1], v[2], v[3]);
-    else if (KC == 2) *(float2 *)q = make_float2(v[0], v[KC > 1 ? 1 : 0]);
-    else q[0] = v[0];
-}
-template <int KC>
-__device__ __forceinline__ void ls_load(const float *q, float (&v)[KC]) {
-    if (KC == 4) { const float4 f = *(const float4 *)q; v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w; }
-    else if (KC == 2) { const float2 f = *(const float2 *)q; v[0] = f.x; v[KC > 1 ? 1 : 0] = f.y; }
-    else v[0] = q[0];
-}
 
 // Token classes as wave-uniform bit masks (bit t of the low word, bit t-64 of the high
 // word): the common classes dispatch on a scalar bit test, with no vector-to-scalar
@@ -310,127 +202,251 @@ __device__ __forceinline__ OpMasks op_masks(const WaveProg &p) {
     return m;
 }
 
+// ---------------------------------------------------------------- wave interpreter
+// The tape is interpreted once per chunk of points; the program is wave-uniform, so every
+// token is one scalar dispatch for all 64 lanes.  That dispatch is what bounds the sampler
+// (the scalar unit, which the four SIMDs of a CU share): tests of token-class masks, as the
+// compiler lays them out, took some 22 scalar instructions and 8 branches a token.  Here
+// the hot tokens (x, constant, + - * with a leaf or a stack operand, negation) are handlers
+// of equal size in one asm block, and a token's word, held in its lane like the token itself
+// (prog_code), is the byte offset of its handler: a dispatch is one v_readlane, an add with
+// carry and s_setpc, and a handler ends in the dispatch of the next token.  A leaf followed
+// by +, - or * is one handler.  Division, powers and library functions (and the last lane's
+// token) leave the block; the caller runs them and enters again at the next token.
+//
+// The value stack's top two entries stay in VGPRs (T, U) and the rest live in this wave's
+// LDS slab, [level][k][lane] with GPR_MAX_DEPTH + 2 levels for any program; levels 0 and 1
+// take the stores and loads of an empty U, so pushes and pops need no test.  p is this
+// lane's LDS address of the level that the next push stores U to.  The tape must be well
+// formed with stack depth at most GPR_MAX_DEPTH: the sampler's programs are (init,
+// proposals and gpr_write_state check it).
+//
+// Against the mask tests, whole runs with their set-up and state copies: random walk,
+// 131072 chains at n = 250 and cap 64, 150.5 -> 123.0 ms; 48 uneven datasets of 2048 chains,
+// 47.1 -> 41.3 ms; MALA, whose gradients have interpreters of their own, 107.8 -> 103.0 ms.
+enum {
+    GPR_U_EXIT = 0, GPR_U_X, GPR_U_C, GPR_U_XADD, GPR_U_XSUB, GPR_U_XMUL, GPR_U_CADD, GPR_U_CSUB, GPR_U_CMUL, GPR_U_ADD,
+    GPR_U_SUB, GPR_U_MUL, GPR_U_NEG
+};
+// Handler words of a half tape: lane l holds token l's.  Lanes past the program, and lane
+// 63 (whose successor the block could not read), hold the exit; so does every token
+// without a handler.  Tokens advance by one, or two for a leaf fused with lane l + 1 <= 62,
+// so the block always reaches an exit.
+template <int KC>
+__device__ __forceinline__ int half_code(int o, int n) {
+    const int l = lane_id();
+    const int nx = shfl_all(o, l + 1);
+    const bool leaf = o <= GPR_OP_CONST, cheap = o >= GPR_OP_ADD && o <= GPR_OP_MUL;
+    const bool fuse = l + 1 < min(n, 63) && nx >= GPR_OP_ADD && nx <= GPR_OP_MUL;
+    int u = leaf ? (fuse ? GPR_U_XADD + 3 * o + (nx - GPR_OP_ADD) : GPR_U_X + o)
+                 : (cheap ? GPR_U_ADD + (o - GPR_OP_ADD) : (o == GPR_OP_NEG ? GPR_U_NEG : GPR_U_EXIT));
+    u = l < min(n, 63) ? u : GPR_U_EXIT;
+    return u << (KC == 1 ? 6 : 7);
+}
+static_assert(GPR_OP_X == 0 && GPR_OP_CONST == 1 && GPR_OP_SUB == GPR_OP_ADD + 1 && GPR_OP_MUL == GPR_OP_ADD + 2,
+              "half_code's arithmetic on op codes");
+struct ProgCode {
+    int w0, w1;
+};
+template <int KC, bool HI>
+__device__ __forceinline__ ProgCode prog_code(const WaveProg &p) {
+    ProgCode c;
+    c.w0 = half_code<KC>(p.o0, p.len);
+    c.w1 = 0;
+    if (HI && p.len > 64) c.w1 = half_code<KC>(p.o1, p.len - 64);
+    return c;
+}
+
+// LDS by byte address, as the asm blocks use it
+typedef __attribute__((address_space(3))) float *gpr_lds_f;
+__device__ __forceinline__ uint32_t lds_addr(const float *q) {
+    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const float *)q;
+}
+__device__ __forceinline__ float lds_ld(uint32_t a) { return *(gpr_lds_f)(uintptr_t)a; }
+__device__ __forceinline__ void lds_st(uint32_t a, float v) { *(gpr_lds_f)(uintptr_t)a = v; }
+
+// Pieces of the handlers.  GT_NEXT reads the next token's word early; GT_JUMP adds it to
+// the handlers' base.  Wait states (the compiler does not look into the block): a lane read
+// into a scalar register and its use by a vector instruction are two instructions apart; a
+// vector register written by the vector unit is read by v_readlane only after others
+// (nothing in the block writes the word and constant registers, and the entry runs four
+// scalar instructions first).  Every LDS load is waited for before its register is used,
+// and before the block ends.
+#define GT_NEXT(N) "s_add_i32 %[t], %[t], " #N "\n\tv_readlane_b32 %[w], %[word], %[t]\n\t"
+#define GT_JUMP "s_add_u32 vcc_lo, %[blo], %[w]\n\ts_addc_u32 vcc_hi, %[bhi], 0\n\ts_setpc_b64 vcc\n\t"
+#define GT_CONST "v_readlane_b32 %[s], %[c], %[t]\n\t"
+#define GT_WAIT "s_waitcnt lgkmcnt(0)\n\t"
+// entry: the base of the handlers, then the dispatch of token t
+#define GT_ENTRY                                                                            \
+    "s_getpc_b64 vcc\n.Lp%=:\n\t"                                                           \
+    "s_add_u32 %[blo], vcc_lo, .Lh%=-.Lp%=\n\t"                                             \
+    "s_addc_u32 %[bhi], vcc_hi, 0\n\t"                                                      \
+    "v_readlane_b32 %[w], %[word], %[t]\n\t" GT_JUMP
+#define GT_EXIT GT_WAIT "s_branch .Lx%=\n\t"
+
+#define GT1(OP, A, B) OP " %[T0], " A ", " B "\n\t"
+#define GT1_PUSH GT_WAIT "ds_write_b32 %[p], %[U0]\n\tv_add_u32 %[p], 0x100, %[p]\n\tv_mov_b32 %[U0], %[T0]\n\t"
+#define GT1_POP "v_add_u32 %[p], 0xffffff00, %[p]\n\tds_read_b32 %[U0], %[p]\n\t"
+// one point per lane, handlers of 64 bytes
+__device__ __forceinline__ void tape_run(int word, float c, const float (&x)[1], float (&T)[1], float (&U)[1], uint32_t &p,
+                                         int &t) {
+    uint32_t blo, bhi, w, s;
+#define GT_H(BODY) ".p2align 6\n\t" BODY
+    __asm__ volatile(
+        GT_ENTRY
+        ".p2align 6\n.Lh%=:\n\t" GT_EXIT
+        GT_H(GT_NEXT(1) GT1_PUSH "v_mov_b32 %[T0], %[x0]\n\t" GT_JUMP)
+        GT_H(GT_CONST GT_NEXT(1) GT1_PUSH "v_mov_b32 %[T0], %[s]\n\t" GT_JUMP)
+        GT_H(GT_NEXT(2) GT1("v_add_f32", "%[x0]", "%[T0]") GT_JUMP)
+        GT_H(GT_NEXT(2) GT1("v_sub_f32", "%[T0]", "%[x0]") GT_JUMP)
+        GT_H(GT_NEXT(2) GT1("v_mul_f32", "%[x0]", "%[T0]") GT_JUMP)
+        GT_H(GT_CONST GT_NEXT(2) GT1("v_add_f32", "%[s]", "%[T0]") GT_JUMP)
+        GT_H(GT_CONST GT_NEXT(2) GT1("v_subrev_f32", "%[s]", "%[T0]") GT_JUMP)
+        GT_H(GT_CONST GT_NEXT(2) GT1("v_mul_f32", "%[s]", "%[T0]") GT_JUMP)
+        GT_H(GT_NEXT(1) GT_WAIT GT1("v_add_f32", "%[U0]", "%[T0]") GT1_POP GT_JUMP)
+        GT_H(GT_NEXT(1) GT_WAIT GT1("v_sub_f32", "%[U0]", "%[T0]") GT1_POP GT_JUMP)
+        GT_H(GT_NEXT(1) GT_WAIT GT1("v_mul_f32", "%[U0]", "%[T0]") GT1_POP GT_JUMP)
+        GT_H(GT_NEXT(1) "v_xor_b32 %[T0], 0x80000000, %[T0]\n\t" GT_JUMP)
+        ".Lx%=:"
+        : [T0] "+&v"(T[0]), [U0] "+&v"(U[0]), [p] "+&v"(p), [t] "+&s"(t), [blo] "=&s"(blo), [bhi] "=&s"(bhi), [w] "=&s"(w),
+          [s] "=&s"(s)
+        : [word] "v"(word), [c] "v"(c), [x0] "v"(x[0])
+        : "vcc", "scc", "memory");
+#undef GT_H
+}
+
+#define GT_H(BODY) ".p2align 7\n\t" BODY
+#define GT2(OP, A, B) OP " %[T0], " A(0) ", " B(0) "\n\t" OP " %[T1], " A(1) ", " B(1) "\n\t"
+#define GT4(OP, A, B) GT2(OP, A, B) OP " %[T2], " A(2) ", " B(2) "\n\t" OP " %[T3], " A(3) ", " B(3) "\n\t"
+#define GT_T(k) "%[T" #k "]"
+#define GT_U(k) "%[U" #k "]"
+#define GT_X(k) "%[x" #k "]"
+#define GT_S(k) "%[s]"
+#define GT_NEGMASK(k) "0x80000000"
+#define GT2_MOV(D, S) "v_mov_b32 " D(0) ", " S(0) "\n\tv_mov_b32 " D(1) ", " S(1) "\n\t"
+#define GT4_MOV(D, S) GT2_MOV(D, S) "v_mov_b32 " D(2) ", " S(2) "\n\tv_mov_b32 " D(3) ", " S(3) "\n\t"
+#define GT2_PUSH GT_WAIT "ds_write2_b32 %[p], %[U0], %[U1] offset1:64\n\tv_add_u32 %[p], 0x200, %[p]\n\t" GT2_MOV(GT_U, GT_T)
+#define GT2_POP "v_add_u32 %[p], 0xfffffe00, %[p]\n\tds_read_b32 %[U0], %[p]\n\tds_read_b32 %[U1], %[p] offset:256\n\t"
+#define GT4_PUSH                                                                                             \
+    GT_WAIT "ds_write2_b32 %[p], %[U0], %[U1] offset1:64\n\tds_write2_b32 %[p], %[U2], %[U3] offset0:128 offset1:192\n\t" \
+            "v_add_u32 %[p], 0x400, %[p]\n\t" GT4_MOV(GT_U, GT_T)
+#define GT4_POP                                                                                              \
+    "v_add_u32 %[p], 0xfffffc00, %[p]\n\tds_read_b32 %[U0], %[p]\n\tds_read_b32 %[U1], %[p] offset:256\n\t"     \
+    "ds_read_b32 %[U2], %[p] offset:512\n\tds_read_b32 %[U3], %[p] offset:768\n\t"
+// several points per lane, handlers of 128 bytes
+#define GT_TABLE(GT, MOV, PUSH, POP)                                             \
+    GT_ENTRY                                                                     \
+    ".p2align 7\n.Lh%=:\n\t" GT_EXIT                                             \
+    GT_H(GT_NEXT(1) PUSH MOV(GT_T, GT_X) GT_JUMP)                                \
+    GT_H(GT_CONST GT_NEXT(1) PUSH MOV(GT_T, GT_S) GT_JUMP)                       \
+    GT_H(GT_NEXT(2) GT("v_add_f32", GT_X, GT_T) GT_JUMP)                         \
+    GT_H(GT_NEXT(2) GT("v_sub_f32", GT_T, GT_X) GT_JUMP)                         \
+    GT_H(GT_NEXT(2) GT("v_mul_f32", GT_X, GT_T) GT_JUMP)                         \
+    GT_H(GT_CONST GT_NEXT(2) GT("v_add_f32", GT_S, GT_T) GT_JUMP)                \
+    GT_H(GT_CONST GT_NEXT(2) GT("v_subrev_f32", GT_S, GT_T) GT_JUMP)             \
+    GT_H(GT_CONST GT_NEXT(2) GT("v_mul_f32", GT_S, GT_T) GT_JUMP)                \
+    GT_H(GT_NEXT(1) GT_WAIT GT("v_add_f32", GT_U, GT_T) POP GT_JUMP)             \
+    GT_H(GT_NEXT(1) GT_WAIT GT("v_sub_f32", GT_U, GT_T) POP GT_JUMP)             \
+    GT_H(GT_NEXT(1) GT_WAIT GT("v_mul_f32", GT_U, GT_T) POP GT_JUMP)             \
+    GT_H(GT_NEXT(1) GT("v_xor_b32", GT_NEGMASK, GT_T) GT_JUMP)                   \
+    ".Lx%=:"
+__device__ __forceinline__ void tape_run(int word, float c, const float (&x)[2], float (&T)[2], float (&U)[2], uint32_t &p,
+                                         int &t) {
+    uint32_t blo, bhi, w, s;
+    __asm__ volatile(GT_TABLE(GT2, GT2_MOV, GT2_PUSH, GT2_POP)
+                     : [T0] "+&v"(T[0]), [T1] "+&v"(T[1]), [U0] "+&v"(U[0]), [U1] "+&v"(U[1]), [p] "+&v"(p), [t] "+&s"(t),
+                       [blo] "=&s"(blo), [bhi] "=&s"(bhi), [w] "=&s"(w), [s] "=&s"(s)
+                     : [word] "v"(word), [c] "v"(c), [x0] "v"(x[0]), [x1] "v"(x[1])
+                     : "vcc", "scc", "memory");
+}
+__device__ __forceinline__ void tape_run(int word, float c, const float (&x)[4], float (&T)[4], float (&U)[4], uint32_t &p,
+                                         int &t) {
+    uint32_t blo, bhi, w, s;
+    __asm__ volatile(GT_TABLE(GT4, GT4_MOV, GT4_PUSH, GT4_POP)
+                     : [T0] "+&v"(T[0]), [T1] "+&v"(T[1]), [T2] "+&v"(T[2]), [T3] "+&v"(T[3]), [U0] "+&v"(U[0]),
+                       [U1] "+&v"(U[1]), [U2] "+&v"(U[2]), [U3] "+&v"(U[3]), [p] "+&v"(p), [t] "+&s"(t), [blo] "=&s"(blo),
+                       [bhi] "=&s"(bhi), [w] "=&s"(w), [s] "=&s"(s)
+                     : [word] "v"(word), [c] "v"(c), [x0] "v"(x[0]), [x1] "v"(x[1]), [x2] "v"(x[2]), [x3] "v"(x[3])
+                     : "vcc", "scc", "memory");
+}
+#undef GT_H
+
+// One token outside the block (any op: the last lane's token may be a cheap one).
+template <int KC>
+__device__ __forceinline__ void tape_slow(int op, float c, const float (&xs)[KC], float (&T)[KC], float (&U)[KC],
+                                          uint32_t &p) {
+    if (op <= GPR_OP_ONE) {
+#pragma unroll
+        for (int k = 0; k < KC; k++) { lds_st(p + 256 * k, U[k]); U[k] = T[k]; }
+        p += 256 * KC;
+        const float sv = op == GPR_OP_CONST ? c : 1.0f;
+        const bool isx = op == GPR_OP_X;
+        GPR_KLOOP(isx ? xs[k] : sv);
+    } else if (op <= GPR_OP_RPOW) {
+        if (op <= GPR_OP_MUL) {
+            const bool mul = op == GPR_OP_MUL;
+            const float sgn = op == GPR_OP_SUB ? -1.0f : 1.0f;
+#pragma unroll
+            for (int k = 0; k < KC; k++) {
+                const float pm = __builtin_fmaf(sgn, T[k], U[k]);
+                const float pr = U[k] * T[k];
+                T[k] = mul ? pr : pm;
+            }
+        } else {
+            switch (op) {
+            case GPR_OP_DIV: GPR_KLOOP(U[k] / T[k]); break;
+            case GPR_OP_RSUB: GPR_KLOOP(T[k] - U[k]); break;
+            case GPR_OP_RDIV: GPR_KLOOP(T[k] / U[k]); break;
+            case GPR_OP_POW: GPR_KLOOP(powf(U[k], T[k])); break;
+            default: GPR_KLOOP(powf(T[k], U[k])); break;
+            }
+        }
+        p -= 256 * KC;
+#pragma unroll
+        for (int k = 0; k < KC; k++) U[k] = lds_ld(p + 256 * k);   // the new second entry
+    } else {
+        switch (op) {
+        case GPR_OP_NEG: GPR_KLOOP(-T[k]); break;
+        case GPR_OP_EXP: GPR_KLOOP(expf(T[k])); break;
+        case GPR_OP_LOG: GPR_KLOOP(logf(T[k])); break;
+        case GPR_OP_INV: GPR_KLOOP(1.0f / T[k]); break;
+        case GPR_OP_SQRT: GPR_KLOOP(sqrtf(T[k])); break;
+        case GPR_OP_SIN: GPR_KLOOP(sinf(T[k])); break;
+        case GPR_OP_ASIN: GPR_KLOOP(asinf(T[k])); break;
+        case GPR_OP_COS: GPR_KLOOP(cosf(T[k])); break;
+        case GPR_OP_ACOS: GPR_KLOOP(acosf(T[k])); break;
+        case GPR_OP_TAN: GPR_KLOOP(tanf(T[k])); break;
+        case GPR_OP_ATAN: GPR_KLOOP(atanf(T[k])); break;
+        case GPR_OP_ABS: GPR_KLOOP(fabsf(T[k])); break;
+        case GPR_OP_CADD: GPR_KLOOP(T[k] + c); break;
+        case GPR_OP_CMUL: GPR_KLOOP(c * T[k]); break;
+        case GPR_OP_CPOW: GPR_KLOOP(powf(T[k], c)); break;
+        case GPR_OP_CRPOW: GPR_KLOOP(powf(c, T[k])); break;
+        default: GPR_KLOOP(__builtin_nanf("")); break;
+        }
+    }
+}
+
+// Values of the tape at KC points per lane.  ls: this wave's slab, levels of 64 * KC floats.
 template <int KC, bool HI>
 __device__ __forceinline__ void wave_eval_ls(const WaveProg &p, const float (&xs)[KC], float (&T)[KC], float *ls,
-                                             const OpMasks &m) {
+                                             const ProgCode &m) {
     float U[KC];
-    float *lane = ls + 2 * 64 * KC + lane_id() * KC;   // level -2 of the stack below T, U
-    int sp = 0;   // entries on the stack, T and U included
+    uint32_t a = lds_addr(ls) + 4u * (uint32_t)lane_id();   // level -2 of the stack below T, U
 #pragma unroll
     for (int k = 0; k < KC; k++) { T[k] = 0.0f; U[k] = 0.0f; }
-    for (int t = 0; t < p.len; t++) {
-        const int l = t & 63;
-        const int h = (HI && t >= 64) ? 1 : 0;
-        const uint64_t bit = 1ull << l;
-        // a leaf followed by +, - or * within the same half: push and pop cancel, so
-        // T = T op leaf with the stack untouched (the same operation on the same operands)
-        if (m.leaf[h] & (m.cheap[h] >> 1) & bit) {
-            // the leaf and the op are wave-uniform: scalar branches pick one vector
-            // instruction per point (the same operation on the same operands)
-            if (m.x[h] & bit) {
-                if ((m.mul[h] >> 1) & bit) {
-#pragma unroll
-                    for (int k = 0; k < KC; k++) T[k] = T[k] * xs[k];
-                } else if ((m.sub[h] >> 1) & bit) {
-#pragma unroll
-                    for (int k = 0; k < KC; k++) T[k] = __builtin_fmaf(-1.0f, xs[k], T[k]);
-                } else {
-#pragma unroll
-                    for (int k = 0; k < KC; k++) T[k] = __builtin_fmaf(1.0f, xs[k], T[k]);
-                }
-            } else {
-                const float cv = h ? rl_f(p.c1, l) : rl_f(p.c0, l);
-                if ((m.mul[h] >> 1) & bit) {
-#pragma unroll
-                    for (int k = 0; k < KC; k++) T[k] = T[k] * cv;
-                } else if ((m.sub[h] >> 1) & bit) {
-#pragma unroll
-                    for (int k = 0; k < KC; k++) T[k] = __builtin_fmaf(-1.0f, cv, T[k]);
-                } else {
-#pragma unroll
-                    for (int k = 0; k < KC; k++) T[k] = __builtin_fmaf(1.0f, cv, T[k]);
-                }
-            }
-            t++;
-            continue;
-        }
-        if (m.leaf[h] & bit) {
-            // level sp-2 receives U (an unused level while U is empty)
-            ls_store<KC>(lane + (sp - 2) * 64 * KC, U);
-#pragma unroll
-            for (int k = 0; k < KC; k++) U[k] = T[k];
-            sp++;
-            const float cv = h ? rl_f(p.c1, l) : rl_f(p.c0, l);
-            const bool isx = (m.x[h] & bit) != 0;
-            GPR_KLOOP(isx ? xs[k] : cv);
-        } else if (m.cheap[h] & bit) {
-            if (m.mul[h] & bit) {
-#pragma unroll
-                for (int k = 0; k < KC; k++) T[k] = U[k] * T[k];
-            } else if (m.sub[h] & bit) {
-#pragma unroll
-                for (int k = 0; k < KC; k++) T[k] = __builtin_fmaf(-1.0f, T[k], U[k]);
-            } else {
-#pragma unroll
-                for (int k = 0; k < KC; k++) T[k] = __builtin_fmaf(1.0f, T[k], U[k]);
-            }
-            ls_load<KC>(lane + (sp - 3) * 64 * KC, U);   // the new second entry (level sp-3)
-            sp--;
-            continue;
-        } else {
-        const int op = h ? rl_i(p.o1, l) : rl_i(p.o0, l);
-        if (op <= GPR_OP_ONE) {
-            ls_store<KC>(lane + (sp - 2) * 64 * KC, U);
-#pragma unroll
-            for (int k = 0; k < KC; k++) U[k] = T[k];
-            sp++;
-            const float cv = h ? rl_f(p.c1, l) : rl_f(p.c0, l);
-            const float sv = op == GPR_OP_CONST ? cv : 1.0f;
-            const bool isx = op == GPR_OP_X;
-            GPR_KLOOP(isx ? xs[k] : sv);
-        } else if (op <= GPR_OP_RPOW) {
-            if (op <= GPR_OP_MUL) {
-                const bool mul = op == GPR_OP_MUL;
-                const float sgn = op == GPR_OP_SUB ? -1.0f : 1.0f;
-#pragma unroll
-                for (int k = 0; k < KC; k++) {
-                    const float pm = __builtin_fmaf(sgn, T[k], U[k]);
-                    const float pr = U[k] * T[k];
-                    T[k] = mul ? pr : pm;
-                }
-            } else {
-                switch (op) {
-                case GPR_OP_DIV: GPR_KLOOP(U[k] / T[k]); break;
-                case GPR_OP_RSUB: GPR_KLOOP(T[k] - U[k]); break;
-                case GPR_OP_RDIV: GPR_KLOOP(T[k] / U[k]); break;
-                case GPR_OP_POW: GPR_KLOOP(powf(U[k], T[k])); break;
-                default: GPR_KLOOP(powf(T[k], U[k])); break;
-                }
-            }
-            ls_load<KC>(lane + (sp - 3) * 64 * KC, U);   // the new second entry (level sp-3)
-            sp--;
-        } else {
-            const float c = op >= GPR_OP_CADD ? (h ? rl_f(p.c1, l) : rl_f(p.c0, l)) : 0.0f;
-            switch (op) {
-            case GPR_OP_NEG: GPR_KLOOP(-T[k]); break;
-            case GPR_OP_EXP: GPR_KLOOP(expf(T[k])); break;
-            case GPR_OP_LOG: GPR_KLOOP(logf(T[k])); break;
-            case GPR_OP_INV: GPR_KLOOP(1.0f / T[k]); break;
-            case GPR_OP_SQRT: GPR_KLOOP(sqrtf(T[k])); break;
-            case GPR_OP_SIN: GPR_KLOOP(sinf(T[k])); break;
-            case GPR_OP_ASIN: GPR_KLOOP(asinf(T[k])); break;
-            case GPR_OP_COS: GPR_KLOOP(cosf(T[k])); break;
-            case GPR_OP_ACOS: GPR_KLOOP(acosf(T[k])); break;
-            case GPR_OP_TAN: GPR_KLOOP(tanf(T[k])); break;
-            case GPR_OP_ATAN: GPR_KLOOP(atanf(T[k])); break;
-            case GPR_OP_ABS: GPR_KLOOP(fabsf(T[k])); break;
-            case GPR_OP_CADD: GPR_KLOOP(T[k] + c); break;
-            case GPR_OP_CMUL: GPR_KLOOP(c * T[k]); break;
-            case GPR_OP_CPOW: GPR_KLOOP(powf(T[k], c)); break;
-            case GPR_OP_CRPOW: GPR_KLOOP(powf(c, T[k])); break;
-            default: GPR_KLOOP(__builtin_nanf("")); break;
-            }
-        }
+    // one copy of the block and of the slow path for both halves of the tape
+#pragma unroll 1
+    for (int h = 0; h == 0 || (HI && 64 * h < p.len); h++) {
+        // (uni: wave-uniform in any case, but the block needs it in a scalar register)
+        const int n = uni(min(p.len - 64 * h, 64)), word = HI && h ? m.w1 : m.w0, o = HI && h ? p.o1 : p.o0;
+        const float c = HI && h ? p.c1 : p.c0;
+        for (int t = 0; t < n; t++) {
+            t = uni(t);
+            tape_run(word, c, xs, T, U, a, t);
+            t = uni(t);
+            if (t >= n) break;
+            tape_slow<KC>(rl_i(o, t), rl_f(c, t), xs, T, U, a);
         }
     }
 }
@@ -454,8 +470,7 @@ struct Chunk {
 
 // Gaussian log-likelihood of the wave's program: lconst - sum_i (f_i - y_i)^2 w_i.
 // Per-lane Kahan sums, wave tree reduction; -inf if any term is not finite.
-// LS: the value stack in LDS, ls = this wave's slab of (GPR_MAX_DEPTH + 2) * 64 * KC floats,
-// pm = the program's token-class masks; else the VGPR stack.
+// ls: this wave's value-stack slab, pc: the program's handler words for KC points per lane.
 // reject_below: the caller rejects the proposal whenever the LL lies below this value.
 // Every term of the sum is >= 0, so after each chunk but the last the sum so far bounds
 // the LL from above; when that bound (with a relative margin of 1e-4 on the partial sum,
@@ -520,10 +535,10 @@ __device__ __forceinline__ bool batch_ok(const WaveProg &p, int mk) {
     return __popcll(m) <= 16 && ballot(l < p.len && gpr_has_const(p.o0)) == m;
 }
 
-template <int KC, bool HI, bool LS = false>
+template <int KC, bool HI>
 __device__ __forceinline__ double wave_loglik(const WaveProg &p, const GprDataset &d, const float *dx, const float *dy,
-                              const float *dw, const Chunk<KC> &c0, int nchunks, float *ls = nullptr,
-                              const OpMasks *pm = nullptr, double reject_below = -GPR_INF, int *points = nullptr) {
+                              const float *dw, const Chunk<KC> &c0, int nchunks, float *ls, const ProgCode &pc,
+                              double reject_below = -GPR_INF, int *points = nullptr) {
     float acc = 0.0f, comp = 0.0f;
     const int l = lane_id();
     if (points) *points = d.n;
@@ -531,8 +546,7 @@ __device__ __forceinline__ double wave_loglik(const WaveProg &p, const GprDatase
         Chunk<KC> c;
         if (ch == 0) c = c0; else c.load(dx, dy, dw, d.n, ch * 64 * KC);
         float T[KC];
-        if (LS) wave_eval_ls<KC, HI>(p, c.x, T, ls, *pm);
-        else wave_eval<KC, HI>(p, c.x, T);
+        wave_eval_ls<KC, HI>(p, c.x, T, ls, pc);
 #pragma unroll
         for (int k = 0; k < KC; k++) {
             const float r = T[k] - c.y[k];
@@ -598,6 +612,17 @@ __device__ __forceinline__ double wave_loglik(const WaveProg &p, const GprDatase
     (GPR_DUAL_PACKED_FLOATS > GPR_DUAL_SPLIT_FLOATS                                      \
          ? (GPR_DUAL_PACKED_FLOATS > GPR_DUAL_SPLIT6_FLOATS ? GPR_DUAL_PACKED_FLOATS : GPR_DUAL_SPLIT6_FLOATS) \
          : (GPR_DUAL_SPLIT_FLOATS > GPR_DUAL_SPLIT6_FLOATS ? GPR_DUAL_SPLIT_FLOATS : GPR_DUAL_SPLIT6_FLOATS))
+
+template <int N>
+__device__ __forceinline__ void ls_store(float *q, const float (&v)[N]) {
+    if constexpr (N == 4) *(float4 *)q = make_float4(v[0], v[1], v[2], v[3]);
+    else *(float2 *)q = make_float2(v[0], v[1]);
+}
+template <int N>
+__device__ __forceinline__ void ls_load(const float *q, float (&v)[N]) {
+    if constexpr (N == 4) { const float4 f = *(const float4 *)q; v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w; }
+    else { const float2 f = *(const float2 *)q; v[0] = f.x; v[1] = f.y; }
+}
 
 // One stack entry of the dual stack at level lv >= -2 (lane, laneb, lanec: this lane's
 // level 0 in each plane): packed W floats per lane; for NT = 4 four floats per lane in the
@@ -916,85 +941,63 @@ __device__ __forceinline__ void dual_grad_lanes(const WaveProg &p, const uint64_
 // evaluation changes nothing).  ls: the wave's value-stack region (KC = 1 layout).
 // out[g] receives the LL of group g's proposal, for g < gn (groups g >= gn repeat the
 // proposal of group gn - 1).
+// As tape_run for one point per lane, with a lane's constants taken from cb in token order:
+// ca is the byte index (ds_bpermute) of the lane holding the next one.  T may still be
+// loading when a handler ends, so every handler waits first.
+__device__ __forceinline__ void tape_run_groups(int word, float cb, float x, float &T, float &U, uint32_t &p, uint32_t &ca,
+                                                int &t) {
+    uint32_t blo, bhi, w;
+    float v;
+#define GT_H(BODY) ".p2align 6\n\t" BODY
+#define GG_TAKE(D) "ds_bpermute_b32 " D ", %[ca], %[cb]\n\tv_add_u32 %[ca], 4, %[ca]\n\t"
+    __asm__ volatile(
+        GT_ENTRY
+        ".p2align 6\n.Lh%=:\n\t" GT_EXIT
+        GT_H(GT_NEXT(1) GT1_PUSH "v_mov_b32 %[T0], %[x]\n\t" GT_JUMP)
+        GT_H(GT_NEXT(1) GT1_PUSH GG_TAKE("%[T0]") GT_JUMP)
+        GT_H(GT_NEXT(2) GT_WAIT GT1("v_add_f32", "%[x]", "%[T0]") GT_JUMP)
+        GT_H(GT_NEXT(2) GT_WAIT GT1("v_sub_f32", "%[T0]", "%[x]") GT_JUMP)
+        GT_H(GT_NEXT(2) GT_WAIT GT1("v_mul_f32", "%[x]", "%[T0]") GT_JUMP)
+        GT_H(GT_NEXT(2) GG_TAKE("%[v]") GT_WAIT GT1("v_add_f32", "%[v]", "%[T0]") GT_JUMP)
+        GT_H(GT_NEXT(2) GG_TAKE("%[v]") GT_WAIT GT1("v_sub_f32", "%[T0]", "%[v]") GT_JUMP)
+        GT_H(GT_NEXT(2) GG_TAKE("%[v]") GT_WAIT GT1("v_mul_f32", "%[v]", "%[T0]") GT_JUMP)
+        GT_H(GT_NEXT(1) GT_WAIT GT1("v_add_f32", "%[U0]", "%[T0]") GT1_POP GT_JUMP)
+        GT_H(GT_NEXT(1) GT_WAIT GT1("v_sub_f32", "%[U0]", "%[T0]") GT1_POP GT_JUMP)
+        GT_H(GT_NEXT(1) GT_WAIT GT1("v_mul_f32", "%[U0]", "%[T0]") GT1_POP GT_JUMP)
+        GT_H(GT_NEXT(1) GT_WAIT "v_xor_b32 %[T0], 0x80000000, %[T0]\n\t" GT_JUMP)
+        ".Lx%=:"
+        : [T0] "+&v"(T), [U0] "+&v"(U), [p] "+&v"(p), [ca] "+&v"(ca), [t] "+&s"(t), [blo] "=&s"(blo), [bhi] "=&s"(bhi),
+          [w] "=&s"(w), [v] "=&v"(v)
+        : [word] "v"(word), [cb] "v"(cb), [x] "v"(x)
+        : "vcc", "scc", "memory");
+#undef GG_TAKE
+#undef GT_H
+}
+
 __device__ __forceinline__ void wave_loglik_groups(const WaveProg &p, const GprDataset &d, const float *dx,
-                                                   const float *dy, const float *dw, float *ls, const OpMasks &m,
-                                                   uint64_t cm, float cb, int ks, int u0, int G, int gn,
-                                                   double (&out)[4]) {
+                                                   const float *dy, const float *dw, float *ls, const ProgCode &m,
+                                                   float cb, int ks, int u0, int G, int gn, double (&out)[4]) {
     const int l = opaque_lane_i32(lane_id());       // what follows is computed here, not kept live
     const int lgs = G == 4 ? 4 : 5;                  // log2 of the group size
     const int gl = l >> lgs;
     const int i = l & ((1 << lgs) - 1);
     const bool valid = i < d.n;
     const float xv = valid ? dx[i] : 0.0f, yv = valid ? dy[i] : 0.0f, wv = valid ? dw[i] : 0.0f;
-    const int src = ks * (u0 + min(gl, gn - 1));    // lane of cb holding rank 0 of this group's step
-    float *lane = ls + 2 * 64 + l;                   // level -2 of the stack below T, U
-    float T = 0.0f, U = 0.0f;
-    int sp = 0;
-    for (int t = 0; t < p.len; t++) {
-        const uint64_t bit = 1ull << t;
-        if (m.leaf[0] & bit) {
-            const bool isx = (m.x[0] & bit) != 0;
-            float b = xv;
-            if (!isx) b = shfl_all(cb, src + __popcll(cm & (bit - 1)));
-            if (m.cheap[0] & (bit << 1)) {
-                // leaf followed by +, - or *: T = T op leaf, stack untouched
-                const uint64_t nb = bit << 1;
-                const bool mul = (m.mul[0] & nb) != 0;
-                const float sgn = (m.sub[0] & nb) ? -1.0f : 1.0f;
-                const float pm = __builtin_fmaf(sgn, b, T), pr = T * b;
-                T = mul ? pr : pm;
-                t++;
-                continue;
-            }
-            lane[(sp - 2) * 64] = U;
-            U = T;
-            sp++;
-            T = b;
-            continue;
-        }
-        if (m.cheap[0] & bit) {
-            const bool mul = (m.mul[0] & bit) != 0;
-            const float sgn = (m.sub[0] & bit) ? -1.0f : 1.0f;
-            const float pm = __builtin_fmaf(sgn, T, U), pr = U * T;
-            T = mul ? pr : pm;
-            U = lane[(sp - 3) * 64];
-            sp--;
-            continue;
-        }
-        const int op = rl_i(p.o0, t);
-        if (op == GPR_OP_ONE) {
-            lane[(sp - 2) * 64] = U;
-            U = T;
-            sp++;
-            T = 1.0f;
-        } else if (op <= GPR_OP_RPOW) {
-            switch (op) {
-            case GPR_OP_DIV: T = U / T; break;
-            case GPR_OP_RSUB: T = T - U; break;
-            case GPR_OP_RDIV: T = T / U; break;
-            case GPR_OP_POW: T = powf(U, T); break;
-            default: T = powf(T, U); break;
-            }
-            U = lane[(sp - 3) * 64];
-            sp--;
-        } else {
-            switch (op) {
-            case GPR_OP_NEG: T = -T; break;
-            case GPR_OP_EXP: T = expf(T); break;
-            case GPR_OP_LOG: T = logf(T); break;
-            case GPR_OP_INV: T = 1.0f / T; break;
-            case GPR_OP_SQRT: T = sqrtf(T); break;
-            case GPR_OP_SIN: T = sinf(T); break;
-            case GPR_OP_ASIN: T = asinf(T); break;
-            case GPR_OP_COS: T = cosf(T); break;
-            case GPR_OP_ACOS: T = acosf(T); break;
-            case GPR_OP_TAN: T = tanf(T); break;
-            case GPR_OP_ATAN: T = atanf(T); break;
-            case GPR_OP_ABS: T = fabsf(T); break;
-            default: T = __builtin_nanf(""); break;   // constant-operand ops never reach here
-            }
-        }
+    uint32_t ca = 4u * (uint32_t)(ks * (u0 + min(gl, gn - 1)));   // lane of cb holding rank 0 of this group's step
+    uint32_t a = lds_addr(ls) + 4u * (uint32_t)l;                 // level -2 of the stack below T, U
+    float Ts[1] = {0.0f}, U[1] = {0.0f};
+    const float xs[1] = {xv};
+    const int n = uni(p.len);
+    for (int t = 0; t < n; t++) {
+        t = uni(t);
+        tape_run_groups(m.w0, cb, xv, Ts[0], U[0], a, ca, t);
+        t = uni(t);
+        if (t >= n) break;
+        // (no constant reaches this: the last lane's token of a full tape is an operator, and a
+        // batched program has no constant-operand token)
+        tape_slow<1>(rl_i(p.o0, t), 0.0f, xs, Ts, U, a);
     }
+    const float T = Ts[0];
     const float r = T - yv;
     const float term = valid ? (r * r) * wv : 0.0f;
     double v = (double)term;
@@ -1049,7 +1052,7 @@ __device__ __forceinline__ void wave_depths(const WaveProg &p, int &D0, int &D1,
     D0 = wave_scan_i(d0);
     dmax = wave_max_i(l < p.len ? D0 : 0);
     D1 = 0;
-    if (HI) {
+    if (HI && p.len > 64) {
         const int tot = rl_i(D0, 63);
         const int d1 = l + 64 < p.len ? 1 - gpr_arity(p.o1) : 0;
         D1 = wave_scan_i(d1) + tot;

@@ -106,6 +106,7 @@ struct GprEvalArgs {
     const GprDataset *dd;
     double *ll;
     float *grad;            // gradient output (grad kernel)
+    int per_wave;           // consecutive tapes a wave evaluates (set by the launcher)
     double lnsym;
 };
 

@@ -167,11 +167,13 @@ k_mh_config_wave(GprMHArgs a) {
         float cg0 = 0.0f, cg1 = 0.0f, pg0 = 0.0f, pg1 = 0.0f, cmg = 0.0f, pmg = 0.0f;
         bool grad_ok = false;
         AcceptDraws adraw;
-        // token classes of the current program (MALA: with the sweeps' plan for programs
-        // without the forward-mode pass; only proposals that survive early rejection need
-        // their gradient)
+        // handler words of the current program (MALA: with its token classes for the
+        // forward-mode pass, or the sweeps' plan for programs without one; only proposals that
+        // survive early rejection need their gradient)
         GradPlan gplan{};
-        OpMasks cmask = op_masks<HI>(cur);
+        OpMasks cmask{};
+        if (MALA) cmask = op_masks<HI>(cur);
+        ProgCode ccode = prog_code<KC, HI>(cur);
         // per-program values that change only with the structure: (operator tokens + 4)
         // and constants of the current program for the work counters, and whether its
         // random-walk moves can be batched (see BATCH below)
@@ -350,7 +352,7 @@ k_mh_config_wave(GprMHArgs a) {
                             win = min(win, (1 << lg) - u);
                             if (win > 1) {
                                 double o[4];
-                                wave_loglik_groups(cur, d, dx, dy, dw, ls, cmask, mk0, cb, ks, u, G, win, o);
+                                wave_loglik_groups(cur, d, dx, dy, dw, ls, ccode, cb, ks, u, G, win, o);
                                 if (l == 0) {
 #pragma unroll
                                     for (int g = 0; g < 4; g++) sll[g] = o[g];
@@ -536,11 +538,8 @@ k_mh_config_wave(GprMHArgs a) {
                     else if (cur_dual)
                         pll_m = dual_passes4<HI>(prop, d, dx, dy, dw, *(const Chunk<1> *)&c0, nchunks, ls, cmask, ccm,
                                                  rb, &mala_pts, cur_nt == GPR_DUAL_NTMAX ? 2 : 1, dgs);
-                    else if (precheck && HI && prop.len <= 64)
-                        pll_m = wave_loglik<KC, false, true>(prop, d, dx, dy, dw, c0, nchunks, ls, &cmask, rb,
-                                                             &mala_pts);
                     else if (precheck)
-                        pll_m = wave_loglik<KC, HI, true>(prop, d, dx, dy, dw, c0, nchunks, ls, &cmask, rb,
+                        pll_m = wave_loglik<KC, HI>(prop, d, dx, dy, dw, c0, nchunks, ls, ccode, rb,
                                                           &mala_pts);
                     bool rejected = (cur_dual || precheck) && !__builtin_isfinite(pll_m) && __builtin_isfinite(post);
                     if (!cur_dual && !rejected) {
@@ -577,27 +576,22 @@ k_mh_config_wave(GprMHArgs a) {
                 }
             }
             const double pprior = bprior ? bpri[bu] : (have_prior ? pre_prior : wave_prior<HI>(prop, a.lnsym));
-            // token classes: the current program's, or the structural proposal's
-            OpMasks pmask{};
+            // handler words: the current program's, or the structural proposal's
+            ProgCode pcode = ccode;
             double pll;
             int pts = d.n;
             if (have_pll) {
                 pll = pll_m;
                 pts = min(mala_pts, d.n);
             } else {
-                pmask = structural ? op_masks<HI>(prop) : cmask;
+                if (structural) pcode = prog_code<KC, HI>(prop);
                 // a = pprior + pll - post + extra < -17 rejects without a draw (cfg_accept);
                 // an LL below this bound gives a < -18 after any FP64 rounding of a
                 double reject_below = -GPR_INF;
                 if (i >= 0 && __builtin_isfinite(post) && __builtin_isfinite(pprior) && __builtin_isfinite(extra))
                     reject_below = post - pprior - extra - 18.0 -
                                    1e-12 * (__builtin_fabs(post) + __builtin_fabs(pprior) + __builtin_fabs(extra));
-                // tapes within 64 tokens evaluate with the one-register interpreter (the high
-                // words of the tape and of its masks are zero)
-                if (HI && prop.len <= 64)
-                    pll = wave_loglik<KC, false, true>(prop, d, dx, dy, dw, c0, nchunks, ls, &pmask, reject_below, &pts);
-                else
-                    pll = wave_loglik<KC, HI, true>(prop, d, dx, dy, dw, c0, nchunks, ls, &pmask, reject_below, &pts);
+                pll = wave_loglik<KC, HI>(prop, d, dx, dy, dw, c0, nchunks, ls, pcode, reject_below, &pts);
                 pts = min(pts, d.n);
             }
             int p_opq = cur_opq, p_nc = cur_nc;
@@ -630,7 +624,7 @@ k_mh_config_wave(GprMHArgs a) {
                     grad_ok = false;
                     zblk = 0xffffffffu;
                     zmblk = 0xffffffffu;
-                    cmask = pmask;
+                    ccode = pcode;
                     cur_opq = p_opq;
                     cur_nc = p_nc;
                     cur_bok = batch_ok<BATCH, HI>(cur, mk);
@@ -641,7 +635,8 @@ k_mh_config_wave(GprMHArgs a) {
                         ccm[0] = ballot(l < cur.len && cur.o0 == GPR_OP_CONST);
                         ccm[1] = HI ? ballot(l + 64 < cur.len && cur.o1 == GPR_OP_CONST) : 0;
                         cur_nt = dual_nt(__popcll(ccm[0]) + __popcll(ccm[1]), dm);
-                        if (!cur_dual) gplan = grad_plan<HI>(cur);
+                        if (cur_dual) cmask = op_masks<HI>(cur);
+                        else gplan = grad_plan<HI>(cur);
                     }
                     cur_b16 = cur_bok && const_count<HI>(cur) <= 4;
                 } else {
@@ -1025,33 +1020,153 @@ hipError_t gpr_launch_mh_config_lane(const GprMHArgs &a, int cap_max, hipStream_
 }
 
 // ---------------------------------------------------------------- standalone evaluator
-template <int KC, bool HI>
-__global__ void __launch_bounds__(GPR_WG) k_eval_wave(GprEvalArgs a) {
-    const int wave = uni((int)(threadIdx.x >> 6));
+// Value-stack rows (256 bytes) of one wave: 18 hold the deepest program at one point per
+// lane; 24 hold one of depth 6 at four.  Deeper programs of a larger dataset run at one
+// point per lane in the same rows, so that the common ones keep five waves per SIMD.
+#define GPR_EVAL_ROWS(KC) ((KC) == 4 ? 24 : GPR_MAX_DEPTH + 2)
+
+// A tape's registers and lengths: lane l holds tokens l and l + 64.  A length outside
+// [0, cap] is clamped: the kernels never read or write past the caller's cap rows (a
+// malformed tape yields a meaningless value).
+template <bool HI>
+__device__ __forceinline__ WaveProg eval_load(const GprEvalArgs &a, int chain) {
     const int l = lane_id();
-    const int chain = uni((int)blockIdx.x * GPR_WAVES_PER_WG + wave);
-    if (chain >= a.nchains) return;
-    const int N = a.nchains;
-    const GprDataset d = a.dd ? *a.dd : a.d;
+    const size_t N = (size_t)a.nchains;
     WaveProg p;
-    // a length outside [0, cap] is clamped: the kernel never reads or writes past the
-    // caller's cap rows or its LDS slab (a malformed tape yields a meaningless value)
     p.len = min(max(uni(a.len[chain]), 0), a.cap);
     p.o0 = l < p.len ? a.ops[(size_t)l * N + chain] : 0;
     p.c0 = l < p.len ? a.cs[(size_t)l * N + chain] : 0.0f;
     p.o1 = (HI && l + 64 < p.len) ? a.ops[(size_t)(l + 64) * N + chain] : 0;
     p.c1 = (HI && l + 64 < p.len) ? a.cs[(size_t)(l + 64) * N + chain] : 0.0f;
-    const int nchunks = (d.n + 64 * KC - 1) / (64 * KC);
-    Chunk<KC> c0;
-    c0.load(a.dx + d.off, a.dy + d.off, a.dw + d.off, d.n, 0);
-    const double ll = wave_loglik<KC, HI>(p, d, a.dx + d.off, a.dy + d.off, a.dw + d.off, c0, nchunks);
-    if (l == 0) a.ll[chain] = ll;
+    return p;
+}
+// The tape's stack depth, or 0 when it pops an empty stack or passes GPR_MAX_DEPTH (it
+// would leave the wave's rows); an empty tape has depth 1.
+template <bool HI>
+__device__ __forceinline__ int eval_depth(const WaveProg &p) {
+    const int l = lane_id();
+    int D0, D1, dm;
+    wave_depths<HI>(p, D0, D1, dm);
+    if (dm > GPR_MAX_DEPTH || ballot((l < p.len && D0 < 1) || (HI && l + 64 < p.len && D1 < 1))) return 0;
+    return max(dm, 1);
 }
 
-hipError_t gpr_launch_eval_wave(const GprEvalArgs &a, hipStream_t s) {
-    const int grid = (a.nchains + GPR_WAVES_PER_WG - 1) / GPR_WAVES_PER_WG;
+// One wave per tape.  A wave takes a.per_wave consecutive tapes: the dataset's first chunk
+// stays in its registers, and a tape's tokens are loaded while the one before it is
+// evaluated (a tape of some ten tokens is evaluated in the time of one trip to memory).
+template <int KC, bool HI>
+__global__ void __launch_bounds__(GPR_WG) __attribute__((amdgpu_waves_per_eu(KC == 4 ? 5 : (KC == 2 ? 6 : 7))))
+k_eval_wave(GprEvalArgs a) {
+    __shared__ float s_stack[GPR_WAVES_PER_WG][GPR_EVAL_ROWS(KC) * 64];
+    const int wave = uni((int)(threadIdx.x >> 6));
+    const int first = uni(((int)blockIdx.x * GPR_WAVES_PER_WG + wave) * a.per_wave);
+    const int last = min(first + a.per_wave, a.nchains);
+    if (first >= last) return;
+    const GprDataset d = uni_dataset(a.dd ? *a.dd : a.d);
+    const float *dx = a.dx + d.off, *dy = a.dy + d.off, *dw = a.dw + d.off;
+    float *ls = s_stack[wave];
+    WaveProg nx = eval_load<HI>(a, first);
+    Chunk<KC> c0;
+    c0.load(dx, dy, dw, d.n, 0);
+    for (int chain = first; chain < last; chain++) {
+        const WaveProg p = nx;
+        if (chain + 1 < last) nx = eval_load<HI>(a, chain + 1);
+        const int dm = eval_depth<HI>(p);
+        double ll = -GPR_INF;
+        if (dm == 0) {
+        } else if (KC == 1 || dm * KC <= GPR_EVAL_ROWS(KC)) {
+            ll = wave_loglik<KC, HI>(p, d, dx, dy, dw, c0, (d.n + 64 * KC - 1) / (64 * KC), ls, prog_code<KC, HI>(p));
+        } else {
+            Chunk<1> c1;
+            c1.load(dx, dy, dw, d.n, 0);
+            ll = wave_loglik<1, HI>(p, d, dx, dy, dw, c1, (d.n + 63) / 64, ls, prog_code<1, HI>(p));
+        }
+        if (lane_id() == 0) a.ll[chain] = ll;
+    }
+}
+
+// One workgroup per tape, for datasets of more than 256 points: its four waves interpret
+// the tape over 256 points each, and the terms of 1024 points meet in LDS, where one wave
+// adds them in the order of wave_loglik (every lane's points in increasing order, so the
+// sum is bit-identical).  With few tapes the GPU is filled four times better, and with many
+// the longest tape ends the launch sooner: 30000 tapes (cap 64) at n = 1024 222 us, and 362
+// by one wave per tape; 500 tapes at n = 500 42 and 66.  At n = 300 two of the waves have
+// little to do: 30000 tapes 191 us, and 136 by one wave per tape, which therefore keeps
+// datasets of up to 512 points where 4096 tapes or more fill the GPU.
+template <bool HI>
+__global__ void __launch_bounds__(GPR_WG) k_eval_split(GprEvalArgs a) {
+    __shared__ float s_stack[GPR_WAVES_PER_WG][GPR_EVAL_ROWS(4) * 64];
+    __shared__ float s_term[16][64];
+    const int wave = uni((int)(threadIdx.x >> 6));
+    const int l = lane_id();
+    const int chain = (int)blockIdx.x;
+    const GprDataset d = uni_dataset(a.dd ? *a.dd : a.d);
+    const float *dx = a.dx + d.off, *dy = a.dy + d.off, *dw = a.dw + d.off;
+    float *ls = s_stack[wave];
+    const WaveProg p = eval_load<HI>(a, chain);
+    const int dm = eval_depth<HI>(p);       // the same in every wave
+    if (dm == 0) {
+        if (threadIdx.x == 0) a.ll[chain] = -GPR_INF;
+        return;
+    }
+    const bool four = dm * 4 <= GPR_EVAL_ROWS(4);
+    const ProgCode pc = four ? prog_code<4, HI>(p) : prog_code<1, HI>(p);
+    float acc = 0.0f, comp = 0.0f;
+    for (int base = 0; base < d.n; base += 1024) {
+        const int mine = base + 256 * wave;
+        if (mine >= d.n) {
+        } else if (four) {
+            Chunk<4> c;
+            c.load(dx, dy, dw, d.n, mine);
+            float T[4];
+            wave_eval_ls<4, HI>(p, c.x, T, ls, pc);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const float r = T[k] - c.y[k];
+                s_term[4 * wave + k][l] = mine + 64 * k + l < d.n ? (r * r) * c.w[k] : 0.0f;
+            }
+        } else {
+            for (int k = 0; k < 4 && mine + 64 * k < d.n; k++) {
+                Chunk<1> c;
+                c.load(dx, dy, dw, d.n, mine + 64 * k);
+                float T[1];
+                wave_eval_ls<1, HI>(p, c.x, T, ls, pc);
+                const float r = T[0] - c.y[0];
+                s_term[4 * wave + k][l] = mine + 64 * k + l < d.n ? (r * r) * c.w[0] : 0.0f;
+            }
+        }
+        __syncthreads();
+        if (wave == 0) {
+            const int m = min((d.n - base + 63) / 64, 16);
+            for (int k = 0; k < m; k++) {
+                const float yv = s_term[k][l] - comp;
+                const float tv = acc + yv;
+                comp = (tv - acc) - yv;
+                acc = tv;
+            }
+        }
+        __syncthreads();
+    }
+    if (wave == 0) {
+        const double s = wave_sum_d((double)acc - (double)comp);
+        if (l == 0) a.ll[chain] = !__builtin_isfinite(s) ? -GPR_INF : d.lconst - (d.wconst > 0.0 ? d.wconst * s : s);
+    }
+}
+
+// Tapes per wave: as many as still leave every wave slot of the GPU (256 CUs, 20 waves
+// each) several waves to balance unequal tapes with.
+hipError_t gpr_launch_eval_wave(const GprEvalArgs &args, hipStream_t s) {
+    GprEvalArgs a = args;
     const bool hi = a.cap > 64;
     const int kc = a.d.kc;
+    if (a.d.n > 512 || (a.d.n > 256 && a.nchains < 4096)) {
+        if (hi) hipLaunchKernelGGL(k_eval_split<true>, dim3(a.nchains), dim3(GPR_WG), 0, s, a);
+        else hipLaunchKernelGGL(k_eval_split<false>, dim3(a.nchains), dim3(GPR_WG), 0, s, a);
+        return hipGetLastError();
+    }
+    a.per_wave = std::max(1, std::min(4, a.nchains / 20480));
+    const int waves = (a.nchains + a.per_wave - 1) / a.per_wave;
+    const int grid = (waves + GPR_WAVES_PER_WG - 1) / GPR_WAVES_PER_WG;
 #define GPR_L(K, H) hipLaunchKernelGGL((k_eval_wave<K, H>), dim3(grid), dim3(GPR_WG), 0, s, a)
     if (kc == 1) { if (hi) GPR_L(1, true); else GPR_L(1, false); }
     else if (kc == 2) { if (hi) GPR_L(2, true); else GPR_L(2, false); }

@@ -461,7 +461,7 @@ __device__ __forceinline__ int r_struct_draw(D &dr, bool valid, int hop, int ops
 // program with an LL near -1e22 is accepted or not by the last bit of it), through the 64
 // doubles of S.
 template <int KC>
-__device__ __forceinline__ double r_loglik64(const WaveProg &p, const OpMasks &m, float *ls, double *S, const float *x,
+__device__ __forceinline__ double r_loglik64(const WaveProg &p, const ProgCode &m, float *ls, double *S, const float *x,
                                              const float *y, const float *sd, const double *lnc, int n) {
 #pragma clang fp contract(off)
     const int l = lane_id();
@@ -529,7 +529,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_
         int hop = live ? a.ops[(size_t)l * N + chain] : 0;
         float hc = live ? a.cs[(size_t)l * N + chain] : 0.0f;
         RefTape cur = r_decode_wave(hop, hc);
-        OpMasks cm = op_masks<false>(cur.p);
+        ProgCode cm = prog_code<KC, false>(cur.p);
         double cur_prior = r_prior_wave(cur.dl, gpr_lcauchy(hc), a.ref_lnops, S);
         double cur_ll = r_loglik64<KC>(cur.p, cm, ls, S, x, y, sdv, lc, n);
         double cur_post = cur_prior + cur_ll;
@@ -543,7 +543,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_
             int php = hop;
             float phc = hc;
             RefTape prop = cur;
-            OpMasks pm = cm;
+            ProgCode pm = cm;
             double pp;
             const bool structural = phase == 0;
             phase = phase == 4 ? 0 : phase + 1;
@@ -557,7 +557,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_
                     php = r_struct_draw(ph, r_valid(cur_post), hop, a.opset, nops, buf);
                 }
                 prop = r_decode_wave(php, hc);
-                pm = op_masks<false>(prop.p);
+                pm = prog_code<KC, false>(prop.p);
                 backward = -(double)gpr_ref_logint[prop.count];
                 pp = r_prior_wave(prop.dl, gpr_lcauchy(hc), a.ref_lnops, S);
             } else {
@@ -687,11 +687,11 @@ __global__ void __launch_bounds__(GPR_WG) __attribute__((amdgpu_waves_per_eu(4))
         int hop = l < GPR_REF_SLOTS ? a.ops[(size_t)l * N + chain] : 0;
         float hc = live ? a.cs[(size_t)slot * N + chain] : 0.0f;
         RefTape cur = r_decode_wave(hop, hc);
-        OpMasks cm = op_masks<false>(cur.p);
+        ProgCode cm = prog_code<KC, false>(cur.p);
         int opq, nconst;
         prog_counts<false>(cur.p, opq, nconst);
         double cur_prior = r_prior_wave(cur.dl, gpr_lcauchy(hc), a.ref_lnops, S);
-        double cur_ll = wave_loglik<KC, false, true>(cur.p, d, dx, dy, dw, c0, nchunks, ls, &cm);
+        double cur_ll = wave_loglik<KC, false>(cur.p, d, dx, dy, dw, c0, nchunks, ls, cm);
         double cur_post = cur_prior + cur_ll;
         double bt, bt0;
         r_const_back(hc, bt, bt0);
@@ -704,7 +704,7 @@ __global__ void __launch_bounds__(GPR_WG) __attribute__((amdgpu_waves_per_eu(4))
             const uint32_t step = step0 + (uint32_t)mcmci;
             int php = hop;
             RefTape prop = cur;
-            OpMasks pm = cm;
+            ProgCode pm = cm;
             double pp;
             int p_opq = opq, p_nconst = nconst;
             const int ph5 = phase;
@@ -716,7 +716,7 @@ __global__ void __launch_bounds__(GPR_WG) __attribute__((amdgpu_waves_per_eu(4))
                 WaveDraws<PhiloxWords> ph = philox_draws(a.seed, chain, step, GPR_P_STRUCT);
                 php = r_struct_draw(ph, r_valid(cur_post), hop, a.opset, nops, (int *)S);
                 prop = r_decode_wave(php, hc);
-                pm = op_masks<false>(prop.p);
+                pm = prog_code<KC, false>(prop.p);
                 prog_counts<false>(prop.p, p_opq, p_nconst);
                 backward = -(double)gpr_ref_logint[prop.count];
                 pp = r_prior_wave(prop.dl, gpr_lcauchy(hc), a.ref_lnops, S);
@@ -785,7 +785,7 @@ __global__ void __launch_bounds__(GPR_WG) __attribute__((amdgpu_waves_per_eu(4))
                                             __builtin_fabs(forward) + __builtin_fabs(pp));
             }
             int pts = d.n;
-            const double pl = wave_loglik<KC, false, true>(prop.p, d, dx, dy, dw, c0, nchunks, ls, &pm, reject_below, &pts);
+            const double pl = wave_loglik<KC, false>(prop.p, d, dx, dy, dw, c0, nchunks, ls, pm, reject_below, &pts);
             pts = min(pts, d.n);
             n_evals += (unsigned long long)prop.p.len * (unsigned long long)pts;
             n_flops += (unsigned long long)p_opq * (unsigned long long)pts + (unsigned long long)p_nconst;

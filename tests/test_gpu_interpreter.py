@@ -1,0 +1,106 @@
+"""The wave interpreter at the edges of its registers and rows: tapes that end, or hold a
+fused leaf and operator, around tokens 62-64 and 127, stacks at the depths where the
+evaluator changes its points per lane, datasets around its chunks, and MH blocks on
+programs that fill their cap."""
+import numpy as np
+import pytest
+
+from gpu_util import check_paths, dev, say
+
+pytestmark = pytest.mark.gpu
+
+LENGTHS = [1, 2, 3, 5, 61, 62, 63, 64, 65, 66, 67, 126, 127, 128]
+DEPTHS = [2, 5, 6, 7, 9, 10, 15, 16]
+
+
+def chain_tape(length, shift):
+    """x, then leaf/operator pairs; `shift` negations in front move the pairs by a token, and
+    negations at the end (a handler without a second token) fill an even length."""
+    toks = ["X"] + ["NEG"] * min(shift, length - 1)
+    k = 0
+    while len(toks) + 2 <= length:
+        leaf, op = [(("CONST", 0.5), "ADD"), ("X", "MUL"), (("CONST", 0.75), "MUL"), ("X", "SUB"), ("X", "ADD"),
+                    (("CONST", 0.25), "SUB")][k % 6]
+        toks += [leaf, op]
+        k += 1
+    return toks + ["NEG"] * (length - len(toks))
+
+
+def deep_tape(depth):
+    """`depth` leaves, then the operators: every push and pop of the stack's rows."""
+    leaves = [("CONST", 0.5) if k % 2 else "X" for k in range(depth)]
+    return leaves + [("ADD", "MUL", "SUB")[k % 3] for k in range(depth - 1)]
+
+
+def batch(oracle, cap):
+    tapes = [chain_tape(n, s) for n in LENGTHS if n <= cap for s in (0, 1)] + [deep_tape(d) for d in DEPTHS if 2 * d <= cap]
+    # a token without a handler between the others, also as the last of a half tape
+    tapes += [chain_tape(n, 0)[:-1] + ["EXP"] for n in (62, 64, 66, 126) if n <= cap]
+    tapes += [["X", ("CONST", 3.0), "ADD", "EXP", "X", "X", "MUL", ("CONST", 2.0), "ADD", "DIV", "NEG", "X", "SUB"]]
+    arrs = [oracle.tape_arrays(t) for t in tapes]
+    O = np.zeros((cap, len(arrs)), dtype=np.uint8)
+    V = np.zeros((cap, len(arrs)), dtype=np.float32)
+    for i, (o, v) in enumerate(arrs):
+        O[:len(o), i] = o
+        V[:len(o), i] = v
+    return O, V, np.array([len(o) for o, _ in arrs], dtype=np.int32)
+
+
+def dataset(n, uneven):
+    rng = np.random.default_rng(n)
+    x = rng.uniform(-1, 1, n)
+    sd = rng.uniform(0.5, 1.0, n) if uneven else np.full(n, 0.5)
+    return x.astype(np.float32), (x + rng.normal(0, 0.5, n)).astype(np.float32), sd.astype(np.float32)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 128, 129, 256, 257, 513, 1024, 1025, 2100])
+@pytest.mark.parametrize("cap", [64, 128])
+def test_eval_at_the_edges(oracle, gpr, n, cap):
+    """Every operation of these tapes is exactly rounded on both sides and the sums differ in
+    order only: 1e-6 of max(|LL|, n), against FP32 sums of n terms in the oracle's order."""
+    import torch
+    O, V, L = batch(oracle, cap)
+    d = dataset(n, uneven=n % 2 == 1)
+    N = O.shape[1]
+    with gpr.Context(cap=cap) as ctx:
+        ctx.set_data([d], [1])
+        out = torch.zeros(N, dtype=torch.float64, device="cuda")
+        say(f"interpreter edges n={n} cap={cap} tapes={N}")
+        dO, dV, dL = dev(O), dev(V), dev(L)
+        ctx.eval_loglik_dev(0, dO.data_ptr(), dV.data_ptr(), dL.data_ptr(), N, cap, gpr.SCHED_WAVE, out.data_ptr())
+        got = out.cpu().numpy()
+    ref = np.array([oracle.tape_loglik(O[:L[i], i], V[:L[i], i], *d) for i in range(N)])
+    assert np.all(np.isfinite(ref))
+    exp = np.array([gpr.OP["EXP"] in O[:L[i], i] for i in range(N)])
+    tol = np.where(exp, 1e-5, 1e-6) * np.maximum(np.abs(ref), n)      # exp: the device's libm
+    assert np.all(np.abs(got - ref) <= tol), np.flatnonzero(np.abs(got - ref) > tol)
+
+
+@pytest.mark.parametrize("cap,n,mala", [(64, 20, 0), (64, 40, 0), (64, 150, 0), (128, 20, 0), (128, 150, 0), (64, 150, 1),
+                                        (128, 150, 1)])
+def test_blocks_on_full_programs(oracle, gpr, cap, n, mala):
+    """Constant steps on programs of 62 to cap tokens (all sizes of one register, and of two),
+    one point per lane and with speculative steps (n <= 32): the oracle's trajectories."""
+    O, V, L = batch(oracle, cap)
+    keep = np.flatnonzero((L >= 60) | (L <= 13))
+    O, V, L = O[:, keep].copy(), V[:, keep].copy(), L[keep].copy()
+    x, y, sd = dataset(n, uneven=True)
+    steps, nch = 24, len(L)
+    cfg = oracle.make_cfg(cap=cap, seed=5, fixed_structure=1, proposal=mala, eps=0.01, sigma=0.05)
+    o_ops, o_cs, o_ln = O.copy(), V.copy(), L.copy()
+    m = np.zeros(nch)
+    p_ref, _, _ = oracle.cfg_run_block(cfg, o_ops, o_cs, o_ln, x, y, sd, 0, steps, margin=m)
+    with gpr.Context(cap=cap, seed=5, fixed_structure=1, proposal=mala, eps=0.01, sigma=0.05,
+                     schedule=gpr.SCHED_WAVE) as ctx:
+        ctx.set_data([(x, y, sd)], [nch])
+        ctx.write_state(O, V, L)
+        say(f"blocks on full programs cap={cap} n={n} mala={mala}")
+        ctx.run_block(steps)
+        g_ops, g_cs, g_ln, g_pr, _ = ctx.read_state()
+    if mala:      # the device sums gradients in FP32: within 1e-3 of the oracle's constants
+        ok = np.all(np.abs(g_cs - o_cs) <= 1e-3 * np.maximum(1.0, np.abs(o_cs)), axis=0)
+        assert ok.mean() >= 0.9
+        return
+    same = np.all(g_cs.view(np.uint32) == o_cs.view(np.uint32), axis=0)
+    check_paths(same, m, f"full programs cap={cap} n={n}:")
+    assert np.array_equal(g_pr[same], p_ref[same])
