@@ -1120,253 +1120,279 @@ __device__ __forceinline__ float gather_f(float v0, float v1, int src, bool hi) 
 }
 
 // ---------------------------------------------------------------- reverse-mode adjoint
-// One point per lane (KC = 1), no value stack: the forward sweep stores the value of
-// every operator token in this wave's LDS slab lv[t * 64 + lane]; leaves (x, constant,
-// one) are not stored, their values come from the token, and a binary token finds its
-// left operand through a per-structure plan.  The reverse sweep walks the tape backwards
-// carrying the adjoint of the current token.  Reverse postfix order visits a node, then
-// its right subtree (ending at t-1), then its left subtree, so a binary token carries its
-// right operand's adjoint and leaves its left operand's in a mailbox: the slot of the
-// first token of its own subtree, always a leaf, which the left subtree's root reads
-// when the sweep arrives there (the next token after a leaf).  Pending mailboxes are
-// distinct slots (nested subtrees pending at once start at distinct tokens), and a
-// constant leaf's mailbox is read before the sweep reaches the leaf itself, whose slot
-// then receives the leaf's per-point gradient; a token with a constant operand (c+, c*,
-// ^c, c^) overwrites its value slot with its gradient once it is done.
+// KC points per lane and sweep pair.  The forward sweep stores the value of every operator
+// token in the wave's rows, lv[row][k][lane], at the row of its rank among the operators;
+// leaves (x, constant, one) are not stored, their values come from the token.  A binary
+// token finds its left operand through a per-structure plan (its right operand is the token
+// before it, whose value the sweep carries).  The reverse sweep walks the tape backwards
+// carrying the adjoint of the current token.  Reverse postfix order visits a node, then its
+// right subtree (ending at t-1), then its left subtree, so a binary token carries its right
+// operand's adjoint on and pushes its left operand's onto a stack in the rows after the
+// operators'; a leaf pops the next one.  The adjoint of a constant is summed over the wave as
+// soon as it is known.  A program needs fewer rows than it has tokens: operators and pending
+// left operands are at most len - 1.
 
-// Per-structure plan of the two sweeps: token-class masks (bit t of word 0, bit t-64 of
-// word 1); for every token t (lane t of the *0 words, lane t-64 of the *1 words) the left
-// operand lc of a binary token and the first token st of the subtree ending at t.
+// Per-structure plan of the two sweeps.  Word t (lane t of w0, lane t-64 of w1): op code
+// (bits 0-4), row of the operator's value (5-12), and the left and right operand of a binary
+// token (13-20, 21-28; a unary token's operand in the right field): a row, or GPR_G_X, GPR_G_ONE
+// or GPR_G_C + token for a leaf.  rows: rows of the sweeps.
+#define GPR_G_X 127
+#define GPR_G_C 128
+#define GPR_G_ONE 255
 struct GradPlan {
-    uint64_t leaf[2], x[2], cnst[2], cheap[2], mul[2], sub[2];
-    int lc0, lc1, st0, st1;
+    int w0, w1;
+    int nops, rows;
 };
 
 template <bool HI>
 __device__ __forceinline__ GradPlan grad_plan(const WaveProg &p) {
     const int l = lane_id();
     GradPlan g;
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-        const bool v = (h == 0 || HI) && l + 64 * h < p.len;
-        const int o = h ? p.o1 : p.o0;
-        g.leaf[h] = ballot(v && o <= GPR_OP_ONE);
-        g.x[h] = ballot(v && o == GPR_OP_X);
-        g.cnst[h] = ballot(v && o == GPR_OP_CONST);
-        g.cheap[h] = ballot(v && o >= GPR_OP_ADD && o <= GPR_OP_MUL);
-        g.mul[h] = ballot(v && o == GPR_OP_MUL);
-        g.sub[h] = ballot(v && o == GPR_OP_SUB);
+    int D0, D1, dm;
+    wave_depths<HI>(p, D0, D1, dm);
+    const bool v0 = l < p.len, v1 = HI && l + 64 < p.len;
+    const uint64_t m0 = ballot(v0 && p.o0 > GPR_OP_ONE), m1 = HI ? ballot(v1 && p.o1 > GPR_OP_ONE) : 0;
+    const uint64_t below = (1ull << l) - 1ull;
+    const int s0 = __popcll(m0 & below), s1 = __popcll(m0) + __popcll(m1 & below);
+    // this token as an operand
+    const int r0 = p.o0 == GPR_OP_X ? GPR_G_X : (p.o0 == GPR_OP_ONE ? GPR_G_ONE : (p.o0 == GPR_OP_CONST ? GPR_G_C + l : s0));
+    const int r1 = p.o1 == GPR_OP_X ? GPR_G_X
+                                    : (p.o1 == GPR_OP_ONE ? GPR_G_ONE : (p.o1 == GPR_OP_CONST ? GPR_G_C + 64 + l : s1));
+    // the left operand of a binary token is the last token before it whose stack depth is its
+    // own: the tokens between them, the right operand's, lie deeper
+    int lc0 = 0, lc1 = 0;
+    for (int k = 1; k <= min(dm, GPR_MAX_DEPTH); k++) {
+        const uint64_t d0 = ballot(v0 && D0 == k), d1 = HI ? ballot(v1 && D1 == k) : 0;
+        const uint64_t q0 = d0 & below, q1 = d1 & below;
+        if (D0 == k) lc0 = q0 ? 63 - __builtin_clzll(q0) : 0;
+        if (HI && D1 == k) lc1 = q1 ? 127 - __builtin_clzll(q1) : (d0 ? 63 - __builtin_clzll(d0) : 0);
     }
-    // replay the stack on token indices: lane k of idx / sdx holds the token whose value
-    // is at level k and the first token of its subtree (levels are bounded for malformed
-    // tapes; valid ones stay below GPR_MAX_DEPTH)
-    int idx = 0, sdx = 0, sp = 0;
-    g.lc0 = 0;
-    g.lc1 = 0;
-    g.st0 = 0;
-    g.st1 = 0;
-    for (int t = 0; t < p.len; t++) {
-        const int li = t & 63;
-        const bool h = HI && t >= 64;
-        const int ar = gpr_arity(h ? rl_i(p.o1, li) : rl_i(p.o0, li));
-        int lev, st = t;
-        if (ar == 0) {
-            lev = min(sp, 63);
-            sp = min(sp + 1, 64);
-        } else {
-            lev = max(sp - ar, 0);
-            st = rl_i(sdx, lev);
-            if (ar == 2) {
-                const int lc = rl_i(idx, lev);
-                if (h) g.lc1 = l == li ? lc : g.lc1; else g.lc0 = l == li ? lc : g.lc0;
-                sp = max(sp - 1, 1);
-            }
-        }
-        if (h) g.st1 = l == li ? st : g.st1; else g.st0 = l == li ? st : g.st0;
-        idx = l == lev ? t : idx;
-        sdx = l == lev ? st : sdx;
+    const int left0 = gather_i(r0, r1, lc0, HI), right0 = gather_i(r0, r1, max(l - 1, 0), HI);
+    g.w0 = (p.o0 & 31) | (s0 << 5) | (left0 << 13) | (right0 << 21);
+    g.w1 = 0;
+    if (HI) {
+        const int left1 = gather_i(r0, r1, lc1, HI), right1 = gather_i(r0, r1, l + 63, HI);
+        g.w1 = (p.o1 & 31) | (s1 << 5) | (left1 << 13) | (right1 << 21);
     }
+    g.nops = __popcll(m0) + __popcll(m1);
+    // pending left operands: at most one per level above the first
+    g.rows = g.nops + max(dm - 1, 0);
     return g;
 }
 
-// value of leaf token u (x, its constant, or one) at this lane's point
-template <bool HI>
-__device__ __forceinline__ float leaf_val(const WaveProg &p, const GradPlan &g, int u, float x) {
-    const int li = u & 63;
-    const int h = (HI && u >= 64) ? 1 : 0;
-    const uint64_t bit = 1ull << li;
-    const float c = h ? rl_f(p.c1, li) : rl_f(p.c0, li);
-    return (g.x[h] & bit) ? x : ((g.cnst[h] & bit) ? c : 1.0f);
-}
-// value of token u: a leaf from the token, an operator from the slab (lvl = lv + lane)
-template <bool HI>
-__device__ __forceinline__ float tok_val(const WaveProg &p, const GradPlan &g, int u, float x, const float *lvl) {
-    const int h = (HI && u >= 64) ? 1 : 0;
-    const float s = lvl[u * 64];
-    return (g.leaf[h] & (1ull << (u & 63))) ? leaf_val<HI>(p, g, u, x) : s;
-}
-template <bool HI>
-__device__ __forceinline__ int left_of(const GradPlan &g, int t) {
-    return (HI && t >= 64) ? rl_i(g.lc1, t & 63) : rl_i(g.lc0, t & 63);
-}
-template <bool HI>
-__device__ __forceinline__ int start_of(const GradPlan &g, int t) {
-    return (HI && t >= 64) ? rl_i(g.st1, t & 63) : rl_i(g.st0, t & 63);
+// operand r (a row or a leaf) at this lane's points
+template <int KC, bool HI>
+__device__ __forceinline__ void grad_val(const WaveProg &p, int r, const float (&x)[KC], const float *lvl, float (&v)[KC]) {
+    if (r < GPR_G_X) {
+#pragma unroll
+        for (int k = 0; k < KC; k++) v[k] = lvl[(r * KC + k) * 64];
+    } else {
+        const int u = r - GPR_G_C;
+        const float c = r == GPR_G_ONE ? 1.0f : ((HI && u >= 64) ? rl_f(p.c1, u & 63) : rl_f(p.c0, max(u, 0) & 63));
+        const bool isx = r == GPR_G_X;
+#pragma unroll
+        for (int k = 0; k < KC; k++) v[k] = isx ? x[k] : c;
+    }
 }
 
-// Forward sweep: the same operations on the same operands as wave_eval, so the value is
-// bit-identical.  A leaf followed by +, - or * in the same half is applied at once.
-template <bool HI>
-__device__ __forceinline__ float grad_forward(const WaveProg &p, const GradPlan &g, float x, float *lvl) {
-    float T = 0.0f;
+// Forward sweep: the same operations on the same operands as wave_eval_ls, so the value is
+// bit-identical.  P: the value before the last leaf, the left operand of a binary token
+// right after a leaf.
+template <int KC, bool HI>
+__device__ __forceinline__ void grad_forward(const WaveProg &p, const GradPlan &g, const float (&x)[KC], float *lvl,
+                                             float (&T)[KC]) {
+    float P[KC];
+#pragma unroll
+    for (int k = 0; k < KC; k++) T[k] = P[k] = 0.0f;
     for (int t = 0; t < p.len; t++) {
         const int li = t & 63;
-        const int h = (HI && t >= 64) ? 1 : 0;
-        const uint64_t bit = 1ull << li;
-        if (g.leaf[h] & bit) {
-            const float b = leaf_val<HI>(p, g, t, x);
-            const uint64_t nb = bit << 1;
-            if (g.cheap[h] & nb) {
-                const bool mul = (g.mul[h] & nb) != 0;
-                const float sgn = (g.sub[h] & nb) ? -1.0f : 1.0f;
-                const float pm = __builtin_fmaf(sgn, b, T), pr = T * b;
-                T = mul ? pr : pm;
-                t++;
-                lvl[t * 64] = T;
-            } else {
-                T = b;
-            }
+        const bool h = HI && t >= 64;
+        const int w = h ? rl_i(g.w1, li) : rl_i(g.w0, li);
+        const int op = w & 31;
+        if (op <= GPR_OP_ONE) {
+            const float cv = h ? rl_f(p.c1, li) : rl_f(p.c0, li);
+            const float sv = op == GPR_OP_CONST ? cv : 1.0f;
+            const bool isx = op == GPR_OP_X;
+#pragma unroll
+            for (int k = 0; k < KC; k++) { P[k] = T[k]; T[k] = isx ? x[k] : sv; }
             continue;
         }
-        if (g.cheap[h] & bit) {
-            const float a = tok_val<HI>(p, g, left_of<HI>(g, t), x, lvl);
-            const bool mul = (g.mul[h] & bit) != 0;
-            const float sgn = (g.sub[h] & bit) ? -1.0f : 1.0f;
-            const float pm = __builtin_fmaf(sgn, T, a), pr = a * T;
-            T = mul ? pr : pm;
-        } else {
-            const int op = h ? rl_i(p.o1, li) : rl_i(p.o0, li);
-            if (op <= GPR_OP_RPOW) {
-                T = op_bin(op, tok_val<HI>(p, g, left_of<HI>(g, t), x, lvl), T);
+        if (op <= GPR_OP_RPOW) {
+            float A[KC];
+            if (((w >> 21) & 255) >= GPR_G_X) {
+#pragma unroll
+                for (int k = 0; k < KC; k++) A[k] = P[k];
             } else {
-                const float c = op >= GPR_OP_CADD ? (h ? rl_f(p.c1, li) : rl_f(p.c0, li)) : 0.0f;
-                T = op_un(op, T, c);
+                grad_val<KC, HI>(p, (w >> 13) & 255, x, lvl, A);
             }
+            if (op == GPR_OP_ADD) GPR_KLOOP(A[k] + T[k]);
+            else if (op == GPR_OP_SUB) GPR_KLOOP(A[k] - T[k]);
+            else if (op == GPR_OP_MUL) GPR_KLOOP(A[k] * T[k]);
+            else GPR_KLOOP(op_bin(op, A[k], T[k]));
+        } else {
+            const float c = op >= GPR_OP_CADD ? (h ? rl_f(p.c1, li) : rl_f(p.c0, li)) : 0.0f;
+            GPR_KLOOP(op_un(op, T[k], c));
         }
-        lvl[t * 64] = T;
+        const int row = (w >> 5) & 255;
+#pragma unroll
+        for (int k = 0; k < KC; k++) lvl[(row * KC + k) * 64] = T[k];
     }
-    return T;
 }
 
-// Reverse sweep from adjoint G of the program's value.
-template <bool HI>
-__device__ __forceinline__ void grad_reverse(const WaveProg &p, const GradPlan &g, float x, float *lvl, float G) {
+// Reverse sweep from the adjoints G of the program's value.  The wave sums of the constants'
+// adjoints over the lanes with a valid point land at lane t of s0[k] (token t < 64) or s1[k].
+template <int KC, bool HI>
+__device__ __forceinline__ void grad_reverse(const WaveProg &p, const GradPlan &g, const float (&x)[KC], float *lvl,
+                                             float (&G)[KC], const bool (&valid)[KC], float (&s0)[KC], float (&s1)[KC]) {
+    const int l = lane_id();
+    int top = g.nops;   // row of the next push
+    auto constant = [&](int t, const float (&v)[KC]) {
+#pragma unroll
+        for (int k = 0; k < KC; k++) {
+            const float s = wave_sum_f(valid[k] ? v[k] : 0.0f);
+            if (HI && t >= 64) s1[k] = l == t - 64 ? s : s1[k];
+            else s0[k] = l == t ? s : s0[k];
+        }
+    };
     for (int t = p.len - 1; t >= 0; t--) {
         const int li = t & 63;
-        const int h = (HI && t >= 64) ? 1 : 0;
-        const uint64_t bit = 1ull << li;
-        if (g.leaf[h] & bit) {
-            if (g.cnst[h] & bit) lvl[t * 64] = G;
-            // the next token roots a left operand: its adjoint waits in its mailbox
-            if (t > 0) G = lvl[start_of<HI>(g, t - 1) * 64];
+        const bool h = HI && t >= 64;
+        const int w = h ? rl_i(g.w1, li) : rl_i(g.w0, li);
+        const int op = w & 31;
+        if (op <= GPR_OP_ONE) {
+            if (op == GPR_OP_CONST) constant(t, G);
+            // the next token roots a left operand: its adjoint waits on the stack
+            if (t > 0) {
+                top--;
+#pragma unroll
+                for (int k = 0; k < KC; k++) G[k] = lvl[(top * KC + k) * 64];
+            }
             continue;
         }
-        float ga, gb;
-        if (g.cheap[h] & bit) {
-            const bool mul = (g.mul[h] & bit) != 0;
-            ga = G;
-            gb = (g.sub[h] & bit) ? -G : G;
-            const uint64_t rb = bit >> 1;
-            if (g.leaf[h] & rb) {
+        const int lr = (w >> 13) & 255, rr = (w >> 21) & 255;
+        if (op <= GPR_OP_RPOW) {
+            float ga[KC], gb[KC];
+            if (op <= GPR_OP_SUB) {
+                const bool sub = op == GPR_OP_SUB;
+#pragma unroll
+                for (int k = 0; k < KC; k++) { ga[k] = G[k]; gb[k] = sub ? -G[k] : G[k]; }
+            } else {
+                float A[KC], B[KC];
+                grad_val<KC, HI>(p, lr, x, lvl, A);
+                grad_val<KC, HI>(p, rr, x, lvl, B);
+                const int row = (w >> 5) & 255;
+#pragma unroll
+                for (int k = 0; k < KC; k++) {
+                    const float a = A[k], b = B[k], q = G[k];
+                    if (op == GPR_OP_MUL) {
+                        ga[k] = q * b;
+                        gb[k] = q * a;
+                        continue;
+                    }
+                    switch (op) {
+                    case GPR_OP_DIV: ga[k] = q / b; gb[k] = -(q * a) / (b * b); break;
+                    case GPR_OP_RSUB: ga[k] = -q; gb[k] = q; break;
+                    case GPR_OP_RDIV: gb[k] = q / a; ga[k] = -(q * b) / (a * a); break;
+                    case GPR_OP_POW: {
+                        const float v = lvl[(row * KC + k) * 64];
+                        ga[k] = q * b * pow_bm1(a, b, v);
+                        gb[k] = q * v * logf(a);
+                        break;
+                    }
+                    default: {  // RPOW: b^a
+                        const float v = lvl[(row * KC + k) * 64];
+                        gb[k] = q * a * pow_bm1(b, a, v);
+                        ga[k] = q * v * logf(b);
+                        break;
+                    }
+                    }
+                }
+            }
+            if (rr >= GPR_G_X) {
                 // right operand is a leaf: its adjoint is final now, and the left operand's
                 // subtree ends at t-2 and comes next, so its adjoint is carried
-                if (mul) {
-                    const float b = leaf_val<HI>(p, g, t - 1, x);
-                    const float a = tok_val<HI>(p, g, max(t - 2, 0), x, lvl);
-                    ga = G * b;
-                    gb = G * a;
-                }
-                if (g.cnst[h] & rb) lvl[(t - 1) * 64] = gb;
-                G = ga;
+                if (rr >= GPR_G_C && rr != GPR_G_ONE) constant(t - 1, gb);
+#pragma unroll
+                for (int k = 0; k < KC; k++) G[k] = ga[k];
                 t--;
                 continue;
             }
-            if (mul) {
-                const float a = tok_val<HI>(p, g, left_of<HI>(g, t), x, lvl);
-                const float b = tok_val<HI>(p, g, t - 1, x, lvl);
-                ga = G * b;
-                gb = G * a;
-            }
+#pragma unroll
+            for (int k = 0; k < KC; k++) { lvl[(top * KC + k) * 64] = ga[k]; G[k] = gb[k]; }
+            top++;
         } else {
-            const int op = h ? rl_i(p.o1, li) : rl_i(p.o0, li);
-            const float v = lvl[t * 64];
-            if (op <= GPR_OP_RPOW) {
-                const float a = tok_val<HI>(p, g, left_of<HI>(g, t), x, lvl);
-                const float b = tok_val<HI>(p, g, t - 1, x, lvl);
+            const float c = op >= GPR_OP_CADD ? (h ? rl_f(p.c1, li) : rl_f(p.c0, li)) : 0.0f;
+            float A[KC], gc[KC];
+            grad_val<KC, HI>(p, rr, x, lvl, A);
+            const int row = (w >> 5) & 255;
+#pragma unroll
+            for (int k = 0; k < KC; k++) {
+                const float a = A[k], v = lvl[(row * KC + k) * 64], q = G[k];
+                gc[k] = 0.0f;
                 switch (op) {
-                case GPR_OP_DIV: ga = G / b; gb = -(G * a) / (b * b); break;
-                case GPR_OP_RSUB: ga = -G; gb = G; break;
-                case GPR_OP_RDIV: gb = G / a; ga = -(G * b) / (a * a); break;
-                case GPR_OP_POW: ga = G * b * pow_bm1(a, b, v); gb = G * v * logf(a); break;
-                default: gb = G * a * pow_bm1(b, a, v); ga = G * v * logf(b); break;  // RPOW: b^a
+                case GPR_OP_NEG: G[k] = -q; break;
+                case GPR_OP_EXP: G[k] = q * v; break;
+                case GPR_OP_LOG: G[k] = q / a; break;
+                case GPR_OP_INV: G[k] = -q / (a * a); break;
+                case GPR_OP_SQRT: G[k] = q * 0.5f / v; break;
+                case GPR_OP_SIN: G[k] = q * cosf(a); break;
+                case GPR_OP_COS: G[k] = -q * sinf(a); break;
+                case GPR_OP_TAN: G[k] = q * (1.0f + v * v); break;
+                case GPR_OP_ASIN: G[k] = q / sqrtf(1.0f - a * a); break;
+                case GPR_OP_ACOS: G[k] = -q / sqrtf(1.0f - a * a); break;
+                case GPR_OP_ATAN: G[k] = q / (1.0f + a * a); break;
+                case GPR_OP_ABS: G[k] = a < 0.0f ? -q : q; break;
+                case GPR_OP_CADD: gc[k] = q; break;
+                case GPR_OP_CMUL: G[k] = q * c; gc[k] = q * a; break;
+                case GPR_OP_CPOW: G[k] = q * c * pow_bm1(a, c, v); gc[k] = q * v * logf(a); break;
+                case GPR_OP_CRPOW: G[k] = q * v * logf(c); gc[k] = q * a * pow_bm1(c, a, v); break;
+                default: G[k] = __builtin_nanf(""); break;
                 }
-            } else {
-                const float a = tok_val<HI>(p, g, t - 1, x, lvl);
-                const float c = op >= GPR_OP_CADD ? (h ? rl_f(p.c1, li) : rl_f(p.c0, li)) : 0.0f;
-                float gc = 0.0f;
-                switch (op) {
-                case GPR_OP_NEG: ga = -G; break;
-                case GPR_OP_EXP: ga = G * v; break;
-                case GPR_OP_LOG: ga = G / a; break;
-                case GPR_OP_INV: ga = -G / (a * a); break;
-                case GPR_OP_SQRT: ga = G * 0.5f / v; break;
-                case GPR_OP_SIN: ga = G * cosf(a); break;
-                case GPR_OP_COS: ga = -G * sinf(a); break;
-                case GPR_OP_TAN: ga = G * (1.0f + v * v); break;
-                case GPR_OP_ASIN: ga = G / sqrtf(1.0f - a * a); break;
-                case GPR_OP_ACOS: ga = -G / sqrtf(1.0f - a * a); break;
-                case GPR_OP_ATAN: ga = G / (1.0f + a * a); break;
-                case GPR_OP_ABS: ga = a < 0.0f ? -G : G; break;
-                case GPR_OP_CADD: ga = G; gc = G; break;
-                case GPR_OP_CMUL: ga = G * c; gc = G * a; break;
-                case GPR_OP_CPOW: ga = G * c * pow_bm1(a, c, v); gc = G * v * logf(a); break;
-                case GPR_OP_CRPOW: ga = G * v * logf(c); gc = G * a * pow_bm1(c, a, v); break;
-                default: ga = __builtin_nanf(""); break;
-                }
-                if (op >= GPR_OP_CADD) lvl[t * 64] = gc;
-                G = ga;
-                continue;
             }
+            if (op >= GPR_OP_CADD) constant(t, gc);
         }
-        // binary: the left operand's adjoint goes to the mailbox, the right one is carried
-        lvl[start_of<HI>(g, t) * 64] = ga;
-        G = gb;
     }
 }
 
-// FP32 wave sums of the per-point gradients in the slots of the constant-carrying tokens
-// (lanes with valid points only), placed at lane t of s0 (t < 64) or s1.  Two tokens per
-// pass so their reductions overlap.
-template <bool HI>
-__device__ __forceinline__ void grad_chunk_sums(uint64_t m0, uint64_t m1, const float *lvl, bool valid, float &s0,
-                                                float &s1) {
+// Both sweeps over KC chunks of 64 points from point `base`: their terms of the LL
+// ((f - y)^2 w, 0 past the last point) and the constants' sums of each chunk.
+template <int KC, bool HI>
+__device__ __forceinline__ void grad_sweeps(const WaveProg &p, const GradPlan &g, const GprDataset &d, const float *dx,
+                                            const float *dy, const float *dw, int base, float *lvl, float (&term)[KC],
+                                            float (&s0)[KC], float (&s1)[KC]) {
     const int l = lane_id();
+    const bool folded = d.wconst > 0.0;
+    const float wf = (float)d.wconst;
+    float x[KC], T[KC], G[KC];
+    bool valid[KC];
 #pragma unroll
-    for (int h = 0; h < (HI ? 2 : 1); h++) {
-        uint64_t m = h ? m1 : m0;
-        float s = 0.0f;
-        while (m) {
-            const int ta = __builtin_ctzll(m);
-            m &= m - 1;
-            const int tb = m ? __builtin_ctzll(m) : ta;
-            if (m) m &= m - 1;
-            const float va = lvl[(ta + 64 * h) * 64], vb = lvl[(tb + 64 * h) * 64];
-            const float sa = wave_sum_f(valid ? va : 0.0f), sb = wave_sum_f(valid ? vb : 0.0f);
-            s = l == ta ? sa : s;
-            s = l == tb ? sb : s;
-        }
-        if (h) s1 = s; else s0 = s;
+    for (int k = 0; k < KC; k++) {
+        const int i = base + 64 * k + l;
+        valid[k] = i < d.n;
+        x[k] = valid[k] ? dx[i] : 0.0f;
     }
+    grad_forward<KC, HI>(p, g, x, lvl, T);
+#pragma unroll
+    for (int k = 0; k < KC; k++) {
+        const int i = base + 64 * k + l;
+        const float y = valid[k] ? dy[i] : 0.0f, w = valid[k] ? dw[i] : 0.0f;
+        const float r = T[k] - y;
+        term[k] = valid[k] ? (r * r) * w : 0.0f;
+        // d/df of -(f - y)^2 w, with w = wconst when the weights are folded into it
+        G[k] = valid[k] ? (-2.0f * r) * (folded ? wf : w) : 0.0f;
+        s0[k] = s1[k] = 0.0f;
+    }
+    grad_reverse<KC, HI>(p, g, x, lvl, G, valid, s0, s1);
+}
+
+// the prior's -2c/(1+c^2) on the constant tokens of g0, g1; false when a gradient is not finite
+template <bool HI>
+__device__ __forceinline__ bool grad_prior(const WaveProg &p, double &g0, double &g1) {
+    const int l = lane_id();
+    const bool c0 = l < p.len && gpr_has_const(p.o0), c1 = HI && l + 64 < p.len && gpr_has_const(p.o1);
+    if (c0) g0 += -2.0 * (double)p.c0 / (1.0 + (double)p.c0 * (double)p.c0);
+    if (c1) g1 += -2.0 * (double)p.c1 / (1.0 + (double)p.c1 * (double)p.c1);
+    return ballot((c0 && !__builtin_isfinite(g0)) || (c1 && !__builtin_isfinite(g1))) == 0;
 }
 
 // Log-likelihood and d(log posterior)/d(constant) of the wave's program (g: its plan).
@@ -1374,47 +1400,29 @@ __device__ __forceinline__ void grad_chunk_sums(uint64_t m0, uint64_t m1, const 
 // c*64 + l in increasing c, the same per-lane order and Kahan updates.  The gradient
 // holds the wave sums of the per-point adjoints (FP32) accumulated over chunks in FP64,
 // plus the Cauchy prior's -2c/(1+c^2); token t sits at lane t of g0 (t < 64) or g1.
-// lv: this wave's LDS slab of at least len * 64 floats.  Returns false in ok when the
+// lv: this wave's slab of at least g.rows * 64 floats.  Returns false in ok when the
 // LL or a constant's gradient is not finite.
 template <bool HI>
 __device__ __forceinline__ double wave_loglik_grad(const WaveProg &p, const GradPlan &g, const GprDataset &d, const float *dx,
                                    const float *dy, const float *dw, float *lv, double &g0, double &g1, bool &ok) {
-    const int l = lane_id();
-    float *lvl = lv + l;
-    const bool c0 = l < p.len && gpr_has_const(p.o0), c1 = HI && l + 64 < p.len && gpr_has_const(p.o1);
-    const uint64_t m0 = ballot(c0), m1 = HI ? ballot(c1) : 0;
+    float *lvl = lv + lane_id();
     g0 = 0.0;
     g1 = 0.0;
     float acc = 0.0f, comp = 0.0f;
-    const bool folded = d.wconst > 0.0;
-    const float wf = (float)d.wconst;
-    const int nch = (d.n + 63) / 64;
-    for (int ch = 0; ch < nch; ch++) {
-        const int i = ch * 64 + l;
-        const bool valid = i < d.n;
-        const float x = valid ? dx[i] : 0.0f, y = valid ? dy[i] : 0.0f, w = valid ? dw[i] : 0.0f;
-        const float f = grad_forward<HI>(p, g, x, lvl);
-        const float r = f - y;
-        const float term = valid ? (r * r) * w : 0.0f;
-        const float yv = term - comp;
+    for (int base = 0; base < d.n; base += 64) {
+        float term[1], s0[1], s1[1];
+        grad_sweeps<1, HI>(p, g, d, dx, dy, dw, base, lvl, term, s0, s1);
+        const float yv = term[0] - comp;
         const float tv = acc + yv;
         comp = (tv - acc) - yv;
         acc = tv;
-        // d/df of -(f - y)^2 w, with w = wconst when the weights are folded into it
-        const float G = valid ? (-2.0f * r) * (folded ? wf : w) : 0.0f;
-        grad_reverse<HI>(p, g, x, lvl, G);
-        float s0 = 0.0f, s1 = 0.0f;
-        grad_chunk_sums<HI>(m0, m1, lvl, valid, s0, s1);
-        g0 += (double)s0;
-        if (HI) g1 += (double)s1;
+        g0 += (double)s0[0];
+        if (HI) g1 += (double)s1[0];
     }
     const double s = wave_sum_d((double)acc - (double)comp);
-    if (c0) g0 += -2.0 * (double)p.c0 / (1.0 + (double)p.c0 * (double)p.c0);
-    if (c1) g1 += -2.0 * (double)p.c1 / (1.0 + (double)p.c1 * (double)p.c1);
-    const bool bad = ballot((c0 && !__builtin_isfinite(g0)) || (c1 && !__builtin_isfinite(g1))) != 0;
-    ok = !bad && __builtin_isfinite(s);
+    ok = grad_prior<HI>(p, g0, g1) && __builtin_isfinite(s);
     if (!__builtin_isfinite(s)) return -GPR_INF;
-    return d.lconst - (folded ? d.wconst * s : s);
+    return d.lconst - (d.wconst > 0.0 ? d.wconst * s : s);
 }
 
 // FP64 sum of the Gaussian log-density terms -f^2 r2 (r2 = 1 / (2 e^2)) over the lanes where m holds, in

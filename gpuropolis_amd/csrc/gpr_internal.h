@@ -40,9 +40,10 @@ struct GprTile {
 };
 
 #define GPR_WAVES_PER_WG 4
-// MALA: token-value rows each wave of the MH kernel keeps in LDS (8 KB, the size the
-// forward-mode interpreter's stack takes anyway); the adjoint sweeps of longer programs
-// use the wave's slab in global memory (GprMHArgs::mala_gslab)
+// MALA: rows of the adjoint sweeps (operator values and pending adjoints) each wave of the
+// MH kernel keeps in LDS (8 KB, the size the forward-mode interpreter's stack takes anyway);
+// the sweeps of programs that need more use the wave's slab in global memory
+// (GprMHArgs::mala_gslab)
 #define GPR_MALA_LDS_ROWS 32
 #define GPR_WG 256
 
@@ -107,6 +108,7 @@ struct GprEvalArgs {
     double *ll;
     float *grad;            // gradient output (grad kernel)
     int per_wave;           // consecutive tapes a wave evaluates (set by the launcher)
+    int rows;               // gradient: LDS rows of a workgroup (set by the launcher)
     double lnsym;
 };
 

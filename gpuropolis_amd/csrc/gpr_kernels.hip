@@ -26,10 +26,10 @@
 // with early rejection.  Programs of at most three constants and stack depth 9, or eight
 // and depth 8, get the proposal's LL and gradient from one forward-mode
 // interpreter pass (value and tangents per stack entry); the others are pre-checked by
-// the plain interpreter, and the survivors get the stack-free adjoint sweeps, whose token values sit in the wave's LDS
-// region for programs of at most GPR_MALA_LDS_ROWS tokens and in the wave's slab in
-// global memory for longer ones (LDS rows for every token of a 128-token cap, 32 KB per
-// wave, would leave room for five waves per CU).  The current structure's sweep plan
+// the plain interpreter, and the survivors get the adjoint sweeps, whose rows sit in the
+// wave's LDS region for programs that need at most GPR_MALA_LDS_ROWS of them and in the wave's
+// slab in global memory for longer ones (LDS rows for every token of a 128-token cap, 32 KB
+// per wave, would leave room for five waves per CU).  The current structure's sweep plan
 // stays in registers.
 extern __shared__ float gpr_lds_slab[];
 
@@ -70,10 +70,9 @@ k_mh_config_wave(GprMHArgs a) {
     const int l = lane_id();
     const int N = a.nchains;
     // dynamic LDS: the value stacks of the wpg waves.  Under MALA each wave's LDS region
-    // (MROWS rows of 64 floats) also holds the token values of the adjoint sweeps of
-    // programs of at most GPR_MALA_LDS_ROWS tokens (the interpreter's stack and the sweeps
-    // are never in use at once); longer programs sweep through the wave's slab in global
-    // memory, lvg.
+    // (MROWS rows of 64 floats) also holds the rows of the adjoint sweeps of programs that
+    // need at most GPR_MALA_LDS_ROWS of them (the interpreter's stack and the sweeps are never
+    // in use at once); longer programs sweep through the wave's slab in global memory, lvg.
     constexpr int SROWS = GPR_MAX_DEPTH + 2;
     constexpr int MROWS = SROWS > GPR_MALA_LDS_ROWS ? SROWS : GPR_MALA_LDS_ROWS;
     // (the forward-mode interpreter's stack of value + tangents shares it too)
@@ -470,7 +469,7 @@ k_mh_config_wave(GprMHArgs a) {
                             gok = gok && __builtin_isfinite(cl);
                         } else {
                             (void)wave_loglik_grad<HI>(cur, gplan, d, dx, dy, dw,
-                                                       cur.len <= GPR_MALA_LDS_ROWS ? ls : lvg, h0, h1, gok);
+                                                       gplan.rows <= GPR_MALA_LDS_ROWS ? ls : lvg, h0, h1, gok);
                         }
                         c_fl += (unsigned long long)(cur_opq - 2 + cur_nc) * (unsigned long long)d.n;
                         cg0 = gok ? (float)h0 : 0.0f;
@@ -544,7 +543,7 @@ k_mh_config_wave(GprMHArgs a) {
                     bool rejected = (cur_dual || precheck) && !__builtin_isfinite(pll_m) && __builtin_isfinite(post);
                     if (!cur_dual && !rejected) {
                         const double gl = wave_loglik_grad<HI>(prop, gplan, d, dx, dy, dw,
-                                                               prop.len <= GPR_MALA_LDS_ROWS ? ls : lvg, h0, h1, pok);
+                                                               gplan.rows <= GPR_MALA_LDS_ROWS ? ls : lvg, h0, h1, pok);
                         if (!precheck) {
                             pll_m = gl;
                             mala_pts = d.n;
@@ -1175,30 +1174,92 @@ hipError_t gpr_launch_eval_wave(const GprEvalArgs &args, hipStream_t s) {
     return hipGetLastError();
 }
 
-// Gradient of the log posterior of each tape (one wave per tape, LDS slab of cap * 64
-// floats per wave for the token values and adjoint mailboxes).  grad rows t < cap: d/dc_t, 0 where token t
-// has no constant or t >= len.  ll receives the log posterior.
+// Gradient of the log posterior of each tape: one workgroup per tape, whose waves (1 to 8,
+// by the dataset's size) share its chunks of points.  grad rows t < cap: d/dc_t, 0 where
+// token t has no constant or t >= len.  ll receives the log posterior.
+//
+// The sweeps are bound by scalar instructions and the latency of one token after another, so
+// they want waves, and LDS rows are what limits those (rows for every token of a 128-token
+// cap in every wave left one wave per SIMD).  The workgroup has a.rows rows of 64 floats, at
+// least what the longest program of the cap needs by itself.  A program runs two points per
+// lane, which halves the scalar work per point, when the rows hold that in every wave, else
+// one point per lane in as many waves as they allow.  The waves take their chunks in turn, a
+// round of at most 16 chunks at a time; the terms of the LL meet in LDS and are added in chunk
+// order (bit-identical to wave_loglik), the constants' FP64 sums wave by wave.  6007 tapes
+// (cap 128, every op) at n = 1021 took 2831 us with a wave per tape and a row per token, 772
+// with two points per lane wherever one wave holds them, and take 602.
+template <int KC, bool HI>
+__device__ __forceinline__ void grad_rounds(const GprEvalArgs &a, const WaveProg &p, const GradPlan &g, const float *dx,
+                                            const float *dy, const float *dw, float *rows, int wave, int waves,
+                                            float *term_lds, double &g0, double &g1, float &acc, float &comp) {
+    const int l = lane_id();
+    const int use = min(waves, a.rows / (KC * uni(g.rows)));     // waves that have rows (at least one point's: g.rows >= 1)
+    float *lvl = rows + (size_t)(wave < use ? wave : 0) * (KC * g.rows * 64) + l;
+    for (int base = 0; base < a.d.n; base += 1024) {
+        if (wave < use) {
+            for (int c = KC * wave; c < 16 && base + 64 * c < a.d.n; c += KC * use) {
+                float term[KC], s0[KC], s1[KC];
+                grad_sweeps<KC, HI>(p, g, a.d, dx, dy, dw, base + 64 * c, lvl, term, s0, s1);
+#pragma unroll
+                for (int k = 0; k < KC; k++) {
+                    if (base + 64 * (c + k) >= a.d.n) break;
+                    term_lds[64 * (c + k) + l] = term[k];
+                    g0 += (double)s0[k];
+                    if (HI) g1 += (double)s1[k];
+                }
+            }
+        }
+        __syncthreads();
+        if (wave == 0) {
+            const int m = min((a.d.n - base + 63) / 64, 16);
+            for (int k = 0; k < m; k++) {
+                const float yv = term_lds[64 * k + l] - comp;
+                const float tv = acc + yv;
+                comp = (tv - acc) - yv;
+                acc = tv;
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// LDS floats: the rows, then one term per point of a round (the waves' gradients meet in the
+// rows afterwards: 128 doubles a wave)
 template <bool HI>
-__global__ void __launch_bounds__(GPR_WG) k_grad_wave(GprEvalArgs a) {
+__global__ void __launch_bounds__(512) k_grad_wave(GprEvalArgs a) {
+    float *term_lds = gpr_lds_slab + a.rows * 64;
+    double *s_g = (double *)gpr_lds_slab;
+    const int waves = (int)(blockDim.x >> 6);
     const int wave = uni((int)(threadIdx.x >> 6));
     const int l = lane_id();
-    const int chain = uni((int)blockIdx.x * GPR_WAVES_PER_WG + wave);
-    if (chain >= a.nchains) return;
-    const int N = a.nchains;
-    float *lv = gpr_lds_slab + (size_t)wave * a.cap * 64;
-    WaveProg p;
-    // a length outside [0, cap] is clamped: the kernel never reads or writes past the
-    // caller's cap rows or its LDS slab (a malformed tape yields a meaningless value)
-    p.len = min(max(uni(a.len[chain]), 0), a.cap);
-    p.o0 = l < p.len ? a.ops[(size_t)l * N + chain] : 0;
-    p.c0 = l < p.len ? a.cs[(size_t)l * N + chain] : 0.0f;
-    p.o1 = (HI && l + 64 < p.len) ? a.ops[(size_t)(l + 64) * N + chain] : 0;
-    p.c1 = (HI && l + 64 < p.len) ? a.cs[(size_t)(l + 64) * N + chain] : 0.0f;
-    double g0, g1;
-    bool ok;
+    const int chain = (int)blockIdx.x;
+    const size_t N = (size_t)a.nchains;
+    const WaveProg p = eval_load<HI>(a, chain);
     const float *dx = a.dx + a.d.off, *dy = a.dy + a.d.off, *dw = a.dw + a.d.off;
-    const GradPlan g = grad_plan<HI>(p);
-    const double ll = wave_loglik_grad<HI>(p, g, a.d, dx, dy, dw, lv, g0, g1, ok);
+    double g0 = 0.0, g1 = 0.0, ll = -GPR_INF;
+    float acc = 0.0f, comp = 0.0f;
+    if (eval_depth<HI>(p)) {                 // the same in every wave
+        GradPlan g = grad_plan<HI>(p);
+        g.rows = max(uni(g.rows), 1);
+        if (a.d.n > 64 && 2 * g.rows * waves <= a.rows)
+            grad_rounds<2, HI>(a, p, g, dx, dy, dw, gpr_lds_slab, wave, waves, term_lds, g0, g1, acc, comp);
+        else
+            grad_rounds<1, HI>(a, p, g, dx, dy, dw, gpr_lds_slab, wave, waves, term_lds, g0, g1, acc, comp);
+        const double s = wave_sum_d((double)acc - (double)comp);     // wave 0's
+        if (__builtin_isfinite(s)) ll = a.d.lconst - (a.d.wconst > 0.0 ? a.d.wconst * s : s);
+    }
+    if (waves > 1) {
+        s_g[128 * wave + l] = g0;
+        s_g[128 * wave + 64 + l] = g1;
+        __syncthreads();
+        if (wave != 0) return;
+        g0 = g1 = 0.0;
+        for (int w = 0; w < waves; w++) {
+            g0 += s_g[128 * w + l];
+            g1 += s_g[128 * w + 64 + l];
+        }
+    }
+    (void)grad_prior<HI>(p, g0, g1);
     const double pr = wave_prior<HI>(p, a.lnsym);
     if (l < a.cap) a.grad[(size_t)l * N + chain] = (l < p.len && gpr_has_const(p.o0)) ? (float)g0 : 0.0f;
     if (HI && l + 64 < a.cap)
@@ -1206,15 +1267,20 @@ __global__ void __launch_bounds__(GPR_WG) k_grad_wave(GprEvalArgs a) {
     if (l == 0) a.ll[chain] = pr + ll;
 }
 
-hipError_t gpr_launch_grad_wave(const GprEvalArgs &a, hipStream_t s) {
-    const int grid = (a.nchains + GPR_WAVES_PER_WG - 1) / GPR_WAVES_PER_WG;
-    const size_t sh = sizeof(float) * 64 * (size_t)a.cap * GPR_WAVES_PER_WG;
-    const bool hi = a.cap > 64;
-    const void *f = hi ? (const void *)k_grad_wave<true> : (const void *)k_grad_wave<false>;
-    hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh);
-    if (e != hipSuccess) return e;
-    if (hi) hipLaunchKernelGGL(k_grad_wave<true>, dim3(grid), dim3(GPR_WG), sh, s, a);
-    else hipLaunchKernelGGL(k_grad_wave<false>, dim3(grid), dim3(GPR_WG), sh, s, a);
+hipError_t gpr_launch_grad_wave(const GprEvalArgs &args, hipStream_t s) {
+    GprEvalArgs a = args;
+    // waves: one per two chunks of 64 points.  Eight share their rows at 16 each, which a
+    // cap over 64 outgrows (6007 tapes of cap 128 at n = 1021: 602 us by four, 694 by eight; 30000
+    // of cap 64 at 1024: 915 and 870), unless so few tapes are asked for that their latency counts
+    // (one tape of cap 64 at n = 1000: 56 and 36).
+    const bool eight = a.d.n > 512 && (a.cap <= 64 || a.nchains < 1024);
+    const int waves = a.d.n <= 128 ? 1 : (a.d.n <= 256 ? 2 : (eight ? 8 : 4));
+    // a program needs at most cap - 1 rows; 16 rows a wave hold the common ones at two points
+    // per lane, and the waves' gradients (4 rows a wave)
+    a.rows = std::max(a.cap, 16 * waves);
+    const size_t sh = sizeof(float) * 64 * ((size_t)a.rows + std::min((a.d.n + 63) / 64, 16));
+    if (a.cap > 64) hipLaunchKernelGGL(k_grad_wave<true>, dim3(a.nchains), dim3(64 * waves), sh, s, a);
+    else hipLaunchKernelGGL(k_grad_wave<false>, dim3(a.nchains), dim3(64 * waves), sh, s, a);
     return hipGetLastError();
 }
 
