@@ -9,10 +9,10 @@ adjoint inside the MH kernel.
 The constants cross the C ABI as float32 (the kernels' arithmetic type); a float64 cs
 is rounded on the way in and its gradient returned as float64.
 
-The arguments are checked before anything reaches the device: ops, cs and length are
-tensors on the context's GPU, ops is uint8 of the shape of cs, [cap, N] with
-1 <= cap <= 128, length holds N lengths in [1, cap], and every tape is well-formed
-postfix whose evaluation stack stays within 16 entries.
+The arguments are checked: ops, cs and length are tensors on the context's GPU, ops is
+uint8 of the shape of cs, [cap, N] with 1 <= cap <= 128, and (on the device, by the kernel
+that uses the tapes) length holds N lengths in [1, cap], and every tape is well-formed
+postfix of known ops whose evaluation stack stays within 16 entries.
 """
 import torch
 
@@ -33,19 +33,24 @@ def _check(gctx, ops, cs, length):
         raise G.GprError(f"cap must be in [1, {G.MAX_CAP}] and N >= 1; got cap {cap}, N {n}")
     if length.dim() != 1 or length.shape[0] != n:
         raise G.GprError(f"length must hold N = {n} entries")
-    check_tapes(ops.cpu(), length.cpu())
+
+
+TAPE_ERRORS = ((G.TAPE_LENGTH, "every length must lie in [1, cap]"), (G.TAPE_OP, "bad op code"),
+               (G.TAPE_POSTFIX, "every tape must be well-formed postfix"),
+               (G.TAPE_DEPTH, f"tape evaluation stacks must stay within {G.MAX_DEPTH} entries"))
 
 
 def check_tapes(ops, length):
     """Host check of tapes ops [cap, N] (uint8) with lengths [N]: lengths in [1, cap],
-    known op codes, well-formed postfix, evaluation stack within MAX_DEPTH entries."""
+    known op codes, well-formed postfix, evaluation stack within MAX_DEPTH entries (what
+    gpr_grad_logpost_checked checks on the device)."""
     cap, n = ops.shape
     ln = length.to(torch.int64)
     if int(ln.min()) < 1 or int(ln.max()) > cap:
-        raise G.GprError("every length must lie in [1, cap]")
+        raise G.GprError(TAPE_ERRORS[0][1])
     o = ops.to(torch.int64)
     if int(o.max()) >= len(G.OPS):
-        raise G.GprError("bad op code")
+        raise G.GprError(TAPE_ERRORS[1][1])
     arity = torch.tensor([_arity(k) for k in range(len(G.OPS))], dtype=torch.int64)
     step = 1 - arity[o]                                           # stack change per token, [cap, N]
     live = torch.arange(cap)[:, None] < ln[None, :]
@@ -53,9 +58,9 @@ def check_tapes(ops, length):
     need = torch.where(live, torch.cat([torch.zeros(1, n, dtype=torch.int64), depth[:-1]]) - arity[o],
                        torch.zeros_like(step))
     if int(need.min()) < 0 or not bool(torch.all(depth[-1] == 1)):
-        raise G.GprError("every tape must be well-formed postfix")
+        raise G.GprError(TAPE_ERRORS[2][1])
     if int(depth.max()) > G.MAX_DEPTH:
-        raise G.GprError(f"tape evaluation stacks must stay within {G.MAX_DEPTH} entries")
+        raise G.GprError(TAPE_ERRORS[3][1])
 
 
 def _arity(op):
@@ -73,14 +78,19 @@ class LogPosterior(torch.autograd.Function):
         _check(gctx, ops, cs, length)
         cap, n = ops.shape
         ops = ops.contiguous()
-        length = length.to(torch.int32).contiguous()
+        if length.dtype != torch.int32:       # (lengths that int32 cannot hold stay outside [1, cap])
+            length = length.to(torch.int64).clamp(0, cap + 1).to(torch.int32)
+        length = length.contiguous()
         cs32 = cs.detach().to(torch.float32).contiguous()
         grad = torch.empty_like(cs32)
         lp = torch.empty(n, dtype=torch.float64, device=cs.device)
         # the library runs on its own stream: inputs made on torch's stream must be ready
         torch.cuda.current_stream(cs.device).synchronize()
-        gctx.grad_logpost_dev(dataset, ops.data_ptr(), cs32.data_ptr(), length.data_ptr(), n, cap,
-                              grad.data_ptr(), lp.data_ptr())
+        faults = gctx.grad_logpost_checked_dev(dataset, ops.data_ptr(), cs32.data_ptr(), length.data_ptr(), n, cap,
+                                               grad.data_ptr(), lp.data_ptr())
+        for bit, what in TAPE_ERRORS:
+            if faults & bit:
+                raise G.GprError(what)
         fctx.save_for_backward(grad)
         fctx.in_dtype = cs.dtype
         return lp

@@ -71,6 +71,7 @@ struct gpr_ctx {
     bool any_metric = false;
     int *d_tile_counter = nullptr;  // one per bucket
     unsigned long long *d_counters = nullptr;
+    int32_t *d_faults = nullptr;       // gpr_grad_logpost_checked
     int32_t *d_good = nullptr, *d_ngood = nullptr, *d_map_chain = nullptr, *d_nres = nullptr;
     float *d_gslab = nullptr;          // MALA token slabs of programs beyond the LDS rows
     size_t gslab_floats = 0;
@@ -126,7 +127,7 @@ static void free_state(gpr_ctx *c) {
     drop_graph(c);
     void *ps[] = {c->d_ds, c->d_x, c->d_y, c->d_w, c->d_sd, c->d_lnc, c->d_ops, c->d_cs, c->d_len, c->d_prior, c->d_ll,
                   c->d_tiles, c->d_tile_counter, c->d_counters, c->d_good, c->d_ngood, c->d_map_chain,
-                  c->d_nres, c->d_map_post, c->d_cutoff, c->d_clock, c->d_metric, c->d_gslab};
+                  c->d_nres, c->d_map_post, c->d_cutoff, c->d_clock, c->d_metric, c->d_gslab, c->d_faults};
     for (void *p : ps)
         if (p) (void)hipFree(p);
     c->d_ds = nullptr; c->d_x = c->d_y = c->d_w = c->d_sd = nullptr; c->d_lnc = nullptr; c->d_ops = nullptr; c->d_cs = nullptr;
@@ -134,6 +135,7 @@ static void free_state(gpr_ctx *c) {
     c->d_tile_counter = nullptr; c->d_counters = nullptr; c->d_good = c->d_ngood = c->d_map_chain = nullptr;
     c->d_nres = nullptr; c->d_map_post = c->d_cutoff = nullptr; c->d_clock = nullptr; c->d_metric = nullptr;
     c->d_gslab = nullptr;
+    c->d_faults = nullptr;
     c->gslab_floats = 0;
     c->hmetric.clear();
     c->any_metric = false;
@@ -366,6 +368,7 @@ extern "C" int gpr_set_data(gpr_ctx *c, int nd, const int32_t *n, const float *x
     for (GprMetric &m : c->hmetric) memset(m.slot, -1, sizeof(m.slot));
     ALLOC(c->d_cutoff, (size_t)nd);
     ALLOC(c->d_nres, 1);
+    ALLOC(c->d_faults, 1);
     // everything on the context stream (non-blocking, so not ordered with the null
     // stream's asynchronous memsets), finished before returning
     const hipStream_t st = c->stream;
@@ -985,8 +988,8 @@ extern "C" int gpr_eval_loglik(gpr_ctx *c, int dataset, const uint8_t *d_ops, co
     return GPR_OK;
 }
 
-extern "C" int gpr_grad_logpost(gpr_ctx *c, int dataset, const uint8_t *d_ops, const float *d_cs,
-                                const int32_t *d_len, int nchains, int cap, float *d_grad, double *d_lp) {
+static int grad_logpost(gpr_ctx *c, int dataset, const uint8_t *d_ops, const float *d_cs, const int32_t *d_len,
+                        int nchains, int cap, float *d_grad, double *d_lp, int32_t *faults) {
     if (!c || !c->have_data) return fail(GPR_E_STATE, "gpr_set_data must come first");
     if (dataset < 0 || dataset >= c->nd) return fail(GPR_E_ARG, "dataset index out of range");
     if (!d_ops || !d_cs || !d_len || !d_grad || !d_lp || nchains < 1) return fail(GPR_E_ARG, "null or empty arrays");
@@ -999,9 +1002,26 @@ extern "C" int gpr_grad_logpost(gpr_ctx *c, int dataset, const uint8_t *d_ops, c
     a.ll = d_lp;
     a.grad = d_grad;
     a.lnsym = log((double)c->cfg.nsym);
+    if (faults) {
+        a.faults = c->d_faults;
+        HIP_TRY(gpr_launch_fill_i32(c->d_faults, 1, 0, c->stream));
+    }
     HIP_TRY(gpr_launch_grad_wave(a, c->stream));
+    if (faults) HIP_TRY(hipMemcpyAsync(faults, c->d_faults, sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     return GPR_OK;
+}
+
+extern "C" int gpr_grad_logpost(gpr_ctx *c, int dataset, const uint8_t *d_ops, const float *d_cs,
+                                const int32_t *d_len, int nchains, int cap, float *d_grad, double *d_lp) {
+    return grad_logpost(c, dataset, d_ops, d_cs, d_len, nchains, cap, d_grad, d_lp, nullptr);
+}
+
+extern "C" int gpr_grad_logpost_checked(gpr_ctx *c, int dataset, const uint8_t *d_ops, const float *d_cs,
+                                        const int32_t *d_len, int nchains, int cap, float *d_grad, double *d_lp,
+                                        int32_t *faults) {
+    if (!faults) return fail(GPR_E_ARG, "null faults");
+    return grad_logpost(c, dataset, d_ops, d_cs, d_len, nchains, cap, d_grad, d_lp, faults);
 }
 
 // ---------------------------------------------------------------- no-allocation evaluation

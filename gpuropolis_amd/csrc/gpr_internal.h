@@ -109,6 +109,8 @@ struct GprEvalArgs {
     float *grad;            // gradient output (grad kernel)
     int per_wave;           // consecutive tapes a wave evaluates (set by the launcher)
     int rows;               // gradient: LDS rows of a workgroup (set by the launcher)
+    int32_t *faults;        // gradient: when set, tapes are checked and what they break (GPR_TAPE_*)
+                            // is or-ed in here
     double lnsym;
 };
 

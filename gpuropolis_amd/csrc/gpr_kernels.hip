@@ -1188,6 +1188,25 @@ hipError_t gpr_launch_eval_wave(const GprEvalArgs &args, hipStream_t s) {
 // order (bit-identical to wave_loglik), the constants' FP64 sums wave by wave.  6007 tapes
 // (cap 128, every op) at n = 1021 took 2831 us with a wave per tape and a row per token, 772
 // with two points per lane wherever one wave holds them, and take 602.
+// What a tape breaks (GPR_TAPE_*): its length, an op code (anywhere in its cap rows), postfix
+// form, or the stack's bound, in the order a host check of all tapes would report them.
+template <bool HI>
+__device__ __forceinline__ int tape_faults(const GprEvalArgs &a, int chain, const WaveProg &p) {
+    const int l = lane_id();
+    const size_t N = (size_t)a.nchains;
+    const int len = uni(a.len[chain]);
+    const int o0 = l < a.cap ? a.ops[(size_t)l * N + chain] : 0;
+    const int o1 = HI && l + 64 < a.cap ? a.ops[(size_t)(l + 64) * N + chain] : 0;
+    const int f = (len < 1 || len > a.cap ? GPR_TAPE_LENGTH : 0) |
+                  (ballot(o0 >= GPR_NUM_OPS || o1 >= GPR_NUM_OPS) ? GPR_TAPE_OP : 0);
+    if (f) return f;
+    int D0, D1, dm;
+    wave_depths<HI>(p, D0, D1, dm);
+    const int end = HI && len > 64 ? rl_i(D1, (len - 1) & 63) : rl_i(D0, (len - 1) & 63);
+    if (end != 1 || ballot((l < len && D0 < 1) || (HI && l + 64 < len && D1 < 1))) return GPR_TAPE_POSTFIX;
+    return dm > GPR_MAX_DEPTH ? GPR_TAPE_DEPTH : 0;
+}
+
 template <int KC, bool HI>
 __device__ __forceinline__ void grad_rounds(const GprEvalArgs &a, const WaveProg &p, const GradPlan &g, const float *dx,
                                             const float *dy, const float *dw, float *rows, int wave, int waves,
@@ -1238,6 +1257,13 @@ __global__ void __launch_bounds__(512) k_grad_wave(GprEvalArgs a) {
     const float *dx = a.dx + a.d.off, *dy = a.dy + a.d.off, *dw = a.dw + a.d.off;
     double g0 = 0.0, g1 = 0.0, ll = -GPR_INF;
     float acc = 0.0f, comp = 0.0f;
+    if (a.faults) {                          // the same in every wave
+        const int f = tape_faults<HI>(a, chain, p);
+        if (f) {
+            if (threadIdx.x == 0) atomicOr(a.faults, f);
+            return;
+        }
+    }
     if (eval_depth<HI>(p)) {                 // the same in every wave
         GradPlan g = grad_plan<HI>(p);
         g.rows = max(uni(g.rows), 1);

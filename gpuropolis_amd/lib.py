@@ -36,7 +36,8 @@ EXPORTS = ["gpr_config_default", "gpr_create", "gpr_destroy", "gpr_last_error", 
            "gpr_eval_loglik", "gpr_grad_logpost", "gpr_ref_decode", "gpr_test_ref_decode", "gpr_test_draws",
            "gpr_autotune", "gpr_set_tuning", "gpr_get_tuning", "gpr_set_metric", "gpr_ref_op_set",
            "gpr_get_clock", "gpr_set_clock", "gpr_eval_loglik_noalloc_async", "gpr_write_heap_i32",
-           "gpr_read_heap_i32"]
+           "gpr_read_heap_i32", "gpr_grad_logpost_checked"]
+TAPE_LENGTH, TAPE_OP, TAPE_POSTFIX, TAPE_DEPTH = 1, 2, 4, 8
 NOALLOC_MAX_POINTS = 65536
 
 
@@ -101,6 +102,8 @@ def load():
         "gpr_stream": (vp, [vp]),
         "gpr_eval_loglik": (C.c_int, [vp, C.c_int, vp, vp, vp, C.c_int, C.c_int, C.c_int, vp]),
         "gpr_grad_logpost": (C.c_int, [vp, C.c_int, vp, vp, vp, C.c_int, C.c_int, vp, vp]),
+        "gpr_grad_logpost_checked": (C.c_int, [vp, C.c_int, vp, vp, vp, C.c_int, C.c_int, vp, vp,
+                                               C.POINTER(C.c_int32)]),
         "gpr_autotune": (C.c_int, [vp, C.c_int, C.POINTER(Tune), C.c_int, C.POINTER(C.c_int)]),
         "gpr_set_metric": (C.c_int, [vp, C.c_int, C.c_int, vp, vp]),
         "gpr_set_tuning": (C.c_int, [vp, C.POINTER(Tune), C.c_int, C.c_int]),
@@ -294,6 +297,13 @@ class Context:
 
     def grad_logpost_dev(self, dataset, d_ops, d_cs, d_len, nchains, cap, d_grad, d_lp):
         check(load().gpr_grad_logpost(self.h, dataset, d_ops, d_cs, d_len, nchains, cap, d_grad, d_lp))
+
+    def grad_logpost_checked_dev(self, dataset, d_ops, d_cs, d_len, nchains, cap, d_grad, d_lp):
+        """grad_logpost_dev on tapes that may be wrong; returns their TAPE_* bits (0: all sound)."""
+        faults = C.c_int32(0)
+        check(load().gpr_grad_logpost_checked(self.h, dataset, d_ops, d_cs, d_len, nchains, cap, d_grad, d_lp,
+                                              C.byref(faults)))
+        return faults.value
 
 
 def eval_loglik_noalloc_async(device, d_x, d_y, d_sd, n, d_ops, d_cs, d_len, nchains, cap, schedule, d_ll,

@@ -238,6 +238,15 @@ int gpr_eval_loglik(gpr_ctx *ctx, int dataset, const uint8_t *d_ops, const float
 int gpr_grad_logpost(gpr_ctx *ctx, int dataset, const uint8_t *d_ops, const float *d_cs,
                      const int32_t *d_len, int nchains, int cap, float *d_grad, double *d_lp);
 
+/* The same for tapes that may be wrong: gpr_grad_logpost's preconditions are checked on the
+ * device, by the kernel that would use the tape.  *faults receives the GPR_TAPE_* bits of all
+ * tapes (0: every tape is sound); when it is not 0 the contents of d_grad and d_lp are
+ * unspecified.  Op codes are checked in all cap rows.  No reference counterpart. */
+enum { GPR_TAPE_LENGTH = 1, GPR_TAPE_OP = 2, GPR_TAPE_POSTFIX = 4, GPR_TAPE_DEPTH = 8 };
+int gpr_grad_logpost_checked(gpr_ctx *ctx, int dataset, const uint8_t *d_ops, const float *d_cs,
+                             const int32_t *d_len, int nchains, int cap, float *d_grad, double *d_lp,
+                             int32_t *faults);
+
 /* gpr_eval_loglik without a context and without allocating anything.  No counterpart in
  * the reference (which allocates everything up front, main.cu:1123-1147); it is for
  * callers that cannot allocate device memory: code under HIP graph capture, serving

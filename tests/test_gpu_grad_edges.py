@@ -40,3 +40,51 @@ def test_gradients_at_the_edges(oracle, gpr, cap, n, copies):
         assert not g[L[i]:, i].any()
     for c in range(1, copies):      # a tape's result does not depend on its place
         assert np.array_equal(g[:, :k], g[:, c * k:(c + 1) * k]) and np.array_equal(lp[:k], lp[c * k:(c + 1) * k])
+
+
+@pytest.mark.parametrize("fault", ["none", "zero length", "length over cap", "op past the end", "pops an empty stack",
+                                   "two values left", "depth 17"])
+@pytest.mark.parametrize("cap", [40, 100])
+def test_tapes_checked_on_the_device(oracle, gpr, cap, fault):
+    """gpr_grad_logpost_checked reports what the host check of the same tapes reports, and the
+    torch function raises its message, with one bad tape among many."""
+    import torch
+    from gpuropolis_amd import autograd
+    n = 130
+    O = np.zeros((cap, n), dtype=np.uint8)
+    L = np.full(n, 5, dtype=np.int64)
+    x, c, add, mul = (gpr.OP[k] for k in ("X", "CONST", "ADD", "MUL"))
+    O[:5] = np.array([c, x, mul, c, add], dtype=np.uint8)[:, None]
+    bad = 77
+    if fault == "zero length":
+        L[bad] = 0
+    elif fault == "length over cap":
+        L[bad] = cap + 1
+    elif fault == "op past the end":
+        O[cap - 1, bad] = len(gpr.OPS)
+    elif fault == "pops an empty stack":
+        O[:5, bad] = [x, add, x, x, add]
+    elif fault == "two values left":
+        L[bad] = 4
+    elif fault == "depth 17":
+        O[:33, bad] = [x] * 17 + [add] * 16
+        L[bad] = 33
+    want = None
+    try:
+        autograd.check_tapes(torch.from_numpy(O), torch.from_numpy(L))
+    except gpr.GprError as e:
+        want = str(e)
+    assert (want is None) == (fault == "none")
+    with gpr.Context(cap=cap) as ctx:
+        ctx.set_data([dataset(70, False)], [1])
+        say(f"device check: {fault}, cap {cap}")
+        for dtype in (torch.int32, torch.int64):
+            cs = torch.full((cap, n), 0.5, device="cuda", requires_grad=True)
+            args = (ctx, 0, dev(O), cs, dev(L).to(dtype))
+            if want is None:
+                autograd.log_posterior(*args).sum().backward()
+                assert bool(torch.isfinite(cs.grad).all())
+            else:
+                with pytest.raises(gpr.GprError) as e:
+                    autograd.log_posterior(*args)
+                assert str(e.value) == want
