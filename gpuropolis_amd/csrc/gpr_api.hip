@@ -1072,7 +1072,6 @@ extern "C" int gpr_eval_loglik_noalloc_async(int device, const float *d_x, const
     float *w = (float *)(sp + GPR_NOALLOC_HDR_BYTES);
     const hipStream_t s = (hipStream_t)stream;
     const int kc = kc_for(n);
-    HIP_TRY(gpr_launch_dataset_prep(d_sd, n, nchains, cap, kc, hdr, w, s));
     GprEvalArgs a{};
     a.ops = d_ops; a.cs = d_cs; a.len = d_len; a.nchains = nchains; a.cap = cap;
     a.dx = d_x; a.dy = d_y; a.dw = w;
@@ -1080,8 +1079,16 @@ extern "C" int gpr_eval_loglik_noalloc_async(int device, const float *d_x, const
     a.d.kc = kc;
     a.d.cap = cap;
     a.d.nchains = nchains;
-    a.dd = hdr;
     a.ll = d_ll;
+    // A launch costs about 5 us on the stream.  A small dataset's constants are formed by the
+    // evaluator's own workgroups instead, while they are few enough to run at once.
+    a.raw = schedule != GPR_SCHED_LANE && n <= GPR_RAW_POINTS && nchains <= 4096;
+    if (a.raw) {
+        a.dw = d_sd;
+    } else {
+        HIP_TRY(gpr_launch_dataset_prep(d_sd, n, nchains, cap, kc, hdr, w, s));
+        a.dd = hdr;
+    }
     if (schedule == GPR_SCHED_LANE) HIP_TRY(gpr_launch_eval_lane(a, s));
     else HIP_TRY(gpr_launch_eval_wave(a, s));
     return GPR_OK;

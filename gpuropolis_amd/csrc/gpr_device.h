@@ -441,12 +441,16 @@ __device__ __forceinline__ void wave_eval_ls(const WaveProg &p, const float (&xs
         // (uni: wave-uniform in any case, but the block needs it in a scalar register)
         const int n = uni(min(p.len - 64 * h, 64)), word = HI && h ? m.w1 : m.w0, o = HI && h ? p.o1 : p.o0;
         const float c = HI && h ? p.c1 : p.c0;
-        for (int t = 0; t < n; t++) {
+        for (int t = 0; t < n;) {
             t = uni(t);
             tape_run(word, c, xs, T, U, a, t);
             t = uni(t);
-            if (t >= n) break;
-            tape_slow<KC>(rl_i(o, t), rl_f(c, t), xs, T, U, a);
+            // tokens without a handler, until one that has one
+            while (t < n) {
+                tape_slow<KC>(rl_i(o, t), rl_f(c, t), xs, T, U, a);
+                t++;
+                if (rl_i(word, t & 63) != GPR_U_EXIT) break;
+            }
         }
     }
 }

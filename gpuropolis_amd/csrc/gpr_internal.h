@@ -94,6 +94,7 @@ struct GprMHArgs {
     double ref_lnops;
 };
 
+#define GPR_RAW_POINTS 256
 struct GprEvalArgs {
     const uint8_t *ops;
     const float *cs;
@@ -108,7 +109,10 @@ struct GprEvalArgs {
     double *ll;
     float *grad;            // gradient output (grad kernel)
     int per_wave;           // consecutive tapes a wave evaluates (set by the launcher)
-    int rows;               // gradient: LDS rows of a workgroup (set by the launcher)
+    bool eager;             // load all cap rows of a tape at once (set by the launchers)
+    bool raw;               // dw holds sd of a dataset of at most GPR_RAW_POINTS points, d no constants
+    int rows;               // LDS rows of 64 floats: of a wave (evaluator) or a workgroup (gradient),
+                            // set by the launchers
     int32_t *faults;        // gradient: when set, tapes are checked and what they break (GPR_TAPE_*)
                             // is or-ed in here
     double lnsym;

@@ -1019,20 +1019,48 @@ hipError_t gpr_launch_mh_config_lane(const GprMHArgs &a, int cap_max, hipStream_
 }
 
 // ---------------------------------------------------------------- standalone evaluator
-// Value-stack rows (256 bytes) of one wave: 18 hold the deepest program at one point per
-// lane; 24 hold one of depth 6 at four.  Deeper programs of a larger dataset run at one
-// point per lane in the same rows, so that the common ones keep five waves per SIMD.
+// Value-stack rows (256 bytes) of one wave.  18 hold the deepest program at one point per
+// lane, and 24 one of depth 6 at four or 12 at two: programs deeper than the rows allow run
+// at fewer points per lane, so that the common ones keep five waves per SIMD.
 #define GPR_EVAL_ROWS(KC) ((KC) == 4 ? 24 : GPR_MAX_DEPTH + 2)
+// the LL at the most points per lane, KC or fewer, that the rows hold
+template <int KC, bool HI>
+__device__ __forceinline__ double eval_loglik(const WaveProg &p, int dm, int rows, const GprDataset &d, const float *dx,
+                                              const float *dy, const float *dw, const Chunk<KC> &c0, float *ls) {
+    if constexpr (KC > 1) {
+        if (dm * KC > rows) {
+            Chunk<KC / 2> c;
+            c.load(dx, dy, dw, d.n, 0);
+            return eval_loglik<KC / 2, HI>(p, dm, rows, d, dx, dy, dw, c, ls);
+        }
+    }
+    return wave_loglik<KC, HI>(p, d, dx, dy, dw, c0, (d.n + 64 * KC - 1) / (64 * KC), ls, prog_code<KC, HI>(p));
+}
 
 // A tape's registers and lengths: lane l holds tokens l and l + 64.  A length outside
 // [0, cap] is clamped: the kernels never read or write past the caller's cap rows (a
 // malformed tape yields a meaningless value).
+// With few tapes (a.eager) every cap row is loaded at once with the length, one trip to
+// memory instead of two; with many, only the rows below the length, a sixth of the traffic.
 template <bool HI>
 __device__ __forceinline__ WaveProg eval_load(const GprEvalArgs &a, int chain) {
     const int l = lane_id();
     const size_t N = (size_t)a.nchains;
     WaveProg p;
-    p.len = min(max(uni(a.len[chain]), 0), a.cap);
+    const int len = a.len[chain];
+    if (a.eager) {
+        const int o0 = l < a.cap ? a.ops[(size_t)l * N + chain] : 0;
+        const float c0 = l < a.cap ? a.cs[(size_t)l * N + chain] : 0.0f;
+        const int o1 = (HI && l + 64 < a.cap) ? a.ops[(size_t)(l + 64) * N + chain] : 0;
+        const float c1 = (HI && l + 64 < a.cap) ? a.cs[(size_t)(l + 64) * N + chain] : 0.0f;
+        p.len = min(max(uni(len), 0), a.cap);
+        p.o0 = l < p.len ? o0 : 0;
+        p.c0 = l < p.len ? c0 : 0.0f;
+        p.o1 = (HI && l + 64 < p.len) ? o1 : 0;
+        p.c1 = (HI && l + 64 < p.len) ? c1 : 0.0f;
+        return p;
+    }
+    p.len = min(max(uni(len), 0), a.cap);
     p.o0 = l < p.len ? a.ops[(size_t)l * N + chain] : 0;
     p.c0 = l < p.len ? a.cs[(size_t)l * N + chain] : 0.0f;
     p.o1 = (HI && l + 64 < p.len) ? a.ops[(size_t)(l + 64) * N + chain] : 0;
@@ -1050,21 +1078,94 @@ __device__ __forceinline__ int eval_depth(const WaveProg &p) {
     return max(dm, 1);
 }
 
+// Dataset constants and weights from the sd column, as gpr_set_data forms them on the host:
+// lconst = -sum_i 0.5 (logf(2 pi) + 2 logf(sd_i)) in FP64, and either w_i = 1 with
+// wconst = 1 / (2 sd^2) when every sd is equal, or w_i = 1 / (2 sd_i^2) rounded to float
+// and wconst = 0.  logf is the float rounding of the FP64 log (both correctly rounded);
+// the FP64 sum runs per thread, then as a fixed tree.  A sd that is not finite and
+// positive makes lconst NaN, so every likelihood of the call is NaN.  Run by a whole
+// workgroup of 256; part: 256 doubles of LDS; w may be LDS or global memory.
+#define GPR_PREP_WG 256
+static_assert(GPR_PREP_WG == GPR_WG, "the evaluator's workgroups prepare small datasets themselves");
+__device__ __forceinline__ void dataset_prep(const float *sd, int n, double *part, float *w, double &lconst, double &wconst) {
+    const int tid = threadIdx.x;
+    const float s0 = sd[0];
+    double lc = 0.0;
+    bool diff = false, bad = false;
+    for (int i = tid; i < n; i += GPR_PREP_WG) {
+        const float s = sd[i];
+        bad = bad || !(s > 0.0f) || !__builtin_isfinite(s);
+        diff = diff || s != s0;
+        const float ls = (float)log((double)s);
+        lc -= 0.5 * ((double)0x1.d67f1ep+0f + 2.0 * (double)ls);
+    }
+    part[tid] = lc;
+    const bool same = !__syncthreads_or(diff);
+    const bool any_bad = __syncthreads_or(bad);
+    for (int o = GPR_PREP_WG / 2; o > 0; o >>= 1) {
+        if (tid < o) part[tid] += part[tid + o];
+        __syncthreads();
+    }
+    for (int i = tid; i < n; i += GPR_PREP_WG) {
+        const double s = sd[i];
+        w[i] = same ? 1.0f : (float)(1.0 / (2.0 * s * s));
+    }
+    lconst = any_bad ? __builtin_nan("") : part[0];
+    wconst = same ? 1.0 / (2.0 * (double)s0 * (double)s0) : 0.0;
+}
+
+__global__ void __launch_bounds__(GPR_PREP_WG) k_dataset_prep(const float *sd, int n, int nchains, int cap, int kc,
+                                                              GprDataset *hdr, float *w) {
+    __shared__ double s_part[GPR_PREP_WG];
+    double lconst, wconst;
+    dataset_prep(sd, n, s_part, w, lconst, wconst);
+    if (threadIdx.x == 0) {
+        GprDataset g{};
+        g.n = n;
+        g.off = 0;
+        g.chain0 = 0;
+        g.nchains = nchains;
+        g.cap = cap;
+        g.kc = kc;
+        g.lconst = lconst;
+        g.wconst = wconst;
+        *hdr = g;
+    }
+}
+
+hipError_t gpr_launch_dataset_prep(const float *sd, int n, int nchains, int cap, int kc, GprDataset *hdr, float *w,
+                                   hipStream_t s) {
+    hipLaunchKernelGGL(k_dataset_prep, dim3(1), dim3(GPR_PREP_WG), 0, s, sd, n, nchains, cap, kc, hdr, w);
+    return hipGetLastError();
+}
+
 // One wave per tape.  A wave takes a.per_wave consecutive tapes: the dataset's first chunk
 // stays in its registers, and a tape's tokens are loaded while the one before it is
 // evaluated (a tape of some ten tokens is evaluated in the time of one trip to memory).
-template <int KC, bool HI>
+// RAW: the dataset is the caller's (at most 256 points, a.dw holds its sd column): every
+// workgroup forms its constants and weights itself, in place of a launch before this one.
+template <int KC, bool HI, bool RAW>
 __global__ void __launch_bounds__(GPR_WG) __attribute__((amdgpu_waves_per_eu(KC == 4 ? 5 : (KC == 2 ? 6 : 7))))
 k_eval_wave(GprEvalArgs a) {
-    __shared__ float s_stack[GPR_WAVES_PER_WG][GPR_EVAL_ROWS(KC) * 64];
+    __shared__ double s_part[RAW ? GPR_PREP_WG : 1];
+    __shared__ float s_w[RAW ? GPR_PREP_WG : 1];
     const int wave = uni((int)(threadIdx.x >> 6));
     const int first = uni(((int)blockIdx.x * GPR_WAVES_PER_WG + wave) * a.per_wave);
     const int last = min(first + a.per_wave, a.nchains);
+    WaveProg nx{};
+    if (first < last) nx = eval_load<HI>(a, first);
+    GprDataset d;
+    if (RAW) {
+        d = a.d;
+        dataset_prep(a.dw, d.n, s_part, s_w, d.lconst, d.wconst);
+        __syncthreads();
+        d = uni_dataset(d);
+    } else {
+        d = uni_dataset(a.dd ? *a.dd : a.d);
+    }
     if (first >= last) return;
-    const GprDataset d = uni_dataset(a.dd ? *a.dd : a.d);
-    const float *dx = a.dx + d.off, *dy = a.dy + d.off, *dw = a.dw + d.off;
-    float *ls = s_stack[wave];
-    WaveProg nx = eval_load<HI>(a, first);
+    const float *dx = a.dx + d.off, *dy = a.dy + d.off, *dw = RAW ? s_w : a.dw + d.off;
+    float *ls = gpr_lds_slab + (size_t)wave * a.rows * 64;
     Chunk<KC> c0;
     c0.load(dx, dy, dw, d.n, 0);
     for (int chain = first; chain < last; chain++) {
@@ -1072,73 +1173,76 @@ k_eval_wave(GprEvalArgs a) {
         if (chain + 1 < last) nx = eval_load<HI>(a, chain + 1);
         const int dm = eval_depth<HI>(p);
         double ll = -GPR_INF;
-        if (dm == 0) {
-        } else if (KC == 1 || dm * KC <= GPR_EVAL_ROWS(KC)) {
-            ll = wave_loglik<KC, HI>(p, d, dx, dy, dw, c0, (d.n + 64 * KC - 1) / (64 * KC), ls, prog_code<KC, HI>(p));
-        } else {
-            Chunk<1> c1;
-            c1.load(dx, dy, dw, d.n, 0);
-            ll = wave_loglik<1, HI>(p, d, dx, dy, dw, c1, (d.n + 63) / 64, ls, prog_code<1, HI>(p));
-        }
+        if (dm) ll = eval_loglik<KC, HI>(p, dm, a.rows, d, dx, dy, dw, c0, ls);
         if (lane_id() == 0) a.ll[chain] = ll;
     }
 }
 
-// One workgroup per tape, for datasets of more than 256 points: its four waves interpret
-// the tape over 256 points each, and the terms of 1024 points meet in LDS, where one wave
-// adds them in the order of wave_loglik (every lane's points in increasing order, so the
-// sum is bit-identical).  With few tapes the GPU is filled four times better, and with many
-// the longest tape ends the launch sooner: 30000 tapes (cap 64) at n = 1024 222 us, and 362
-// by one wave per tape; 500 tapes at n = 500 42 and 66.  At n = 300 two of the waves have
-// little to do: 30000 tapes 191 us, and 136 by one wave per tape, which therefore keeps
-// datasets of up to 512 points where 4096 tapes or more fill the GPU.
-template <bool HI>
+// LL terms (chunk k of 64 points at term[64 k + lane]) of KC chunks from point `first`, at the
+// most points per lane, KC or fewer, that the rows hold.
+template <int KC, bool HI>
+__device__ __forceinline__ void eval_terms(const WaveProg &p, int dm, int rows, const GprDataset &d, const float *dx,
+                                           const float *dy, const float *dw, int first, float *ls, float *term) {
+    if (first >= d.n) return;
+    if constexpr (KC > 1) {
+        if (dm * KC > rows) {
+#pragma unroll 1
+            for (int h = 0; h < 2; h++)
+                eval_terms<KC / 2, HI>(p, dm, rows, d, dx, dy, dw, first + 32 * KC * h, ls, term + 32 * KC * h);
+            return;
+        }
+    }
+    const int l = lane_id();
+    Chunk<KC> c;
+    c.load(dx, dy, dw, d.n, first);
+    float T[KC];
+    wave_eval_ls<KC, HI>(p, c.x, T, ls, prog_code<KC, HI>(p));
+#pragma unroll
+    for (int k = 0; k < KC; k++) {
+        const float r = T[k] - c.y[k];
+        term[64 * k + l] = first + 64 * k + l < d.n ? (r * r) * c.w[k] : 0.0f;
+    }
+}
+
+// One workgroup per tape: its four waves interpret the tape over 64 KC points each, and the
+// terms of such a round meet in LDS, where one wave adds them in the order of wave_loglik
+// (every lane's points in increasing order, so the sum is bit-identical).  With few tapes the
+// GPU is filled four times better and a wave runs fewer points per lane (the longest tape's
+// chain of library functions is what the call waits for), and with many tapes of a large
+// dataset the longest tape ends the launch sooner.
+template <int KC, bool HI, bool RAW>
 __global__ void __launch_bounds__(GPR_WG) k_eval_split(GprEvalArgs a) {
-    __shared__ float s_stack[GPR_WAVES_PER_WG][GPR_EVAL_ROWS(4) * 64];
-    __shared__ float s_term[16][64];
+    __shared__ float s_term[4 * KC * 64];
+    __shared__ double s_part[RAW ? GPR_PREP_WG : 1];
+    __shared__ float s_w[RAW ? GPR_PREP_WG : 1];
     const int wave = uni((int)(threadIdx.x >> 6));
     const int l = lane_id();
     const int chain = (int)blockIdx.x;
-    const GprDataset d = uni_dataset(a.dd ? *a.dd : a.d);
-    const float *dx = a.dx + d.off, *dy = a.dy + d.off, *dw = a.dw + d.off;
-    float *ls = s_stack[wave];
     const WaveProg p = eval_load<HI>(a, chain);
+    GprDataset d;
+    if (RAW) {
+        d = a.d;
+        dataset_prep(a.dw, d.n, s_part, s_w, d.lconst, d.wconst);
+        __syncthreads();
+        d = uni_dataset(d);
+    } else {
+        d = uni_dataset(a.dd ? *a.dd : a.d);
+    }
+    const float *dx = a.dx + d.off, *dy = a.dy + d.off, *dw = RAW ? s_w : a.dw + d.off;
     const int dm = eval_depth<HI>(p);       // the same in every wave
     if (dm == 0) {
         if (threadIdx.x == 0) a.ll[chain] = -GPR_INF;
         return;
     }
-    const bool four = dm * 4 <= GPR_EVAL_ROWS(4);
-    const ProgCode pc = four ? prog_code<4, HI>(p) : prog_code<1, HI>(p);
+    float *ls = gpr_lds_slab + (size_t)wave * a.rows * 64;
     float acc = 0.0f, comp = 0.0f;
-    for (int base = 0; base < d.n; base += 1024) {
-        const int mine = base + 256 * wave;
-        if (mine >= d.n) {
-        } else if (four) {
-            Chunk<4> c;
-            c.load(dx, dy, dw, d.n, mine);
-            float T[4];
-            wave_eval_ls<4, HI>(p, c.x, T, ls, pc);
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const float r = T[k] - c.y[k];
-                s_term[4 * wave + k][l] = mine + 64 * k + l < d.n ? (r * r) * c.w[k] : 0.0f;
-            }
-        } else {
-            for (int k = 0; k < 4 && mine + 64 * k < d.n; k++) {
-                Chunk<1> c;
-                c.load(dx, dy, dw, d.n, mine + 64 * k);
-                float T[1];
-                wave_eval_ls<1, HI>(p, c.x, T, ls, pc);
-                const float r = T[0] - c.y[0];
-                s_term[4 * wave + k][l] = mine + 64 * k + l < d.n ? (r * r) * c.w[0] : 0.0f;
-            }
-        }
+    for (int base = 0; base < d.n; base += 256 * KC) {
+        eval_terms<KC, HI>(p, dm, a.rows, d, dx, dy, dw, base + 64 * KC * wave, ls, s_term + 64 * KC * wave);
         __syncthreads();
         if (wave == 0) {
-            const int m = min((d.n - base + 63) / 64, 16);
+            const int m = min((d.n - base + 63) / 64, 4 * KC);
             for (int k = 0; k < m; k++) {
-                const float yv = s_term[k][l] - comp;
+                const float yv = s_term[64 * k + l] - comp;
                 const float tv = acc + yv;
                 comp = (tv - acc) - yv;
                 acc = tv;
@@ -1152,26 +1256,57 @@ __global__ void __launch_bounds__(GPR_WG) k_eval_split(GprEvalArgs a) {
     }
 }
 
-// Tapes per wave: as many as still leave every wave slot of the GPU (256 CUs, 20 waves
-// each) several waves to balance unequal tapes with.
-hipError_t gpr_launch_eval_wave(const GprEvalArgs &args, hipStream_t s) {
-    GprEvalArgs a = args;
-    const bool hi = a.cap > 64;
-    const int kc = a.d.kc;
-    if (a.d.n > 512 || (a.d.n > 256 && a.nchains < 4096)) {
-        if (hi) hipLaunchKernelGGL(k_eval_split<true>, dim3(a.nchains), dim3(GPR_WG), 0, s, a);
-        else hipLaunchKernelGGL(k_eval_split<false>, dim3(a.nchains), dim3(GPR_WG), 0, s, a);
-        return hipGetLastError();
+template <int KC, bool RAW>
+static hipError_t launch_eval_split(const GprEvalArgs &a, hipStream_t s) {
+    const size_t sh = sizeof(float) * 64 * (size_t)a.rows * GPR_WAVES_PER_WG;
+    const void *f = a.cap > 64 ? (const void *)k_eval_split<KC, true, RAW> : (const void *)k_eval_split<KC, false, RAW>;
+    if (sh > 64 * 1024) {
+        hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh);
+        if (e != hipSuccess) return e;
     }
-    a.per_wave = std::max(1, std::min(4, a.nchains / 20480));
+    if (a.cap > 64) hipLaunchKernelGGL((k_eval_split<KC, true, RAW>), dim3(a.nchains), dim3(GPR_WG), sh, s, a);
+    else hipLaunchKernelGGL((k_eval_split<KC, false, RAW>), dim3(a.nchains), dim3(GPR_WG), sh, s, a);
+    return hipGetLastError();
+}
+template <int KC, bool RAW>
+static hipError_t launch_eval_wave(const GprEvalArgs &a, hipStream_t s) {
     const int waves = (a.nchains + a.per_wave - 1) / a.per_wave;
     const int grid = (waves + GPR_WAVES_PER_WG - 1) / GPR_WAVES_PER_WG;
-#define GPR_L(K, H) hipLaunchKernelGGL((k_eval_wave<K, H>), dim3(grid), dim3(GPR_WG), 0, s, a)
-    if (kc == 1) { if (hi) GPR_L(1, true); else GPR_L(1, false); }
-    else if (kc == 2) { if (hi) GPR_L(2, true); else GPR_L(2, false); }
-    else { if (hi) GPR_L(4, true); else GPR_L(4, false); }
-#undef GPR_L
+    const size_t sh = sizeof(float) * 64 * (size_t)a.rows * GPR_WAVES_PER_WG;
+    const void *f = a.cap > 64 ? (const void *)k_eval_wave<KC, true, RAW> : (const void *)k_eval_wave<KC, false, RAW>;
+    if (sh > 64 * 1024) {
+        hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh);
+        if (e != hipSuccess) return e;
+    }
+    if (a.cap > 64) hipLaunchKernelGGL((k_eval_wave<KC, true, RAW>), dim3(grid), dim3(GPR_WG), sh, s, a);
+    else hipLaunchKernelGGL((k_eval_wave<KC, false, RAW>), dim3(grid), dim3(GPR_WG), sh, s, a);
     return hipGetLastError();
+}
+
+hipError_t gpr_launch_eval_wave(const GprEvalArgs &args, hipStream_t s) {
+    GprEvalArgs a = args;
+    const int n = a.d.n;
+    a.eager = a.nchains <= 2048;
+    // A workgroup per tape while all of them run at once, from three chunks on, and for
+    // datasets of more than 512 points.  One wave per tape / one workgroup, whole calls in us:
+    // 300 tapes at n = 200 31 / 23, 500 at 500 41 / 24, 2000 at 100 24.0 / 25.3, 4096 at 256
+    // 17 / 20, 30000 at 300 136 / 191, 30000 at 1024 362 / 198.
+    if ((n > 128 && a.nchains <= 2048) || n > 512) {
+        const int kc = n <= 256 ? 1 : (n <= 512 ? 2 : 4);
+        // rows for every depth at the full points per lane where that keeps the tapes resident
+        a.rows = kc == 1 || a.nchains * kc <= 2048 ? (GPR_MAX_DEPTH + 2) * kc : GPR_EVAL_ROWS(4);
+        if (kc == 1) return a.raw ? launch_eval_split<1, true>(a, s) : launch_eval_split<1, false>(a, s);
+        return kc == 2 ? launch_eval_split<2, false>(a, s) : launch_eval_split<4, false>(a, s);
+    }
+    // Tapes per wave: as many as still leave every wave slot of the GPU (256 CUs, 20 waves
+    // each) several waves to balance unequal tapes with.
+    a.per_wave = std::max(1, std::min(4, a.nchains / 20480));
+    const int kc = a.d.kc;
+    // 300 tapes at n = 200: 36 us with the rows of many tapes, 22 with all; 30000 at 300: 122 and 217
+    a.rows = a.nchains * kc <= 8192 ? (GPR_MAX_DEPTH + 2) * kc : GPR_EVAL_ROWS(kc);
+    if (kc == 1) return a.raw ? launch_eval_wave<1, true>(a, s) : launch_eval_wave<1, false>(a, s);
+    if (kc == 2) return a.raw ? launch_eval_wave<2, true>(a, s) : launch_eval_wave<2, false>(a, s);
+    return a.raw ? launch_eval_wave<4, true>(a, s) : launch_eval_wave<4, false>(a, s);
 }
 
 // Gradient of the log posterior of each tape: one workgroup per tape, whose waves (1 to 8,
@@ -1295,6 +1430,7 @@ __global__ void __launch_bounds__(512) k_grad_wave(GprEvalArgs a) {
 
 hipError_t gpr_launch_grad_wave(const GprEvalArgs &args, hipStream_t s) {
     GprEvalArgs a = args;
+    a.eager = a.nchains <= 2048;
     // waves: one per two chunks of 64 points.  Eight share their rows at 16 each, which a
     // cap over 64 outgrows (6007 tapes of cap 128 at n = 1021: 602 us by four, 694 by eight; 30000
     // of cap 64 at 1024: 915 and 870), unless so few tapes are asked for that their latency counts
@@ -1384,63 +1520,6 @@ hipError_t gpr_launch_eval_lane(const GprEvalArgs &a, hipStream_t s) {
         if (e != hipSuccess) return e;
     }
     hipLaunchKernelGGL(k_eval_lane, dim3(grid), dim3(GPR_LANE_WG), sh, s, a);
-    return hipGetLastError();
-}
-
-// Dataset header and weights from the sd column, as gpr_set_data forms them on the host:
-// lconst = -sum_i 0.5 (logf(2 pi) + 2 logf(sd_i)) in FP64, and either w_i = 1 with
-// wconst = 1 / (2 sd^2) when every sd is equal, or w_i = 1 / (2 sd_i^2) rounded to float
-// and wconst = 0.  logf is the float rounding of the FP64 log (both correctly rounded);
-// the FP64 sum runs per thread, then as a fixed tree.  A sd that is not finite and
-// positive makes lconst NaN, so every likelihood of the call is NaN.
-#define GPR_PREP_WG 256
-__global__ void __launch_bounds__(GPR_PREP_WG) k_dataset_prep(const float *sd, int n, int nchains, int cap, int kc,
-                                                              GprDataset *hdr, float *w) {
-    __shared__ double s_part[GPR_PREP_WG];
-    __shared__ int s_diff, s_bad;
-    const int tid = threadIdx.x;
-    if (tid == 0) { s_diff = 0; s_bad = 0; }
-    __syncthreads();
-    const float s0 = sd[0];
-    double lc = 0.0;
-    bool diff = false, bad = false;
-    for (int i = tid; i < n; i += GPR_PREP_WG) {
-        const float s = sd[i];
-        bad = bad || !(s > 0.0f) || !__builtin_isfinite(s);
-        diff = diff || s != s0;
-        const float ls = (float)log((double)s);
-        lc -= 0.5 * ((double)0x1.d67f1ep+0f + 2.0 * (double)ls);
-    }
-    s_part[tid] = lc;
-    if (diff) atomicOr(&s_diff, 1);
-    if (bad) atomicOr(&s_bad, 1);
-    __syncthreads();
-    for (int o = GPR_PREP_WG / 2; o > 0; o >>= 1) {
-        if (tid < o) s_part[tid] += s_part[tid + o];
-        __syncthreads();
-    }
-    const bool same = s_diff == 0;
-    for (int i = tid; i < n; i += GPR_PREP_WG) {
-        const double s = sd[i];
-        w[i] = same ? 1.0f : (float)(1.0 / (2.0 * s * s));
-    }
-    if (tid == 0) {
-        GprDataset g{};
-        g.n = n;
-        g.off = 0;
-        g.chain0 = 0;
-        g.nchains = nchains;
-        g.cap = cap;
-        g.kc = kc;
-        g.lconst = s_bad ? __builtin_nan("") : s_part[0];
-        g.wconst = same ? 1.0 / (2.0 * (double)s0 * (double)s0) : 0.0;
-        *hdr = g;
-    }
-}
-
-hipError_t gpr_launch_dataset_prep(const float *sd, int n, int nchains, int cap, int kc, GprDataset *hdr, float *w,
-                                   hipStream_t s) {
-    hipLaunchKernelGGL(k_dataset_prep, dim3(1), dim3(GPR_PREP_WG), 0, s, sd, n, nchains, cap, kc, hdr, w);
     return hipGetLastError();
 }
 

@@ -104,3 +104,40 @@ def test_blocks_on_full_programs(oracle, gpr, cap, n, mala):
     same = np.all(g_cs.view(np.uint32) == o_cs.view(np.uint32), axis=0)
     check_paths(same, m, f"full programs cap={cap} n={n}:")
     assert np.array_equal(g_pr[same], p_ref[same])
+
+
+@pytest.mark.parametrize("n,tapes", [(1, 40), (63, 2049), (65, 100), (128, 4097), (129, 100), (256, 4096), (256, 4097),
+                                     (257, 100), (513, 600)])
+def test_noalloc_eval_prepares_the_dataset(oracle, gpr, n, tapes):
+    """gpr_eval_loglik_noalloc_async where its dataset constants move between the evaluator's
+    workgroups and a launch of their own, with equal deviations and one per point, against
+    gpr_eval_loglik; the normaliser is the same FP64 sum in another order, of logs that may
+    differ by an ulp from the host libm's logf."""
+    import torch
+    cap = 128
+    O, V, L = batch(oracle, cap)
+    idx = np.arange(tapes) % O.shape[1]
+    O, V, L = O[:, idx].copy(), V[:, idx].copy(), L[idx].copy()
+    dO, dV, dL = dev(O), dev(V), dev(L)
+    for uneven in (False, True):
+        data = dataset(n, uneven)
+        ref = torch.zeros(tapes, dtype=torch.float64, device="cuda")
+        with gpr.Context(cap=cap) as ctx:
+            ctx.set_data([data], [1])
+            ctx.eval_loglik_dev(0, dO.data_ptr(), dV.data_ptr(), dL.data_ptr(), tapes, cap, gpr.SCHED_WAVE, ref.data_ptr())
+        x, y, sd = (dev(v) for v in data)
+        out = torch.full((tapes,), 7.0, dtype=torch.float64, device="cuda")
+        say(f"no-alloc dataset n={n} tapes={tapes} uneven={uneven}")
+        gpr.eval_loglik_noalloc_async(0, x.data_ptr(), y.data_ptr(), sd.data_ptr(), n, dO.data_ptr(), dV.data_ptr(),
+                                      dL.data_ptr(), tapes, cap, gpr.SCHED_WAVE, out.data_ptr(),
+                                      torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        ref, out = ref.cpu().numpy(), out.cpu().numpy()
+        assert np.all(np.isfinite(ref)) and np.all(np.abs(out - ref) <= 1e-9 * np.maximum(np.abs(ref), n))
+    # a deviation that is not positive: every result NaN
+    o2 = dev(out)
+    bad = dev(np.where(np.arange(n) == n - 1, 0.0, 1.0).astype(np.float32))
+    gpr.eval_loglik_noalloc_async(0, x.data_ptr(), y.data_ptr(), bad.data_ptr(), n, dO.data_ptr(), dV.data_ptr(),
+                                  dL.data_ptr(), tapes, cap, gpr.SCHED_WAVE, o2.data_ptr(), None)
+    torch.cuda.synchronize()
+    assert not np.any(np.isfinite(o2.cpu().numpy()))
