@@ -94,7 +94,13 @@ __device__ __forceinline__ float wave_sum_f(float v) {
     v += dpp_f<DPP_QP_2301>(v);
     v += dpp_f<DPP_ROW_HALF_MIRROR>(v);
     v += dpp_f<DPP_ROW_MIRROR>(v);
-    return (rl_f(v, 0) + rl_f(v, 16)) + (rl_f(v, 32) + rl_f(v, 48));
+    // rows 0 and 1, rows 2 and 3, then the pairs, in lane 63: (r0 + r1) + (r2 + r3) in two
+    // adds, where lane reads took four and three (s_nop: a DPP operand is read two wait states
+    // after the vector unit wrote it)
+    __asm__("s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+            "s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf\n\ts_nop 0"
+            : "+v"(v));
+    return rl_f(v, 63);
 }
 template <int CTRL>
 __device__ __forceinline__ double dpp_d(double v) {
@@ -211,8 +217,9 @@ __device__ __forceinline__ OpMasks op_masks(const WaveProg &p) {
 // of equal size in one asm block, and a token's word, held in its lane like the token itself
 // (prog_code), is the byte offset of its handler: a dispatch is one v_readlane, an add with
 // carry and s_setpc, and a handler ends in the dispatch of the next token.  A leaf followed
-// by +, - or * is one handler.  Division, powers and library functions (and the last lane's
-// token) leave the block; the caller runs them and enters again at the next token.
+// by +, - or * is one handler, and so are two leaves with their operator.  Division, powers
+// and library functions (and the last lane's token) leave the block; the caller runs them and
+// enters again at the next token with a handler.
 //
 // The value stack's top two entries stay in VGPRs (T, U) and the rest live in this wave's
 // LDS slab, [level][k][lane] with GPR_MAX_DEPTH + 2 levels for any program; levels 0 and 1
@@ -224,26 +231,37 @@ __device__ __forceinline__ OpMasks op_masks(const WaveProg &p) {
 // Against the mask tests, whole runs with their set-up and state copies: random walk,
 // 131072 chains at n = 250 and cap 64, 150.5 -> 123.0 ms; 48 uneven datasets of 2048 chains,
 // 47.1 -> 41.3 ms; MALA, whose gradients have interpreters of their own, 107.8 -> 103.0 ms.
+// Two leaves and their operator in one handler, with the branch-free words below: 122.8 ->
+// 120.3 ms and 39.6 -> 39.1 ms on those two random walks.
 enum {
     GPR_U_EXIT = 0, GPR_U_X, GPR_U_C, GPR_U_XADD, GPR_U_XSUB, GPR_U_XMUL, GPR_U_CADD, GPR_U_CSUB, GPR_U_CMUL, GPR_U_ADD,
-    GPR_U_SUB, GPR_U_MUL, GPR_U_NEG
+    GPR_U_SUB, GPR_U_MUL, GPR_U_NEG, GPR_U_XXADD, GPR_U_XCADD = GPR_U_XXADD + 3, GPR_U_CXADD = GPR_U_XCADD + 3
 };
 // Handler words of a half tape: lane l holds token l's.  Lanes past the program, and lane
 // 63 (whose successor the block could not read), hold the exit; so does every token
-// without a handler.  Tokens advance by one, or two for a leaf fused with lane l + 1 <= 62,
-// so the block always reaches an exit.
+// without a handler.  A handler advances by the one, two (a leaf and its operator) or three
+// tokens (two leaves, not both constants, and their operator) it stands for, all of them
+// before min(n, 63), so the block always reaches an exit.  No branches: per lane they would
+// cost more than the arithmetic.
 template <int KC>
 __device__ __forceinline__ int half_code(int o, int n) {
-    const int l = lane_id();
-    const int nx = shfl_all(o, l + 1);
-    const bool leaf = o <= GPR_OP_CONST, cheap = o >= GPR_OP_ADD && o <= GPR_OP_MUL;
-    const bool fuse = l + 1 < min(n, 63) && nx >= GPR_OP_ADD && nx <= GPR_OP_MUL;
-    int u = leaf ? (fuse ? GPR_U_XADD + 3 * o + (nx - GPR_OP_ADD) : GPR_U_X + o)
-                 : (cheap ? GPR_U_ADD + (o - GPR_OP_ADD) : (o == GPR_OP_NEG ? GPR_U_NEG : GPR_U_EXIT));
-    u = l < min(n, 63) ? u : GPR_U_EXIT;
+    const int l = lane_id(), end = min(n, 63);
+    const int n1 = shfl_all(o, l + 1), n2 = shfl_all(o, l + 2);
+    // the handler of a token by itself, five bits an op: x, constant, (one), + - *, (five
+    // operators), negation; nothing from op 12 on
+    constexpr uint64_t ALONE = (uint64_t)GPR_U_X | ((uint64_t)GPR_U_C << 5) | ((uint64_t)GPR_U_ADD << 15) |
+                               ((uint64_t)GPR_U_SUB << 20) | ((uint64_t)GPR_U_MUL << 25) | ((uint64_t)GPR_U_NEG << 55);
+    int u = (int)(ALONE >> (5 * min(o, 12))) & 31;
+    const bool leaf = o <= GPR_OP_CONST;
+    const bool one = leaf & (l + 1 < end) & ((unsigned)(n1 - GPR_OP_ADD) < 3u);
+    const bool two = leaf & (l + 2 < end) & (o + n1 < 2) & ((unsigned)(n2 - GPR_OP_ADD) < 3u);
+    u = one ? GPR_U_XADD - GPR_OP_ADD + 3 * o + n1 : u;
+    u = two ? GPR_U_XXADD - GPR_OP_ADD + 3 * (2 * o + n1) + n2 : u;
+    u = l < end ? u : GPR_U_EXIT;
     return u << (KC == 1 ? 6 : 7);
 }
-static_assert(GPR_OP_X == 0 && GPR_OP_CONST == 1 && GPR_OP_SUB == GPR_OP_ADD + 1 && GPR_OP_MUL == GPR_OP_ADD + 2,
+static_assert(GPR_OP_X == 0 && GPR_OP_CONST == 1 && GPR_OP_ONE == 2 && GPR_OP_SUB == GPR_OP_ADD + 1 &&
+                  GPR_OP_MUL == GPR_OP_ADD + 2 && GPR_OP_NEG == 11,
               "half_code's arithmetic on op codes");
 struct ProgCode {
     int w0, w1;
@@ -275,6 +293,8 @@ __device__ __forceinline__ void lds_st(uint32_t a, float v) { *(gpr_lds_f)(uintp
 #define GT_NEXT(N) "s_add_i32 %[t], %[t], " #N "\n\tv_readlane_b32 %[w], %[word], %[t]\n\t"
 #define GT_JUMP "s_add_u32 vcc_lo, %[blo], %[w]\n\ts_addc_u32 vcc_hi, %[bhi], 0\n\ts_setpc_b64 vcc\n\t"
 #define GT_CONST "v_readlane_b32 %[s], %[c], %[t]\n\t"
+// the constant of the token after this one
+#define GT_CONST2 "s_add_i32 %[s], %[t], 1\n\tv_readlane_b32 %[s], %[c], %[s]\n\t"
 #define GT_WAIT "s_waitcnt lgkmcnt(0)\n\t"
 // entry: the base of the handlers, then the dispatch of token t
 #define GT_ENTRY                                                                            \
@@ -307,6 +327,15 @@ __device__ __forceinline__ void tape_run(int word, float c, const float (&x)[1],
         GT_H(GT_NEXT(1) GT_WAIT GT1("v_sub_f32", "%[U0]", "%[T0]") GT1_POP GT_JUMP)
         GT_H(GT_NEXT(1) GT_WAIT GT1("v_mul_f32", "%[U0]", "%[T0]") GT1_POP GT_JUMP)
         GT_H(GT_NEXT(1) "v_xor_b32 %[T0], 0x80000000, %[T0]\n\t" GT_JUMP)
+        GT_H(GT_NEXT(3) GT1_PUSH GT1("v_add_f32", "%[x0]", "%[x0]") GT_JUMP)
+        GT_H(GT_NEXT(3) GT1_PUSH GT1("v_sub_f32", "%[x0]", "%[x0]") GT_JUMP)
+        GT_H(GT_NEXT(3) GT1_PUSH GT1("v_mul_f32", "%[x0]", "%[x0]") GT_JUMP)
+        GT_H(GT_CONST2 GT_NEXT(3) GT1_PUSH GT1("v_add_f32", "%[s]", "%[x0]") GT_JUMP)
+        GT_H(GT_CONST2 GT_NEXT(3) GT1_PUSH GT1("v_subrev_f32", "%[s]", "%[x0]") GT_JUMP)
+        GT_H(GT_CONST2 GT_NEXT(3) GT1_PUSH GT1("v_mul_f32", "%[s]", "%[x0]") GT_JUMP)
+        GT_H(GT_CONST GT_NEXT(3) GT1_PUSH GT1("v_add_f32", "%[s]", "%[x0]") GT_JUMP)
+        GT_H(GT_CONST GT_NEXT(3) GT1_PUSH GT1("v_sub_f32", "%[s]", "%[x0]") GT_JUMP)
+        GT_H(GT_CONST GT_NEXT(3) GT1_PUSH GT1("v_mul_f32", "%[s]", "%[x0]") GT_JUMP)
         ".Lx%=:"
         : [T0] "+&v"(T[0]), [U0] "+&v"(U[0]), [p] "+&v"(p), [t] "+&s"(t), [blo] "=&s"(blo), [bhi] "=&s"(bhi), [w] "=&s"(w),
           [s] "=&s"(s)
@@ -349,6 +378,15 @@ __device__ __forceinline__ void tape_run(int word, float c, const float (&x)[1],
     GT_H(GT_NEXT(1) GT_WAIT GT("v_sub_f32", GT_U, GT_T) POP GT_JUMP)             \
     GT_H(GT_NEXT(1) GT_WAIT GT("v_mul_f32", GT_U, GT_T) POP GT_JUMP)             \
     GT_H(GT_NEXT(1) GT("v_xor_b32", GT_NEGMASK, GT_T) GT_JUMP)                   \
+    GT_H(GT_NEXT(3) PUSH GT("v_add_f32", GT_X, GT_X) GT_JUMP)                    \
+    GT_H(GT_NEXT(3) PUSH GT("v_sub_f32", GT_X, GT_X) GT_JUMP)                    \
+    GT_H(GT_NEXT(3) PUSH GT("v_mul_f32", GT_X, GT_X) GT_JUMP)                    \
+    GT_H(GT_CONST2 GT_NEXT(3) PUSH GT("v_add_f32", GT_S, GT_X) GT_JUMP)          \
+    GT_H(GT_CONST2 GT_NEXT(3) PUSH GT("v_subrev_f32", GT_S, GT_X) GT_JUMP)       \
+    GT_H(GT_CONST2 GT_NEXT(3) PUSH GT("v_mul_f32", GT_S, GT_X) GT_JUMP)          \
+    GT_H(GT_CONST GT_NEXT(3) PUSH GT("v_add_f32", GT_S, GT_X) GT_JUMP)           \
+    GT_H(GT_CONST GT_NEXT(3) PUSH GT("v_sub_f32", GT_S, GT_X) GT_JUMP)           \
+    GT_H(GT_CONST GT_NEXT(3) PUSH GT("v_mul_f32", GT_S, GT_X) GT_JUMP)           \
     ".Lx%=:"
 __device__ __forceinline__ void tape_run(int word, float c, const float (&x)[2], float (&T)[2], float (&U)[2], uint32_t &p,
                                          int &t) {
@@ -733,12 +771,20 @@ __device__ __forceinline__ void dual_token(const WaveProg &p, const OpMasks &m, 
                 const float tv = T[0];
                 T[0] = T[0] * b;
 #pragma unroll
-                for (int j = 1; j < W; j++) T[j] = tmul(T[j], b) + (rk == j - 1 ? tv : 0.0f);
+                for (int j = 1; j < W; j++) T[j] = tmul(T[j], b);
+                if (!isx) {
+#pragma unroll
+                    for (int j = 1; j < W; j++)
+                        if (rk == j - 1) T[j] = T[j] + tv;
+                }
             } else {
                 const float sgn = (m.sub[h] & nb) ? -1.0f : 1.0f;
                 T[0] = __builtin_fmaf(sgn, b, T[0]);
+                if (!isx) {
 #pragma unroll
-                for (int j = 1; j < W; j++) T[j] = rk == j - 1 ? T[j] + sgn : T[j];
+                    for (int j = 1; j < W; j++)
+                        if (rk == j - 1) T[j] = T[j] + sgn;
+                }
             }
             t++;
             return;
@@ -969,6 +1015,15 @@ __device__ __forceinline__ void tape_run_groups(int word, float cb, float x, flo
         GT_H(GT_NEXT(1) GT_WAIT GT1("v_sub_f32", "%[U0]", "%[T0]") GT1_POP GT_JUMP)
         GT_H(GT_NEXT(1) GT_WAIT GT1("v_mul_f32", "%[U0]", "%[T0]") GT1_POP GT_JUMP)
         GT_H(GT_NEXT(1) GT_WAIT "v_xor_b32 %[T0], 0x80000000, %[T0]\n\t" GT_JUMP)
+        GT_H(GT_NEXT(3) GT1_PUSH GT1("v_add_f32", "%[x]", "%[x]") GT_JUMP)
+        GT_H(GT_NEXT(3) GT1_PUSH GT1("v_sub_f32", "%[x]", "%[x]") GT_JUMP)
+        GT_H(GT_NEXT(3) GT1_PUSH GT1("v_mul_f32", "%[x]", "%[x]") GT_JUMP)
+        GT_H(GT_NEXT(3) GG_TAKE("%[v]") GT1_PUSH GT1("v_add_f32", "%[v]", "%[x]") GT_JUMP)
+        GT_H(GT_NEXT(3) GG_TAKE("%[v]") GT1_PUSH GT1("v_sub_f32", "%[x]", "%[v]") GT_JUMP)
+        GT_H(GT_NEXT(3) GG_TAKE("%[v]") GT1_PUSH GT1("v_mul_f32", "%[v]", "%[x]") GT_JUMP)
+        GT_H(GT_NEXT(3) GG_TAKE("%[v]") GT1_PUSH GT1("v_add_f32", "%[v]", "%[x]") GT_JUMP)
+        GT_H(GT_NEXT(3) GG_TAKE("%[v]") GT1_PUSH GT1("v_sub_f32", "%[v]", "%[x]") GT_JUMP)
+        GT_H(GT_NEXT(3) GG_TAKE("%[v]") GT1_PUSH GT1("v_mul_f32", "%[v]", "%[x]") GT_JUMP)
         ".Lx%=:"
         : [T0] "+&v"(T), [U0] "+&v"(U), [p] "+&v"(p), [ca] "+&v"(ca), [t] "+&s"(t), [blo] "=&s"(blo), [bhi] "=&s"(bhi),
           [w] "=&s"(w), [v] "=&v"(v)

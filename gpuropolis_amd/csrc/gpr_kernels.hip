@@ -78,11 +78,6 @@ k_mh_config_wave(GprMHArgs a) {
     // (the forward-mode interpreter's stack of value + tangents shares it too)
     constexpr int MFLOATS = MROWS * 64 > GPR_DUAL_LDS_FLOATS ? MROWS * 64 : GPR_DUAL_LDS_FLOATS;
     float *ls = gpr_lds_slab + (size_t)wave * (MALA ? MFLOATS : SROWS * 64 * KC);
-    // after the wpg value stacks: each wave's priors of the (up to 16) steps of its draw
-    // batch, then the LLs of its (up to 4) speculatively evaluated steps
-    double *bpri = MALA ? nullptr
-                        : (double *)(gpr_lds_slab + (size_t)a.wpg * ((GPR_MAX_DEPTH + 2) * 64 * KC)) + wave * 20;
-    double *sll = MALA ? nullptr : bpri + 16;
     float *lvg = (MALA && a.mala_gslab) ? a.mala_gslab + ((size_t)blockIdx.x * a.wpg + wave) * (size_t)a.dmax_cap * 64
                                         : nullptr;
     const uint32_t step0 = a.clock ? (uint32_t)uni((int)a.clock[0]) : a.step0;
@@ -108,10 +103,11 @@ k_mh_config_wave(GprMHArgs a) {
         const int nchunks = (d.n + 64 * KC - 1) / (64 * KC);
         // speculative constant steps of small datasets: G proposals per interpreter pass
         // (wave_loglik_groups); the window of the last pass starts at step spec_lo and
-        // holds spec_n cached LLs in sll, valid while the state does not change
+        // holds spec_n LLs in lanes 0 .. spec_n - 1 of sll, valid while the state does not change
         const int G = (SPEC && !MALA && KC == 1) ? (d.n <= 16 ? 4 : (d.n <= 32 ? 2 : 1)) : 1;
         uint32_t spec_lo = 0;
         int spec_n = 0;
+        double sll = 0.0;
 
         WaveProg cur;
         cur.len = uni(a.len[chain]);
@@ -155,11 +151,12 @@ k_mh_config_wave(GprMHArgs a) {
         // most 4 constants, 16 steps (4 lanes each).  At the first constant step of a batch,
         // lane j = ks u + r takes the normal of step u's word for the r-th constant token
         // and, from the current constants, the proposed constant and its Cauchy term; the
-        // batch also sums each step's prior into bpri.  Each step then reads its proposal
-        // lanes and its prior, the same values as the per-step path.  Any accepted move drops the batch (the next constant step
+        // batch also sums each step's prior (bpri, at the step's first lane).  Each step then reads
+        // its proposal lanes and its prior, the same values as the per-step path.  Any accepted move drops the batch (the next constant step
         // recomputes it).
         constexpr bool BATCH = !MALA;
         float cb = 0.0f;
+        double bpri = 0.0;
         uint32_t zblk = 0xffffffffu;
         // MALA: gradient of the current state (lane-distributed like the constants) and its
         // metric drift M g at the metric rows
@@ -220,10 +217,8 @@ k_mh_config_wave(GprMHArgs a) {
             bool have_pll = false;   // MALA constant step: the LL (pll_m, over mala_pts points) is known
             double pll_m = 0.0;
             int mala_pts = 0;
-            bool have_prior = false; // MALA constant step: the prior (pre_prior) is known
+            bool have_prior = false; // constant step of MALA or a batch: the prior (pre_prior) is known
             double pre_prior = 0.0;
-            bool bprior = false;   // the prior comes from the batch: bpri[bu]
-            int bu = 0;
             const bool structural = struct_slot && !a.fixed_structure;
             if (i < 0) {
             } else if (structural) {
@@ -329,17 +324,17 @@ k_mh_config_wave(GprMHArgs a) {
                         const int K = __popcll(mk0);
                         double sacc = 0.0;
                         for (int q = 0; q < K; q++) sacc += shfl_all_d(t, (l & ~(ks - 1)) + q);
-                        if (r == 0) bpri[l >> (6 - lg)] = gpr_dl_prior(cur.len, a.lnsym, sacc);
+                        bpri = gpr_dl_prior(cur.len, a.lnsym, sacc);
                     }
                     const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mk0 >> 32),
                                                                     __builtin_amdgcn_mbcnt_lo((uint32_t)mk0, 0u));
                     const float cv = shfl_all(cb, ks * u + rank);
                     if (k0) prop.c0 = cv;
-                    bprior = true;
-                    bu = u;
+                    pre_prior = rl_d(bpri, ks * u);
+                    have_prior = true;
                     if (G > 1) {
                         if (spec_n > 0 && step >= spec_lo && step < spec_lo + (uint32_t)spec_n) {
-                            pll_m = rl_d(sll[step - spec_lo], 0);   // evaluated by the window's pass
+                            pll_m = rl_d(sll, (int)(step - spec_lo));   // evaluated by the window's pass
                             have_pll = true;
                             mala_pts = d.n;
                         } else {
@@ -352,10 +347,7 @@ k_mh_config_wave(GprMHArgs a) {
                             if (win > 1) {
                                 double o[4];
                                 wave_loglik_groups(cur, d, dx, dy, dw, ls, ccode, cb, ks, u, G, win, o);
-                                if (l == 0) {
-#pragma unroll
-                                    for (int g = 0; g < 4; g++) sll[g] = o[g];
-                                }
+                                sll = l == 0 ? o[0] : (l == 1 ? o[1] : (l == 2 ? o[2] : o[3]));
                                 spec_lo = step;
                                 spec_n = win;
                                 pll_m = o[0];
@@ -574,7 +566,7 @@ k_mh_config_wave(GprMHArgs a) {
                 }
                 }
             }
-            const double pprior = bprior ? bpri[bu] : (have_prior ? pre_prior : wave_prior<HI>(prop, a.lnsym));
+            const double pprior = have_prior ? pre_prior : wave_prior<HI>(prop, a.lnsym);
             // handler words: the current program's, or the structural proposal's
             ProgCode pcode = ccode;
             double pll;
@@ -687,7 +679,7 @@ static hipError_t launch_mh_wave(const GprMHArgs &a, int grid, hipStream_t s) {
     const size_t mfloats = std::max((size_t)std::max(GPR_MALA_LDS_ROWS, GPR_MAX_DEPTH + 2) * 64,
                                     (size_t)GPR_DUAL_LDS_FLOATS);
     const size_t sh = MALA ? sizeof(float) * mfloats * a.wpg
-                           : (sizeof(float) * (GPR_MAX_DEPTH + 2) * 64 * KC + sizeof(double) * 20) * (size_t)a.wpg;
+                           : sizeof(float) * (GPR_MAX_DEPTH + 2) * 64 * KC * (size_t)a.wpg;
     if (sh > 64 * 1024) {
         hipError_t e = hipFuncSetAttribute((const void *)k_mh_config_wave<KC, HI, MALA, MET, SPEC>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh);

@@ -141,3 +141,42 @@ def test_noalloc_eval_prepares_the_dataset(oracle, gpr, n, tapes):
                                   dL.data_ptr(), tapes, cap, gpr.SCHED_WAVE, o2.data_ptr(), None)
     torch.cuda.synchronize()
     assert not np.any(np.isfinite(o2.cpu().numpy()))
+
+
+def pairs_tape(length, shift):
+    """x, then two leaves, their operator and an addition, moved a token at a time by the
+    negations in front; negations fill the rest."""
+    toks = ["X"] + ["NEG"] * shift
+    c = ("CONST", 0.5)
+    k = 0
+    while len(toks) + 4 <= length:
+        a, b = [("X", "X"), ("X", c), (c, "X"), (c, c)][k % 4]
+        toks += [a, b, ("SUB", "MUL", "ADD")[k % 3], ("ADD", "SUB")[k % 2]]
+        k += 1
+    return toks + ["NEG"] * (length - len(toks))
+
+
+@pytest.mark.parametrize("n", [20, 64, 65, 200, 700])
+def test_two_leaves_and_their_operator(oracle, gpr, n):
+    """Every pair of leaves with every operator, at every offset from the last lane of each half
+    tape: exactly rounded operations, 1e-6 of max(|LL|, n) as above."""
+    import torch
+    cap = 128
+    tapes = [pairs_tape(length, s) for length in (4, 61, 62, 63, 64, 65, 66, 126, 127, 128) for s in range(min(length, 13))]
+    arrs = [oracle.tape_arrays(t) for t in tapes]
+    N = len(arrs)
+    O, V = np.zeros((cap, N), dtype=np.uint8), np.zeros((cap, N), dtype=np.float32)
+    for i, (o, v) in enumerate(arrs):
+        O[:len(o), i], V[:len(v), i] = o, v
+    L = np.array([len(o) for o, _ in arrs], dtype=np.int32)
+    d = dataset(n, uneven=True)
+    with gpr.Context(cap=cap) as ctx:
+        ctx.set_data([d], [1])
+        out = torch.zeros(N, dtype=torch.float64, device="cuda")
+        say(f"two leaves and an operator n={n} tapes={N}")
+        dO, dV, dL = dev(O), dev(V), dev(L)
+        ctx.eval_loglik_dev(0, dO.data_ptr(), dV.data_ptr(), dL.data_ptr(), N, cap, gpr.SCHED_WAVE, out.data_ptr())
+        got = out.cpu().numpy()
+    ref = np.array([oracle.tape_loglik(O[:L[i], i], V[:L[i], i], *d) for i in range(N)])
+    assert np.all(np.isfinite(ref))
+    assert np.all(np.abs(got - ref) <= 1e-6 * np.maximum(np.abs(ref), n))
