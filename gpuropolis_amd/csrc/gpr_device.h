@@ -217,9 +217,10 @@ __device__ __forceinline__ OpMasks op_masks(const WaveProg &p) {
 // of equal size in one asm block, and a token's word, held in its lane like the token itself
 // (prog_code), is the byte offset of its handler: a dispatch is one v_readlane, an add with
 // carry and s_setpc, and a handler ends in the dispatch of the next token.  A leaf followed
-// by +, - or * is one handler, and so are two leaves with their operator.  Division, powers
-// and library functions (and the last lane's token) leave the block; the caller runs them and
-// enters again at the next token with a handler.
+// by +, - or * is one handler, and so are two leaves with their operator.  Division, exp and
+// log, the frequent ones of the remaining operators, are larger handlers at the end of the table.
+// The others (and the last lane's token, and exp where a value is not below 88) leave the
+// block; the caller runs them and enters again at the next token with a handler.
 //
 // The value stack's top two entries stay in VGPRs (T, U) and the rest live in this wave's
 // LDS slab, [level][k][lane] with GPR_MAX_DEPTH + 2 levels for any program; levels 0 and 1
@@ -232,11 +233,20 @@ __device__ __forceinline__ OpMasks op_masks(const WaveProg &p) {
 // 131072 chains at n = 250 and cap 64, 150.5 -> 123.0 ms; 48 uneven datasets of 2048 chains,
 // 47.1 -> 41.3 ms; MALA, whose gradients have interpreters of their own, 107.8 -> 103.0 ms.
 // Two leaves and their operator in one handler, with the branch-free words below: 122.8 ->
-// 120.3 ms and 39.6 -> 39.1 ms on those two random walks.
+// 120.3 ms and 39.6 -> 39.1 ms on those two random walks; division, exp and log inside the
+// block, where each left it through some ten branches and thirty scalar instructions:
+// 120.5 -> 103.0 ms, 39.3 -> 36.4 ms, MALA 102.9 -> 98.5 ms, and 100003 tapes at n = 250
+// evaluated in 185 -> 161 us.
 enum {
     GPR_U_EXIT = 0, GPR_U_X, GPR_U_C, GPR_U_XADD, GPR_U_XSUB, GPR_U_XMUL, GPR_U_CADD, GPR_U_CSUB, GPR_U_CMUL, GPR_U_ADD,
-    GPR_U_SUB, GPR_U_MUL, GPR_U_NEG, GPR_U_XXADD, GPR_U_XCADD = GPR_U_XXADD + 3, GPR_U_CXADD = GPR_U_XCADD + 3
+    GPR_U_SUB, GPR_U_MUL, GPR_U_NEG, GPR_U_XXADD, GPR_U_XCADD = GPR_U_XXADD + 3, GPR_U_CXADD = GPR_U_XCADD + 3,
+    GPR_U_EXP = GPR_U_CXADD + 3
 };
+// (the last three handlers take two or three places of the table)
+template <int KC>
+constexpr int GPR_U_DIV = GPR_U_EXP + (KC == 4 ? 3 : 2);
+template <int KC>
+constexpr int GPR_U_LOG = GPR_U_DIV<KC> + (KC == 4 ? 3 : 2);
 // Handler words of a half tape: lane l holds token l's.  Lanes past the program, and lane
 // 63 (whose successor the block could not read), hold the exit; so does every token
 // without a handler.  A handler advances by the one, two (a leaf and its operator) or three
@@ -247,11 +257,13 @@ template <int KC>
 __device__ __forceinline__ int half_code(int o, int n) {
     const int l = lane_id(), end = min(n, 63);
     const int n1 = shfl_all(o, l + 1), n2 = shfl_all(o, l + 2);
-    // the handler of a token by itself, five bits an op: x, constant, (one), + - *, (five
-    // operators), negation; nothing from op 12 on
+    // the handler of a token by itself, five bits an op: x, constant, (one), + - * /, (four
+    // operators), negation; nothing from op 12 on but exp and log
     constexpr uint64_t ALONE = (uint64_t)GPR_U_X | ((uint64_t)GPR_U_C << 5) | ((uint64_t)GPR_U_ADD << 15) |
-                               ((uint64_t)GPR_U_SUB << 20) | ((uint64_t)GPR_U_MUL << 25) | ((uint64_t)GPR_U_NEG << 55);
+                               ((uint64_t)GPR_U_SUB << 20) | ((uint64_t)GPR_U_MUL << 25) |
+                               ((uint64_t)GPR_U_DIV<KC> << 30) | ((uint64_t)GPR_U_NEG << 55);
     int u = (int)(ALONE >> (5 * min(o, 12))) & 31;
+    u = o == GPR_OP_EXP ? GPR_U_EXP : o == GPR_OP_LOG ? GPR_U_LOG<KC> : u;
     const bool leaf = o <= GPR_OP_CONST;
     const bool one = leaf & (l + 1 < end) & ((unsigned)(n1 - GPR_OP_ADD) < 3u);
     const bool two = leaf & (l + 2 < end) & (o + n1 < 2) & ((unsigned)(n2 - GPR_OP_ADD) < 3u);
@@ -261,7 +273,7 @@ __device__ __forceinline__ int half_code(int o, int n) {
     return u << (KC == 1 ? 6 : 7);
 }
 static_assert(GPR_OP_X == 0 && GPR_OP_CONST == 1 && GPR_OP_ONE == 2 && GPR_OP_SUB == GPR_OP_ADD + 1 &&
-                  GPR_OP_MUL == GPR_OP_ADD + 2 && GPR_OP_NEG == 11,
+                  GPR_OP_MUL == GPR_OP_ADD + 2 && GPR_OP_DIV == 6 && GPR_OP_NEG == 11,
               "half_code's arithmetic on op codes");
 struct ProgCode {
     int w0, w1;
@@ -289,7 +301,8 @@ __device__ __forceinline__ void lds_st(uint32_t a, float v) { *(gpr_lds_f)(uintp
 // vector register written by the vector unit is read by v_readlane only after others
 // (nothing in the block writes the word and constant registers, and the entry runs four
 // scalar instructions first).  Every LDS load is waited for before its register is used,
-// and before the block ends.
+// and before the block ends.  v_exp and v_rcp are one instruction away from the use of their
+// result, v_div_scale's vcc six from v_div_fmas, and a compare's vcc two from a select.
 #define GT_NEXT(N) "s_add_i32 %[t], %[t], " #N "\n\tv_readlane_b32 %[w], %[word], %[t]\n\t"
 #define GT_JUMP "s_add_u32 vcc_lo, %[blo], %[w]\n\ts_addc_u32 vcc_hi, %[bhi], 0\n\ts_setpc_b64 vcc\n\t"
 #define GT_CONST "v_readlane_b32 %[s], %[c], %[t]\n\t"
@@ -304,6 +317,37 @@ __device__ __forceinline__ void lds_st(uint32_t a, float v) { *(gpr_lds_f)(uintp
     "v_readlane_b32 %[w], %[word], %[t]\n\t" GT_JUMP
 #define GT_EXIT GT_WAIT "s_branch .Lx%=\n\t"
 
+// exp of T: 2^k e^r from the product with log2(e), its rounding error and the constant's
+// low part in one correction; for |T| < 88 neither end of the range needs a test, and every
+// such value gives the bits of expf (all 2^32 inputs compared).
+#define GT_LOG2E "s_mov_b32 %[s], 0x3fb8aa3b\n\t"
+#define GT_EXP(T)                                                                                               \
+    "v_mul_f32 %[q0], %[s], " T "\n\tv_rndne_f32 %[q1], %[q0]\n\tv_fma_f32 %[q2], " T ", %[s], -%[q0]\n\t"      \
+    "v_sub_f32 %[q0], %[q0], %[q1]\n\tv_fmac_f32 %[q2], 0x32a5705f, " T "\n\tv_add_f32 %[q0], %[q0], %[q2]\n\t" \
+    "v_exp_f32 %[q0], %[q0]\n\tv_cvt_i32_f32 %[q1], %[q1]\n\tv_ldexp_f32 " T ", %[q0], %[q1]\n\t"
+// leave at this token when the largest magnitude M is not below 88
+#define GT_EXP_TEST(M)                                                                                          \
+    "s_mov_b32 %[s], 0x42b00000\n\tv_cmp_nlt_f32 vcc, |" M "|, %[s]\n\ts_cbranch_vccnz .Lh%=\n\t"
+// log of T: log2 (of T 2^32 below the normal range, less 32 log(2) at the end) times log(2)
+// in two parts, where it is finite.  Bits of logf for all 2^32 inputs.
+#define GT_LOG(T)                                                                                               \
+    "s_mov_b32 %[s], 0x800000\n\tv_cmp_gt_f32 vcc, %[s], " T "\n\ts_mov_b32 %[s], 0x3f317217\n\t"                 \
+    "v_mov_b32 %[q2], 0x41b17218\n\tv_cndmask_b32 %[q0], 0, 32, vcc\n\tv_ldexp_f32 %[q0], " T ", %[q0]\n\t"       \
+    "v_log_f32 %[q0], %[q0]\n\tv_cndmask_b32 %[q2], 0, %[q2], vcc\n\tv_mul_f32 %[q1], %[s], %[q0]\n\t"          \
+    "v_fma_f32 %[q1], %[q0], %[s], -%[q1]\n\ts_mov_b32 %[s], 0x7f800000\n\tv_cmp_lt_f32 vcc, |%[q0]|, %[s]\n\t" \
+    "v_fmac_f32 %[q1], 0x3377d1cf, %[q0]\n\tv_fmac_f32 %[q1], 0x3f317217, %[q0]\n\t"                            \
+    "v_cndmask_b32 %[q0], %[q0], %[q1], vcc\n\tv_sub_f32 " T ", %[q0], %[q2]\n\t"
+// U / T, correctly rounded: scaled operands, a reciprocal with one step, a quotient with two
+#define GT_DIV(U, T)                                                                                            \
+    "v_div_scale_f32 %[q0], vcc, " T ", " T ", " U "\n\tv_rcp_f32 %[q1], %[q0]\n\t"                             \
+    "v_div_scale_f32 %[q2], vcc, " U ", " T ", " U "\n\tv_fma_f32 %[q3], -%[q0], %[q1], 1.0\n\t"                \
+    "v_fmac_f32 %[q1], %[q3], %[q1]\n\tv_mul_f32 %[q3], %[q2], %[q1]\n\t"                                       \
+    "v_fma_f32 %[q4], -%[q0], %[q3], %[q2]\n\tv_fmac_f32 %[q3], %[q4], %[q1]\n\t"                               \
+    "v_fma_f32 %[q0], -%[q0], %[q3], %[q2]\n\tv_div_fmas_f32 %[q0], %[q0], %[q1], %[q3]\n\t"                    \
+    "v_div_fixup_f32 " T ", %[q0], " T ", " U "\n\t"
+#define GT_TEMPS float q0, q1, q2, q3, q4
+#define GT_TEMP_OUT [q0] "=&v"(q0), [q1] "=&v"(q1), [q2] "=&v"(q2), [q3] "=&v"(q3), [q4] "=&v"(q4)
+
 #define GT1(OP, A, B) OP " %[T0], " A ", " B "\n\t"
 #define GT1_PUSH GT_WAIT "ds_write_b32 %[p], %[U0]\n\tv_add_u32 %[p], 0x100, %[p]\n\tv_mov_b32 %[U0], %[T0]\n\t"
 #define GT1_POP "v_add_u32 %[p], 0xffffff00, %[p]\n\tds_read_b32 %[U0], %[p]\n\t"
@@ -311,6 +355,7 @@ __device__ __forceinline__ void lds_st(uint32_t a, float v) { *(gpr_lds_f)(uintp
 __device__ __forceinline__ void tape_run(int word, float c, const float (&x)[1], float (&T)[1], float (&U)[1], uint32_t &p,
                                          int &t) {
     uint32_t blo, bhi, w, s;
+    GT_TEMPS;
 #define GT_H(BODY) ".p2align 6\n\t" BODY
     __asm__ volatile(
         GT_ENTRY
@@ -336,9 +381,12 @@ __device__ __forceinline__ void tape_run(int word, float c, const float (&x)[1],
         GT_H(GT_CONST GT_NEXT(3) GT1_PUSH GT1("v_add_f32", "%[s]", "%[x0]") GT_JUMP)
         GT_H(GT_CONST GT_NEXT(3) GT1_PUSH GT1("v_sub_f32", "%[s]", "%[x0]") GT_JUMP)
         GT_H(GT_CONST GT_NEXT(3) GT1_PUSH GT1("v_mul_f32", "%[s]", "%[x0]") GT_JUMP)
+        GT_H(GT_EXP_TEST("%[T0]") GT_NEXT(1) GT_LOG2E GT_EXP("%[T0]") GT_JUMP)
+        GT_H(GT_WAIT GT_NEXT(1) GT_DIV("%[U0]", "%[T0]") GT1_POP GT_JUMP)
+        GT_H(GT_WAIT GT_NEXT(1) GT_LOG("%[T0]") GT_JUMP)
         ".Lx%=:"
         : [T0] "+&v"(T[0]), [U0] "+&v"(U[0]), [p] "+&v"(p), [t] "+&s"(t), [blo] "=&s"(blo), [bhi] "=&s"(bhi), [w] "=&s"(w),
-          [s] "=&s"(s)
+          [s] "=&s"(s), GT_TEMP_OUT
         : [word] "v"(word), [c] "v"(c), [x0] "v"(x[0])
         : "vcc", "scc", "memory");
 #undef GT_H
@@ -362,8 +410,17 @@ __device__ __forceinline__ void tape_run(int word, float c, const float (&x)[1],
 #define GT4_POP                                                                                              \
     "v_add_u32 %[p], 0xfffffc00, %[p]\n\tds_read_b32 %[U0], %[p]\n\tds_read_b32 %[U1], %[p] offset:256\n\t"     \
     "ds_read_b32 %[U2], %[p] offset:512\n\tds_read_b32 %[U3], %[p] offset:768\n\t"
+#define GT2_EXP                                                                                              \
+    "v_max_f32 %[q0], |%[T0]|, |%[T1]|\n\t" GT_EXP_TEST("%[q0]") GT_NEXT(1) GT_LOG2E GT_EXP("%[T0]") GT_EXP("%[T1]")
+#define GT4_EXP                                                                                              \
+    "v_max_f32 %[q0], |%[T0]|, |%[T1]|\n\tv_max3_f32 %[q0], %[q0], |%[T2]|, |%[T3]|\n\t" GT_EXP_TEST("%[q0]")  \
+        GT_NEXT(1) GT_LOG2E GT_EXP("%[T0]") GT_EXP("%[T1]") GT_EXP("%[T2]") GT_EXP("%[T3]")
+#define GT2_DIV GT_DIV("%[U0]", "%[T0]") GT_DIV("%[U1]", "%[T1]")
+#define GT4_DIV GT2_DIV GT_DIV("%[U2]", "%[T2]") GT_DIV("%[U3]", "%[T3]")
+#define GT2_LOG GT_LOG("%[T0]") GT_LOG("%[T1]")
+#define GT4_LOG GT2_LOG GT_LOG("%[T2]") GT_LOG("%[T3]")
 // several points per lane, handlers of 128 bytes
-#define GT_TABLE(GT, MOV, PUSH, POP)                                             \
+#define GT_TABLE(GT, MOV, PUSH, POP, EXP, DIV, LOG)                                             \
     GT_ENTRY                                                                     \
     ".p2align 7\n.Lh%=:\n\t" GT_EXIT                                             \
     GT_H(GT_NEXT(1) PUSH MOV(GT_T, GT_X) GT_JUMP)                                \
@@ -387,23 +444,28 @@ __device__ __forceinline__ void tape_run(int word, float c, const float (&x)[1],
     GT_H(GT_CONST GT_NEXT(3) PUSH GT("v_add_f32", GT_S, GT_X) GT_JUMP)           \
     GT_H(GT_CONST GT_NEXT(3) PUSH GT("v_sub_f32", GT_S, GT_X) GT_JUMP)           \
     GT_H(GT_CONST GT_NEXT(3) PUSH GT("v_mul_f32", GT_S, GT_X) GT_JUMP)           \
+    GT_H(EXP GT_JUMP)                                                            \
+    GT_H(GT_WAIT GT_NEXT(1) DIV POP GT_JUMP)                                     \
+    GT_H(GT_NEXT(1) LOG GT_JUMP)                                                 \
     ".Lx%=:"
 __device__ __forceinline__ void tape_run(int word, float c, const float (&x)[2], float (&T)[2], float (&U)[2], uint32_t &p,
                                          int &t) {
     uint32_t blo, bhi, w, s;
-    __asm__ volatile(GT_TABLE(GT2, GT2_MOV, GT2_PUSH, GT2_POP)
+    GT_TEMPS;
+    __asm__ volatile(GT_TABLE(GT2, GT2_MOV, GT2_PUSH, GT2_POP, GT2_EXP, GT2_DIV, GT2_LOG)
                      : [T0] "+&v"(T[0]), [T1] "+&v"(T[1]), [U0] "+&v"(U[0]), [U1] "+&v"(U[1]), [p] "+&v"(p), [t] "+&s"(t),
-                       [blo] "=&s"(blo), [bhi] "=&s"(bhi), [w] "=&s"(w), [s] "=&s"(s)
+                       [blo] "=&s"(blo), [bhi] "=&s"(bhi), [w] "=&s"(w), [s] "=&s"(s), GT_TEMP_OUT
                      : [word] "v"(word), [c] "v"(c), [x0] "v"(x[0]), [x1] "v"(x[1])
                      : "vcc", "scc", "memory");
 }
 __device__ __forceinline__ void tape_run(int word, float c, const float (&x)[4], float (&T)[4], float (&U)[4], uint32_t &p,
                                          int &t) {
     uint32_t blo, bhi, w, s;
-    __asm__ volatile(GT_TABLE(GT4, GT4_MOV, GT4_PUSH, GT4_POP)
+    GT_TEMPS;
+    __asm__ volatile(GT_TABLE(GT4, GT4_MOV, GT4_PUSH, GT4_POP, GT4_EXP, GT4_DIV, GT4_LOG)
                      : [T0] "+&v"(T[0]), [T1] "+&v"(T[1]), [T2] "+&v"(T[2]), [T3] "+&v"(T[3]), [U0] "+&v"(U[0]),
                        [U1] "+&v"(U[1]), [U2] "+&v"(U[2]), [U3] "+&v"(U[3]), [p] "+&v"(p), [t] "+&s"(t), [blo] "=&s"(blo),
-                       [bhi] "=&s"(bhi), [w] "=&s"(w), [s] "=&s"(s)
+                       [bhi] "=&s"(bhi), [w] "=&s"(w), [s] "=&s"(s), GT_TEMP_OUT
                      : [word] "v"(word), [c] "v"(c), [x0] "v"(x[0]), [x1] "v"(x[1]), [x2] "v"(x[2]), [x3] "v"(x[3])
                      : "vcc", "scc", "memory");
 }
@@ -996,8 +1058,9 @@ __device__ __forceinline__ void dual_grad_lanes(const WaveProg &p, const uint64_
 // loading when a handler ends, so every handler waits first.
 __device__ __forceinline__ void tape_run_groups(int word, float cb, float x, float &T, float &U, uint32_t &p, uint32_t &ca,
                                                 int &t) {
-    uint32_t blo, bhi, w;
+    uint32_t blo, bhi, w, s;
     float v;
+    GT_TEMPS;
 #define GT_H(BODY) ".p2align 6\n\t" BODY
 #define GG_TAKE(D) "ds_bpermute_b32 " D ", %[ca], %[cb]\n\tv_add_u32 %[ca], 4, %[ca]\n\t"
     __asm__ volatile(
@@ -1024,9 +1087,12 @@ __device__ __forceinline__ void tape_run_groups(int word, float cb, float x, flo
         GT_H(GT_NEXT(3) GG_TAKE("%[v]") GT1_PUSH GT1("v_add_f32", "%[v]", "%[x]") GT_JUMP)
         GT_H(GT_NEXT(3) GG_TAKE("%[v]") GT1_PUSH GT1("v_sub_f32", "%[v]", "%[x]") GT_JUMP)
         GT_H(GT_NEXT(3) GG_TAKE("%[v]") GT1_PUSH GT1("v_mul_f32", "%[v]", "%[x]") GT_JUMP)
+        GT_H(GT_WAIT GT_EXP_TEST("%[T0]") GT_NEXT(1) GT_LOG2E GT_EXP("%[T0]") GT_JUMP)
+        GT_H(GT_WAIT GT_NEXT(1) GT_DIV("%[U0]", "%[T0]") GT1_POP GT_JUMP)
+        GT_H(GT_WAIT GT_NEXT(1) GT_LOG("%[T0]") GT_JUMP)
         ".Lx%=:"
         : [T0] "+&v"(T), [U0] "+&v"(U), [p] "+&v"(p), [ca] "+&v"(ca), [t] "+&s"(t), [blo] "=&s"(blo), [bhi] "=&s"(bhi),
-          [w] "=&s"(w), [v] "=&v"(v)
+          [w] "=&s"(w), [s] "=&s"(s), [v] "=&v"(v), GT_TEMP_OUT
         : [word] "v"(word), [cb] "v"(cb), [x] "v"(x)
         : "vcc", "scc", "memory");
 #undef GG_TAKE

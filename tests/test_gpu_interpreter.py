@@ -180,3 +180,40 @@ def test_two_leaves_and_their_operator(oracle, gpr, n):
     ref = np.array([oracle.tape_loglik(O[:L[i], i], V[:L[i], i], *d) for i in range(N)])
     assert np.all(np.isfinite(ref))
     assert np.all(np.abs(got - ref) <= 1e-6 * np.maximum(np.abs(ref), n))
+
+
+@pytest.mark.parametrize("overflow", [False, True])
+@pytest.mark.parametrize("n", [7, 64, 130, 300, 700])
+def test_exp_log_and_division(oracle, gpr, n, overflow):
+    """The handlers of exp, log and division around the magnitude where exp leaves the block, at
+    every place of the second half tape's edge: 1e-5 of max(|LL|, n) for the device's exp and
+    log; a point where exp overflows makes every LL with it -inf."""
+    import torch
+    cap = 128
+    one, half = ("CONST", 1.0), ("CONST", 0.5)
+    bodies = [["X", "EXP", "LOG"], ["X", half, "MUL", "EXP", "X", "X", "MUL", one, "ADD", "DIV", "LOG"],
+              ["X", "X", "X", "MUL", one, "ADD", "DIV", "EXP", "X", "ADD"]]
+    tapes = [b[:1] + ["NEG"] * pad + b[1:] for b in bodies for pad in (0, 52, 54, 56, 58, 60, 62, 64)]
+    arrs = [oracle.tape_arrays(t) for t in tapes]
+    N = len(arrs)
+    O, V = np.zeros((cap, N), dtype=np.uint8), np.zeros((cap, N), dtype=np.float32)
+    for i, (o, v) in enumerate(arrs):
+        O[:len(o), i], V[:len(v), i] = o, v
+    L = np.array([len(o) for o, _ in arrs], dtype=np.int32)
+    x = np.linspace(-20, 20, n).astype(np.float32)
+    x[:6] = [87.9, 88.0, 88.3, -87.9, -88.0, -88.3]
+    if overflow:
+        x[-1] = 89.0
+    d = (x, np.zeros(n, dtype=np.float32), np.full(n, 0.5, dtype=np.float32))
+    with gpr.Context(cap=cap) as ctx:
+        ctx.set_data([d], [1])
+        out = torch.zeros(N, dtype=torch.float64, device="cuda")
+        say(f"exp, log and division n={n} overflow={overflow}")
+        dO, dV, dL = dev(O), dev(V), dev(L)
+        ctx.eval_loglik_dev(0, dO.data_ptr(), dV.data_ptr(), dL.data_ptr(), N, cap, gpr.SCHED_WAVE, out.data_ptr())
+        got = out.cpu().numpy()
+    ref = np.array([oracle.tape_loglik(O[:L[i], i], V[:L[i], i], *d) for i in range(N)])
+    fin = np.isfinite(ref)
+    assert fin.any() and fin.all() == (not overflow) and np.array_equal(fin, np.isfinite(got))
+    assert np.all(got[~fin] == -np.inf)
+    assert np.all(np.abs(got - ref)[fin] <= 1e-5 * np.maximum(np.abs(ref[fin]), n))
