@@ -9,8 +9,10 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "gpr_internal.h"
@@ -46,6 +48,11 @@ struct KernelBucket {
 // x 2 register forms), forked from and joined back to the context stream.
 #define GPR_MAX_BUCKETS 6
 
+// State copies larger than one piece go through a ring of pinned pieces.
+#define GPR_STAGE_PIECE ((size_t)2 << 20)
+#define GPR_STAGE_SLOTS 8
+#define GPR_STAGE_THREADS 4
+
 struct gpr_ctx {
     gpr_config cfg;
     hipStream_t stream = nullptr;
@@ -57,10 +64,17 @@ struct gpr_ctx {
     GprDataset *d_ds = nullptr;
     float *d_x = nullptr, *d_y = nullptr, *d_w = nullptr, *d_sd = nullptr;
     double *d_lnc = nullptr;
+    // chain state: one allocation, the arrays one after another (state_layout)
+    char *d_state = nullptr;
     uint8_t *d_ops = nullptr;
     float *d_cs = nullptr;
     int32_t *d_len = nullptr;
     double *d_prior = nullptr, *d_ll = nullptr;
+    // pinned buffer that gpr_read_state and gpr_write_state go through (stage_get)
+    std::mutex stage_mu;
+    char *stage = nullptr;
+    size_t stage_bytes = 0;
+    hipEvent_t stage_ev[GPR_STAGE_SLOTS] = {};
     std::vector<GprTile> htiles;
     std::vector<KernelBucket> buckets;
     ClassTune ct[3][2];
@@ -125,12 +139,13 @@ static void drop_graph(gpr_ctx *c) {
 
 static void free_state(gpr_ctx *c) {
     drop_graph(c);
-    void *ps[] = {c->d_ds, c->d_x, c->d_y, c->d_w, c->d_sd, c->d_lnc, c->d_ops, c->d_cs, c->d_len, c->d_prior, c->d_ll,
+    void *ps[] = {c->d_ds, c->d_x, c->d_y, c->d_w, c->d_sd, c->d_lnc, c->d_state,
                   c->d_tiles, c->d_tile_counter, c->d_counters, c->d_good, c->d_ngood, c->d_map_chain,
                   c->d_nres, c->d_map_post, c->d_cutoff, c->d_clock, c->d_metric, c->d_gslab, c->d_faults};
     for (void *p : ps)
         if (p) (void)hipFree(p);
     c->d_ds = nullptr; c->d_x = c->d_y = c->d_w = c->d_sd = nullptr; c->d_lnc = nullptr; c->d_ops = nullptr; c->d_cs = nullptr;
+    c->d_state = nullptr;
     c->d_len = nullptr; c->d_prior = c->d_ll = nullptr; c->d_tiles = nullptr;
     c->d_tile_counter = nullptr; c->d_counters = nullptr; c->d_good = c->d_ngood = c->d_map_chain = nullptr;
     c->d_nres = nullptr; c->d_map_post = c->d_cutoff = nullptr; c->d_clock = nullptr; c->d_metric = nullptr;
@@ -203,9 +218,30 @@ extern "C" int gpr_destroy(gpr_ctx *c) {
     if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
+    for (hipEvent_t e : c->stage_ev)
+        if (e) (void)hipEventDestroy(e);
+    if (c->stage) (void)hipHostFree(c->stage);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return GPR_OK;
+}
+
+// Byte offsets of the state arrays in their allocation.  gpr_write_state's arrays are
+// neighbours, len last (reference semantics has none), so a small state is one copy either way.
+struct StateLayout {
+    size_t prior, ll, cs, ops, len, end;
+};
+static StateLayout state_layout(const gpr_ctx *c) {
+    const size_t N = (size_t)c->N, R = (size_t)c->rows;
+    const auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
+    StateLayout s;
+    s.prior = 0;
+    s.ll = s.prior + up(sizeof(double) * N);
+    s.cs = s.ll + up(sizeof(double) * N);
+    s.ops = s.cs + up(sizeof(float) * R * N);
+    s.len = s.ops + up(R * N);
+    s.end = s.len + up(sizeof(int32_t) * N);
+    return s;
 }
 
 static int kc_for(int n) { return n <= 64 ? 1 : (n <= 128 ? 2 : 4); }
@@ -248,7 +284,7 @@ static void build_tiles(gpr_ctx *c) {
         }
 }
 
-// MALA token slabs of programs longer than GPR_MALA_LDS_ROWS tokens live in global
+// MALA token slabs of programs of more than GPR_MALA_LDS_ROWS rows live in global
 // memory, one per resident wave (workgroups x waves per workgroup) of each launch; the
 // launches of a block run concurrently, so each has its own region.  Sized whenever the
 // tiles change, before any launch, so never inside a graph capture.
@@ -350,11 +386,13 @@ extern "C" int gpr_set_data(gpr_ctx *c, int nd, const int32_t *n, const float *x
     ALLOC(c->d_w, (size_t)total_pts);
     ALLOC(c->d_sd, (size_t)total_pts);
     ALLOC(c->d_lnc, (size_t)total_pts);
-    ALLOC(c->d_ops, (size_t)c->rows * N);
-    ALLOC(c->d_cs, (size_t)c->rows * N);
-    ALLOC(c->d_len, N);
-    ALLOC(c->d_prior, N);
-    ALLOC(c->d_ll, N);
+    const StateLayout sl = state_layout(c);
+    ALLOC(c->d_state, sl.end);
+    c->d_prior = (double *)(c->d_state + sl.prior);
+    c->d_ll = (double *)(c->d_state + sl.ll);
+    c->d_cs = (float *)(c->d_state + sl.cs);
+    c->d_ops = (uint8_t *)(c->d_state + sl.ops);
+    c->d_len = (int32_t *)(c->d_state + sl.len);
     ALLOC(c->d_tiles, N);                  // enough for one chain per tile
     ALLOC(c->d_tile_counter, GPR_MAX_BUCKETS);
     ALLOC(c->d_counters, (size_t)GPR_NCNT);
@@ -382,11 +420,7 @@ extern "C" int gpr_set_data(gpr_ctx *c, int nd, const int32_t *n, const float *x
                            st));
     c->gexec_stale = true;
     HIP_TRY(hipMemsetAsync(c->d_counters, 0, sizeof(unsigned long long) * GPR_NCNT, st));
-    HIP_TRY(hipMemsetAsync(c->d_ops, 0, (size_t)c->rows * N, st));
-    HIP_TRY(hipMemsetAsync(c->d_cs, 0, sizeof(float) * c->rows * N, st));
-    HIP_TRY(hipMemsetAsync(c->d_len, 0, sizeof(int32_t) * N, st));
-    HIP_TRY(hipMemsetAsync(c->d_prior, 0, sizeof(double) * N, st));
-    HIP_TRY(hipMemsetAsync(c->d_ll, 0, sizeof(double) * N, st));
+    HIP_TRY(hipMemsetAsync(c->d_state, 0, sl.end, st));
     HIP_TRY(hipStreamSynchronize(st));
     if (int r = ensure_gslab(c)) return r;
     c->step = 0;
@@ -438,39 +472,225 @@ extern "C" int gpr_init_chains(gpr_ctx *c) {
     return GPR_OK;
 }
 
+// ---------------------------------------------------------------- state copies
+// The caller's arrays are pageable, and most often fresh from the allocator: a read spends
+// its time on page faults and on the one thread that copies out of the runtime's own pinned
+// buffer, not on the link.  So copies go through a pinned buffer of the context: a state of at
+// most one piece in one transfer, a larger one in pieces through a ring of GPR_STAGE_SLOTS,
+// with a few threads between the ring and the caller's arrays.  The buffer is at most
+// GPR_STAGE_SLOTS pieces (16 MB), is kept with the context and holds nothing between calls.
+// Whole runs, before and after: 98304 chains of cap 128 (66 MB read) 36.7 -> 32.3 ms, 57337
+// chains of cap 64 written and read (19 MB) 10.9 -> 9.6 ms, 1024 chains of cap 32 (0.2 MB)
+// 0.95 -> 0.83 ms.
+struct HostCopy {
+    char *host, *dev;
+    size_t bytes;
+};
+
+// Whether the pinned buffer, of at least min(bytes, the whole ring), is there; the caller
+// holds stage_mu.
+static bool stage_get(gpr_ctx *c, size_t bytes) {
+    const bool ring = bytes > GPR_STAGE_PIECE;
+    const size_t want = ring ? GPR_STAGE_PIECE * GPR_STAGE_SLOTS : (bytes + 0xffff) & ~(size_t)0xffff;
+    if (ring)
+        for (hipEvent_t &e : c->stage_ev)
+            if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return false;
+    if (c->stage_bytes >= want) return true;
+    if (c->stage) (void)hipHostFree(c->stage);
+    c->stage = nullptr;
+    c->stage_bytes = 0;
+    if (hipHostMalloc((void **)&c->stage, want, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        c->stage = nullptr;
+        return false;
+    }
+    c->stage_bytes = want;
+    return true;
+}
+
+// Helper threads for `bytes` of host copying or checking: one per 8 MB (starting a thread costs
+// some 20 us; 8 and 12 threads, one per 4 MB, read no faster).
+static int helpers_for(size_t bytes) { return (int)std::min<size_t>(GPR_STAGE_THREADS, 1 + (bytes >> 23)); }
+
+// Threads that are joined when the scope ends; as many of n as the system starts.
+struct Helpers {
+    std::vector<std::thread> t;
+    template <class F>
+    Helpers(int n, F f) {
+        try {
+            t.reserve((size_t)n);
+            for (int k = 0; k < n; k++) t.emplace_back(f, k);
+        } catch (...) {
+        }
+    }
+    ~Helpers() {
+        for (std::thread &x : t) x.join();
+    }
+};
+
+// The copies without the pinned buffer, when there is no memory or no thread for it.
+static int plain_copies(gpr_ctx *c, const HostCopy *cp, int ncp, bool to_host) {
+    for (int k = 0; k < ncp; k++)
+        HIP_TRY(to_host ? hipMemcpyAsync(cp[k].host, cp[k].dev, cp[k].bytes, hipMemcpyDeviceToHost, c->stream)
+                        : hipMemcpyAsync(cp[k].dev, cp[k].host, cp[k].bytes, hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    return GPR_OK;
+}
+
+// Copies through the ring, complete on return.  Piece i uses slot i % GPR_STAGE_SLOTS; st[i]:
+// 0, then 1 when its slot is full (transferred, or filled by a helper), then 2 when the slot
+// is free again.
+static int stage_ring(gpr_ctx *c, const HostCopy *cp, int ncp, bool to_host) {
+    size_t total = 0;
+    std::vector<HostCopy> pc;
+    std::vector<std::atomic<int>> st;
+    try {
+        for (int k = 0; k < ncp; k++) {
+            total += cp[k].bytes;
+            for (size_t o = 0; o < cp[k].bytes; o += GPR_STAGE_PIECE)
+                pc.push_back({cp[k].host + o, cp[k].dev + o, std::min(GPR_STAGE_PIECE, cp[k].bytes - o)});
+        }
+        st = std::vector<std::atomic<int>>(pc.size());
+    } catch (...) {
+        return plain_copies(c, cp, ncp, to_host);
+    }
+    const size_t n = pc.size(), S = GPR_STAGE_SLOTS;
+    for (std::atomic<int> &x : st) x.store(0, std::memory_order_relaxed);
+    const auto slot = [&](size_t i) { return c->stage + (i % S) * GPR_STAGE_PIECE; };
+    std::atomic<size_t> next{0};
+    std::atomic<bool> stop{false};
+    hipError_t err = hipSuccess;
+    const auto wait = [&](size_t i, int v) {
+        while (st[i].load(std::memory_order_acquire) < v && !stop.load(std::memory_order_acquire)) std::this_thread::yield();
+    };
+    const auto helper = [&](int) {
+        for (size_t i; (i = next.fetch_add(1)) < n && !stop.load(std::memory_order_acquire);) {
+            if (to_host) wait(i, 1);
+            else if (i >= S) wait(i - S, 2);
+            if (stop.load(std::memory_order_acquire)) return;
+            if (to_host) memcpy(pc[i].host, slot(i), pc[i].bytes);
+            else memcpy(slot(i), pc[i].host, pc[i].bytes);
+            st[i].store(to_host ? 2 : 1, std::memory_order_release);
+        }
+    };
+    {
+        Helpers h(helpers_for(total), helper);
+        if (h.t.empty()) return plain_copies(c, cp, ncp, to_host);
+        const auto issue = [&](size_t i) {
+            if (err == hipSuccess)
+                err = to_host ? hipMemcpyAsync(slot(i), pc[i].dev, pc[i].bytes, hipMemcpyDeviceToHost, c->stream)
+                              : hipMemcpyAsync(pc[i].dev, slot(i), pc[i].bytes, hipMemcpyHostToDevice, c->stream);
+            if (err == hipSuccess) err = hipEventRecord(c->stage_ev[i % S], c->stream);
+        };
+        const auto arrived = [&](size_t i, int v) {
+            if (err == hipSuccess) err = hipEventSynchronize(c->stage_ev[i % S]);
+            if (err == hipSuccess) st[i].store(v, std::memory_order_release);
+        };
+        for (size_t i = 0, sent = 0; i < n && err == hipSuccess; i++) {
+            if (to_host) {
+                for (; sent < n && sent < i + S; sent++) {
+                    if (sent >= S) {
+                        if (sent > i && st[sent - S].load(std::memory_order_acquire) < 2) break;
+                        wait(sent - S, 2);
+                    }
+                    issue(sent);
+                }
+                arrived(i, 1);
+            } else {
+                wait(i, 1);
+                issue(i);
+                if (i >= S / 2) arrived(i - S / 2, 2);
+            }
+        }
+        if (err != hipSuccess) stop.store(true, std::memory_order_release);
+    }
+    const hipError_t e = hipStreamSynchronize(c->stream);
+    if (err == hipSuccess) err = e;
+    return err == hipSuccess ? GPR_OK : fail(GPR_E_HIP, std::string("state copy: ") + hipGetErrorString(err));
+}
+
+// Copies of state arrays in the order of their addresses on the device, complete on return.
+static int state_copies(gpr_ctx *c, const HostCopy *cp, int ncp, bool to_host) {
+    if (ncp == 0) return plain_copies(c, cp, 0, to_host);
+    const size_t span = (size_t)(cp[ncp - 1].dev - cp[0].dev) + cp[ncp - 1].bytes;
+    std::lock_guard<std::mutex> lk(c->stage_mu);
+    if (!stage_get(c, span)) return plain_copies(c, cp, ncp, to_host);
+    if (span > GPR_STAGE_PIECE) return stage_ring(c, cp, ncp, to_host);
+    if (to_host) {
+        HIP_TRY(hipMemcpyAsync(c->stage, cp[0].dev, span, hipMemcpyDeviceToHost, c->stream));
+        HIP_TRY(hipStreamSynchronize(c->stream));
+        for (int k = 0; k < ncp; k++) memcpy(cp[k].host, c->stage + (cp[k].dev - cp[0].dev), cp[k].bytes);
+    } else {
+        for (int k = 0; k < ncp; k++) memcpy(c->stage + (cp[k].dev - cp[0].dev), cp[k].host, cp[k].bytes);
+        HIP_TRY(hipMemcpyAsync(cp[0].dev, c->stage, span, hipMemcpyHostToDevice, c->stream));
+        HIP_TRY(hipStreamSynchronize(c->stream));
+    }
+    return GPR_OK;
+}
+
+// Why chains [i0, i1) of the caller's arrays are not valid programs: the first chain that is
+// not (its text in why), or -1.
+static long bad_chain(const gpr_ctx *c, const uint8_t *ops, const int32_t *len, size_t i0, size_t i1, const char *&why) {
+    const size_t N = (size_t)c->N;
+    int ds = 0;
+    for (size_t i = i0; i < i1; i++) {
+        while (ds + 1 < c->nd && c->hds[ds + 1].chain0 <= (int)i) ds++;
+        const int L = len[i];
+        why = "len out of [1, cap]";
+        if (L < 1 || L > c->hds[ds].cap) return (long)i;
+        int depth = 0, dm = 0;
+        for (int t = 0; t < L; t++) {
+            const int o = ops[(size_t)t * N + i];
+            why = "bad op code";
+            if (o >= GPR_NUM_OPS) return (long)i;
+            const int ar = gpr_arity(o);
+            why = "malformed postfix";
+            if (depth < ar) return (long)i;
+            depth += 1 - ar;
+            dm = std::max(dm, depth);
+        }
+        if (depth != 1) return (long)i;
+        why = "stack depth above dmax";
+        if (dm > c->cfg.dmax) return (long)i;
+    }
+    return -1;
+}
+
 extern "C" int gpr_write_state(gpr_ctx *c, const uint8_t *ops, const float *cs, const int32_t *len) {
     if (!c || !c->have_data) return fail(GPR_E_STATE, "gpr_set_data must come first");
     if (!ops || !cs) return fail(GPR_E_ARG, "null state arrays");
     const bool ref = c->cfg.semantics == GPR_SEM_REFERENCE;
-    const size_t N = (size_t)c->N;
+    const size_t N = (size_t)c->N, R = (size_t)c->rows;
     if (!ref) {
         if (!len) return fail(GPR_E_ARG, "null len");
-        for (size_t i = 0; i < N; i++) {
-            int ds = 0;
-            while (ds + 1 < c->nd && c->hds[ds + 1].chain0 <= (int)i) ds++;
-            const int L = len[i];
-            if (L < 1 || L > c->hds[ds].cap) return fail(GPR_E_ARG, "chain " + std::to_string(i) + ": len out of [1, cap]");
-            int depth = 0, dm = 0;
-            for (int t = 0; t < L; t++) {
-                const int o = ops[(size_t)t * N + i];
-                if (o >= GPR_NUM_OPS) return fail(GPR_E_ARG, "chain " + std::to_string(i) + ": bad op code");
-                const int ar = gpr_arity(o);
-                if (depth < ar) return fail(GPR_E_ARG, "chain " + std::to_string(i) + ": malformed postfix");
-                depth += 1 - ar;
-                dm = std::max(dm, depth);
-            }
-            if (depth != 1) return fail(GPR_E_ARG, "chain " + std::to_string(i) + ": malformed postfix");
-            if (dm > c->cfg.dmax) return fail(GPR_E_ARG, "chain " + std::to_string(i) + ": stack depth above dmax");
+        // the checks of a large state are shared out in ranges of chains; the lowest bad chain
+        // is reported, as by one loop
+        constexpr int MAXP = GPR_STAGE_THREADS + 1;
+        const int np = R * N <= GPR_STAGE_PIECE / 4 ? 1 : std::min(MAXP, 1 + helpers_for(5 * R * N));
+        long bad[MAXP];
+        const char *why[MAXP] = {};
+        std::atomic<int> next{0};
+        for (long &b : bad) b = -1;
+        const auto part = [&](int) {
+            for (int k; (k = next.fetch_add(1)) < np;)
+                bad[k] = bad_chain(c, ops, len, N * (size_t)k / (size_t)np, N * (size_t)(k + 1) / (size_t)np, why[k]);
+        };
+        {
+            Helpers h(np - 1, part);
+            part(0);
         }
+        for (int k = 0; k < np; k++)
+            if (bad[k] >= 0) return fail(GPR_E_ARG, "chain " + std::to_string(bad[k]) + ": " + why[k]);
     } else {
         for (size_t i = 0; i < N * GPR_REF_SLOTS; i++)
             if (ops[i] >= GPR_REF_NCODES) return fail(GPR_E_ARG, "bad heap op code");
     }
     HIP_TRY(hipSetDevice(c->cfg.device));
-    HIP_TRY(hipMemcpyAsync(c->d_ops, ops, (size_t)c->rows * N, hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(hipMemcpyAsync(c->d_cs, cs, sizeof(float) * c->rows * N, hipMemcpyHostToDevice, c->stream));
-    if (!ref) HIP_TRY(hipMemcpyAsync(c->d_len, len, sizeof(int32_t) * N, hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    const StateLayout s = state_layout(c);
+    const HostCopy cp[3] = {{(char *)cs, c->d_state + s.cs, sizeof(float) * R * N},
+                            {(char *)ops, c->d_state + s.ops, R * N},
+                            {(char *)len, c->d_state + s.len, sizeof(int32_t) * N}};
+    if (int r = state_copies(c, cp, ref ? 2 : 3, false)) return r;
     c->have_state = true;
     return GPR_OK;
 }
@@ -478,14 +698,18 @@ extern "C" int gpr_write_state(gpr_ctx *c, const uint8_t *ops, const float *cs, 
 extern "C" int gpr_read_state(gpr_ctx *c, uint8_t *ops, float *cs, int32_t *len, double *prior, double *ll) {
     if (!c || !c->have_data) return fail(GPR_E_STATE, "no state");
     HIP_TRY(hipSetDevice(c->cfg.device));
-    const size_t N = (size_t)c->N;
-    if (ops) HIP_TRY(hipMemcpyAsync(ops, c->d_ops, (size_t)c->rows * N, hipMemcpyDeviceToHost, c->stream));
-    if (cs) HIP_TRY(hipMemcpyAsync(cs, c->d_cs, sizeof(float) * c->rows * N, hipMemcpyDeviceToHost, c->stream));
-    if (len) HIP_TRY(hipMemcpyAsync(len, c->d_len, sizeof(int32_t) * N, hipMemcpyDeviceToHost, c->stream));
-    if (prior) HIP_TRY(hipMemcpyAsync(prior, c->d_prior, sizeof(double) * N, hipMemcpyDeviceToHost, c->stream));
-    if (ll) HIP_TRY(hipMemcpyAsync(ll, c->d_ll, sizeof(double) * N, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return GPR_OK;
+    const size_t N = (size_t)c->N, R = (size_t)c->rows;
+    const StateLayout s = state_layout(c);
+    const HostCopy all[5] = {{(char *)prior, c->d_state + s.prior, sizeof(double) * N},
+                             {(char *)ll, c->d_state + s.ll, sizeof(double) * N},
+                             {(char *)cs, c->d_state + s.cs, sizeof(float) * R * N},
+                             {(char *)ops, c->d_state + s.ops, R * N},
+                             {(char *)len, c->d_state + s.len, sizeof(int32_t) * N}};
+    HostCopy cp[5];
+    int ncp = 0;
+    for (const HostCopy &k : all)
+        if (k.host) cp[ncp++] = k;
+    return state_copies(c, cp, ncp, true);
 }
 
 // Heap state in main.cu's types (int op codes), converted on the host.
