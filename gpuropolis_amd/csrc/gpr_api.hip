@@ -437,6 +437,7 @@ static GprMHArgs mh_args(gpr_ctx *c, int steps, int32_t block_seed) {
     a.dsd = c->d_sd;
     a.lnc = c->d_lnc;
     a.ds = c->d_ds;
+    a.ndatasets = c->nd;
     a.metric = c->any_metric ? c->d_metric : nullptr;
     a.tiles = c->d_tiles;
     a.ntiles = (int)c->htiles.size();
@@ -463,7 +464,9 @@ extern "C" int gpr_init_chains(gpr_ctx *c) {
     HIP_TRY(hipSetDevice(c->cfg.device));
     GprMHArgs a = mh_args(c, 0, 0);
     if (c->cfg.semantics == GPR_SEM_CONFIG) {
-        HIP_TRY(gpr_launch_init_config(a, c->stream));
+        int rows = 1;
+        for (const GprDataset &d : c->hds) rows = std::max(rows, d.cap);
+        HIP_TRY(gpr_launch_init_config(a, rows, c->stream));
     } else {
         HIP_TRY(gpr_launch_init_ref(a, c->stream));
     }

@@ -171,6 +171,17 @@ __device__ __forceinline__ float op_un(int op, float a, float c) {
     }
 }
 
+// The dataset of a chain: the last one that starts at or before it.
+__device__ __forceinline__ int chain_dataset(const GprDataset *ds, int nd, int chain) {
+    int lo = 0, hi = nd;
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (ds[mid].chain0 <= chain) lo = mid;
+        else hi = mid;
+    }
+    return lo;
+}
+
 // ---------------------------------------------------------------- wave program state
 // Lane l holds token l in (o0, c0) and token l+64 in (o1, c1); tokens >= len are 0.
 struct WaveProg {

@@ -65,6 +65,7 @@ struct GprMHArgs {
     const float *dsd;       // sd per point (reference lane schedule)
     const double *lnc;      // 0.5*(logf(2 pi) + 2 logf(sd)) per point, host libm (main.cu:300)
     const GprDataset *ds;
+    int ndatasets;
     const GprMetric *metric;  // [ndatasets] or null (identity metric everywhere)
     const GprTile *tiles;
     int ntiles;
@@ -157,7 +158,7 @@ hipError_t gpr_launch_dataset_prep(const float *sd, int n, int nchains, int cap,
                                    hipStream_t s);
 hipError_t gpr_launch_eval_lane(const GprEvalArgs &a, hipStream_t s);
 hipError_t gpr_launch_grad_wave(const GprEvalArgs &a, hipStream_t s);
-hipError_t gpr_launch_init_config(const GprMHArgs &a, hipStream_t s);
+hipError_t gpr_launch_init_config(const GprMHArgs &a, int rows, hipStream_t s);
 hipError_t gpr_launch_init_ref(const GprMHArgs &a, hipStream_t s);
 hipError_t gpr_launch_resample(const GprResampleArgs &a, hipStream_t s);
 hipError_t gpr_launch_resample_quantile(const GprResampleArgs &a, hipStream_t s);

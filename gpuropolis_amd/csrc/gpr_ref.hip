@@ -850,27 +850,75 @@ hipError_t gpr_launch_mh_ref_wave(const GprMHArgs &a, int kc, int grid, hipStrea
 // ---------------------------------------------------------------- init and median resampling
 // initial draw (main.cu:1133-1137): 31 ops ~ U{0..NOPS-2}, then 31 constants
 // 10^U{-4..3} N(0,1), host transforms, stream (chain, step, purpose, 0)
-// The op set is a template parameter of the draw kernels: each one-lane-per-chain draw
-// loop sees a constant table row.
+// The op set is a template parameter: the draw sees a constant table row.
+// Word k of the stream, halved as rand31 does.
+struct WordSrc {
+    uint32_t chain, step, purpose, klo, khi, k;
+    __device__ __forceinline__ uint32_t at(uint32_t i) const {
+        return gpr_u4_word(gpr_philox(chain, step, purpose << 24, i >> 2, klo, khi), (int)(i & 3)) >> 1;
+    }
+    __device__ __forceinline__ uint32_t rand31() { return at(k++); }
+};
 template <int SET>
-__device__ void r_draw_chain(uint64_t seed, uint32_t chain, uint32_t step, uint32_t purpose, uint8_t *ops, float *cs,
-                             int N) {
+__device__ __forceinline__ void r_draw_serial(WordSrc s, uint8_t *ops, float *cs, int stride) {
 #pragma clang fp contract(off)
-    PhiloxSrc s;
-    s.st.init(seed, chain, step, purpose, 0);
     for (int i = 0; i < GPR_REF_SLOTS; i++)
-        ops[(size_t)i * N + chain] = (uint8_t)gpr_opset_code(SET, r_host_random_int(gpr_opset_nops(SET) - 1, s));
+        ops[i * stride] = (uint8_t)gpr_opset_code(SET, r_host_random_int(gpr_opset_nops(SET) - 1, s));
     for (int i = 0; i < GPR_REF_SLOTS; i++) {
         const int order = r_host_random_int(8, s) - 4;
-        cs[(size_t)i * N + chain] = 1.0f * r_pow10(order) * r_host_random_normal(s);
+        cs[i * stride] = 1.0f * r_pow10(order) * r_host_random_normal(s);
+    }
+}
+
+// The draws of the chains of one workgroup (32 of them, from c0 on; those in `who`).  Drawn by
+// one thread a chain waits for 31 Philox blocks and 31 normals in a row (1024 chains drawn in 50
+// us with the call; 20 us this way).  Here
+// a half wave draws a chain, a slot per lane: unless one of the 62 integer draws is
+// rejected, op i takes word i of the stream and constant i the words 31 + 3 i .. 33 + 3 i.
+// After a rejection (some 3e-7 of chains) the words move, and one lane draws in order.  The
+// tapes are staged in LDS so that the state's rows are written 32 chains at a time.
+#define R_DRAW_WG 512
+#define R_DRAW_CHAINS 32
+#define R_DRAW_STRIDE (R_DRAW_CHAINS + 1)
+template <int SET>
+__device__ void r_draw_chains(uint64_t seed, int c0, uint32_t who, uint32_t step, uint32_t purpose, uint8_t *ops,
+                              float *cs, int N) {
+#pragma clang fp contract(off)
+    __shared__ float lc[GPR_REF_SLOTS * R_DRAW_STRIDE];
+    __shared__ uint8_t lo[GPR_REF_SLOTS * R_DRAW_STRIDE];
+    const int i = threadIdx.x & 31;
+    const uint32_t klo = (uint32_t)uni((int)(uint32_t)seed), khi = (uint32_t)uni((int)(uint32_t)(seed >> 32));
+    for (int p = 0; p < R_DRAW_CHAINS / (R_DRAW_WG / 32); p++) {
+        const int h = p * (R_DRAW_WG / 32) + (int)(threadIdx.x >> 5);
+        const bool drawn = (who >> h) & 1u;
+        const WordSrc src{(uint32_t)(c0 + h), step, purpose, klo, khi, 0u};
+        const uint32_t NOPS = (uint32_t)gpr_opset_nops(SET) - 1, ODIV = 0x7fffffffu / NOPS, EDIV = 0x7fffffffu / 8u;
+        const int slot = min(i, GPR_REF_SLOTS - 1);
+        const uint32_t op = src.at((uint32_t)slot) / ODIV, e = src.at((uint32_t)(GPR_REF_SLOTS + 3 * slot)) / EDIV;
+        const float u = (float)src.at((uint32_t)(GPR_REF_SLOTS + 3 * slot + 1)) / (float)0x7fffffff;
+        const float v = (float)src.at((uint32_t)(GPR_REF_SLOTS + 3 * slot + 2)) / (float)0x7fffffff;
+        const uint64_t rejected = ballot(op >= NOPS || e >= 8u);
+        if (((uint32_t)(rejected >> (threadIdx.x & 32))) == 0) {
+            if (drawn && i < GPR_REF_SLOTS) {
+                lo[i * R_DRAW_STRIDE + h] = (uint8_t)gpr_opset_code(SET, (int)op);
+                lc[i * R_DRAW_STRIDE + h] = 1.0f * r_pow10((int)e - 4) * (sqrtf(-2.0f * gpr_logf(u)) * gpr_sin2pi(v));
+            }
+        } else if (drawn && i == 0) {
+            r_draw_serial<SET>(src, lo + h, lc + h, R_DRAW_STRIDE);
+        }
+    }
+    __syncthreads();
+    if (!((who >> i) & 1u)) return;
+    for (int t = threadIdx.x >> 5; t < GPR_REF_SLOTS; t += R_DRAW_WG / 32) {
+        ops[(size_t)t * N + c0 + i] = lo[t * R_DRAW_STRIDE + i];
+        cs[(size_t)t * N + c0 + i] = lc[t * R_DRAW_STRIDE + i];
     }
 }
 
 template <int SET>
-__global__ void k_init_ref(GprMHArgs a) {
-    const int chain = blockIdx.x * blockDim.x + threadIdx.x;
-    if (chain >= a.nchains) return;
-    r_draw_chain<SET>(a.seed, (uint32_t)chain, 0, GPR_P_INIT, a.ops, a.cs, a.nchains);
+__global__ void __launch_bounds__(R_DRAW_WG) k_init_ref(GprMHArgs a) {
+    const int c0 = blockIdx.x * R_DRAW_CHAINS, n = min(R_DRAW_CHAINS, a.nchains - c0);
+    r_draw_chains<SET>(a.seed, c0, n == 32 ? ~0u : (1u << n) - 1u, 0, GPR_P_INIT, a.ops, a.cs, a.nchains);
 }
 
 #define GPR_OPSET_LAUNCH(KERNEL, SET, GRID, BLOCK, S, ARGS)                                                        \
@@ -883,7 +931,7 @@ __global__ void k_init_ref(GprMHArgs a) {
     }
 
 hipError_t gpr_launch_init_ref(const GprMHArgs &a, hipStream_t s) {
-    GPR_OPSET_LAUNCH(k_init_ref, a.opset, dim3((a.nchains + 255) / 256), dim3(256), s, a);
+    GPR_OPSET_LAUNCH(k_init_ref, a.opset, dim3((a.nchains + R_DRAW_CHAINS - 1) / R_DRAW_CHAINS), dim3(R_DRAW_WG), s, a);
     return hipGetLastError();
 }
 
@@ -899,41 +947,78 @@ __device__ __forceinline__ double r_unkey(uint64_t k) {
     return __builtin_bit_cast(double, b);
 }
 
+// Adds 1 to hist[bin] for the lanes of `mine`: posteriors share their leading bytes (and the
+// NaN ones all bytes), so the lanes with the first lane's bin count as one atomic, a few
+// times, before the rest add theirs one by one.
+__device__ __forceinline__ void r_hist_add(unsigned int *hist, int bin, bool mine) {
+    uint64_t m = ballot(mine);
+    for (int k = 0; k < 3 && m; k++) {
+        const int lead = __builtin_ctzll(m), b = rl_i(bin, lead);
+        const uint64_t same = ballot(mine && bin == b) & m;
+        if (lane_id() == lead) atomicAdd(&hist[b], (unsigned int)__popcll(same));
+        m &= ~same;
+    }
+    if ((m >> lane_id()) & 1) atomicAdd(&hist[bin], 1u);
+}
+
 // One workgroup per dataset: radix select (8 passes of 8 bits) of the element of rank
-// floor(nchains * quantile) in the NaN-first order; cutoff[d] is its value.
+// floor(nchains * quantile) in the NaN-first order; cutoff[d] is its value.  Latency bounds
+// the passes: the keys of up to R_SEL_KEYS chains per thread stay in registers between
+// them, and one wave scans the 256 bins, four per lane, where a single thread walked them
+// (1024 chains selected and re-drawn in 103 us with the
+// call before, 29 us now).
 #define R_SEL_WG 1024
+#define R_SEL_KEYS 4
 __global__ void __launch_bounds__(R_SEL_WG) k_rs_quantile_select(GprResampleArgs a) {
     const GprDataset d = a.ds[blockIdx.x];
     __shared__ unsigned int hist[256];
     __shared__ uint64_t s_prefix;
     __shared__ int s_rank;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, l = lane_id();
+    const auto key = [&](int i) { return r_key(a.prior[d.chain0 + i] + a.ll[d.chain0 + i]); };
+    const bool held = d.nchains <= R_SEL_WG * R_SEL_KEYS;
+    uint64_t kept[R_SEL_KEYS];
+#pragma unroll
+    for (int q = 0; q < R_SEL_KEYS; q++) kept[q] = held && tid + q * R_SEL_WG < d.nchains ? key(tid + q * R_SEL_WG) : 0;
     if (tid == 0) {
         s_prefix = 0;
         // the rank of the cutoff, cutoff = sorted[(int)(N * q)] (main.cu:1219); gpr_create
         // keeps q in [0, 1), and the clamp keeps the select inside the keys regardless
         s_rank = min(max((int)((float)d.nchains * a.quantile), 0), d.nchains - 1);
     }
-    __syncthreads();
     for (int pass = 7; pass >= 0; pass--) {
-        for (int b = tid; b < 256; b += R_SEL_WG) hist[b] = 0;
+        if (tid < 256) hist[tid] = 0;
         __syncthreads();
         const uint64_t prefix = s_prefix;
         const uint64_t hmask = pass == 7 ? 0 : (~0ull << ((pass + 1) * 8));
-        for (int i = tid; i < d.nchains; i += R_SEL_WG) {
-            const uint64_t k = r_key(a.prior[d.chain0 + i] + a.ll[d.chain0 + i]);
-            if ((k & hmask) == prefix) atomicAdd(&hist[(k >> (pass * 8)) & 255], 1u);
+        const auto add = [&](uint64_t k, bool in) {
+            r_hist_add(hist, (int)(k >> (pass * 8)) & 255, in && (k & hmask) == prefix);
+        };
+        if (held) {
+#pragma unroll
+            for (int q = 0; q < R_SEL_KEYS; q++)
+                if (q * R_SEL_WG < d.nchains) add(kept[q], tid + q * R_SEL_WG < d.nchains);
+        } else {
+            for (int i0 = 0; i0 < d.nchains; i0 += R_SEL_WG) {
+                const bool in = i0 + tid < d.nchains;
+                add(in ? key(i0 + tid) : 0, in);
+            }
         }
         __syncthreads();
-        if (tid == 0) {
-            int r = s_rank;
-            int b = 0;
-            for (; b < 256; b++) {
-                if (r < (int)hist[b]) break;
-                r -= (int)hist[b];
+        if (tid < 64) {
+            const int r = s_rank;
+            int h[4], below = 0;
+#pragma unroll
+            for (int q = 0; q < 4; q++) below += h[q] = (int)hist[4 * l + q];
+            below = wave_scan_i(below) - below;       // keys in the bins of the lanes before
+            const int own = h[0] + h[1] + h[2] + h[3];
+            if (r >= below && r < below + own) {      // one lane: the rank is below the sum of all
+                int b = 0;
+                int left = r - below;
+                for (; b < 3 && left >= h[b]; b++) left -= h[b];
+                s_rank = left;
+                s_prefix = prefix | ((uint64_t)(4 * l + b) << (pass * 8));
             }
-            s_rank = r;
-            s_prefix = prefix | ((uint64_t)b << (pass * 8));
         }
         __syncthreads();
     }
@@ -941,21 +1026,21 @@ __global__ void __launch_bounds__(R_SEL_WG) k_rs_quantile_select(GprResampleArgs
 }
 
 template <int SET>
-__global__ void k_rs_quantile_redraw(GprResampleArgs a) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= a.nchains) return;
-    int di = 0;
-    while (di + 1 < a.ndatasets && a.ds[di + 1].chain0 <= c) di++;
-    if (!(a.prior[c] + a.ll[c] < a.cutoff[di])) return;   // NaN posteriors never resampled
-    r_draw_chain<SET>(a.seed, (uint32_t)c, a.clock ? a.clock[1] : a.block, GPR_P_RESAMPLE, a.ops, a.cs, a.nchains);
-    atomicAdd(a.nresampled, 1);
+__global__ void __launch_bounds__(R_DRAW_WG) k_rs_quantile_redraw(GprResampleArgs a) {
+    const int c0 = blockIdx.x * R_DRAW_CHAINS, c = c0 + (int)(threadIdx.x & 31);
+    bool low = false;      // NaN posteriors never resampled
+    if (c < a.nchains) low = a.prior[c] + a.ll[c] < a.cutoff[chain_dataset(a.ds, a.ndatasets, c)];
+    const uint32_t who = (uint32_t)ballot(low);       // each half of each wave: the same 32 chains
+    if (!who) return;
+    r_draw_chains<SET>(a.seed, c0, who, a.clock ? a.clock[1] : a.block, GPR_P_RESAMPLE, a.ops, a.cs, a.nchains);
+    if (threadIdx.x == 0) atomicAdd(a.nresampled, __popc(who));
 }
 
 hipError_t gpr_launch_resample_quantile(const GprResampleArgs &a, hipStream_t s) {
     hipLaunchKernelGGL(k_rs_quantile_select, dim3(a.ndatasets), dim3(R_SEL_WG), 0, s, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    GPR_OPSET_LAUNCH(k_rs_quantile_redraw, a.opset, dim3((a.nchains + 255) / 256), dim3(256), s, a);
+    GPR_OPSET_LAUNCH(k_rs_quantile_redraw, a.opset, dim3((a.nchains + R_DRAW_CHAINS - 1) / R_DRAW_CHAINS), dim3(R_DRAW_WG), s, a);
     return hipGetLastError();
 }
 
