@@ -87,19 +87,17 @@ __device__ __forceinline__ int dpp_i(int v) {
     return __builtin_amdgcn_mov_dpp(v, CTRL, 0xf, 0xf, false);
 }
 
-// Sum over the 64 lanes, returned uniform.  Butterflies inside each 16-lane row, then
-// the four row sums combined in a fixed order.
+// Sum over the 64 lanes, returned uniform.  Butterflies inside each 16-lane row, then rows 0
+// and 1, rows 2 and 3, and the pairs, in lane 63: one add a step, with the other lane's value
+// as its DPP operand (s_nop: that operand is read two wait states after the vector unit wrote
+// it, and the lane one after).
 __device__ __forceinline__ float wave_sum_f(float v) {
-    v += dpp_f<DPP_QP_1032>(v);
-    v += dpp_f<DPP_QP_2301>(v);
-    v += dpp_f<DPP_ROW_HALF_MIRROR>(v);
-    v += dpp_f<DPP_ROW_MIRROR>(v);
-    // rows 0 and 1, rows 2 and 3, then the pairs, in lane 63: (r0 + r1) + (r2 + r3) in two
-    // adds, where lane reads took four and three (s_nop: a DPP operand is read two wait states
-    // after the vector unit wrote it)
-    __asm__("s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
-            "s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf\n\ts_nop 0"
+#define GPR_DPP_ADD(CTRL) "s_nop 1\n\tv_add_f32_dpp %0, %0, %0 " CTRL " bank_mask:0xf\n\t"
+    __asm__(GPR_DPP_ADD("quad_perm:[1,0,3,2] row_mask:0xf") GPR_DPP_ADD("quad_perm:[2,3,0,1] row_mask:0xf")
+            GPR_DPP_ADD("row_half_mirror row_mask:0xf") GPR_DPP_ADD("row_mirror row_mask:0xf")
+            GPR_DPP_ADD("row_bcast:15 row_mask:0xa") GPR_DPP_ADD("row_bcast:31 row_mask:0xc") "s_nop 0"
             : "+v"(v));
+#undef GPR_DPP_ADD
     return rl_f(v, 63);
 }
 template <int CTRL>
@@ -566,7 +564,10 @@ __device__ __forceinline__ void wave_eval_ls(const WaveProg &p, const float (&xs
     }
 }
 
-// Dataset points of one chunk: point index base + k*64 + lane.
+// Dataset points of one chunk: point index base + k*64 + lane, the last point again past the
+// data (the sums take no term of these lanes).  A clamped 32-bit offset for the three loads costs
+// a quarter of a mask and three 64-bit addresses; with the sums' DPP adds, 99.5 -> 96.6 ms
+// on 131072 chains at n = 250, MALA 97.2 -> 94.7 ms.
 template <int KC>
 struct Chunk {
     float x[KC], y[KC], w[KC];
@@ -574,11 +575,10 @@ struct Chunk {
         const int l = opaque_lane_i32(lane_id());   // the point's offset is computed here, not kept live
 #pragma unroll
         for (int k = 0; k < KC; k++) {
-            const int i = base + k * 64 + l;
-            const bool v = i < n;
-            x[k] = v ? dx[i] : 0.0f;
-            y[k] = v ? dy[i] : 0.0f;
-            w[k] = v ? dw[i] : 0.0f;
+            const uint32_t o = 4u * (uint32_t)min(base + k * 64 + l, n - 1);
+            x[k] = *(const float *)((const char *)dx + o);
+            y[k] = *(const float *)((const char *)dy + o);
+            w[k] = *(const float *)((const char *)dw + o);
         }
     }
 };
@@ -656,6 +656,7 @@ __device__ __forceinline__ double wave_loglik(const WaveProg &p, const GprDatase
                               double reject_below = -GPR_INF, int *points = nullptr) {
     float acc = 0.0f, comp = 0.0f;
     const int l = lane_id();
+    const double wc = d.wconst > 0.0 ? d.wconst : 1.0;
     if (points) *points = d.n;
     for (int ch = 0; ch < nchunks; ch++) {
         Chunk<KC> c;
@@ -673,7 +674,7 @@ __device__ __forceinline__ double wave_loglik(const WaveProg &p, const GprDatase
         }
         if (ch + 1 < nchunks && reject_below > -GPR_INF) {
             const double lb = (double)wave_sum_f(acc - comp) * (1.0 - 1e-4);
-            const double ub = d.lconst - (d.wconst > 0.0 ? d.wconst * lb : lb);
+            const double ub = d.lconst - wc * lb;
             if (!(ub >= reject_below)) {
                 if (points) *points = (ch + 1) * 64 * KC;
                 return -GPR_INF;
@@ -956,12 +957,16 @@ __device__ __forceinline__ double wave_loglik_dual(const WaveProg &p, const GprD
     for (int j = 0; j < NT; j++) ga[j] = 0.0f;
     const bool folded = d.wconst > 0.0;
     const float wf = (float)d.wconst;
+    const double wc = folded ? d.wconst : 1.0;
     const int nlo = __popcll(cm[0]);
     if (points) *points = d.n;
     for (int ch = 0; ch < nchunks; ch++) {
         Chunk<1> c;
         if (ch == 0) c = c0; else c.load(dx, dy, dw, d.n, ch * 64);
-        const float xv = c.x[0];
+        const int i = ch * 64 + l;
+        const bool valid = i < d.n;
+        // (0 past the data: pow_bm1 looks at every lane)
+        const float xv = valid ? c.x[0] : 0.0f;
         float T[W], U[W];
         // token 0 (x, a constant of rank 0 or one) starts the stack in T
         const bool t0x = (m.x[0] & 1ull) != 0, t0c = (cm[0] & 1ull) != 0;
@@ -976,8 +981,6 @@ __device__ __forceinline__ double wave_loglik_dual(const WaveProg &p, const GprD
         for (int t = 1; t < lo_end; t++) dual_token<0, NT>(p, m, cm, nlo, j0, xv, lane, laneb, lanec, T, U, sp, t);
         if (HI)
             for (int t = 64; t < p.len; t++) dual_token<1, NT>(p, m, cm, nlo, j0, xv, lane, laneb, lanec, T, U, sp, t);
-        const int i = ch * 64 + l;
-        const bool valid = i < d.n;
         const float r = T[0] - c.y[0];
         const float term = valid ? (r * r) * c.w[0] : 0.0f;
         const float yv = term - comp;
@@ -989,7 +992,7 @@ __device__ __forceinline__ double wave_loglik_dual(const WaveProg &p, const GprD
         for (int j = 0; j < NT; j++) ga[j] = valid ? __builtin_fmaf(G, T[j + 1], ga[j]) : ga[j];
         if (ch + 1 < nchunks && reject_below > -GPR_INF) {
             const double lb = (double)wave_sum_f(acc - comp) * (1.0 - 1e-4);
-            const double ub = d.lconst - (d.wconst > 0.0 ? d.wconst * lb : lb);
+            const double ub = d.lconst - wc * lb;
             if (!(ub >= reject_below)) {
                 if (points) *points = (ch + 1) * 64;
                 return -GPR_INF;
