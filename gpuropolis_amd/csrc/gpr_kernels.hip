@@ -52,7 +52,10 @@ __global__ void k_fill_logint() {
 // unconstrained it takes 138 VGPRs and three waves, 20 % slower.
 // MET: some dataset of the launch has a proposal metric.  The metric path holds many
 // wave-uniform values (matrix rows, pointers), so launches without a metric use a
-// build without it, whose scalar registers then fit with far fewer spills.
+// build without it, whose scalar registers then fit with far fewer spills.  With SPEC too its
+// random-walk moves run at five waves per SIMD, since at six the step loop spills (a rational
+// of 7 constants, n = 37: 9.12e8 steps/s at six, 9.90e8 at five, 9.17e8 at four); without
+// SPEC six stay faster (59 datasets of 6 to 250 points: 1.14e9 against 1.11e9).
 #ifndef GPR_MALA_WAVES_PER_EU
 #define GPR_MALA_WAVES_PER_EU 4
 #endif
@@ -64,7 +67,7 @@ __global__ void k_fill_logint() {
 // larger datasets keep their registers.
 template <int KC, bool HI, bool MALA, bool MET, bool SPEC = false>
 __global__ void __launch_bounds__(GPR_WG)
-__attribute__((amdgpu_waves_per_eu(MALA ? (MET ? GPR_MALA_MET_WAVES_PER_EU : GPR_MALA_WAVES_PER_EU) : (KC == 1 ? 6 : 1))))
+__attribute__((amdgpu_waves_per_eu(MALA ? (MET ? GPR_MALA_MET_WAVES_PER_EU : GPR_MALA_WAVES_PER_EU) : (KC == 1 ? (MET && SPEC ? 5 : 6) : 1))))
 k_mh_config_wave(GprMHArgs a) {
     const int wave = uni((int)(threadIdx.x >> 6));
     const int l = lane_id();
