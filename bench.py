@@ -47,18 +47,18 @@ HBM_PEAK = 8.0e12
 # were measured on.  For the batched workload a "launch" is one block's six concurrent
 # size-class launches.
 MEASURED_TRAFFIC = {
-    ("full", 1048576, 1000, 0): 1_323_373_952,
-    ("large", 131072, 1000, 0): 163_308_256,
-    ("batched", 262144, 1000, 0): 384_401_216,
+    ("full", 1048576, 1000, 0): 1_344_635_552,
+    ("large", 131072, 1000, 0): 137_598_080,
+    ("batched", 262144, 1000, 0): 15_994_380_864,
 }
 # VALU and SALU instructions per chain-step of the same launches (rocprofv3 --pmc
 # SQ_INSTS_VALU, SQ_INSTS_SALU over chains x steps).  With the live launch time they give
 # the share of issue slots each unit is busy: one wave64 instruction per SIMD every 4
 # cycles, 1024 SIMDs at 2.4 GHz.
 MEASURED_ISSUE = {
-    ("full", 1048576, 1000, 0): (1116.28, 758.48),
-    ("large", 131072, 1000, 0): (281.12, 288.25),
-    ("batched", 262144, 1000, 0): (319.92, 296.77),
+    ("full", 1048576, 1000, 0): (1054.96, 694.64),
+    ("large", 131072, 1000, 0): (247.40, 179.35),
+    ("batched", 262144, 1000, 0): (289.40, 199.07),
 }
 
 METRIC = "MH steps/sec + node×datapoint evals/sec (% VALU peak); ESS/sec MALA vs RW"
