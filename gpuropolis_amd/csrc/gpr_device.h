@@ -19,8 +19,6 @@ __device__ __forceinline__ double rl_d(double v, int l) {
     int hi = __builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), l);
     return __builtin_bit_cast(double, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
 }
-__device__ __forceinline__ int wl_i(int old, int v, int l) { return lane_id() == l ? v : old; }
-__device__ __forceinline__ float wl_f(float old, float v, int l) { return lane_id() == l ? v : old; }
 __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 __device__ __forceinline__ double uni_d(double v) {
     const unsigned long long b = (unsigned long long)__double_as_longlong(v);
@@ -78,10 +76,6 @@ __device__ __forceinline__ uint64_t ballot(bool p) { return __ballot(p); }
 #define DPP_ROW_BCAST15 0x142
 #define DPP_ROW_BCAST31 0x143
 
-template <int CTRL>
-__device__ __forceinline__ float dpp_f(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
-}
 template <int CTRL>
 __device__ __forceinline__ int dpp_i(int v) {
     return __builtin_amdgcn_mov_dpp(v, CTRL, 0xf, 0xf, false);
