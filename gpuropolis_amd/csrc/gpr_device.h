@@ -3,6 +3,7 @@
 // wave-uniform tape interpreter with its VGPR value stack, the Gaussian
 // log-likelihood and description-length prior of a wave-resident program.
 #pragma once
+#include "gpr_index.h"
 #include "gpr_internal.h"
 
 #define GPR_INF (__builtin_inf())
@@ -561,18 +562,20 @@ __device__ __forceinline__ void wave_eval_ls(const WaveProg &p, const float (&xs
 // Dataset points of one chunk: point index base + k*64 + lane, the last point again past the
 // data (the sums take no term of these lanes).  A clamped 32-bit offset for the three loads costs
 // a quarter of a mask and three 64-bit addresses; with the sums' DPP adds, 99.5 -> 96.6 ms
-// on 131072 chains at n = 250, MALA 97.2 -> 94.7 ms.
+// on 131072 chains at n = 250, MALA 97.2 -> 94.7 ms.  base < n is wave-uniform: it goes to
+// the scalar addresses.
 template <int KC>
 struct Chunk {
     float x[KC], y[KC], w[KC];
     __device__ __forceinline__ void load(const float *dx, const float *dy, const float *dw, int n, int base) {
         const int l = opaque_lane_i32(lane_id());   // the point's offset is computed here, not kept live
+        const float *px = dx + base, *py = dy + base, *pw = dw + base;
 #pragma unroll
         for (int k = 0; k < KC; k++) {
-            const uint32_t o = 4u * (uint32_t)min(base + k * 64 + l, n - 1);
-            x[k] = *(const float *)((const char *)dx + o);
-            y[k] = *(const float *)((const char *)dy + o);
-            w[k] = *(const float *)((const char *)dw + o);
+            const uint32_t o = gpr_point_offset(k * 64 + l, n - 1 - base);
+            x[k] = *(const float *)((const char *)px + o);
+            y[k] = *(const float *)((const char *)py + o);
+            w[k] = *(const float *)((const char *)pw + o);
         }
     }
 };

@@ -1,0 +1,9 @@
+// Index arithmetic of the kernels in plain constexpr functions, which the host's tests
+// compile as they stand.
+#pragma once
+#include <stdint.h>
+
+// Byte offset of point i of a chunk, from the chunk's first point; last: the index of the
+// dataset's last point from there, which lanes past it load again.  The chunk's own offset,
+// which passes 32 bits from 2^30 points on, stays out of it: it goes to the base address.
+constexpr uint32_t gpr_point_offset(int i, int last) { return 4u * (uint32_t)(i < last ? i : last); }

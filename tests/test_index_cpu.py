@@ -1,0 +1,30 @@
+"""The kernels' index arithmetic on the CPU, at sizes that a GPU test would take minutes on."""
+import ctypes as C
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def shim(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("index") / "libindex.so")
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", os.path.join(HERE, "index_shim.cpp"), "-o", out])
+    L = C.CDLL(out)
+    L.shim_point_offset.restype = C.c_uint32
+    return L
+
+
+@pytest.mark.parametrize("kc", [1, 2, 4])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 1000, (1 << 29) + 5, 1 << 30, (1 << 30) + 130, (1 << 31) - 1])
+def test_a_chunk_loads_its_own_points(shim, n, kc):
+    """Lane l of chunk `base` loads point base + 64 k + l, or the last one: past 2^30 points too,
+    where a point's byte offset in the dataset no longer fits 32 bits."""
+    chunk = 64 * kc
+    last = (n - 1) // chunk * chunk
+    for base in sorted({0, last, max(last - chunk, 0), min(last, (1 << 30) // chunk * chunk)}):
+        for i in range(chunk):
+            at = 4 * base + shim.shim_point_offset(i, n - 1 - base)
+            assert at == 4 * min(base + i, n - 1), (n, base, i)
