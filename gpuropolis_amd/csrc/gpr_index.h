@@ -7,3 +7,7 @@
 // dataset's last point from there, which lanes past it load again.  The chunk's own offset,
 // which passes 32 bits from 2^30 points on, stays out of it: it goes to the base address.
 constexpr uint32_t gpr_point_offset(int i, int last) { return 4u * (uint32_t)(i < last ? i : last); }
+
+// Most workgroups of a launch of `threads` threads each.  A launch's size in threads has 32
+// bits: HIP starts what is left of a larger one modulo 2^32, and reports no error.
+constexpr int gpr_max_groups(int threads) { return (int)(0xffffffffu / (unsigned)threads); }

@@ -1254,6 +1254,26 @@ __global__ void __launch_bounds__(GPR_WG) k_eval_split(GprEvalArgs a) {
     }
 }
 
+// Launches of one workgroup of `threads` per tape, as many as their size takes (8.4 million tapes
+// fill a launch of 512 threads each): launch(a, groups) starts `groups` of them on the first
+// tapes of a's arrays, a column per tape.
+template <class F>
+static hipError_t launch_per_tape(GprEvalArgs a, int threads, F launch) {
+    for (int left = a.nchains; left > 0;) {
+        const int groups = std::min(left, gpr_max_groups(threads));
+        launch(a, groups);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        a.ops += groups;
+        a.cs += groups;
+        a.len += groups;
+        a.ll += groups;
+        if (a.grad) a.grad += groups;
+        left -= groups;
+    }
+    return hipSuccess;
+}
+
 template <int KC, bool RAW>
 static hipError_t launch_eval_split(const GprEvalArgs &a, hipStream_t s) {
     const size_t sh = sizeof(float) * 64 * (size_t)a.rows * GPR_WAVES_PER_WG;
@@ -1262,9 +1282,10 @@ static hipError_t launch_eval_split(const GprEvalArgs &a, hipStream_t s) {
         hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh);
         if (e != hipSuccess) return e;
     }
-    if (a.cap > 64) hipLaunchKernelGGL((k_eval_split<KC, true, RAW>), dim3(a.nchains), dim3(GPR_WG), sh, s, a);
-    else hipLaunchKernelGGL((k_eval_split<KC, false, RAW>), dim3(a.nchains), dim3(GPR_WG), sh, s, a);
-    return hipGetLastError();
+    return launch_per_tape(a, GPR_WG, [&](const GprEvalArgs &b, int groups) {
+        if (b.cap > 64) hipLaunchKernelGGL((k_eval_split<KC, true, RAW>), dim3(groups), dim3(GPR_WG), sh, s, b);
+        else hipLaunchKernelGGL((k_eval_split<KC, false, RAW>), dim3(groups), dim3(GPR_WG), sh, s, b);
+    });
 }
 template <int KC, bool RAW>
 static hipError_t launch_eval_wave(const GprEvalArgs &a, hipStream_t s) {
@@ -1439,9 +1460,10 @@ hipError_t gpr_launch_grad_wave(const GprEvalArgs &args, hipStream_t s) {
     // per lane, and the waves' gradients (4 rows a wave)
     a.rows = std::max(a.cap, 16 * waves);
     const size_t sh = sizeof(float) * 64 * ((size_t)a.rows + std::min((a.d.n + 63) / 64, 16));
-    if (a.cap > 64) hipLaunchKernelGGL(k_grad_wave<true>, dim3(a.nchains), dim3(64 * waves), sh, s, a);
-    else hipLaunchKernelGGL(k_grad_wave<false>, dim3(a.nchains), dim3(64 * waves), sh, s, a);
-    return hipGetLastError();
+    return launch_per_tape(a, 64 * waves, [&](const GprEvalArgs &b, int groups) {
+        if (b.cap > 64) hipLaunchKernelGGL(k_grad_wave<true>, dim3(groups), dim3(64 * waves), sh, s, b);
+        else hipLaunchKernelGGL(k_grad_wave<false>, dim3(groups), dim3(64 * waves), sh, s, b);
+    });
 }
 
 // Lane schedule: one lane per chain; tape staged in LDS [token][lane], value stack in

@@ -28,3 +28,9 @@ def test_a_chunk_loads_its_own_points(shim, n, kc):
         for i in range(chunk):
             at = 4 * base + shim.shim_point_offset(i, n - 1 - base)
             assert at == 4 * min(base + i, n - 1), (n, base, i)
+
+
+@pytest.mark.parametrize("threads", [64, 128, 256, 512, 1024])
+def test_a_launch_holds_fewer_than_2_32_threads(shim, threads):
+    groups = shim.shim_max_groups(threads)
+    assert groups * threads < 1 << 32 <= (groups + 1) * threads
