@@ -11,3 +11,14 @@ constexpr uint32_t gpr_point_offset(int i, int last) { return 4u * (uint32_t)(i 
 // Most workgroups of a launch of `threads` threads each.  A launch's size in threads has 32
 // bits: HIP starts what is left of a larger one modulo 2^32, and reports no error.
 constexpr int gpr_max_groups(int threads) { return (int)(0xffffffffu / (unsigned)threads); }
+
+// `groups` workgroups of `threads` in as many launches as that takes: launch(first, count),
+// which returns 0 or an error, starts `count` of them from `first` on.
+template <class F>
+inline int gpr_launches(int groups, int threads, F launch) {
+    for (int first = 0, count; first < groups; first += count) {
+        count = groups - first < gpr_max_groups(threads) ? groups - first : gpr_max_groups(threads);
+        if (const int e = launch(first, count)) return e;
+    }
+    return 0;
+}

@@ -1254,24 +1254,21 @@ __global__ void __launch_bounds__(GPR_WG) k_eval_split(GprEvalArgs a) {
     }
 }
 
-// Launches of one workgroup of `threads` per tape, as many as their size takes (8.4 million tapes
-// fill a launch of 512 threads each): launch(a, groups) starts `groups` of them on the first
-// tapes of a's arrays, a column per tape.
+// One workgroup of `threads` per tape, in as many launches as that takes (8.4 million tapes fill a
+// launch of 512 threads each): launch(a, groups) starts `groups` of them on the first tapes of
+// a's arrays, a column per tape.
 template <class F>
-static hipError_t launch_per_tape(GprEvalArgs a, int threads, F launch) {
-    for (int left = a.nchains; left > 0;) {
-        const int groups = std::min(left, gpr_max_groups(threads));
-        launch(a, groups);
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-        a.ops += groups;
-        a.cs += groups;
-        a.len += groups;
-        a.ll += groups;
-        if (a.grad) a.grad += groups;
-        left -= groups;
-    }
-    return hipSuccess;
+static hipError_t launch_per_tape(const GprEvalArgs &a, int threads, F launch) {
+    return (hipError_t)gpr_launches(a.nchains, threads, [&](int first, int count) {
+        GprEvalArgs b = a;
+        b.ops += first;
+        b.cs += first;
+        b.len += first;
+        b.ll += first;
+        if (b.grad) b.grad += first;
+        launch(b, count);
+        return (int)hipGetLastError();
+    });
 }
 
 template <int KC, bool RAW>
@@ -1665,9 +1662,9 @@ __global__ void __launch_bounds__(GPR_RS_WG) k_rs_map_scan(GprResampleArgs a) {
 // nothing writes it here; every wave reads its chains' posteriors before the barrier, and
 // the first one replaces them after it.
 #define GPR_GATHER_WAVES 8
-__global__ void __launch_bounds__(64 * GPR_GATHER_WAVES) k_rs_map_gather(GprResampleArgs a) {
+__global__ void __launch_bounds__(64 * GPR_GATHER_WAVES) k_rs_map_gather(GprResampleArgs a, int first) {
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int c = blockIdx.x * 64 + l, N = a.nchains;
+    const int c = (first + (int)blockIdx.x) * 64 + l, N = a.nchains;
     int j = -1;
     if (c < N) {
         const int di = chain_dataset(a.ds, a.ndatasets, c);
@@ -1713,8 +1710,10 @@ hipError_t gpr_launch_resample(const GprResampleArgs &a, hipStream_t s) {
     hipLaunchKernelGGL(k_rs_map_scan, dim3(a.ndatasets), dim3(GPR_RS_WG), 0, s, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_rs_map_gather, dim3((a.nchains + 63) / 64), dim3(64 * GPR_GATHER_WAVES), 0, s, a);
-    return hipGetLastError();
+    return (hipError_t)gpr_launches((a.nchains + 63) / 64, 64 * GPR_GATHER_WAVES, [&](int first, int count) {
+        hipLaunchKernelGGL(k_rs_map_gather, dim3(count), dim3(64 * GPR_GATHER_WAVES), 0, s, a, first);
+        return (int)hipGetLastError();
+    });
 }
 
 // ---------------------------------------------------------------- small utilities

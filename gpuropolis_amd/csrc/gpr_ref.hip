@@ -916,23 +916,28 @@ __device__ void r_draw_chains(uint64_t seed, int c0, uint32_t who, uint32_t step
 }
 
 template <int SET>
-__global__ void __launch_bounds__(R_DRAW_WG) k_init_ref(GprMHArgs a) {
-    const int c0 = blockIdx.x * R_DRAW_CHAINS, n = min(R_DRAW_CHAINS, a.nchains - c0);
+__global__ void __launch_bounds__(R_DRAW_WG) k_init_ref(GprMHArgs a, int first) {
+    const int c0 = (first + (int)blockIdx.x) * R_DRAW_CHAINS, n = min(R_DRAW_CHAINS, a.nchains - c0);
     r_draw_chains<SET>(a.seed, c0, n == 32 ? ~0u : (1u << n) - 1u, 0, GPR_P_INIT, a.ops, a.cs, a.nchains);
 }
 
-#define GPR_OPSET_LAUNCH(KERNEL, SET, GRID, BLOCK, S, ARGS)                                                        \
-    switch (SET) {                                                                                                \
-    case GPR_OPS_SIMPLIFIED: hipLaunchKernelGGL(KERNEL<GPR_OPS_SIMPLIFIED>, GRID, BLOCK, 0, S, ARGS); break;      \
-    case GPR_OPS_POLYNOMIAL: hipLaunchKernelGGL(KERNEL<GPR_OPS_POLYNOMIAL>, GRID, BLOCK, 0, S, ARGS); break;      \
-    case GPR_OPS_LINEAR: hipLaunchKernelGGL(KERNEL<GPR_OPS_LINEAR>, GRID, BLOCK, 0, S, ARGS); break;              \
-    case GPR_OPS_PHYSICAL: hipLaunchKernelGGL(KERNEL<GPR_OPS_PHYSICAL>, GRID, BLOCK, 0, S, ARGS); break;          \
-    default: hipLaunchKernelGGL(KERNEL<GPR_OPS_DEFAULT>, GRID, BLOCK, 0, S, ARGS); break;                         \
-    }
+// KERNEL over the chains, R_DRAW_CHAINS a workgroup (16 threads a chain: from 2^28 chains on
+// they pass the size of one launch)
+#define GPR_DRAW_LAUNCH(KERNEL, SET, S, ARGS)                                                                     \
+    return (hipError_t)gpr_launches((ARGS.nchains + R_DRAW_CHAINS - 1) / R_DRAW_CHAINS, R_DRAW_WG, [&](int first, int count) { \
+        const dim3 grid(count), wg(R_DRAW_WG);                                                                    \
+        switch (SET) {                                                                                            \
+        case GPR_OPS_SIMPLIFIED: hipLaunchKernelGGL(KERNEL<GPR_OPS_SIMPLIFIED>, grid, wg, 0, S, ARGS, first); break; \
+        case GPR_OPS_POLYNOMIAL: hipLaunchKernelGGL(KERNEL<GPR_OPS_POLYNOMIAL>, grid, wg, 0, S, ARGS, first); break; \
+        case GPR_OPS_LINEAR: hipLaunchKernelGGL(KERNEL<GPR_OPS_LINEAR>, grid, wg, 0, S, ARGS, first); break;        \
+        case GPR_OPS_PHYSICAL: hipLaunchKernelGGL(KERNEL<GPR_OPS_PHYSICAL>, grid, wg, 0, S, ARGS, first); break;    \
+        default: hipLaunchKernelGGL(KERNEL<GPR_OPS_DEFAULT>, grid, wg, 0, S, ARGS, first); break;                   \
+        }                                                                                                         \
+        return (int)hipGetLastError();                                                                            \
+    })
 
 hipError_t gpr_launch_init_ref(const GprMHArgs &a, hipStream_t s) {
-    GPR_OPSET_LAUNCH(k_init_ref, a.opset, dim3((a.nchains + R_DRAW_CHAINS - 1) / R_DRAW_CHAINS), dim3(R_DRAW_WG), s, a);
-    return hipGetLastError();
+    GPR_DRAW_LAUNCH(k_init_ref, a.opset, s, a);
 }
 
 // Order-preserving key of a double with NaN below everything (cmp, main.cu:987-995).
@@ -1026,8 +1031,8 @@ __global__ void __launch_bounds__(R_SEL_WG) k_rs_quantile_select(GprResampleArgs
 }
 
 template <int SET>
-__global__ void __launch_bounds__(R_DRAW_WG) k_rs_quantile_redraw(GprResampleArgs a) {
-    const int c0 = blockIdx.x * R_DRAW_CHAINS, c = c0 + (int)(threadIdx.x & 31);
+__global__ void __launch_bounds__(R_DRAW_WG) k_rs_quantile_redraw(GprResampleArgs a, int first) {
+    const int c0 = (first + (int)blockIdx.x) * R_DRAW_CHAINS, c = c0 + (int)(threadIdx.x & 31);
     bool low = false;      // NaN posteriors never resampled
     if (c < a.nchains) low = a.prior[c] + a.ll[c] < a.cutoff[chain_dataset(a.ds, a.ndatasets, c)];
     const uint32_t who = (uint32_t)ballot(low);       // each half of each wave: the same 32 chains
@@ -1040,8 +1045,7 @@ hipError_t gpr_launch_resample_quantile(const GprResampleArgs &a, hipStream_t s)
     hipLaunchKernelGGL(k_rs_quantile_select, dim3(a.ndatasets), dim3(R_SEL_WG), 0, s, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    GPR_OPSET_LAUNCH(k_rs_quantile_redraw, a.opset, dim3((a.nchains + R_DRAW_CHAINS - 1) / R_DRAW_CHAINS), dim3(R_DRAW_WG), s, a);
-    return hipGetLastError();
+    GPR_DRAW_LAUNCH(k_rs_quantile_redraw, a.opset, s, a);
 }
 
 // ---------------------------------------------------------------- test hooks

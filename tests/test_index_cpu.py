@@ -34,3 +34,19 @@ def test_a_chunk_loads_its_own_points(shim, n, kc):
 def test_a_launch_holds_fewer_than_2_32_threads(shim, threads):
     groups = shim.shim_max_groups(threads)
     assert groups * threads < 1 << 32 <= (groups + 1) * threads
+
+
+@pytest.mark.parametrize("groups,threads", [(1, 512), (8388607, 512), (8388608, 512), (1 << 25, 512), (1 << 24, 512),
+                                            ((1 << 31) - 1, 64), ((1 << 31) - 1, 512), (16777216, 256)])
+def test_launches_cover_every_workgroup_once(shim, groups, threads):
+    """The draws (16 threads a chain), MAP copies (8) and per-tape kernels past 2^32 threads."""
+    out = (C.c_int * 1024)()
+    n = shim.shim_launches(groups, threads, -1, out, 512)
+    assert n == -(-groups // (((1 << 32) - 1) // threads))
+    at = 0
+    for k in range(n):
+        assert out[2 * k] == at and out[2 * k + 1] >= 1 and out[2 * k + 1] * threads < 1 << 32
+        at += out[2 * k + 1]
+    assert at == groups
+    if n > 1:
+        assert shim.shim_launches(groups, threads, out[2], out, 512) == -5      # an error ends the walk
