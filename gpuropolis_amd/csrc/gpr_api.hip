@@ -85,7 +85,8 @@ struct gpr_ctx {
     bool any_metric = false;
     int *d_tile_counter = nullptr;  // one per bucket
     unsigned long long *d_counters = nullptr;
-    int32_t *d_faults = nullptr;       // gpr_grad_logpost_checked
+    int32_t *d_faults = nullptr;       // gpr_grad_logpost_checked, whose calls hold faults_mu until
+    std::mutex faults_mu;              // their clear, kernel and copy are on the stream, in that order
     int32_t *d_good = nullptr, *d_ngood = nullptr, *d_map_chain = nullptr, *d_nres = nullptr;
     float *d_gslab = nullptr;          // MALA token slabs of programs beyond the LDS rows
     size_t gslab_floats = 0;
@@ -1230,11 +1231,16 @@ static int grad_logpost(gpr_ctx *c, int dataset, const uint8_t *d_ops, const flo
     a.grad = d_grad;
     a.lnsym = log((double)c->cfg.nsym);
     if (faults) {
+        // threads that share the context share the word: one call's three operations on it follow
+        // each other on the stream
+        std::lock_guard<std::mutex> lk(c->faults_mu);
         a.faults = c->d_faults;
         HIP_TRY(gpr_launch_fill_i32(c->d_faults, 1, 0, c->stream));
+        HIP_TRY(gpr_launch_grad_wave(a, c->stream));
+        HIP_TRY(hipMemcpyAsync(faults, c->d_faults, sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
+    } else {
+        HIP_TRY(gpr_launch_grad_wave(a, c->stream));
     }
-    HIP_TRY(gpr_launch_grad_wave(a, c->stream));
-    if (faults) HIP_TRY(hipMemcpyAsync(faults, c->d_faults, sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     return GPR_OK;
 }
