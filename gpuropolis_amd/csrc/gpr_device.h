@@ -1268,13 +1268,12 @@ __device__ __forceinline__ float gather_f(float v0, float v1, int src, bool hi) 
 // soon as it is known.  A program needs fewer rows than it has tokens: operators and pending
 // left operands are at most len - 1.
 
-// Per-structure plan of the two sweeps.  Word t (lane t of w0, lane t-64 of w1): op code
-// (bits 0-4), row of the operator's value (5-12), and the left and right operand of a binary
-// token (13-20, 21-28; a unary token's operand in the right field): a row, or GPR_G_X, GPR_G_ONE
-// or GPR_G_C + token for a leaf.  rows: rows of the sweeps.
+// Per-structure plan of the two sweeps.  Word t (lane t of w0, lane t-64 of w1): a gpr_gtok, its
+// operands a row, or GPR_G_X, GPR_G_ONE or GPR_G_C + token for a leaf.  rows: rows of the sweeps.
 #define GPR_G_X 127
 #define GPR_G_C 128
 #define GPR_G_ONE 255
+static_assert(GPR_NUM_OPS <= 31, "gpr_gtok keeps 31 for an unknown op");
 struct GradPlan {
     int w0, w1;
     int nops, rows;
@@ -1304,11 +1303,11 @@ __device__ __forceinline__ GradPlan grad_plan(const WaveProg &p) {
         if (HI && D1 == k) lc1 = q1 ? 127 - __builtin_clzll(q1) : (d0 ? 63 - __builtin_clzll(d0) : 0);
     }
     const int left0 = gather_i(r0, r1, lc0, HI), right0 = gather_i(r0, r1, max(l - 1, 0), HI);
-    g.w0 = (p.o0 & 31) | (s0 << 5) | (left0 << 13) | (right0 << 21);
+    g.w0 = gpr_gtok(p.o0, s0, left0, right0);
     g.w1 = 0;
     if (HI) {
         const int left1 = gather_i(r0, r1, lc1, HI), right1 = gather_i(r0, r1, l + 63, HI);
-        g.w1 = (p.o1 & 31) | (s1 << 5) | (left1 << 13) | (right1 << 21);
+        g.w1 = gpr_gtok(p.o1, s1, left1, right1);
     }
     g.nops = __popcll(m0) + __popcll(m1);
     // pending left operands: at most one per level above the first
@@ -1344,7 +1343,7 @@ __device__ __forceinline__ void grad_forward(const WaveProg &p, const GradPlan &
         const int li = t & 63;
         const bool h = HI && t >= 64;
         const int w = h ? rl_i(g.w1, li) : rl_i(g.w0, li);
-        const int op = w & 31;
+        const int op = gpr_gtok_op(w);
         if (op <= GPR_OP_ONE) {
             float L[KC];
             if (op == GPR_OP_X) {
@@ -1358,9 +1357,9 @@ __device__ __forceinline__ void grad_forward(const WaveProg &p, const GradPlan &
             // with the +, - or * after it in one step, no copies of the stack's top: MALA with a
             // metric on a rational of 7 constants, n = 37, 2.95e8 -> 3.20e8 steps/s.  At several
             // points per lane the copies are a smaller share and the branches cost 1.5 %
-            const int w2 = HI && t >= 63 ? rl_i(g.w1, (t + 1) & 63) : rl_i(g.w0, (t + 1) & 63), op2 = w2 & 31;
+            const int w2 = HI && t >= 63 ? rl_i(g.w1, (t + 1) & 63) : rl_i(g.w0, (t + 1) & 63), op2 = gpr_gtok_op(w2);
             if (KC == 1 && t + 1 < p.len && (unsigned)(op2 - GPR_OP_ADD) < 3u) {
-                const int row = (w2 >> 5) & 255;
+                const int row = gpr_gtok_row(w2);
 #pragma unroll
                 for (int k = 0; k < KC; k++) {
                     if (op2 == GPR_OP_ADD) T[k] = T[k] + L[k];
@@ -1377,11 +1376,11 @@ __device__ __forceinline__ void grad_forward(const WaveProg &p, const GradPlan &
         }
         if (op <= GPR_OP_RPOW) {
             float A[KC];
-            if (((w >> 21) & 255) >= GPR_G_X) {
+            if (gpr_gtok_right(w) >= GPR_G_X) {
 #pragma unroll
                 for (int k = 0; k < KC; k++) A[k] = P[k];
             } else {
-                grad_val<KC, HI>(p, (w >> 13) & 255, x, lvl, A);
+                grad_val<KC, HI>(p, gpr_gtok_left(w), x, lvl, A);
             }
             if (op == GPR_OP_ADD) GPR_KLOOP(A[k] + T[k]);
             else if (op == GPR_OP_SUB) GPR_KLOOP(A[k] - T[k]);
@@ -1391,7 +1390,7 @@ __device__ __forceinline__ void grad_forward(const WaveProg &p, const GradPlan &
             const float c = op >= GPR_OP_CADD ? (h ? rl_f(p.c1, li) : rl_f(p.c0, li)) : 0.0f;
             GPR_KLOOP(op_un(op, T[k], c));
         }
-        const int row = (w >> 5) & 255;
+        const int row = gpr_gtok_row(w);
 #pragma unroll
         for (int k = 0; k < KC; k++) lvl[(row * KC + k) * 64] = T[k];
     }
@@ -1416,7 +1415,7 @@ __device__ __forceinline__ void grad_reverse(const WaveProg &p, const GradPlan &
         const int li = t & 63;
         const bool h = HI && t >= 64;
         const int w = h ? rl_i(g.w1, li) : rl_i(g.w0, li);
-        const int op = w & 31;
+        const int op = gpr_gtok_op(w);
         if (op <= GPR_OP_ONE) {
             if (op == GPR_OP_CONST) constant(t, G);
             // the next token roots a left operand: its adjoint waits on the stack
@@ -1427,7 +1426,7 @@ __device__ __forceinline__ void grad_reverse(const WaveProg &p, const GradPlan &
             }
             continue;
         }
-        const int lr = (w >> 13) & 255, rr = (w >> 21) & 255;
+        const int lr = gpr_gtok_left(w), rr = gpr_gtok_right(w);
         if (op <= GPR_OP_RPOW) {
             float ga[KC], gb[KC];
             if (op <= GPR_OP_SUB) {
@@ -1438,7 +1437,7 @@ __device__ __forceinline__ void grad_reverse(const WaveProg &p, const GradPlan &
                 float A[KC], B[KC];
                 grad_val<KC, HI>(p, lr, x, lvl, A);
                 grad_val<KC, HI>(p, rr, x, lvl, B);
-                const int row = (w >> 5) & 255;
+                const int row = gpr_gtok_row(w);
 #pragma unroll
                 for (int k = 0; k < KC; k++) {
                     const float a = A[k], b = B[k], q = G[k];
@@ -1482,7 +1481,7 @@ __device__ __forceinline__ void grad_reverse(const WaveProg &p, const GradPlan &
             const float c = op >= GPR_OP_CADD ? (h ? rl_f(p.c1, li) : rl_f(p.c0, li)) : 0.0f;
             float A[KC], gc[KC];
             grad_val<KC, HI>(p, rr, x, lvl, A);
-            const int row = (w >> 5) & 255;
+            const int row = gpr_gtok_row(w);
 #pragma unroll
             for (int k = 0; k < KC; k++) {
                 const float a = A[k], v = lvl[(row * KC + k) * 64], q = G[k];

@@ -22,3 +22,14 @@ inline int gpr_launches(int groups, int threads, F launch) {
     }
     return 0;
 }
+
+// A token of the adjoint's plan: op code (5 bits; every code past the table's is 31, an unknown op
+// as they are, since its low bits alone may be another's), row of its value, and its left
+// and right operands (a unary token's operand on the right), eight bits each.
+constexpr int gpr_gtok(int op, int row, int left, int right) {
+    return (op < 31 ? op : 31) | (row & 255) << 5 | (left & 255) << 13 | (right & 255) << 21;
+}
+constexpr int gpr_gtok_op(int w) { return w & 31; }
+constexpr int gpr_gtok_row(int w) { return (w >> 5) & 255; }
+constexpr int gpr_gtok_left(int w) { return (w >> 13) & 255; }
+constexpr int gpr_gtok_right(int w) { return (w >> 21) & 255; }

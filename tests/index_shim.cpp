@@ -15,3 +15,10 @@ extern "C" int shim_launches(int groups, int threads, int fail, int *out, int ro
     });
     return e ? -e : n;
 }
+extern "C" void shim_gtok(int op, int row, int left, int right, int *out) {
+    const int w = gpr_gtok(op, row, left, right);
+    out[0] = gpr_gtok_op(w);
+    out[1] = gpr_gtok_row(w);
+    out[2] = gpr_gtok_left(w);
+    out[3] = gpr_gtok_right(w);
+}

@@ -47,3 +47,39 @@ def test_faults_of_calls_side_by_side(gpr):
     for k in range(4):
         want = gpr.TAPE_POSTFIX if k % 2 else 0
         assert got[k] == [want] * rounds, (k, sum(f != want for f in got[k]))
+
+
+@pytest.mark.parametrize("cap,n", [(64, 70), (128, 600)])
+def test_op_codes_that_are_no_ops(gpr, cap, n):
+    """The unchecked gradient of a tape with an unknown op code, anywhere in the byte's range: the
+    value is no number, so the posterior is -inf, and the tapes beside it keep their results."""
+    import torch
+    codes = [len(gpr.OPS), 31] + [32 + k for k in range(32)] + [64, 96, 128, 200, 255]
+    x, c, add = (gpr.OP[k] for k in ("X", "CONST", "ADD"))
+    N = 5 * len(codes)
+    ops, cs, ln = sound_tapes(gpr, cap, N)
+    clean = ops.copy()
+    where = []
+    for k, op in enumerate(codes):
+        for at, tape in ((5 * k + 1, [x, op]), (5 * k + 2, [c, x, op, add]), (5 * k + 3, [c] + [op] * (cap - 1))):
+            ops[:, at] = 0
+            ops[:len(tape), at] = tape
+            ln[at] = len(tape)
+            where.append(at)
+    with gpr.Context(cap=cap) as ctx:
+        ctx.set_data([dataset(n, True)], [1])
+        dcs = dev(cs)
+        say(f"unknown op codes, cap {cap}, n {n}")
+
+        def call(o, length):
+            grad = torch.empty((cap, N), dtype=torch.float32, device="cuda")
+            lp = torch.empty(N, dtype=torch.float64, device="cuda")
+            do, dl = dev(o), dev(length)
+            ctx.grad_logpost_dev(0, do.data_ptr(), dcs.data_ptr(), dl.data_ptr(), N, cap, grad.data_ptr(), lp.data_ptr())
+            return grad.cpu().numpy(), lp.cpu().numpy()
+
+        want_g, want = call(clean, np.full(N, 5, dtype=np.int32))
+        got_g, got = call(ops, ln)
+    assert np.all(got[where] == -np.inf)
+    rest = np.setdiff1d(np.arange(N), where)
+    assert np.array_equal(got[rest], want[rest]) and np.array_equal(got_g[:, rest], want_g[:, rest])

@@ -50,3 +50,13 @@ def test_launches_cover_every_workgroup_once(shim, groups, threads):
     assert at == groups
     if n > 1:
         assert shim.shim_launches(groups, threads, out[2], out, 512) == -5      # an error ends the walk
+
+
+def test_adjoint_tokens_keep_their_fields(shim):
+    """Any byte as op code (what is past the table's 27 stays an unknown one: 35 is no ADD), rows
+    to 126, leaf operands to 255."""
+    out = (C.c_int * 4)()
+    for op in range(256):
+        for row, left, right in ((0, 0, 0), (126, 255, 255), (op // 3, 255 - op, op), (127, 128, 254)):
+            shim.shim_gtok(op, row, left, right, out)
+            assert list(out) == [min(op, 31), row, left, right] and (out[0] == op or op >= 27)
