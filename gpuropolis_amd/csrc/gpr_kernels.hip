@@ -1065,14 +1065,22 @@ __device__ __forceinline__ WaveProg eval_load(const GprEvalArgs &a, int chain) {
     p.c1 = (HI && l + 64 < p.len) ? a.cs[(size_t)(l + 64) * N + chain] : 0.0f;
     return p;
 }
-// The tape's stack depth, or 0 when it pops an empty stack or passes GPR_MAX_DEPTH (it
-// would leave the wave's rows); an empty tape has depth 1.
+// Values on the stack after the last of len tokens, from wave_depths (0 for an empty tape).
 template <bool HI>
+__device__ __forceinline__ int values_left(int len, int D0, int D1) {
+    return HI && len > 64 ? rl_i(D1, (len - 1) & 63) : rl_i(D0, (len - 1) & 63);
+}
+// The tape's stack depth, or 0 when it pops an empty stack or passes GPR_MAX_DEPTH (it
+// would leave the wave's rows); an empty tape has depth 1.  The interpreter's rows hold a tape
+// that leaves several values too (its value is the last); the adjoint's do not: its reverse
+// sweep would pop an operand's adjoint for each of them that nothing has pushed (ADJOINT).
+template <bool HI, bool ADJOINT = false>
 __device__ __forceinline__ int eval_depth(const WaveProg &p) {
     const int l = lane_id();
     int D0, D1, dm;
     wave_depths<HI>(p, D0, D1, dm);
     if (dm > GPR_MAX_DEPTH || ballot((l < p.len && D0 < 1) || (HI && l + 64 < p.len && D1 < 1))) return 0;
+    if (ADJOINT && values_left<HI>(p.len, D0, D1) > 1) return 0;
     return max(dm, 1);
 }
 
@@ -1353,8 +1361,7 @@ __device__ __forceinline__ int tape_faults(const GprEvalArgs &a, int chain, cons
     if (f) return f;
     int D0, D1, dm;
     wave_depths<HI>(p, D0, D1, dm);
-    const int end = HI && len > 64 ? rl_i(D1, (len - 1) & 63) : rl_i(D0, (len - 1) & 63);
-    if (end != 1 || ballot((l < len && D0 < 1) || (HI && l + 64 < len && D1 < 1))) return GPR_TAPE_POSTFIX;
+    if (values_left<HI>(len, D0, D1) != 1 || ballot((l < len && D0 < 1) || (HI && l + 64 < len && D1 < 1))) return GPR_TAPE_POSTFIX;
     return dm > GPR_MAX_DEPTH ? GPR_TAPE_DEPTH : 0;
 }
 
@@ -1415,7 +1422,7 @@ __global__ void __launch_bounds__(512) k_grad_wave(GprEvalArgs a) {
             return;
         }
     }
-    if (eval_depth<HI>(p)) {                 // the same in every wave
+    if (eval_depth<HI, true>(p)) {           // the same in every wave
         GradPlan g = grad_plan<HI>(p);
         g.rows = max(uni(g.rows), 1);
         if (a.d.n > 64 && 2 * g.rows * waves <= a.rows)

@@ -83,3 +83,42 @@ def test_op_codes_that_are_no_ops(gpr, cap, n):
     assert np.all(got[where] == -np.inf)
     rest = np.setdiff1d(np.arange(N), where)
     assert np.array_equal(got[rest], want[rest]) and np.array_equal(got_g[:, rest], want_g[:, rest])
+
+
+@pytest.mark.parametrize("cap,n", [(16, 1), (64, 70), (128, 600), (128, 1025)])
+def test_tapes_that_leave_several_values(gpr, cap, n):
+    """The unchecked gradient of tapes that end with 2 to 16 values: no program, so the posterior
+    is -inf and the gradient the prior's, and the tapes beside them keep their results."""
+    import torch
+    x, c, add, neg = (gpr.OP[k] for k in ("X", "CONST", "ADD", "NEG"))
+    wrong = [[c] * k for k in range(2, 17)] + [[x, x, x, neg, add] + [c] * 6, [c, x, add, c], [c] * 8 + [add] * 6]
+    wrong += [[c] * 16 + [neg] * (cap - 16)] if cap > 16 else []
+    N = 3 * len(wrong)
+    ops, cs, ln = sound_tapes(gpr, cap, N)
+    clean = ops.copy()
+    where = np.arange(len(wrong)) * 3 + 1
+    for at, tape in zip(where, wrong):
+        ops[:, at] = 0
+        ops[:len(tape), at] = tape
+        ln[at] = len(tape)
+    with gpr.Context(cap=cap) as ctx:
+        ctx.set_data([dataset(n, True)], [1])
+        dcs = dev(cs)
+        say(f"several values left, cap {cap}, n {n}")
+
+        def call(o, length):
+            grad = torch.empty((cap, N), dtype=torch.float32, device="cuda")
+            lp = torch.empty(N, dtype=torch.float64, device="cuda")
+            do, dl = dev(o), dev(length)
+            ctx.grad_logpost_dev(0, do.data_ptr(), dcs.data_ptr(), dl.data_ptr(), N, cap, grad.data_ptr(), lp.data_ptr())
+            return grad.cpu().numpy(), lp.cpu().numpy()
+
+        want_g, want = call(clean, np.full(N, 5, dtype=np.int32))
+        got_g, got = call(ops, ln)
+    assert np.all(got[where] == -np.inf)
+    for at, tape in zip(where, wrong):       # -2 c / (1 + c^2) at c = 0.5, on the constants only
+        want_col = np.zeros(cap, dtype=np.float32)
+        want_col[:len(tape)] = np.where(np.array(tape) == c, np.float32(-0.8), np.float32(0))
+        assert np.array_equal(got_g[:, at], want_col)
+    rest = np.setdiff1d(np.arange(N), where)
+    assert np.array_equal(got[rest], want[rest]) and np.array_equal(got_g[:, rest], want_g[:, rest])
