@@ -246,11 +246,16 @@ enum {
     GPR_U_SUB, GPR_U_MUL, GPR_U_NEG, GPR_U_XXADD, GPR_U_XCADD = GPR_U_XXADD + 3, GPR_U_CXADD = GPR_U_XCADD + 3,
     GPR_U_EXP = GPR_U_CXADD + 3
 };
-// (the last three handlers take two or three places of the table)
+// (the last three handlers take two or three places of the table; .org stops the assembler
+// at one that has outgrown its place)
 template <int KC>
 constexpr int GPR_U_DIV = GPR_U_EXP + (KC == 4 ? 3 : 2);
 template <int KC>
 constexpr int GPR_U_LOG = GPR_U_DIV<KC> + (KC == 4 ? 3 : 2);
+static_assert(GPR_U_X == 1 && GPR_U_XADD == 3 && GPR_U_CADD == 6 && GPR_U_ADD == 9 && GPR_U_NEG == 12 && GPR_U_XXADD == 13 &&
+                  GPR_U_CXADD == 19 && GPR_U_EXP == 22 && GPR_U_DIV<1> == 24 && GPR_U_LOG<1> == 26 && GPR_U_DIV<2> == 24 &&
+                  GPR_U_LOG<2> == 26 && GPR_U_DIV<4> == 25 && GPR_U_LOG<4> == 28,
+              "the places written in the tables");
 // Handler words of a half tape: lane l holds token l's.  Lanes past the program, and lane
 // 63 (whose successor the block could not read), hold the exit; so does every token
 // without a handler.  A handler advances by the one, two (a leaf and its operator) or three
@@ -360,34 +365,34 @@ __device__ __forceinline__ void tape_run(int word, float c, const float (&x)[1],
                                          int &t) {
     uint32_t blo, bhi, w, s;
     GT_TEMPS;
-#define GT_H(BODY) ".p2align 6\n\t" BODY
+#define GT_H(N, BODY) ".org .Lh%=+64*" #N "\n\t" BODY
     __asm__ volatile(
         GT_ENTRY
         ".p2align 6\n.Lh%=:\n\t" GT_EXIT
-        GT_H(GT_NEXT(1) GT1_PUSH "v_mov_b32 %[T0], %[x0]\n\t" GT_JUMP)
-        GT_H(GT_CONST GT_NEXT(1) GT1_PUSH "v_mov_b32 %[T0], %[s]\n\t" GT_JUMP)
-        GT_H(GT_NEXT(2) GT1("v_add_f32", "%[x0]", "%[T0]") GT_JUMP)
-        GT_H(GT_NEXT(2) GT1("v_sub_f32", "%[T0]", "%[x0]") GT_JUMP)
-        GT_H(GT_NEXT(2) GT1("v_mul_f32", "%[x0]", "%[T0]") GT_JUMP)
-        GT_H(GT_CONST GT_NEXT(2) GT1("v_add_f32", "%[s]", "%[T0]") GT_JUMP)
-        GT_H(GT_CONST GT_NEXT(2) GT1("v_subrev_f32", "%[s]", "%[T0]") GT_JUMP)
-        GT_H(GT_CONST GT_NEXT(2) GT1("v_mul_f32", "%[s]", "%[T0]") GT_JUMP)
-        GT_H(GT_NEXT(1) GT_WAIT GT1("v_add_f32", "%[U0]", "%[T0]") GT1_POP GT_JUMP)
-        GT_H(GT_NEXT(1) GT_WAIT GT1("v_sub_f32", "%[U0]", "%[T0]") GT1_POP GT_JUMP)
-        GT_H(GT_NEXT(1) GT_WAIT GT1("v_mul_f32", "%[U0]", "%[T0]") GT1_POP GT_JUMP)
-        GT_H(GT_NEXT(1) "v_xor_b32 %[T0], 0x80000000, %[T0]\n\t" GT_JUMP)
-        GT_H(GT_NEXT(3) GT1_PUSH GT1("v_add_f32", "%[x0]", "%[x0]") GT_JUMP)
-        GT_H(GT_NEXT(3) GT1_PUSH GT1("v_sub_f32", "%[x0]", "%[x0]") GT_JUMP)
-        GT_H(GT_NEXT(3) GT1_PUSH GT1("v_mul_f32", "%[x0]", "%[x0]") GT_JUMP)
-        GT_H(GT_CONST2 GT_NEXT(3) GT1_PUSH GT1("v_add_f32", "%[s]", "%[x0]") GT_JUMP)
-        GT_H(GT_CONST2 GT_NEXT(3) GT1_PUSH GT1("v_subrev_f32", "%[s]", "%[x0]") GT_JUMP)
-        GT_H(GT_CONST2 GT_NEXT(3) GT1_PUSH GT1("v_mul_f32", "%[s]", "%[x0]") GT_JUMP)
-        GT_H(GT_CONST GT_NEXT(3) GT1_PUSH GT1("v_add_f32", "%[s]", "%[x0]") GT_JUMP)
-        GT_H(GT_CONST GT_NEXT(3) GT1_PUSH GT1("v_sub_f32", "%[s]", "%[x0]") GT_JUMP)
-        GT_H(GT_CONST GT_NEXT(3) GT1_PUSH GT1("v_mul_f32", "%[s]", "%[x0]") GT_JUMP)
-        GT_H(GT_EXP_TEST("%[T0]") GT_NEXT(1) GT_LOG2E GT_EXP("%[T0]") GT_JUMP)
-        GT_H(GT_WAIT GT_NEXT(1) GT_DIV("%[U0]", "%[T0]") GT1_POP GT_JUMP)
-        GT_H(GT_WAIT GT_NEXT(1) GT_LOG("%[T0]") GT_JUMP)
+        GT_H(1, GT_NEXT(1) GT1_PUSH "v_mov_b32 %[T0], %[x0]\n\t" GT_JUMP)
+        GT_H(2, GT_CONST GT_NEXT(1) GT1_PUSH "v_mov_b32 %[T0], %[s]\n\t" GT_JUMP)
+        GT_H(3, GT_NEXT(2) GT1("v_add_f32", "%[x0]", "%[T0]") GT_JUMP)
+        GT_H(4, GT_NEXT(2) GT1("v_sub_f32", "%[T0]", "%[x0]") GT_JUMP)
+        GT_H(5, GT_NEXT(2) GT1("v_mul_f32", "%[x0]", "%[T0]") GT_JUMP)
+        GT_H(6, GT_CONST GT_NEXT(2) GT1("v_add_f32", "%[s]", "%[T0]") GT_JUMP)
+        GT_H(7, GT_CONST GT_NEXT(2) GT1("v_subrev_f32", "%[s]", "%[T0]") GT_JUMP)
+        GT_H(8, GT_CONST GT_NEXT(2) GT1("v_mul_f32", "%[s]", "%[T0]") GT_JUMP)
+        GT_H(9, GT_NEXT(1) GT_WAIT GT1("v_add_f32", "%[U0]", "%[T0]") GT1_POP GT_JUMP)
+        GT_H(10, GT_NEXT(1) GT_WAIT GT1("v_sub_f32", "%[U0]", "%[T0]") GT1_POP GT_JUMP)
+        GT_H(11, GT_NEXT(1) GT_WAIT GT1("v_mul_f32", "%[U0]", "%[T0]") GT1_POP GT_JUMP)
+        GT_H(12, GT_NEXT(1) "v_xor_b32 %[T0], 0x80000000, %[T0]\n\t" GT_JUMP)
+        GT_H(13, GT_NEXT(3) GT1_PUSH GT1("v_add_f32", "%[x0]", "%[x0]") GT_JUMP)
+        GT_H(14, GT_NEXT(3) GT1_PUSH GT1("v_sub_f32", "%[x0]", "%[x0]") GT_JUMP)
+        GT_H(15, GT_NEXT(3) GT1_PUSH GT1("v_mul_f32", "%[x0]", "%[x0]") GT_JUMP)
+        GT_H(16, GT_CONST2 GT_NEXT(3) GT1_PUSH GT1("v_add_f32", "%[s]", "%[x0]") GT_JUMP)
+        GT_H(17, GT_CONST2 GT_NEXT(3) GT1_PUSH GT1("v_subrev_f32", "%[s]", "%[x0]") GT_JUMP)
+        GT_H(18, GT_CONST2 GT_NEXT(3) GT1_PUSH GT1("v_mul_f32", "%[s]", "%[x0]") GT_JUMP)
+        GT_H(19, GT_CONST GT_NEXT(3) GT1_PUSH GT1("v_add_f32", "%[s]", "%[x0]") GT_JUMP)
+        GT_H(20, GT_CONST GT_NEXT(3) GT1_PUSH GT1("v_sub_f32", "%[s]", "%[x0]") GT_JUMP)
+        GT_H(21, GT_CONST GT_NEXT(3) GT1_PUSH GT1("v_mul_f32", "%[s]", "%[x0]") GT_JUMP)
+        GT_H(22, GT_EXP_TEST("%[T0]") GT_NEXT(1) GT_LOG2E GT_EXP("%[T0]") GT_JUMP)
+        GT_H(24, GT_WAIT GT_NEXT(1) GT_DIV("%[U0]", "%[T0]") GT1_POP GT_JUMP)
+        GT_H(26, GT_WAIT GT_NEXT(1) GT_LOG("%[T0]") GT_JUMP)
         ".Lx%=:"
         : [T0] "+&v"(T[0]), [U0] "+&v"(U[0]), [p] "+&v"(p), [t] "+&s"(t), [blo] "=&s"(blo), [bhi] "=&s"(bhi), [w] "=&s"(w),
           [s] "=&s"(s), GT_TEMP_OUT
@@ -396,7 +401,8 @@ __device__ __forceinline__ void tape_run(int word, float c, const float (&x)[1],
 #undef GT_H
 }
 
-#define GT_H(BODY) ".p2align 7\n\t" BODY
+#define GT_H_(N, BODY) ".org .Lh%=+128*" #N "\n\t" BODY
+#define GT_H(N, BODY) GT_H_(N, BODY)
 #define GT2(OP, A, B) OP " %[T0], " A(0) ", " B(0) "\n\t" OP " %[T1], " A(1) ", " B(1) "\n\t"
 #define GT4(OP, A, B) GT2(OP, A, B) OP " %[T2], " A(2) ", " B(2) "\n\t" OP " %[T3], " A(3) ", " B(3) "\n\t"
 #define GT_T(k) "%[T" #k "]"
@@ -424,39 +430,39 @@ __device__ __forceinline__ void tape_run(int word, float c, const float (&x)[1],
 #define GT2_LOG GT_LOG("%[T0]") GT_LOG("%[T1]")
 #define GT4_LOG GT2_LOG GT_LOG("%[T2]") GT_LOG("%[T3]")
 // several points per lane, handlers of 128 bytes
-#define GT_TABLE(GT, MOV, PUSH, POP, EXP, DIV, LOG)                                             \
+#define GT_TABLE(GT, MOV, PUSH, POP, EXP, DIV, LOG, DIVP, LOGP)                                             \
     GT_ENTRY                                                                     \
     ".p2align 7\n.Lh%=:\n\t" GT_EXIT                                             \
-    GT_H(GT_NEXT(1) PUSH MOV(GT_T, GT_X) GT_JUMP)                                \
-    GT_H(GT_CONST GT_NEXT(1) PUSH MOV(GT_T, GT_S) GT_JUMP)                       \
-    GT_H(GT_NEXT(2) GT("v_add_f32", GT_X, GT_T) GT_JUMP)                         \
-    GT_H(GT_NEXT(2) GT("v_sub_f32", GT_T, GT_X) GT_JUMP)                         \
-    GT_H(GT_NEXT(2) GT("v_mul_f32", GT_X, GT_T) GT_JUMP)                         \
-    GT_H(GT_CONST GT_NEXT(2) GT("v_add_f32", GT_S, GT_T) GT_JUMP)                \
-    GT_H(GT_CONST GT_NEXT(2) GT("v_subrev_f32", GT_S, GT_T) GT_JUMP)             \
-    GT_H(GT_CONST GT_NEXT(2) GT("v_mul_f32", GT_S, GT_T) GT_JUMP)                \
-    GT_H(GT_NEXT(1) GT_WAIT GT("v_add_f32", GT_U, GT_T) POP GT_JUMP)             \
-    GT_H(GT_NEXT(1) GT_WAIT GT("v_sub_f32", GT_U, GT_T) POP GT_JUMP)             \
-    GT_H(GT_NEXT(1) GT_WAIT GT("v_mul_f32", GT_U, GT_T) POP GT_JUMP)             \
-    GT_H(GT_NEXT(1) GT("v_xor_b32", GT_NEGMASK, GT_T) GT_JUMP)                   \
-    GT_H(GT_NEXT(3) PUSH GT("v_add_f32", GT_X, GT_X) GT_JUMP)                    \
-    GT_H(GT_NEXT(3) PUSH GT("v_sub_f32", GT_X, GT_X) GT_JUMP)                    \
-    GT_H(GT_NEXT(3) PUSH GT("v_mul_f32", GT_X, GT_X) GT_JUMP)                    \
-    GT_H(GT_CONST2 GT_NEXT(3) PUSH GT("v_add_f32", GT_S, GT_X) GT_JUMP)          \
-    GT_H(GT_CONST2 GT_NEXT(3) PUSH GT("v_subrev_f32", GT_S, GT_X) GT_JUMP)       \
-    GT_H(GT_CONST2 GT_NEXT(3) PUSH GT("v_mul_f32", GT_S, GT_X) GT_JUMP)          \
-    GT_H(GT_CONST GT_NEXT(3) PUSH GT("v_add_f32", GT_S, GT_X) GT_JUMP)           \
-    GT_H(GT_CONST GT_NEXT(3) PUSH GT("v_sub_f32", GT_S, GT_X) GT_JUMP)           \
-    GT_H(GT_CONST GT_NEXT(3) PUSH GT("v_mul_f32", GT_S, GT_X) GT_JUMP)           \
-    GT_H(EXP GT_JUMP)                                                            \
-    GT_H(GT_WAIT GT_NEXT(1) DIV POP GT_JUMP)                                     \
-    GT_H(GT_NEXT(1) LOG GT_JUMP)                                                 \
+    GT_H(1, GT_NEXT(1) PUSH MOV(GT_T, GT_X) GT_JUMP)                                \
+    GT_H(2, GT_CONST GT_NEXT(1) PUSH MOV(GT_T, GT_S) GT_JUMP)                       \
+    GT_H(3, GT_NEXT(2) GT("v_add_f32", GT_X, GT_T) GT_JUMP)                         \
+    GT_H(4, GT_NEXT(2) GT("v_sub_f32", GT_T, GT_X) GT_JUMP)                         \
+    GT_H(5, GT_NEXT(2) GT("v_mul_f32", GT_X, GT_T) GT_JUMP)                         \
+    GT_H(6, GT_CONST GT_NEXT(2) GT("v_add_f32", GT_S, GT_T) GT_JUMP)                \
+    GT_H(7, GT_CONST GT_NEXT(2) GT("v_subrev_f32", GT_S, GT_T) GT_JUMP)             \
+    GT_H(8, GT_CONST GT_NEXT(2) GT("v_mul_f32", GT_S, GT_T) GT_JUMP)                \
+    GT_H(9, GT_NEXT(1) GT_WAIT GT("v_add_f32", GT_U, GT_T) POP GT_JUMP)             \
+    GT_H(10, GT_NEXT(1) GT_WAIT GT("v_sub_f32", GT_U, GT_T) POP GT_JUMP)             \
+    GT_H(11, GT_NEXT(1) GT_WAIT GT("v_mul_f32", GT_U, GT_T) POP GT_JUMP)             \
+    GT_H(12, GT_NEXT(1) GT("v_xor_b32", GT_NEGMASK, GT_T) GT_JUMP)                   \
+    GT_H(13, GT_NEXT(3) PUSH GT("v_add_f32", GT_X, GT_X) GT_JUMP)                    \
+    GT_H(14, GT_NEXT(3) PUSH GT("v_sub_f32", GT_X, GT_X) GT_JUMP)                    \
+    GT_H(15, GT_NEXT(3) PUSH GT("v_mul_f32", GT_X, GT_X) GT_JUMP)                    \
+    GT_H(16, GT_CONST2 GT_NEXT(3) PUSH GT("v_add_f32", GT_S, GT_X) GT_JUMP)          \
+    GT_H(17, GT_CONST2 GT_NEXT(3) PUSH GT("v_subrev_f32", GT_S, GT_X) GT_JUMP)       \
+    GT_H(18, GT_CONST2 GT_NEXT(3) PUSH GT("v_mul_f32", GT_S, GT_X) GT_JUMP)          \
+    GT_H(19, GT_CONST GT_NEXT(3) PUSH GT("v_add_f32", GT_S, GT_X) GT_JUMP)           \
+    GT_H(20, GT_CONST GT_NEXT(3) PUSH GT("v_sub_f32", GT_S, GT_X) GT_JUMP)           \
+    GT_H(21, GT_CONST GT_NEXT(3) PUSH GT("v_mul_f32", GT_S, GT_X) GT_JUMP)           \
+    GT_H(22, EXP GT_JUMP)                                                            \
+    GT_H(DIVP, GT_WAIT GT_NEXT(1) DIV POP GT_JUMP)                                     \
+    GT_H(LOGP, GT_NEXT(1) LOG GT_JUMP)                                                 \
     ".Lx%=:"
 __device__ __forceinline__ void tape_run(int word, float c, const float (&x)[2], float (&T)[2], float (&U)[2], uint32_t &p,
                                          int &t) {
     uint32_t blo, bhi, w, s;
     GT_TEMPS;
-    __asm__ volatile(GT_TABLE(GT2, GT2_MOV, GT2_PUSH, GT2_POP, GT2_EXP, GT2_DIV, GT2_LOG)
+    __asm__ volatile(GT_TABLE(GT2, GT2_MOV, GT2_PUSH, GT2_POP, GT2_EXP, GT2_DIV, GT2_LOG, 24, 26)
                      : [T0] "+&v"(T[0]), [T1] "+&v"(T[1]), [U0] "+&v"(U[0]), [U1] "+&v"(U[1]), [p] "+&v"(p), [t] "+&s"(t),
                        [blo] "=&s"(blo), [bhi] "=&s"(bhi), [w] "=&s"(w), [s] "=&s"(s), GT_TEMP_OUT
                      : [word] "v"(word), [c] "v"(c), [x0] "v"(x[0]), [x1] "v"(x[1])
@@ -466,7 +472,7 @@ __device__ __forceinline__ void tape_run(int word, float c, const float (&x)[4],
                                          int &t) {
     uint32_t blo, bhi, w, s;
     GT_TEMPS;
-    __asm__ volatile(GT_TABLE(GT4, GT4_MOV, GT4_PUSH, GT4_POP, GT4_EXP, GT4_DIV, GT4_LOG)
+    __asm__ volatile(GT_TABLE(GT4, GT4_MOV, GT4_PUSH, GT4_POP, GT4_EXP, GT4_DIV, GT4_LOG, 25, 28)
                      : [T0] "+&v"(T[0]), [T1] "+&v"(T[1]), [T2] "+&v"(T[2]), [T3] "+&v"(T[3]), [U0] "+&v"(U[0]),
                        [U1] "+&v"(U[1]), [U2] "+&v"(U[2]), [U3] "+&v"(U[3]), [p] "+&v"(p), [t] "+&s"(t), [blo] "=&s"(blo),
                        [bhi] "=&s"(bhi), [w] "=&s"(w), [s] "=&s"(s), GT_TEMP_OUT
@@ -1072,35 +1078,35 @@ __device__ __forceinline__ void tape_run_groups(int word, float cb, float x, flo
     uint32_t blo, bhi, w, s;
     float v;
     GT_TEMPS;
-#define GT_H(BODY) ".p2align 6\n\t" BODY
+#define GT_H(N, BODY) ".org .Lh%=+64*" #N "\n\t" BODY
 #define GG_TAKE(D) "ds_bpermute_b32 " D ", %[ca], %[cb]\n\tv_add_u32 %[ca], 4, %[ca]\n\t"
     __asm__ volatile(
         GT_ENTRY
         ".p2align 6\n.Lh%=:\n\t" GT_EXIT
-        GT_H(GT_NEXT(1) GT1_PUSH "v_mov_b32 %[T0], %[x]\n\t" GT_JUMP)
-        GT_H(GT_NEXT(1) GT1_PUSH GG_TAKE("%[T0]") GT_JUMP)
-        GT_H(GT_NEXT(2) GT_WAIT GT1("v_add_f32", "%[x]", "%[T0]") GT_JUMP)
-        GT_H(GT_NEXT(2) GT_WAIT GT1("v_sub_f32", "%[T0]", "%[x]") GT_JUMP)
-        GT_H(GT_NEXT(2) GT_WAIT GT1("v_mul_f32", "%[x]", "%[T0]") GT_JUMP)
-        GT_H(GT_NEXT(2) GG_TAKE("%[v]") GT_WAIT GT1("v_add_f32", "%[v]", "%[T0]") GT_JUMP)
-        GT_H(GT_NEXT(2) GG_TAKE("%[v]") GT_WAIT GT1("v_sub_f32", "%[T0]", "%[v]") GT_JUMP)
-        GT_H(GT_NEXT(2) GG_TAKE("%[v]") GT_WAIT GT1("v_mul_f32", "%[v]", "%[T0]") GT_JUMP)
-        GT_H(GT_NEXT(1) GT_WAIT GT1("v_add_f32", "%[U0]", "%[T0]") GT1_POP GT_JUMP)
-        GT_H(GT_NEXT(1) GT_WAIT GT1("v_sub_f32", "%[U0]", "%[T0]") GT1_POP GT_JUMP)
-        GT_H(GT_NEXT(1) GT_WAIT GT1("v_mul_f32", "%[U0]", "%[T0]") GT1_POP GT_JUMP)
-        GT_H(GT_NEXT(1) GT_WAIT "v_xor_b32 %[T0], 0x80000000, %[T0]\n\t" GT_JUMP)
-        GT_H(GT_NEXT(3) GT1_PUSH GT1("v_add_f32", "%[x]", "%[x]") GT_JUMP)
-        GT_H(GT_NEXT(3) GT1_PUSH GT1("v_sub_f32", "%[x]", "%[x]") GT_JUMP)
-        GT_H(GT_NEXT(3) GT1_PUSH GT1("v_mul_f32", "%[x]", "%[x]") GT_JUMP)
-        GT_H(GT_NEXT(3) GG_TAKE("%[v]") GT1_PUSH GT1("v_add_f32", "%[v]", "%[x]") GT_JUMP)
-        GT_H(GT_NEXT(3) GG_TAKE("%[v]") GT1_PUSH GT1("v_sub_f32", "%[x]", "%[v]") GT_JUMP)
-        GT_H(GT_NEXT(3) GG_TAKE("%[v]") GT1_PUSH GT1("v_mul_f32", "%[v]", "%[x]") GT_JUMP)
-        GT_H(GT_NEXT(3) GG_TAKE("%[v]") GT1_PUSH GT1("v_add_f32", "%[v]", "%[x]") GT_JUMP)
-        GT_H(GT_NEXT(3) GG_TAKE("%[v]") GT1_PUSH GT1("v_sub_f32", "%[v]", "%[x]") GT_JUMP)
-        GT_H(GT_NEXT(3) GG_TAKE("%[v]") GT1_PUSH GT1("v_mul_f32", "%[v]", "%[x]") GT_JUMP)
-        GT_H(GT_WAIT GT_EXP_TEST("%[T0]") GT_NEXT(1) GT_LOG2E GT_EXP("%[T0]") GT_JUMP)
-        GT_H(GT_WAIT GT_NEXT(1) GT_DIV("%[U0]", "%[T0]") GT1_POP GT_JUMP)
-        GT_H(GT_WAIT GT_NEXT(1) GT_LOG("%[T0]") GT_JUMP)
+        GT_H(1, GT_NEXT(1) GT1_PUSH "v_mov_b32 %[T0], %[x]\n\t" GT_JUMP)
+        GT_H(2, GT_NEXT(1) GT1_PUSH GG_TAKE("%[T0]") GT_JUMP)
+        GT_H(3, GT_NEXT(2) GT_WAIT GT1("v_add_f32", "%[x]", "%[T0]") GT_JUMP)
+        GT_H(4, GT_NEXT(2) GT_WAIT GT1("v_sub_f32", "%[T0]", "%[x]") GT_JUMP)
+        GT_H(5, GT_NEXT(2) GT_WAIT GT1("v_mul_f32", "%[x]", "%[T0]") GT_JUMP)
+        GT_H(6, GT_NEXT(2) GG_TAKE("%[v]") GT_WAIT GT1("v_add_f32", "%[v]", "%[T0]") GT_JUMP)
+        GT_H(7, GT_NEXT(2) GG_TAKE("%[v]") GT_WAIT GT1("v_sub_f32", "%[T0]", "%[v]") GT_JUMP)
+        GT_H(8, GT_NEXT(2) GG_TAKE("%[v]") GT_WAIT GT1("v_mul_f32", "%[v]", "%[T0]") GT_JUMP)
+        GT_H(9, GT_NEXT(1) GT_WAIT GT1("v_add_f32", "%[U0]", "%[T0]") GT1_POP GT_JUMP)
+        GT_H(10, GT_NEXT(1) GT_WAIT GT1("v_sub_f32", "%[U0]", "%[T0]") GT1_POP GT_JUMP)
+        GT_H(11, GT_NEXT(1) GT_WAIT GT1("v_mul_f32", "%[U0]", "%[T0]") GT1_POP GT_JUMP)
+        GT_H(12, GT_NEXT(1) GT_WAIT "v_xor_b32 %[T0], 0x80000000, %[T0]\n\t" GT_JUMP)
+        GT_H(13, GT_NEXT(3) GT1_PUSH GT1("v_add_f32", "%[x]", "%[x]") GT_JUMP)
+        GT_H(14, GT_NEXT(3) GT1_PUSH GT1("v_sub_f32", "%[x]", "%[x]") GT_JUMP)
+        GT_H(15, GT_NEXT(3) GT1_PUSH GT1("v_mul_f32", "%[x]", "%[x]") GT_JUMP)
+        GT_H(16, GT_NEXT(3) GG_TAKE("%[v]") GT1_PUSH GT1("v_add_f32", "%[v]", "%[x]") GT_JUMP)
+        GT_H(17, GT_NEXT(3) GG_TAKE("%[v]") GT1_PUSH GT1("v_sub_f32", "%[x]", "%[v]") GT_JUMP)
+        GT_H(18, GT_NEXT(3) GG_TAKE("%[v]") GT1_PUSH GT1("v_mul_f32", "%[v]", "%[x]") GT_JUMP)
+        GT_H(19, GT_NEXT(3) GG_TAKE("%[v]") GT1_PUSH GT1("v_add_f32", "%[v]", "%[x]") GT_JUMP)
+        GT_H(20, GT_NEXT(3) GG_TAKE("%[v]") GT1_PUSH GT1("v_sub_f32", "%[v]", "%[x]") GT_JUMP)
+        GT_H(21, GT_NEXT(3) GG_TAKE("%[v]") GT1_PUSH GT1("v_mul_f32", "%[v]", "%[x]") GT_JUMP)
+        GT_H(22, GT_WAIT GT_EXP_TEST("%[T0]") GT_NEXT(1) GT_LOG2E GT_EXP("%[T0]") GT_JUMP)
+        GT_H(24, GT_WAIT GT_NEXT(1) GT_DIV("%[U0]", "%[T0]") GT1_POP GT_JUMP)
+        GT_H(26, GT_WAIT GT_NEXT(1) GT_LOG("%[T0]") GT_JUMP)
         ".Lx%=:"
         : [T0] "+&v"(T), [U0] "+&v"(U), [p] "+&v"(p), [ca] "+&v"(ca), [t] "+&s"(t), [blo] "=&s"(blo), [bhi] "=&s"(bhi),
           [w] "=&s"(w), [s] "=&s"(s), [v] "=&v"(v), GT_TEMP_OUT
