@@ -1,7 +1,8 @@
 // Device building blocks shared by the config and reference kernels: wave-level
-// primitives (DPP reductions and scans, readlane/writelane), FP32 op semantics, the
-// wave-uniform tape interpreter with its VGPR value stack, the Gaussian
-// log-likelihood and description-length prior of a wave-resident program.
+// primitives (DPP reductions and scans, readlane), FP32 op semantics, the wave-uniform
+// tape interpreter (handlers in one asm block, value stack in LDS under two VGPR entries),
+// the Gaussian log-likelihood, its forward-mode and adjoint gradients, and the
+// description-length prior of a wave-resident program.
 #pragma once
 #include "gpr_index.h"
 #include "gpr_internal.h"
@@ -328,7 +329,10 @@ __device__ __forceinline__ void lds_st(uint32_t a, float v) { *(gpr_lds_f)(uintp
 
 // exp of T: 2^k e^r from the product with log2(e), its rounding error and the constant's
 // low part in one correction; for |T| < 88 neither end of the range needs a test, and every
-// such value gives the bits of expf (all 2^32 inputs compared).
+// such value gives the bits of expf (all 2^32 inputs compared).  The steps and constants of
+// exp, log and the division are those of the code that the AMD compiler emits for expf, logf
+// and a float division on this target: the other paths of a program's value (tape_slow, the
+// adjoint, the forward-mode pass, the lane schedule) call those, and the bits must not differ.
 #define GT_LOG2E "s_mov_b32 %[s], 0x3fb8aa3b\n\t"
 #define GT_EXP(T)                                                                                               \
     "v_mul_f32 %[q0], %[s], " T "\n\tv_rndne_f32 %[q1], %[q0]\n\tv_fma_f32 %[q2], " T ", %[s], -%[q0]\n\t"      \
@@ -586,15 +590,6 @@ struct Chunk {
     }
 };
 
-// Gaussian log-likelihood of the wave's program: lconst - sum_i (f_i - y_i)^2 w_i.
-// Per-lane Kahan sums, wave tree reduction; -inf if any term is not finite.
-// ls: this wave's value-stack slab, pc: the program's handler words for KC points per lane.
-// reject_below: the caller rejects the proposal whenever the LL lies below this value.
-// Every term of the sum is >= 0, so after each chunk but the last the sum so far bounds
-// the LL from above; when that bound (with a relative margin of 1e-4 on the partial sum,
-// far above its FP32 rounding) is below reject_below, or the partial sum is not finite,
-// the evaluation stops and returns -inf: the proposal is rejected either way.  *points
-// receives the number of data points evaluated.
 // Work-counter values of a program: operator tokens + 4 (the per-point FP32 ops of its
 // evaluation and Gaussian term) and its constant-carrying tokens.
 template <bool HI>
@@ -606,33 +601,6 @@ __device__ __forceinline__ void prog_counts(const WaveProg &p, int &opq, int &nc
          (HI ? __popcll(ballot(l + 64 < p.len && gpr_has_const(p.o1))) : 0);
     opq = p.len - nleaf + 4;
 }
-
-// The words of a Philox substream (chain, step, purpose, slot) as gpr_rstream yields
-// them, computed on the vector unit 64 at a time: lane k holds word 64 b + k (block
-// 16 b + k / 4, word k % 4) of the current batch b, and next() reads them in order with
-// v_readlane.  One vector Philox evaluation replaces up to 16 scalar ones, which takes
-// the structure move's draws off the scalar unit.
-struct WaveStream {
-    uint64_t seed;
-    uint32_t chain, step, c2;
-    uint32_t w;     // this lane's word of the current batch
-    int idx, base;  // next word within the batch, batch index
-    __device__ __forceinline__ void fill() {
-        const int k = lane_id();
-        const gpr_u4 b = gpr_philox(chain, step, c2, (uint32_t)(16 * base + (k >> 2)), (uint32_t)seed,
-                                    (uint32_t)(seed >> 32));
-        w = gpr_u4_word(b, k & 3);
-    }
-    __device__ __forceinline__ void init(uint64_t s, uint32_t ch, uint32_t st, uint32_t purpose, uint32_t slot) {
-        seed = s; chain = ch; step = st; c2 = (purpose << 24) | (slot & 0xffffffu);
-        idx = 0; base = 0;
-        fill();
-    }
-    __device__ __forceinline__ uint32_t next() {
-        if (idx == 64) { base++; idx = 0; fill(); }
-        return (uint32_t)rl_i((int)w, idx++);
-    }
-};
 
 // Constant tokens of a program.
 template <bool HI>
@@ -653,6 +621,15 @@ __device__ __forceinline__ bool batch_ok(const WaveProg &p, int mk) {
     return __popcll(m) <= 16 && ballot(l < p.len && gpr_has_const(p.o0)) == m;
 }
 
+// Gaussian log-likelihood of the wave's program: lconst - sum_i (f_i - y_i)^2 w_i.
+// Per-lane Kahan sums, wave tree reduction; -inf if any term is not finite.
+// ls: this wave's value-stack slab, pc: the program's handler words for KC points per lane.
+// reject_below: the caller rejects the proposal whenever the LL lies below this value.
+// Every term of the sum is >= 0, so after each chunk but the last the sum so far bounds
+// the LL from above; when that bound (with a relative margin of 1e-4 on the partial sum,
+// far above its FP32 rounding) is below reject_below, or the partial sum is not finite,
+// the evaluation stops and returns -inf: the proposal is rejected either way.  *points
+// receives the number of data points evaluated.
 template <int KC, bool HI>
 __device__ __forceinline__ double wave_loglik(const WaveProg &p, const GprDataset &d, const float *dx, const float *dy,
                               const float *dw, const Chunk<KC> &c0, int nchunks, float *ls, const ProgCode &pc,
@@ -1052,24 +1029,6 @@ __device__ __forceinline__ void dual_grad_lanes(const WaveProg &p, const uint64_
     ok = ballot((c0 && !__builtin_isfinite(g0)) || (c1 && !__builtin_isfinite(g1))) == 0;
 }
 
-// ---------------------------------------------------------------- speculative constant steps
-// Datasets of at most 32 points fill a fraction of a wave.  The random-walk kernel then
-// evaluates the proposals of G consecutive constant steps in one interpreter pass, one
-// per lane group (G = 4 groups of 16 lanes for n <= 16, 2 of 32 for n <= 32): lane l
-// takes point l mod (64 / G) of the proposal of step u0 + l / (64 / G).  All of them are
-// proposals from the same current state, which is the state each step sees as long as
-// the steps before it reject; the kernel uses them in step order and drops the rest
-// after an accept.  The dispatch of every token serves the G proposals.
-//
-// Proposal constants come from the draw batch: the constant of rank r of step u is lane
-// ks u + r of cb.  The value of each proposal is bit-identical to its own evaluation by
-// wave_loglik<1, false>: the same operations per point, a one-chunk Kahan sum (the term
-// itself), and a group sum whose FP64 additions are those of wave_sum_d over the lanes
-// it would occupy alone (rows of 16 lanes summed by the same DPP steps; a group of two
-// rows adds them as wave_sum_d adds rows 0 and 1, and adding the zero rows of a lone
-// evaluation changes nothing).  ls: the wave's value-stack region (KC = 1 layout).
-// out[g] receives the LL of group g's proposal, for g < gn (groups g >= gn repeat the
-// proposal of group gn - 1).
 // As tape_run for one point per lane, with a lane's constants taken from cb in token order:
 // ca is the byte index (ds_bpermute) of the lane holding the next one.  T may still be
 // loading when a handler ends, so every handler waits first.
@@ -1116,6 +1075,24 @@ __device__ __forceinline__ void tape_run_groups(int word, float cb, float x, flo
 #undef GT_H
 }
 
+// ---------------------------------------------------------------- speculative constant steps
+// Datasets of at most 32 points fill a fraction of a wave.  The random-walk kernel then
+// evaluates the proposals of G consecutive constant steps in one interpreter pass, one
+// per lane group (G = 4 groups of 16 lanes for n <= 16, 2 of 32 for n <= 32): lane l
+// takes point l mod (64 / G) of the proposal of step u0 + l / (64 / G).  All of them are
+// proposals from the same current state, which is the state each step sees as long as
+// the steps before it reject; the kernel uses them in step order and drops the rest
+// after an accept.  The dispatch of every token serves the G proposals.
+//
+// Proposal constants come from the draw batch: the constant of rank r of step u is lane
+// ks u + r of cb.  The value of each proposal is bit-identical to its own evaluation by
+// wave_loglik<1, false>: the same operations per point, a one-chunk Kahan sum (the term
+// itself), and a group sum whose FP64 additions are those of wave_sum_d over the lanes
+// it would occupy alone (rows of 16 lanes summed by the same DPP steps; a group of two
+// rows adds them as wave_sum_d adds rows 0 and 1, and adding the zero rows of a lone
+// evaluation changes nothing).  ls: the wave's value-stack region (KC = 1 layout).
+// out[g] receives the LL of group g's proposal, for g < gn (groups g >= gn repeat the
+// proposal of group gn - 1).
 __device__ __forceinline__ void wave_loglik_groups(const WaveProg &p, const GprDataset &d, const float *dx,
                                                    const float *dy, const float *dw, float *ls, const ProgCode &m,
                                                    float cb, int ks, int u0, int G, int gn, double (&out)[4]) {

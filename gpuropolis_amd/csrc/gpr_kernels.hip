@@ -7,10 +7,10 @@
 //
 // Two evaluator schedules:
 //   wave  one wavefront per chain.  The program is wave-uniform: lane t holds token
-//         t (and t+64) of the tape, the interpreter reads each op with v_readlane into
-//         a scalar register and branches on it without divergence, and the 64 lanes
-//         run over data points, KC points per lane per chunk, with a per-lane value
-//         stack in VGPRs indexed by the uniform stack pointer.  Per-point terms are
+//         t (and t+64) of the tape and the word of its handler, the interpreter jumps
+//         from handler to handler by one v_readlane and s_setpc a token, and the 64 lanes
+//         run over data points, KC points per lane per chunk, with the value stack's top
+//         two entries in VGPRs and the rest in the wave's LDS slab.  Per-point terms are
 //         Kahan-summed per lane and tree-reduced across the wave.
 //   lane  one lane per chain, as the reference.  Every lane interprets its own tape;
 //         the proposal tape and the value stack live in LDS ([slot][lane],
@@ -1313,8 +1313,10 @@ hipError_t gpr_launch_eval_wave(const GprEvalArgs &args, hipStream_t s) {
     a.eager = a.nchains <= 2048;
     // A workgroup per tape while all of them run at once, from three chunks on, and for
     // datasets of more than 512 points.  One wave per tape / one workgroup, whole calls in us:
-    // 300 tapes at n = 200 31 / 23, 500 at 500 41 / 24, 2000 at 100 24.0 / 25.3, 4096 at 256
-    // 17 / 20, 30000 at 300 136 / 191, 30000 at 1024 362 / 198.
+    // 300 tapes at n = 200 31 / 23, 500 at 500 41 / 24, 2000 at 100 24.0 / 25.3, 30000 at 300
+    // 136 / 191, 30000 at 1024 362 / 198.  Tapes of the sampler's ops, cap 64, 300 / 512 / 1024 / 1536 /
+    // 2048 of them: at n = 200 24 29 30 32 32 / 19 21 22 24 25, at 400 37 37 41 42 45 / 22 22 25 28
+    // 30; above 2048 it depends on the tapes (4096 at 200 47 / 28; of every op at 256 17 / 20).
     if ((n > 128 && a.nchains <= 2048) || n > 512) {
         const int kc = n <= 256 ? 1 : (n <= 512 ? 2 : 4);
         // rows for every depth at the full points per lane where that keeps the tapes resident
@@ -1333,20 +1335,6 @@ hipError_t gpr_launch_eval_wave(const GprEvalArgs &args, hipStream_t s) {
     return a.raw ? launch_eval_wave<4, true>(a, s) : launch_eval_wave<4, false>(a, s);
 }
 
-// Gradient of the log posterior of each tape: one workgroup per tape, whose waves (1 to 8,
-// by the dataset's size) share its chunks of points.  grad rows t < cap: d/dc_t, 0 where
-// token t has no constant or t >= len.  ll receives the log posterior.
-//
-// The sweeps are bound by scalar instructions and the latency of one token after another, so
-// they want waves, and LDS rows are what limits those (rows for every token of a 128-token
-// cap in every wave left one wave per SIMD).  The workgroup has a.rows rows of 64 floats, at
-// least what the longest program of the cap needs by itself.  A program runs two points per
-// lane, which halves the scalar work per point, when the rows hold that in every wave, else
-// one point per lane in as many waves as they allow.  The waves take their chunks in turn, a
-// round of at most 16 chunks at a time; the terms of the LL meet in LDS and are added in chunk
-// order (bit-identical to wave_loglik), the constants' FP64 sums wave by wave.  6007 tapes
-// (cap 128, every op) at n = 1021 took 2831 us with a wave per tape and a row per token, 772
-// with two points per lane wherever one wave holds them, and take 602.
 // What a tape breaks (GPR_TAPE_*): its length, an op code (anywhere in its cap rows), postfix
 // form, or the stack's bound, in the order a host check of all tapes would report them.
 template <bool HI>
@@ -1400,6 +1388,20 @@ __device__ __forceinline__ void grad_rounds(const GprEvalArgs &a, const WaveProg
     }
 }
 
+// Gradient of the log posterior of each tape: one workgroup per tape, whose waves (1 to 8,
+// by the dataset's size) share its chunks of points.  grad rows t < cap: d/dc_t, 0 where
+// token t has no constant or t >= len.  ll receives the log posterior.
+//
+// The sweeps are bound by scalar instructions and the latency of one token after another, so
+// they want waves, and LDS rows are what limits those (rows for every token of a 128-token
+// cap in every wave left one wave per SIMD).  The workgroup has a.rows rows of 64 floats, at
+// least what the longest program of the cap needs by itself.  A program runs two points per
+// lane, which halves the scalar work per point, when the rows hold that in every wave, else
+// one point per lane in as many waves as they allow.  The waves take their chunks in turn, a
+// round of at most 16 chunks at a time; the terms of the LL meet in LDS and are added in chunk
+// order (bit-identical to wave_loglik), the constants' FP64 sums wave by wave.  6007 tapes
+// (cap 128, every op) at n = 1021 took 2831 us with a wave per tape and a row per token, 772
+// with two points per lane wherever one wave holds them, and take 602.
 // LDS floats: the rows, then one term per point of a round (the waves' gradients meet in the
 // rows afterwards: 128 doubles a wave)
 template <bool HI>
@@ -1457,7 +1459,9 @@ hipError_t gpr_launch_grad_wave(const GprEvalArgs &args, hipStream_t s) {
     // waves: one per two chunks of 64 points.  Eight share their rows at 16 each, which a
     // cap over 64 outgrows (6007 tapes of cap 128 at n = 1021: 602 us by four, 694 by eight; 30000
     // of cap 64 at 1024: 915 and 870), unless so few tapes are asked for that their latency counts
-    // (one tape of cap 64 at n = 1000: 56 and 36).
+    // (one tape of cap 64 at n = 1000: 56 and 36).  Tapes of the sampler's ops at n = 1021, four /
+    // eight: cap 64, 64 256 1023 2048 6007 of them 101 245 346 361 452 / 59 103 167 189 301; cap 128
+    // 46 137 190 207 312 / 40 138 193 218 356.
     const bool eight = a.d.n > 512 && (a.cap <= 64 || a.nchains < 1024);
     const int waves = a.d.n <= 128 ? 1 : (a.d.n <= 256 ? 2 : (eight ? 8 : 4));
     // a program needs at most cap - 1 rows; 16 rows a wave hold the common ones at two points
