@@ -1320,7 +1320,7 @@ hipError_t gpr_launch_eval_wave(const GprEvalArgs &args, hipStream_t s) {
     if ((n > 128 && a.nchains <= 2048) || n > 512) {
         const int kc = n <= 256 ? 1 : (n <= 512 ? 2 : 4);
         // rows for every depth at the full points per lane where that keeps the tapes resident
-        a.rows = kc == 1 || a.nchains * kc <= 2048 ? (GPR_MAX_DEPTH + 2) * kc : GPR_EVAL_ROWS(4);
+        a.rows = kc == 1 || a.nchains <= 2048 / kc ? (GPR_MAX_DEPTH + 2) * kc : GPR_EVAL_ROWS(4);
         if (kc == 1) return a.raw ? launch_eval_split<1, true>(a, s) : launch_eval_split<1, false>(a, s);
         return kc == 2 ? launch_eval_split<2, false>(a, s) : launch_eval_split<4, false>(a, s);
     }
@@ -1329,7 +1329,7 @@ hipError_t gpr_launch_eval_wave(const GprEvalArgs &args, hipStream_t s) {
     a.per_wave = std::max(1, std::min(4, a.nchains / 20480));
     const int kc = a.d.kc;
     // 300 tapes at n = 200: 36 us with the rows of many tapes, 22 with all; 30000 at 300: 122 and 217
-    a.rows = a.nchains * kc <= 8192 ? (GPR_MAX_DEPTH + 2) * kc : GPR_EVAL_ROWS(kc);
+    a.rows = a.nchains <= 8192 / kc ? (GPR_MAX_DEPTH + 2) * kc : GPR_EVAL_ROWS(kc);
     if (kc == 1) return a.raw ? launch_eval_wave<1, true>(a, s) : launch_eval_wave<1, false>(a, s);
     if (kc == 2) return a.raw ? launch_eval_wave<2, true>(a, s) : launch_eval_wave<2, false>(a, s);
     return a.raw ? launch_eval_wave<4, true>(a, s) : launch_eval_wave<4, false>(a, s);
