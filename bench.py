@@ -47,18 +47,18 @@ HBM_PEAK = 8.0e12
 # were measured on.  For the batched workload a "launch" is one block's six concurrent
 # size-class launches.
 MEASURED_TRAFFIC = {
-    ("full", 1048576, 1000, 0): 1_344_635_552,
-    ("large", 131072, 1000, 0): 137_598_080,
-    ("batched", 262144, 1000, 0): 15_994_380_864,
+    ("full", 1048576, 1000, 0): 1_336_024_928,
+    ("large", 131072, 1000, 0): 136_888_960,
+    ("batched", 262144, 1000, 0): 12_557_262_016,
 }
 # VALU and SALU instructions per chain-step of the same launches (rocprofv3 --pmc
 # SQ_INSTS_VALU, SQ_INSTS_SALU over chains x steps).  With the live launch time they give
 # the share of issue slots each unit is busy: one wave64 instruction per SIMD every 4
 # cycles, 1024 SIMDs at 2.4 GHz.
 MEASURED_ISSUE = {
-    ("full", 1048576, 1000, 0): (1054.96, 694.64),
-    ("large", 131072, 1000, 0): (247.40, 179.35),
-    ("batched", 262144, 1000, 0): (289.40, 199.07),
+    ("full", 1048576, 1000, 0): (1050.34, 709.20),
+    ("large", 131072, 1000, 0): (243.87, 180.30),
+    ("batched", 262144, 1000, 0): (287.16, 200.98),
 }
 
 METRIC = "MH steps/sec + node×datapoint evals/sec (% VALU peak); ESS/sec MALA vs RW"

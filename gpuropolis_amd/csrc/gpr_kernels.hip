@@ -44,7 +44,7 @@ __global__ void k_fill_logint() {
 // The plain one-point-per-lane kernel is latency bound: six waves per SIMD (80 VGPRs) run
 // it faster than the four that fit unspilled, although the compiler then spills per-tile
 // values to scratch at every tile start and reloads some of them in the step loop.
-// (The two-register speculative build also stores some in the loop, 15 GB a block of the
+// (The two-register speculative build also stores some in the loop, 13 GB a block of the
 // batched workload, without cost: five waves store 38 MB there and run 48 datasets of 6 to
 // 250 points 0.5 to 3 % slower.)
 // The MALA kernel: unconstrained it takes about 160 VGPRs (three waves per SIMD), 15 %
