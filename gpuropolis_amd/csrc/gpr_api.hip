@@ -498,7 +498,11 @@ static bool stage_get(gpr_ctx *c, size_t bytes) {
     const size_t want = ring ? GPR_STAGE_PIECE * GPR_STAGE_SLOTS : (bytes + 0xffff) & ~(size_t)0xffff;
     if (ring)
         for (hipEvent_t &e : c->stage_ev)
-            if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return false;
+            if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+                (void)hipGetLastError();    // (the next launch would report it as its own)
+                e = nullptr;
+                return false;
+            }
     if (c->stage_bytes >= want) return true;
     if (c->stage) (void)hipHostFree(c->stage);
     c->stage = nullptr;
