@@ -4,6 +4,7 @@ import ctypes as C
 import os
 import re
 import subprocess
+import threading
 
 import numpy as np
 import pytest
@@ -64,3 +65,25 @@ def test_state_copies_without_the_pinned_buffer(host, chains, fails):
         assert np.array_equal(got[0], ops) and np.array_equal(got[1], cs) and np.array_equal(got[2], ln)
         again = ctx.read_state()                  # with what failed before
         assert np.array_equal(again[1], cs) and np.array_equal(again[2], ln)
+
+
+def test_checked_gradients_side_by_side(host):
+    """Each call gets the faults of its own tapes, where threads share a context for all that (the
+    fault word is the context's)."""
+    G, L = host
+    got = {}
+    one = np.zeros(8, dtype=np.float64)
+    p = one.ctypes.data
+    with G.Context(cap=1) as ctx:
+        ctx.set_data([(np.ones(1, np.float32),) * 3], [1])
+
+        def calls(want):
+            length = np.full(1, want, dtype=np.int32)
+            got[want] = [ctx.grad_logpost_checked_dev(0, p, p, length.ctypes.data, 1, 1, p, p) for _ in range(50)]
+
+        threads = [threading.Thread(target=calls, args=(w,)) for w in (0, G.TAPE_OP, G.TAPE_POSTFIX)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    assert all(set(v) == {want} for want, v in got.items()) and len(got) == 3
